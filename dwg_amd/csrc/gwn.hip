@@ -169,16 +169,15 @@ __global__ void pack_sources_kernel(const float* __restrict__ pts, const float* 
 constexpr int kDirectThreads = 256;
 constexpr int kDirectTile = 64;
 
-template <bool SCREENED, bool KAHAN, bool NEAR64 = false>
-__global__ __launch_bounds__(kDirectThreads) void gwn_direct_kernel(
-    const float4* __restrict__ sa, const float4* __restrict__ sb, int64_t n, const float* __restrict__ q,
-    int64_t nq, float sigma, float* __restrict__ out) {
-    const int64_t i = int64_t(blockIdx.x) * kDirectThreads + threadIdx.x;
-    const bool valid = i < nq;
-    const float qx = valid ? q[3 * i] : 0.f, qy = valid ? q[3 * i + 1] : 0.f, qz = valid ? q[3 * i + 2] : 0.f;
+// the sources [j0, j1) summed at q: the FP32 sum is sum − comp, and near the
+// FP64 sum of the terms inside the screening radius (DWG_NEAR_FP64)
+template <bool SCREENED, bool KAHAN, bool NEAR64>
+__device__ __forceinline__ void direct_value(const float4* __restrict__ sa, const float4* __restrict__ sb, int64_t j0,
+                                             int64_t j1, float qx, float qy, float qz, float sigma, float& sum,
+                                             float& comp, double& near) {
     const float sl2e = sigma * kLog2e;
-    float sum = 0.f, comp = 0.f;
-    double near = 0.0;  // DWG_NEAR_FP64: the terms inside the screening radius, in FP64
+    sum = comp = 0.f;
+    near = 0.0;
     auto term = [&](const float4 a, const float4 b) {
         if constexpr (NEAR64) {
             const float dx = a.x - qx, dy = a.y - qy, dz = a.z - qz;
@@ -190,16 +189,64 @@ __global__ __launch_bounds__(kDirectThreads) void gwn_direct_kernel(
         }
         return gwn_term<SCREENED>(qx, qy, qz, a, b, sigma, sl2e);
     };
-    int64_t j0 = 0;
-    for (; j0 + kDirectTile <= n; j0 += kDirectTile) {
+    for (; j0 + kDirectTile <= j1; j0 += kDirectTile) {
         float part = 0.f;
 #pragma unroll 8
         for (int j = 0; j < kDirectTile; ++j) part += term(sa[j0 + j], sb[j0 + j]);
         if (KAHAN) kahan_add(sum, comp, part); else sum += part;
     }
     float part = 0.f;
-    for (int64_t j = j0; j < n; ++j) part += term(sa[j], sb[j]);
+    for (int64_t j = j0; j < j1; ++j) part += term(sa[j], sb[j]);
     if (KAHAN) kahan_add(sum, comp, part); else sum += part;
+}
+
+// the sources [j0, j1) summed at q, value and gradient: s − c for each
+template <bool SCREENED, bool KAHAN>
+__device__ __forceinline__ void direct_grad(const float4* __restrict__ sa, const float4* __restrict__ sb, int64_t j0,
+                                            int64_t j1, float qx, float qy, float qz, float sigma, float (&s)[4],
+                                            float (&c)[4]) {
+    const float sl2e = sigma * kLog2e;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s[k] = c[k] = 0.f;
+    float p[4];
+    auto term = [&](const float4 a, const float4 b) {
+        float w, gx, gy, gz;
+        gwn_term_grad_d<SCREENED>(a.x - qx, a.y - qy, a.z - qz, a.w, b, sigma, sl2e, w, gx, gy, gz);
+        p[0] += w;
+        p[1] += gx;
+        p[2] += gy;
+        p[3] += gz;
+    };
+    auto fold = [&]() {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (KAHAN) kahan_add(s[k], c[k], p[k]); else s[k] += p[k];
+            p[k] = 0.f;
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < 4; ++k) p[k] = 0.f;
+    for (; j0 + kDirectTile <= j1; j0 += kDirectTile) {
+#pragma unroll 4
+        for (int j = 0; j < kDirectTile; ++j) term(sa[j0 + j], sb[j0 + j]);
+        fold();
+    }
+    if (j0 < j1) {
+        for (int64_t j = j0; j < j1; ++j) term(sa[j], sb[j]);
+        fold();
+    }
+}
+
+template <bool SCREENED, bool KAHAN, bool NEAR64 = false>
+__global__ __launch_bounds__(kDirectThreads) void gwn_direct_kernel(
+    const float4* __restrict__ sa, const float4* __restrict__ sb, int64_t n, const float* __restrict__ q,
+    int64_t nq, float sigma, float* __restrict__ out) {
+    const int64_t i = int64_t(blockIdx.x) * kDirectThreads + threadIdx.x;
+    const bool valid = i < nq;
+    const float qx = valid ? q[3 * i] : 0.f, qy = valid ? q[3 * i + 1] : 0.f, qz = valid ? q[3 * i + 2] : 0.f;
+    float sum, comp;
+    double near;
+    direct_value<SCREENED, KAHAN, NEAR64>(sa, sb, 0, n, qx, qy, qz, sigma, sum, comp, near);
     if (valid) out[i] = NEAR64 ? float(double(sum - comp) + near) : sum - comp;
 }
 
@@ -210,33 +257,78 @@ __global__ __launch_bounds__(kDirectThreads) void gwn_direct_grad_kernel(
     const int64_t i = int64_t(blockIdx.x) * kDirectThreads + threadIdx.x;
     const bool valid = i < nq;
     const float qx = valid ? q[3 * i] : 0.f, qy = valid ? q[3 * i + 1] : 0.f, qz = valid ? q[3 * i + 2] : 0.f;
-    const float sl2e = sigma * kLog2e;
-    float s[4] = {0, 0, 0, 0}, c[4] = {0, 0, 0, 0};
-    for (int64_t j0 = 0; j0 < n; j0 += kDirectTile) {
-        const int64_t j1 = j0 + kDirectTile < n ? j0 + kDirectTile : n;
-        float p[4] = {0, 0, 0, 0};
-        for (int64_t j = j0; j < j1; ++j) {
-            float w, gx, gy, gz;
-            const float4 a = sa[j];
-            gwn_term_grad_d<SCREENED>(a.x - qx, a.y - qy, a.z - qz, a.w, sb[j], sigma, sl2e, w, gx, gy, gz);
-            p[0] += w;
-            p[1] += gx;
-            p[2] += gy;
-            p[3] += gz;
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if (KAHAN) kahan_add(s[k], c[k], p[k]); else s[k] += p[k];
-        }
-    }
+    float s[4], c[4];
+    direct_grad<SCREENED, KAHAN>(sa, sb, 0, n, qx, qy, qz, sigma, s, c);
     if (valid) {
         out_w[i] = s[0] - c[0];
-        if (out_g) {
-            out_g[3 * i] = s[1] - c[1];
-            out_g[3 * i + 1] = s[2] - c[2];
-            out_g[3 * i + 2] = s[3] - c[3];
-        }
+        out_g[3 * i] = s[1] - c[1];
+        out_g[3 * i + 1] = s[2] - c[2];
+        out_g[3 * i + 2] = s[3] - c[3];
     }
+}
+
+// Few queries over many sources leave most of the chip idle (2,000 queries
+// are 32 waves for 1,024 SIMDs), so the sources are split: one wave takes 64
+// queries (blockIdx.x) and one run of sources (blockIdx.y) and writes its
+// sums in FP64 (the Kahan pair and the FP64 near field without a rounding),
+// direct_fold_kernel adds the runs in FP64 in a fixed order and rounds once:
+// no less exact than one chain.  VALU-bound like the unsplit kernels once
+// every SIMD has a few waves.
+template <bool SCREENED, bool KAHAN, bool NEAR64>
+__global__ __launch_bounds__(64) void gwn_direct_split_kernel(const float4* __restrict__ sa,
+                                                              const float4* __restrict__ sb, int64_t n, int64_t run,
+                                                              const float* __restrict__ q, int64_t nq, float sigma,
+                                                              double* __restrict__ part) {
+    const int64_t i = int64_t(blockIdx.x) * 64 + threadIdx.x;
+    const bool valid = i < nq;
+    const float qx = valid ? q[3 * i] : 0.f, qy = valid ? q[3 * i + 1] : 0.f, qz = valid ? q[3 * i + 2] : 0.f;
+    const int64_t j0 = int64_t(blockIdx.y) * run, j1 = j0 + run < n ? j0 + run : n;
+    float sum, comp;
+    double near;
+    direct_value<SCREENED, KAHAN, NEAR64>(sa, sb, j0, j1, qx, qy, qz, sigma, sum, comp, near);
+    if (valid) part[int64_t(blockIdx.y) * nq + i] = (double(sum) - double(comp)) + near;
+}
+
+template <bool SCREENED, bool KAHAN>
+__global__ __launch_bounds__(64) void gwn_direct_grad_split_kernel(const float4* __restrict__ sa,
+                                                                   const float4* __restrict__ sb, int64_t n,
+                                                                   int64_t run, const float* __restrict__ q,
+                                                                   int64_t nq, float sigma,
+                                                                   double* __restrict__ part) {
+    const int64_t i = int64_t(blockIdx.x) * 64 + threadIdx.x;
+    const bool valid = i < nq;
+    const float qx = valid ? q[3 * i] : 0.f, qy = valid ? q[3 * i + 1] : 0.f, qz = valid ? q[3 * i + 2] : 0.f;
+    const int64_t j0 = int64_t(blockIdx.y) * run, j1 = j0 + run < n ? j0 + run : n;
+    float s[4], c[4];
+    direct_grad<SCREENED, KAHAN>(sa, sb, j0, j1, qx, qy, qz, sigma, s, c);
+    if (valid) {
+        double* o = part + int64_t(blockIdx.y) * 4 * nq;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k * nq + i] = double(s[k]) - double(c[k]);
+    }
+}
+
+// out = Σ over the splits of part[split][value]: kFoldValues values and
+// kFoldRows rows of splits a block, the rows added in order.  Values
+// [0, nq) are w, then ∇w by component (nv = 4·nq with a gradient)
+constexpr int kFoldValues = 32, kFoldRows = 8;
+__global__ __launch_bounds__(kFoldValues * kFoldRows) void direct_fold_kernel(const double* __restrict__ part,
+                                                                              int splits, int64_t nq, int64_t nv,
+                                                                              float* __restrict__ out_w,
+                                                                              float* __restrict__ out_g) {
+    __shared__ double lds[kFoldRows][kFoldValues];
+    const int c = threadIdx.x % kFoldValues, r = threadIdx.x / kFoldValues;
+    const int64_t v = int64_t(blockIdx.x) * kFoldValues + c;
+    double s = 0;
+    if (v < nv)
+        for (int k = r; k < splits; k += kFoldRows) s += part[int64_t(k) * nv + v];
+    lds[r][c] = s;
+    __syncthreads();
+    if (r != 0 || v >= nv) return;
+#pragma unroll
+    for (int k = 1; k < kFoldRows; ++k) s += lds[k][c];
+    if (v < nq) out_w[v] = float(s);
+    else out_g[3 * (v % nq) + (v / nq - 1)] = float(s);
 }
 
 static void check_direct_args(int64_t n, int64_t nq, const float* radii, uint32_t flags, const float*) {
@@ -244,40 +336,84 @@ static void check_direct_args(int64_t n, int64_t nq, const float* radii, uint32_
     DWG_REQUIRE(!(flags & DWG_USE_RADII) || radii, "DWG_USE_RADII needs radii");
 }
 
+// The source runs a direct sum of nq queries over n sources is split into.
+// One wave takes 64 queries; below kDirectWaves waves the chip's 1,024 SIMDs
+// hold too few to hide their latencies, and the sources are split until there
+// are that many.  A run has at least kDirectMinRun sources, under which the
+// second launch costs more than the split saves, and the partial sums fit in
+// kDirectPartials doubles.  Depends on the sizes only, so both entry points
+// sum alike.
+constexpr int64_t kDirectWaves = 4096, kDirectMinRun = 2 * kDirectTile, kDirectMaxSplits = 1024;
+constexpr int64_t kDirectPartials = int64_t(1) << 20;
+
+static int64_t direct_splits(int64_t n, int64_t nq, int values) {
+    const int64_t waves = (nq + 63) / 64;
+    int64_t s = std::min({kDirectWaves / waves, n / kDirectMinRun, kDirectMaxSplits, kDirectPartials / (values * nq)});
+    if (s < 2) return 1;
+    const int64_t run = ((n + s - 1) / s + kDirectTile - 1) / kDirectTile * kDirectTile;  // whole tiles
+    return (n + run - 1) / run;
+}
+
 // packs the n sources into sa/sb (room for n + 1 each) and runs the direct
-// kernel; `profile` off records no events (the allocation-free entry point)
-static void direct_sums(dwg_ctx* ctx, float4* sa, float4* sb, const float* pts, const float* nrm, const float* area,
-                        const float* radii, int64_t n, const float* q, int64_t nq, float sigma, uint32_t flags,
-                        float* out_w, float* out_g, bool profile) {
+// kernel; `part`: room for kDirectPartials doubles when the sums are split;
+// `profile` off records no events (the allocation-free entry point)
+static void direct_sums(dwg_ctx* ctx, float4* sa, float4* sb, double* part, const float* pts, const float* nrm,
+                        const float* area, const float* radii, int64_t n, const float* q, int64_t nq, float sigma,
+                        uint32_t flags, float* out_w, float* out_g, bool profile) {
     if (n > 0) {
         ProfileScope ps(profile ? ctx : nullptr, "pack_sources");
         hipLaunchKernelGGL(pack_sources_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, pts, nrm, area,
                            radii, nullptr, n, (flags & DWG_USE_RADII) ? 1 : 0, sa, sb, nullptr);
         check_launch();
     }
-    const bool kahan = flags & DWG_KAHAN;
-    dim3 grid(grid_for(nq, kDirectThreads)), block(kDirectThreads);
+    const bool kahan = flags & DWG_KAHAN, scr = flags & DWG_SCREENED, near64 = scr && (flags & DWG_NEAR_FP64) && !out_g;
     ProfileScope ps(profile ? ctx : nullptr,
-                    out_g ? "gwn_direct_grad" : ((flags & DWG_SCREENED) ? "gwn_direct_screened" : "gwn_direct_plain"));
-    if (out_g) {
-        const bool scr = flags & DWG_SCREENED;
-#define DWG_GRAD_LAUNCH(S, K) \
-    hipLaunchKernelGGL((gwn_direct_grad_kernel<S, K>), grid, block, 0, ctx->stream, sa, sb, n, q, nq, sigma, out_w, out_g)
-        if (scr && kahan) DWG_GRAD_LAUNCH(true, true);
-        else if (scr) DWG_GRAD_LAUNCH(true, false);
-        else if (kahan) DWG_GRAD_LAUNCH(false, true);
-        else DWG_GRAD_LAUNCH(false, false);
-#undef DWG_GRAD_LAUNCH
-    } else if ((flags & DWG_SCREENED) && (flags & DWG_NEAR_FP64)) {
-        if (kahan) hipLaunchKernelGGL((gwn_direct_kernel<true, true, true>), grid, block, 0, ctx->stream, sa, sb, n, q, nq, sigma, out_w);
-        else hipLaunchKernelGGL((gwn_direct_kernel<true, false, true>), grid, block, 0, ctx->stream, sa, sb, n, q, nq, sigma, out_w);
-    } else if (flags & DWG_SCREENED) {
-        if (kahan) hipLaunchKernelGGL((gwn_direct_kernel<true, true>), grid, block, 0, ctx->stream, sa, sb, n, q, nq, sigma, out_w);
-        else hipLaunchKernelGGL((gwn_direct_kernel<true, false>), grid, block, 0, ctx->stream, sa, sb, n, q, nq, sigma, out_w);
-    } else {
-        if (kahan) hipLaunchKernelGGL((gwn_direct_kernel<false, true>), grid, block, 0, ctx->stream, sa, sb, n, q, nq, sigma, out_w);
-        else hipLaunchKernelGGL((gwn_direct_kernel<false, false>), grid, block, 0, ctx->stream, sa, sb, n, q, nq, sigma, out_w);
+                    out_g ? "gwn_direct_grad" : (scr ? "gwn_direct_screened" : "gwn_direct_plain"));
+    const int values = out_g ? 4 : 1;
+    const int64_t splits = direct_splits(n, nq, values);
+    // LAUNCH(screened, kahan) over the two flags
+#define DWG_DIRECT_BY_FLAGS(LAUNCH)         \
+    do {                                    \
+        if (scr && kahan) LAUNCH(true, true);    \
+        else if (scr) LAUNCH(true, false);       \
+        else if (kahan) LAUNCH(false, true);     \
+        else LAUNCH(false, false);               \
+    } while (0)
+    if (splits > 1) {
+        const int64_t run = ((n + splits - 1) / splits + kDirectTile - 1) / kDirectTile * kDirectTile;
+        dim3 grid(grid_for(nq, 64), unsigned(splits)), block(64);
+#define DWG_SPLIT_GRAD(S, K) \
+    hipLaunchKernelGGL((gwn_direct_grad_split_kernel<S, K>), grid, block, 0, ctx->stream, sa, sb, n, run, q, nq, sigma, part)
+#define DWG_SPLIT_VALUE(S, K) \
+    hipLaunchKernelGGL((gwn_direct_split_kernel<S, K, false>), grid, block, 0, ctx->stream, sa, sb, n, run, q, nq, sigma, part)
+#define DWG_SPLIT_NEAR(S, K) \
+    hipLaunchKernelGGL((gwn_direct_split_kernel<true, K, true>), grid, block, 0, ctx->stream, sa, sb, n, run, q, nq, sigma, part)
+        if (out_g) DWG_DIRECT_BY_FLAGS(DWG_SPLIT_GRAD);
+        else if (near64) DWG_DIRECT_BY_FLAGS(DWG_SPLIT_NEAR);
+        else DWG_DIRECT_BY_FLAGS(DWG_SPLIT_VALUE);
+#undef DWG_SPLIT_GRAD
+#undef DWG_SPLIT_VALUE
+#undef DWG_SPLIT_NEAR
+        check_launch();
+        hipLaunchKernelGGL(direct_fold_kernel, dim3(grid_for(values * nq, kFoldValues)), dim3(kFoldValues * kFoldRows),
+                           0, ctx->stream, part, int(splits), nq, values * nq, out_w, out_g);
+        check_launch();
+        return;
     }
+    dim3 grid(grid_for(nq, kDirectThreads)), block(kDirectThreads);
+#define DWG_DIRECT_GRAD(S, K) \
+    hipLaunchKernelGGL((gwn_direct_grad_kernel<S, K>), grid, block, 0, ctx->stream, sa, sb, n, q, nq, sigma, out_w, out_g)
+#define DWG_DIRECT_VALUE(S, K) \
+    hipLaunchKernelGGL((gwn_direct_kernel<S, K>), grid, block, 0, ctx->stream, sa, sb, n, q, nq, sigma, out_w)
+#define DWG_DIRECT_NEAR(S, K) \
+    hipLaunchKernelGGL((gwn_direct_kernel<true, K, true>), grid, block, 0, ctx->stream, sa, sb, n, q, nq, sigma, out_w)
+    if (out_g) DWG_DIRECT_BY_FLAGS(DWG_DIRECT_GRAD);
+    else if (near64) DWG_DIRECT_BY_FLAGS(DWG_DIRECT_NEAR);
+    else DWG_DIRECT_BY_FLAGS(DWG_DIRECT_VALUE);
+#undef DWG_DIRECT_GRAD
+#undef DWG_DIRECT_VALUE
+#undef DWG_DIRECT_NEAR
+#undef DWG_DIRECT_BY_FLAGS
     check_launch();
 }
 
@@ -287,16 +423,20 @@ void gwn_direct(dwg_ctx* ctx, const float* pts, const float* nrm, const float* a
     if (nq == 0) return;
     float4* sa = static_cast<float4*>(ctx->buf("direct_sa", sizeof(float4) * (n + 1)));
     float4* sb = static_cast<float4*>(ctx->buf("direct_sb", sizeof(float4) * (n + 1)));
-    direct_sums(ctx, sa, sb, pts, nrm, area, radii, n, q, nq, sigma, flags, out_w, out_g, true);
+    double* part = direct_splits(n, nq, out_g ? 4 : 1) > 1
+                       ? static_cast<double*>(ctx->buf("direct_part", sizeof(double) * kDirectPartials))
+                       : nullptr;
+    direct_sums(ctx, sa, sb, part, pts, nrm, area, radii, n, q, nq, sigma, flags, out_w, out_g, true);
 }
 
 // ---------------------------------------------------------------------------
 // allocation-free direct sums: the packed sources live in a fixed device
 // array instead of the context's growable buffers
 // ---------------------------------------------------------------------------
-// sa of source i at scratch[i], sb at scratch[kNoAllocSources + 1 + i]
-// (8 MiB on every device the library runs on, held until the process ends)
-static __device__ __align__(256) float4 scratch[2 * (kNoAllocSources + 1)];
+// sa of source i at scratch[i], sb at scratch[kNoAllocSources + 1 + i], then
+// the partial sums of a split call (8 + 8 MiB on every device the library
+// runs on, held until the process ends)
+static __device__ __align__(256) float4 scratch[2 * (kNoAllocSources + 1) + kDirectPartials * sizeof(double) / sizeof(float4)];
 
 namespace {
 std::mutex g_scratch_mu;
@@ -334,7 +474,7 @@ void gwn_direct_noalloc(dwg_ctx* ctx, const float* pts, const float* nrm, const 
         if (size_t(ctx->device) < g_scratch_ptr.size()) base = g_scratch_ptr[size_t(ctx->device)];
     }
     if (!base) throw Error(DWG_ERR_STATE, "allocation-free scratch of this device was not set up");
-    direct_sums(ctx, base, base + (kNoAllocSources + 1), pts, nrm, area, radii, n, q, nq, sigma, flags, out_w, out_g,
+    direct_sums(ctx, base, base + (kNoAllocSources + 1), reinterpret_cast<double*>(base + 2 * (kNoAllocSources + 1)), pts, nrm, area, radii, n, q, nq, sigma, flags, out_w, out_g,
                 false);
 }
 

@@ -88,7 +88,7 @@ int dwg_gwn_direct(dwg_ctx* ctx, const float* d_pts, const float* d_nrm, const f
 /* No counterpart in the reference: dwg_gwn_direct for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same arguments, kernels and results;
- * the packed sources go to a fixed device array of the library (8 MiB per
+ * the packed sources go to a fixed device array of the library (16 MiB per
  * device, held until the process ends) instead of context buffers, so the
  * call allocates nothing.  n ≤ DWG_NOALLOC_MAX_SOURCES, else DWG_ERR_ARG.
  * Every call on one device shares that array: calls that overlap on a

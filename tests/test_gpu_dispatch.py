@@ -1,0 +1,59 @@
+"""The variants a call is dispatched to by its sizes, each at the edges of its
+range, against the FP64 references."""
+import numpy as np
+import pytest
+
+from dwg_amd import shapes
+
+pytestmark = pytest.mark.gpu
+
+EPS_PLAIN, EPS_SCREENED, SCREEN, SIGMA = 1e-8, 1e-7, 0.0015, 10.0
+
+
+def _direct64(P, N, A, Q, screened):
+    """w, ∇w and the sums of the terms' magnitudes, all pairs in FP64."""
+    d = P[None].astype(float) - Q[:, None].astype(float)
+    b = N.astype(float) * A.astype(float)[:, None]
+    r = np.sqrt((d * d).sum(-1))
+    dot = (d * b).sum(-1)
+    if screened:
+        rho = np.maximum(r, float(np.float32(SCREEN)))
+        e = np.exp(SIGMA * rho) * 4 * np.pi
+        den = e * rho ** 3 + EPS_SCREENED
+        g = (SIGMA * rho + 1) / den
+        gp = (SIGMA * EPS_SCREENED - e * rho ** 2 * (SIGMA ** 2 * rho ** 2 + 3 * SIGMA * rho + 3)) / den ** 2
+        c = np.where(r >= rho, -dot * gp / r, 0.0)
+    else:
+        den = 4 * np.pi * r ** 3 + EPS_PLAIN
+        g = 1 / den
+        c = 12 * np.pi * r * dot * g * g
+    grad = c[..., None] * d - g[..., None] * b
+    mag = (np.abs(c)[..., None] * np.abs(d) + np.abs(g)[..., None] * np.abs(b)).sum(1)
+    rb = r * np.sqrt((b * b).sum(-1))[None]
+    return (g * dot).sum(1), grad.sum(1), (g * rb).sum(1), mag
+
+
+# one wave of queries or less, a query past a wave, few sources (no split),
+# the first split sizes, ragged last runs and tiles, many splits
+@pytest.mark.parametrize("n,nq", [(1, 1), (127, 64), (255, 65), (256, 1), (257, 63), (1000, 1000), (8191, 130),
+                                  (8193, 64), (70_001, 33)])
+@pytest.mark.parametrize("screened", [False, True])
+@pytest.mark.parametrize("kahan", [False, True])
+def test_direct_sums_split_over_sources(ctx, n, nq, screened, kahan):
+    P, N = shapes.sphere(n, 5)
+    rng = np.random.default_rng(n + nq)
+    A = rng.uniform(1e-4, 3e-3, n).astype(np.float32)
+    Q = rng.uniform(-1.3, 1.3, (nq, 3)).astype(np.float32)
+    w, g = ctx.gwn_direct(P, N, A, Q, sigma=SIGMA, screened=screened, kahan=kahan, grad=True)
+    w1 = ctx.gwn_direct(P, N, A, Q, sigma=SIGMA, screened=screened, kahan=kahan)
+    w, g, w1 = (t.cpu().numpy().astype(float) for t in (w, g, w1))
+    rw, rg, mw, mg = _direct64(P, N, A, Q, screened)
+    # a term: the rounding of d (up to 3 ulp of r), of r³ and of the factors,
+    # 1-ulp sqrt, exp2 and reciprocal: under 32·2^-24 of |d||b|g; the chain of
+    # 64 terms in FP32 adds at most 64·2^-24 of their magnitudes, without
+    # compensation the tiles' partial sums as many again per tile
+    tiles = 0 if kahan else (n + 63) // 64
+    tol = (32 + 64 + tiles) * 2.0 ** -24
+    assert (np.abs(w - rw) <= tol * mw + 1e-30).all()
+    assert (np.abs(w1 - rw) <= tol * mw + 1e-30).all()
+    assert (np.abs(g - rg) <= 2 * tol * mg + 1e-30).all()
