@@ -32,15 +32,23 @@ struct dwg_octree {
     double4* cell = nullptr;       // cell centre and width (breadth-first node order)
     double4* cm64 = nullptr;       // (CM, ΣA) in FP64
     // 8 words per node, read by the traversal for all 8 children of a node
-    // in one vector load: internal node (EC/4π, s², CM − float(CM), 0) with
-    // s the default screening radius; leaf with one point: that point's
-    // (A·n/4π, s², 0, 0, 0, 0), its position in cm_r
+    // in one vector load: internal node (EC/4π, s², CM − float(CM), bare
+    // floor) with s the default screening radius; leaf with one point: that
+    // point's (A·n/4π, s², 0, 0, 0, bare floor), its position in cm_r
     float4* payload = nullptr;
     bool payload_bf16 = false;  // internal nodes' EC/4π in the payload rounded to BF16
     ~dwg_octree();
 };
 
 namespace dwg {
+
+// The smallest squared distance at which a dipole's term needs neither the
+// r > 1e-10 guard nor the screening maximum, also once its centre has been
+// corrected by its residual δ (|δ|² = d2): r ≥ 2s and r ≥ 4|δ| leave the
+// corrected distance at least 0.75 r ≥ 1.5 s
+__device__ __forceinline__ float bare_floor(float s2, float d2) {
+    return fmaxf(fmaxf(4.f * s2, 16.f * d2), 1e-18f);
+}
 
 void octree_update(dwg_ctx* ctx, dwg_octree* T, const float* nrm, const float* area, const float* radii);
 // re-packs the point terms (A·n, A) with other areas, keeping the far-field

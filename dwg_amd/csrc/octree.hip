@@ -225,7 +225,8 @@ __global__ void node_pack_kernel(const double4* __restrict__ cm, const unsigned 
     // rounding of the difference itself
     cm_lo[i] = make_float4(float(c.x - double(cx)), float(c.y - double(cy)), float(c.z - double(cz)), 0.f);
     payload[2 * i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    payload[2 * i + 1] = cm_lo[i];
+    const float4 lo = cm_lo[i];
+    payload[2 * i + 1] = make_float4(lo.x, lo.y, lo.z, bare_floor(kScreenDefault * kScreenDefault, dist2(lo.x, lo.y, lo.z)));
 }
 
 __global__ void pack_positions_kernel(const double* __restrict__ P, const int* __restrict__ perm, int64_t n,

@@ -2,8 +2,9 @@
 range, against the FP64 references."""
 import numpy as np
 import pytest
+import torch
 
-from dwg_amd import shapes
+from dwg_amd import gpu, shapes
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +58,32 @@ def test_direct_sums_split_over_sources(ctx, n, nq, screened, kahan):
     assert (np.abs(w - rw) <= tol * mw + 1e-30).all()
     assert (np.abs(w1 - rw) <= tol * mw + 1e-30).all()
     assert (np.abs(g - rg) <= 2 * tol * mg + 1e-30).all()
+
+
+# bricks cut by every face of the grid, a grid inside one brick, grids far
+# from and across the cloud, and a cloud far from the origin (large residuals
+# of the rounded centres)
+@pytest.mark.parametrize("res,h,shift", [((8, 4, 8), 0.05, 0.0), ((9, 5, 7), 0.002, 0.0), ((1, 1, 1), 0.1, 0.0),
+                                         ((33, 29, 31), 0.08, 0.0), ((23, 3, 17), 0.3, 0.0),
+                                         ((25, 26, 9), 0.05, 100.0)])
+@pytest.mark.parametrize("screened,bf16,radii", [(True, False, False), (True, True, True), (False, False, False),
+                                                 (False, True, False)])
+def test_grid_walk_equals_the_point_walk(ctx, res, h, shift, screened, bf16, radii):
+    # the brick's whole-box decisions are each point's own, so a grid value is
+    # the explicit point's bit for bit (the same terms in the same order)
+    P, N = shapes.union(3000, 8, 11)
+    P = np.concatenate([P, P[:40], P[:3] + 1e-6]).astype(np.float64) + shift  # leaves of several points
+    N = np.concatenate([N, N[:40], N[:3]]).astype(np.float32)
+    A = np.full(len(P), 2e-6, np.float32)
+    R = np.linspace(0.0, 0.05, len(P), dtype=np.float32) if radii else None
+    tree = gpu.Octree(ctx, P, None, max_depth=10)
+    tree.update(N, A, R)
+    c = P.mean(0)
+    grid = gpu.make_grid([c[d] - 0.5 * h * (res[d] - 1) for d in range(3)], h, res)
+    ax = [np.array([np.float32(np.float64(i) * grid.h + grid.origin[d]) for i in range(res[d])]) for d in range(3)]
+    z, y, x = np.meshgrid(ax[2], ax[1], ax[0], indexing="ij")
+    Q = torch.from_numpy(np.stack([x, y, z], -1).reshape(-1, 3).astype(np.float32)).cuda()
+    kw = dict(sigma=SIGMA, screened=screened, bf16=bf16)
+    got = tree.eval_grid(grid, 2.3, **kw).cpu().numpy()
+    want = tree.eval(Q, 2.3, **kw).cpu().numpy()
+    np.testing.assert_array_equal(got, want)
