@@ -3,12 +3,12 @@
 // The reference builds a left-balanced kd-tree with log2(N) thrust sorts and
 // walks it per query (KNN_GWN.cu:42-66, builder_thrust.h:486-724).  Here the
 // points are bucketed once into a dense cell grid (counting sort: one
-// histogram, one scan, one scatter); a query visits cells in growing
-// Chebyshev shells around its own cell and stops once its k-th key is closer
-// than any cell not yet visited.  Candidates are kept as 64-bit keys
-// (float bits of d² << 32 | index) in a register array, so results are the
-// exact k smallest (d², index) pairs — identical to a brute-force scan with
-// the same float d² formula, ties to the lower index.
+// histogram, one scan, one scatter).  Many queries are answered tile by tile
+// from points staged in LDS; the ones that leaves open, and small query sets,
+// walk the grid's occupancy pyramid.  Candidates are kept as 64-bit keys
+// (float bits of d² << 32 | index) in registers, so results are the exact k
+// smallest (d², index) pairs — identical to a brute-force scan with the same
+// float d² formula, ties to the lower index.
 #include <algorithm>
 #include <cmath>
 
@@ -532,95 +532,6 @@ __device__ __forceinline__ void knn_store(const uint64_t (&best)[K], int k, int6
     }
 }
 
-// Visits shells r = 0..rmax of cells around q on one grid level, keeping
-// the k smallest (d², index) keys.  Returns true once no unvisited cell can
-// hold a closer point (the search is then exact on this level).
-template <int K>
-__device__ bool search_level(const KnnGridArgs& G, const int64_t* __restrict__ cell_start,
-                             const float4* __restrict__ pts, float qx, float qy, float qz, int k,
-                             const uint8_t* __restrict__ skip, uint64_t (&best)[K], int rmax,
-                             const int* __restrict__ empty) {
-    knn_reset<K>(best, k);
-    const int c0x = cell_coord(qx, G.lo[0], G.inv_cell, G.dim[0]);
-    const int c0y = cell_coord(qy, G.lo[1], G.inv_cell, G.dim[1]);
-    const int c0z = cell_coord(qz, G.lo[2], G.inv_cell, G.dim[2]);
-    // every cell closer (Chebyshev) than empty[c0] holds no point: start there
-    const int r0 = empty ? min(empty[c0x + int64_t(G.dim[0]) * (c0y + int64_t(G.dim[1]) * c0z)], rmax) : 0;
-    for (int r = r0; r <= rmax; ++r) {
-        const int zlo = max(c0z - r, 0), zhi = min(c0z + r, G.dim[2] - 1);
-        const int ylo = max(c0y - r, 0), yhi = min(c0y + r, G.dim[1] - 1);
-        for (int z = zlo; z <= zhi; ++z) {
-            const bool zedge = abs(z - c0z) == r;
-            for (int y = ylo; y <= yhi; ++y) {
-                const bool yedge = zedge || abs(y - c0y) == r;
-                // rows on the shell's faces are scanned fully, other rows only at both ends
-                const int xs = yedge ? max(c0x - r, 0) : c0x - r;
-                const int step = yedge ? 1 : 2 * r;
-                const int xe = min(c0x + r, G.dim[0] - 1);
-                for (int x = xs; x <= xe; x += step) {
-                    if (x < 0) continue;
-                    const int64_t c = x + int64_t(G.dim[0]) * (y + int64_t(G.dim[1]) * z);
-                    const int64_t sb = cell_start[c], se = cell_start[c + 1];
-                    for (int64_t s = sb; s < se; ++s) {
-                        const float4 p = pts[s];
-                        const int idx = __float_as_int(p.w);
-                        const float d2 = dist2(qx - p.x, qy - p.y, qz - p.z);
-                        const uint64_t key = (uint64_t(__float_as_uint(d2)) << 32) | uint32_t(idx);
-                        // the skip byte only for a point that would enter the list
-                        if (key < best[0] && !(skip && skip[idx])) knn_insert<K>(best, key);
-                    }
-                }
-            }
-        }
-        const uint64_t kth = best[0];
-        // distance from q to the nearest face of the searched block that is
-        // not on the grid boundary; no unvisited point can be closer
-        float dmin = INFINITY;
-        if (c0x - r > 0) dmin = fminf(dmin, qx - (G.lo[0] + float(c0x - r) * G.cell));
-        if (c0x + r + 1 < G.dim[0]) dmin = fminf(dmin, (G.lo[0] + float(c0x + r + 1) * G.cell) - qx);
-        if (c0y - r > 0) dmin = fminf(dmin, qy - (G.lo[1] + float(c0y - r) * G.cell));
-        if (c0y + r + 1 < G.dim[1]) dmin = fminf(dmin, (G.lo[1] + float(c0y + r + 1) * G.cell) - qy);
-        if (c0z - r > 0) dmin = fminf(dmin, qz - (G.lo[2] + float(c0z - r) * G.cell));
-        if (c0z + r + 1 < G.dim[2]) dmin = fminf(dmin, (G.lo[2] + float(c0z + r + 1) * G.cell) - qz);
-        if (dmin == INFINITY) return true;  // the block covers the whole grid
-        if (kth != kNoKey) {
-            const float kd2 = __uint_as_float(uint32_t(kth >> 32));
-            const float safe = dmin * (1.0f - 1e-5f) - 1e-6f * G.cell;
-            if (safe > 0.f && kd2 < safe * safe) return true;
-        }
-    }
-    return false;
-}
-
-// One query per lane; `qlist` (nullable) lists the queries to answer
-// (nq entries), otherwise queries 0..nq−1.
-template <int K>
-__global__ __launch_bounds__(256) void knn_query_kernel(KnnGridArgs G0, const int64_t* __restrict__ cs0,
-                                                        const float4* __restrict__ p0, KnnGridArgs G1,
-                                                        const int64_t* __restrict__ cs1,
-                                                        const float4* __restrict__ p1, const int* __restrict__ empty1,
-                                                        const float* __restrict__ q, int64_t nq,
-                                                        const int* __restrict__ qlist, int k,
-                                                        const uint8_t* __restrict__ skip,
-                                                        const uint8_t* __restrict__ qmask, int32_t* __restrict__ out_idx,
-                                                        float* __restrict__ out_d2) {
-    const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= nq) return;
-    const int64_t i = qlist ? int64_t(qlist[t]) : t;
-    if (qmask && !qmask[i]) return;
-    const float qx = q[3 * i], qy = q[3 * i + 1], qz = q[3 * i + 2];
-    uint64_t best[K];
-    // a query whose coarse cell is empty skips the fine shells
-    const int c1 = cell_coord(qx, G1.lo[0], G1.inv_cell, G1.dim[0]) +
-                   G1.dim[0] * (cell_coord(qy, G1.lo[1], G1.inv_cell, G1.dim[1]) +
-                                G1.dim[1] * cell_coord(qz, G1.lo[2], G1.inv_cell, G1.dim[2]));
-    if (empty1[c1] > 0 || !search_level<K>(G0, cs0, p0, qx, qy, qz, k, skip, best, 2, nullptr)) {
-        const int maxr = max(G1.dim[0], max(G1.dim[1], G1.dim[2]));
-        (void)search_level<K>(G1, cs1, p1, qx, qy, qz, k, skip, best, maxr, empty1);
-    }
-    knn_store<K>(best, k, i, out_idx, out_d2);
-}
-
 // ---------------------------------------------------------------------------
 // Tiled queries.  Queries are bucketed by tile (kTile³ fine cells); one
 // workgroup per non-empty tile stages the points of the tile plus a kHalo
@@ -628,23 +539,21 @@ __global__ __launch_bounds__(256) void knn_query_kernel(KnnGridArgs G0, const in
 // candidates in lockstep, so LDS reads are broadcasts and no lane diverges.
 // A query is final when its k-th key is closer than every face of the
 // staged box that is not on the grid boundary; the rest (sparse or clustered
-// regions) go to the per-lane shell search above.  Both paths keep the k
-// smallest (d², index) keys, so the result does not depend on the path.
+// regions) walk the pyramid.  All paths keep the k smallest (d², index) keys,
+// so the result does not depend on the path.
 // ---------------------------------------------------------------------------
 constexpr double kScatterFix = 1099511627776.0;  // 2^40
 constexpr int kTile = 4;
 constexpr int kStage = 512;
 constexpr int kTileThreads = 256;
-// halos of the tiled passes: most queries close within 2 cells; the ones
-// that do not (off-surface centroids) get passes with 5 and 9 cells
-constexpr int kHalo1 = 2;
-constexpr int kHalo2 = 5;
-constexpr int kHalo3 = 9;
+// most queries close within 2 cells of their tile.  Wider passes for the
+// others (5 and 9 cells) cost more than walking the pyramid at once: 200,000
+// queries over 1M points, half of them off the surface, 5.6 → 3.4 ms
+constexpr int kHalo = 2;
 // the tiled passes bucket their queries by 2×2×2-cell eighth of the tile
 // (8 buckets per tile), so that the 64 queries of a wave sit close together
 // (first pass 2.07 → 1.97 ms, and the far walk that takes its open queries
-// in this order 1.89 → 1.81 ms); the sparse walk's order keeps one bucket
-// per tile (0.86 instead of 0.93 ms)
+// in this order 1.89 → 1.81 ms)
 constexpr int kSubTiled = 8;
 
 // exclusive sum over the block's threads (NT threads, a multiple of 64);
@@ -667,32 +576,26 @@ __device__ __forceinline__ int block_exclusive_sum(int v, int* wsum) {
 }
 
 struct TileArgs {
-    int tdim[3];   // tiles per axis
-    float margin;  // rounding allowance of cell boundaries (cell_margin)
-    int sub;       // query buckets per tile: 1 or 8 (by eighth of the tile)
+    int tdim[3];  // tiles per axis
 };
 
-// bucket of a point: its tile, times 8 plus the eighth of the tile it lies
-// in when T.sub is 8
+// bucket of a point: its tile, times 8, plus the eighth of the tile it lies in
 __device__ __forceinline__ int bucket_of_point(const KnnGridArgs& G, const TileArgs& T, float x, float y, float z) {
     const int cx = cell_coord(x, G.lo[0], G.inv_cell, G.dim[0]);
     const int cy = cell_coord(y, G.lo[1], G.inv_cell, G.dim[1]);
     const int cz = cell_coord(z, G.lo[2], G.inv_cell, G.dim[2]);
     const int tile = cx / kTile + T.tdim[0] * (cy / kTile + T.tdim[1] * (cz / kTile));
-    if (T.sub == 1) return tile;
     constexpr int h = kTile / 2;
-    return tile * 8 + int(cx % kTile >= h) + 2 * int(cy % kTile >= h) + 4 * int(cz % kTile >= h);
+    return tile * kSubTiled + int(cx % kTile >= h) + 2 * int(cy % kTile >= h) + 4 * int(cz % kTile >= h);
 }
 
-// query t of the pass is qlist[t] (or t); masked queries are left out
-__global__ void tile_count_kernel(const float* __restrict__ q, int64_t nq, const int* __restrict__ qlist,
-                                  const uint8_t* __restrict__ qmask, KnnGridArgs G, TileArgs T,
+// masked queries are left out
+__global__ void tile_count_kernel(const float* __restrict__ q, int64_t nq, const uint8_t* __restrict__ qmask, KnnGridArgs G, TileArgs T,
                                   int* __restrict__ tile_of, unsigned long long* __restrict__ count) {
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     int tl = -1;  // every lane takes part in the run detection
     if (t < nq) {
-        const int64_t i = qlist ? int64_t(qlist[t]) : t;
-        if (!qmask || qmask[i]) tl = bucket_of_point(G, T, q[3 * i], q[3 * i + 1], q[3 * i + 2]);
+        if (!qmask || qmask[t]) tl = bucket_of_point(G, T, q[3 * t], q[3 * t + 1], q[3 * t + 2]);
         tile_of[t] = tl;
     }
     const int lane = threadIdx.x & 63;
@@ -700,7 +603,7 @@ __global__ void tile_count_kernel(const float* __restrict__ q, int64_t nq, const
     if (tl >= 0 && ((starts >> lane) & 1ull)) atomicAdd(&count[tl], (unsigned long long)run_length(starts, lane));
 }
 
-__global__ void tile_scatter_kernel(const int* __restrict__ tile_of, int64_t nq, const int* __restrict__ qlist,
+__global__ void tile_scatter_kernel(const int* __restrict__ tile_of, int64_t nq,
                                     unsigned long long* __restrict__ cursor, int* __restrict__ order) {
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const int tl = t < nq ? tile_of[t] : -1;
@@ -711,14 +614,13 @@ __global__ void tile_scatter_kernel(const int* __restrict__ tile_of, int64_t nq,
         base = int(atomicAdd(&cursor[tl], (unsigned long long)run_length(starts, lane)));
     const int head = run_head(starts, lane);
     const int hb = __shfl(base, head, 64);
-    if (tl >= 0) order[hb + (lane - head)] = qlist ? qlist[t] : int(t);
+    if (tl >= 0) order[hb + (lane - head)] = int(t);
 }
 
-__global__ void tile_flags_kernel(const int64_t* __restrict__ start, int64_t ntiles, int sub,
-                                  int64_t* __restrict__ flags) {
+__global__ void tile_flags_kernel(const int64_t* __restrict__ start, int64_t ntiles, int64_t* __restrict__ flags) {
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (t > ntiles) return;
-    flags[t] = (t < ntiles && start[sub * (t + 1)] > start[sub * t]) ? 1 : 0;
+    flags[t] = (t < ntiles && start[kSubTiled * (t + 1)] > start[kSubTiled * t]) ? 1 : 0;
 }
 
 __global__ void tile_list_kernel(const int64_t* __restrict__ flags, int64_t ntiles, int* __restrict__ list) {
@@ -736,18 +638,19 @@ __global__ void tile_list_kernel(const int64_t* __restrict__ flags, int64_t ntil
 // LDS hash table keyed by point index and flushes each key once with 64-bit
 // global atomics; integer sums are associative, so the result equals
 // per-pair atomics bit for bit.
-template <int K, int HALO, bool SCATTER>
+template <int K, bool SCATTER>
 __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     KnnGridArgs G, TileArgs T, const int64_t* __restrict__ cell_start, const float4* __restrict__ pts,
     const int* __restrict__ tiles, const int64_t* __restrict__ tile_start, const int* __restrict__ order,
     const float* __restrict__ q, int k, const uint8_t* __restrict__ skip, int32_t* __restrict__ out_idx,
-    float* __restrict__ out_d2, int* __restrict__ redo, float* __restrict__ redo_kth, unsigned int* __restrict__ n_redo,
-    int64_t* __restrict__ redo_flag, KnnScatter sc) {
-    constexpr int kRegion = kTile + 2 * HALO;
-    // the first pass splits each row into the tile's own cells and the halo
-    // cells at x distance 1 and 2 on either side, so that the staging order
-    // (by Chebyshev ring from the tile) starts with the tile's own cells
-    constexpr int kParts = HALO == kHalo1 ? 5 : 1;
+    float* __restrict__ out_d2, int* __restrict__ redo, float* __restrict__ redo_kth, int64_t* __restrict__ redo_flag,
+    const int64_t* __restrict__ ntiles, KnnScatter sc) {
+    if (ntiles && int64_t(blockIdx.x) >= *ntiles) return;  // launched for the most tiles there can be
+    constexpr int kRegion = kTile + 2 * kHalo;
+    // each row is split into the tile's own cells and the halo cells at x
+    // distance 1 and 2 on either side, so that the staging order (by
+    // Chebyshev ring from the tile) starts with the tile's own cells
+    constexpr int kParts = 5;
     constexpr int kRows = kRegion * kRegion * kParts;
     constexpr int kHash = SCATTER ? 256 : 1;
     __shared__ int s_hkey[kHash];
@@ -762,46 +665,41 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     __shared__ int64_t s_rb[kRows];
     __shared__ int s_cnt[kRows];
     __shared__ int s_pref[kRows + 1];
-    __shared__ int s_ryz[kRows];  // y | z << 16 of each row
-    __shared__ int s_rx[kRows];   // its cells xa | xb << 16
     __shared__ int s_wsum[kTileThreads / 64];
-    __shared__ int s_ring[HALO + 2];
+    __shared__ int s_ring[kHalo + 2];
     const int tile = tiles[blockIdx.x];
     const int tx = tile % T.tdim[0], ty = (tile / T.tdim[0]) % T.tdim[1], tz = tile / (T.tdim[0] * T.tdim[1]);
-    const int x0 = max(tx * kTile - HALO, 0), x1 = min(tx * kTile + kTile - 1 + HALO, G.dim[0] - 1);
-    const int y0 = max(ty * kTile - HALO, 0), y1 = min(ty * kTile + kTile - 1 + HALO, G.dim[1] - 1);
-    const int z0 = max(tz * kTile - HALO, 0), z1 = min(tz * kTile + kTile - 1 + HALO, G.dim[2] - 1);
+    const int x0 = max(tx * kTile - kHalo, 0), x1 = min(tx * kTile + kTile - 1 + kHalo, G.dim[0] - 1);
+    const int y0 = max(ty * kTile - kHalo, 0), y1 = min(ty * kTile + kTile - 1 + kHalo, G.dim[1] - 1);
+    const int z0 = max(tz * kTile - kHalo, 0), z1 = min(tz * kTile + kTile - 1 + kHalo, G.dim[2] - 1);
     const int ny = y1 - y0 + 1, nrows = ny * (z1 - z0 + 1) * kParts;
-    if (threadIdx.x < HALO + 2) s_ring[threadIdx.x] = 0;
+    if (threadIdx.x < kHalo + 2) s_ring[threadIdx.x] = 0;
     __syncthreads();
     // each (y, z) row of cells x0..x1 (or each of its parts) is one
     // contiguous range of points; a thread takes rows threadIdx.x +
     // h · kTileThreads, h < kRowIters
     constexpr int kRowIters = (kRows + kTileThreads - 1) / kTileThreads;
-    int ring[kRowIters], rank[kRowIters], rc[kRowIters], rx[kRowIters];
+    int ring[kRowIters], rank[kRowIters], rc[kRowIters];
     int64_t rb[kRowIters];
 #pragma unroll
     for (int h = 0; h < kRowIters; ++h) {
-        ring[h] = rank[h] = rc[h] = rx[h] = 0;
+        ring[h] = rank[h] = rc[h] = 0;
         rb[h] = 0;
         const int r = threadIdx.x + h * kTileThreads;
         if (r < nrows) {
             const int row = r / kParts, part = r % kParts;
             const int y = y0 + row % ny, z = z0 + row / ny;
             // the part's cells xa..xb and their x distance from the tile
-            int xa = x0, xb = x1, dx = 0;
-            if (kParts > 1) {
-                const int t0 = tx * kTile, t1 = tx * kTile + kTile - 1;
-                if (part == 0) { xa = t0; xb = t1; }
-                else if (part <= 2) { xa = xb = t0 - part; dx = part; }
-                else { xa = xb = t1 + (part - 2); dx = part - 2; }
-                xa = max(xa, x0);
-                xb = min(xb, x1);
-            }
+            int xa, xb, dx = 0;
+            const int t0 = tx * kTile, t1 = tx * kTile + kTile - 1;
+            if (part == 0) { xa = t0; xb = t1; }
+            else if (part <= 2) { xa = xb = t0 - part; dx = part; }
+            else { xa = xb = t1 + (part - 2); dx = part - 2; }
+            xa = max(xa, x0);
+            xb = min(xb, x1);
             const int64_t c = xa + int64_t(G.dim[0]) * (y + int64_t(G.dim[1]) * z);
             rb[h] = cell_start[c];
             rc[h] = xb >= xa ? int(cell_start[c + (xb - xa) + 1] - rb[h]) : 0;
-            rx[h] = xa | (xb << 16);
             const int dy = max(max(ty * kTile - y, y - (ty * kTile + kTile - 1)), 0);
             const int dz = max(max(tz * kTile - z, z - (tz * kTile + kTile - 1)), 0);
             ring[h] = max(max(dy, dz), dx);
@@ -810,17 +708,14 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     }
     __syncthreads();
     if (threadIdx.x == 0)
-        for (int r = 1; r <= HALO + 1; ++r) s_ring[r] += s_ring[r - 1];
+        for (int r = 1; r <= kHalo + 1; ++r) s_ring[r] += s_ring[r - 1];
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < kRowIters; ++h) {
         if (threadIdx.x + h * kTileThreads < nrows) {
             const int pos = s_ring[ring[h]] + rank[h];
-            const int r = (threadIdx.x + h * kTileThreads) / kParts;
             s_rb[pos] = rb[h];
             s_cnt[pos] = rc[h];
-            s_ryz[pos] = (y0 + r % ny) | ((z0 + r / ny) << 16);
-            s_rx[pos] = rx[h];
         }
     }
     __syncthreads();
@@ -852,7 +747,7 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     const float fhy = y1 + 1 < G.dim[1] ? G.lo[1] + float(y1 + 1) * G.cell : INFINITY;
     const float flz = z0 > 0 ? G.lo[2] + float(z0) * G.cell : -INFINITY;
     const float fhz = z1 + 1 < G.dim[2] ? G.lo[2] + float(z1 + 1) * G.cell : INFINITY;
-    const int64_t qs = tile_start[int64_t(tile) * T.sub], qe = tile_start[int64_t(tile + 1) * T.sub];
+    const int64_t qs = tile_start[int64_t(tile) * kSubTiled], qe = tile_start[int64_t(tile + 1) * kSubTiled];
     for (int64_t qb = qs; qb < qe; qb += kTileThreads) {
         const int64_t t = qb + threadIdx.x;
         const bool active = t < qe;
@@ -889,35 +784,8 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
                     kd2 = best[0] == kNoKey ? INFINITY : __uint_as_float(uint32_t(best[0] >> 32));
                 }
             };
-            if (active && HALO == kHalo1) {
-                // the first pass's small region is nearly all needed
+            if (active)
                 for (int j = 0; j < cnt; ++j) candidate(s_pts[j]);
-            } else if (active) {
-                // row by row in ring order: a row whose box of cells is
-                // farther than the k-th distance of every lane of the wave
-                // is skipped whole
-                int r = 0;
-                for (int hi = nrows - 1; r < hi;) {  // the row holding point cb
-                    const int mid = (r + hi + 1) >> 1;
-                    if (s_pref[mid] <= cb) r = mid;
-                    else hi = mid - 1;
-                }
-                for (; r < nrows; ++r) {
-                    const int a = max(s_pref[r], cb), b = min(s_pref[r + 1], cb + cnt);
-                    if (a >= cb + cnt) break;
-                    if (a >= b) continue;
-                    const int yz = s_ryz[r], xr = s_rx[r];
-                    const float rxlo = __builtin_fmaf(float(xr & 0xFFFF), G.cell, G.lo[0]);
-                    const float rxhi = __builtin_fmaf(float((xr >> 16) + 1), G.cell, G.lo[0]);
-                    const float ylo = __builtin_fmaf(float(yz & 0xFFFF), G.cell, G.lo[1]);
-                    const float zlo = __builtin_fmaf(float(yz >> 16), G.cell, G.lo[2]);
-                    const float gy = fmaxf(fmaxf(ylo - qy, qy - (ylo + G.cell)) - T.margin, 0.f);
-                    const float gz = fmaxf(fmaxf(zlo - qz, qz - (zlo + G.cell)) - T.margin, 0.f);
-                    const float gx = fmaxf(fmaxf(rxlo - qx, qx - rxhi) - T.margin, 0.f);
-                    if (!__builtin_amdgcn_ballot_w64(dist2(gx, gy, gz) <= kd2)) continue;
-                    for (int j = a - cb; j < b - cb; ++j) candidate(s_pts[j]);
-                }
-            }
         }
         if (!active) continue;
         const float dmin = fminf(fminf(fminf(qx - flx, fhx - qx), fminf(qy - fly, fhy - qy)), fminf(qz - flz, fhz - qz));
@@ -926,25 +794,13 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
             const float safe = dmin * (1.0f - 1e-5f) - 1e-6f * G.cell;
             exact = safe > 0.f && kd2 < safe * safe;
         }
-        if (!exact && redo_flag) {
-            // ordered: the query keeps its place in tile order (compacted
-            // afterwards), so the far walk's waves get spatially coherent runs
+        if (!exact) {
+            // the query keeps its place in tile order (compacted afterwards),
+            // so the far walk's waves get spatially coherent runs; the k
+            // candidates it has bound its k-th distance
             redo_flag[t] = 1;
             redo[t] = qi;
-            if (redo_kth) redo_kth[t] = kd2;
-            continue;
-        }
-        if (!exact) {
-            // the wave's lanes that give up here take consecutive slots from
-            // one atomic; the k candidates a lane has bound its k-th distance
-            const uint64_t m = __ballot(1);
-            const int lane = threadIdx.x & 63, leader = __builtin_ctzll(m);
-            unsigned int base = 0;
-            if (lane == leader) base = atomicAdd(n_redo, (unsigned int)__builtin_popcountll(m));
-            base = unsigned(__shfl(int(base), leader, 64));
-            const unsigned int slot = base + unsigned(__builtin_popcountll(m & ((1ull << lane) - 1ull)));
-            redo[slot] = qi;
-            if (redo_kth) redo_kth[slot] = kd2;
+            redo_kth[t] = kd2;
             continue;
         }
         knn_store<K>(best, k, qi, out_idx, out_d2);
@@ -984,12 +840,11 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     }
 }
 
-// acc[neighbour] += value of the query, for the queries of qlist (or all)
-__global__ void scatter_pairs_kernel(const int32_t* __restrict__ knn, int k, const int* __restrict__ qlist, int64_t nq,
-                                     KnnScatter sc) {
+// acc[neighbour] += value of the query, for every query
+__global__ void scatter_pairs_kernel(const int32_t* __restrict__ knn, int k, int64_t nq, KnnScatter sc) {
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (t >= nq * k) return;
-    const int64_t qi = qlist ? int64_t(qlist[t / k]) : t / k;
+    const int64_t qi = t / k;
     const int32_t s = knn[qi * k + t % k];
     if (s < 0) return;
 #pragma unroll
@@ -1005,8 +860,10 @@ __global__ void scatter_pairs_kernel(const int32_t* __restrict__ knn, int k, con
 // flushed once with 64-bit global atomics (integer sums: bit for bit the
 // per-pair result).
 __global__ __launch_bounds__(256) void scatter_pairs_hashed_kernel(const int32_t* __restrict__ knn, int k,
-                                                                   const int* __restrict__ qlist, int64_t nq,
-                                                                   KnnScatter sc) {
+                                                                   const int* __restrict__ qlist,
+                                                                   const int64_t* __restrict__ count, KnnScatter sc) {
+    const int64_t nq = *count;  // launched for every query
+    if (int64_t(blockIdx.x) * 256 >= nq) return;
     constexpr int kHash = 1024;
     __shared__ int s_hkey[kHash];
     __shared__ unsigned long long s_hacc[kHash][3];
@@ -1017,7 +874,7 @@ __global__ __launch_bounds__(256) void scatter_pairs_hashed_kernel(const int32_t
     __syncthreads();
     const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
     if (t < nq) {
-        const int64_t qi = qlist ? int64_t(qlist[t]) : t;
+        const int64_t qi = qlist[t];
         long long v[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) v[d] = __double2ll_rn(double(sc.val[3 * qi + d]) * kScatterFix);
@@ -1063,9 +920,8 @@ __device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
     return v;
 }
 
-// One wave per query, for the queries the tiled passes could not close (far
-// from the points, or inside a cluster of skipped points).  On the coarse
-// level the cells of each Chebyshev shell are read 64 at a time, their
+// One wave per query, for indices without a pyramid (a single cell, or a grid
+// too elongated for one).  On the coarse level the cells of each Chebyshev shell are read 64 at a time, their
 // points flattened and scanned 64 per step (one candidate per lane), each
 // lane keeping its own k best keys.  The smallest lane-local k-th key bounds
 // the wave's k-th key from above, so the search stops once it is closer than
@@ -1095,18 +951,16 @@ template <int K>
 __global__ __launch_bounds__(256) void knn_wave_kernel(KnnGridArgs G, const int64_t* __restrict__ cell_start,
                                                        const float4* __restrict__ pts, const int* __restrict__ empty,
                                                        const float* __restrict__ q, int64_t nq,
+                                                       const int64_t* __restrict__ count,
                                                        const int* __restrict__ qlist, int k,
-                                                       const uint8_t* __restrict__ skip, int32_t* __restrict__ out_idx,
+                                                       const uint8_t* __restrict__ skip,
+                                                       const uint8_t* __restrict__ qmask, int32_t* __restrict__ out_idx,
                                                        float* __restrict__ out_d2) {
     const int lane = threadIdx.x & 63;
-    // wave w takes query w/2 of the list if w is even, else the (w/2)-th
-    // from the end: the long searches, which come in runs along the list,
-    // start early from either end (zero fill 0.61 → 0.57 ms per iteration;
-    // the tiled passes lose L2 reuse that way and keep their order)
-    const int64_t w = int64_t(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (w >= nq) return;  // uniform per wave
-    const int64_t t = (w & 1) ? nq - 1 - (w >> 1) : (w >> 1);
+    const int64_t t = int64_t(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (t >= (count ? *count : nq)) return;  // uniform per wave
     const int64_t i = qlist ? int64_t(qlist[t]) : t;
+    if (qmask && !qmask[i]) return;
     const float qx = q[3 * i], qy = q[3 * i + 1], qz = q[3 * i + 2];
     uint64_t best[K];
     knn_reset<K>(best, k);
@@ -1202,30 +1056,7 @@ __global__ __launch_bounds__(256) void knn_wave_kernel(KnnGridArgs G, const int6
     }
 }
 
-static void launch_wave(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const int* qlist, int k,
-                        const uint8_t* skip, int32_t* out_idx, float* out_d2) {
-    if (nq == 0) return;
-    dim3 grid(grid_for(nq, 4)), block(256);
-    const auto& L = I->lvl[1];
-#define DWG_KNNW(KK)                                                                                               \
-    hipLaunchKernelGGL(knn_wave_kernel<KK>, grid, block, 0, ctx->stream, L.G, L.cell_start, L.pts, L.empty, q, nq, \
-                       qlist, k, skip, out_idx, out_d2)
-    if (k <= 8) DWG_KNNW(8);
-    else if (k <= 10) DWG_KNNW(10);
-    else if (k <= 16) DWG_KNNW(16);
-    else if (k <= 17) DWG_KNNW(17);  // the learned start's 16-point patches with the point itself
-    else DWG_KNNW(32);
-#undef DWG_KNNW
-    check_launch();
-}
-
-// Exact search over the occupancy pyramid of the fine level, one query per
-// lane: a depth-first walk from the top block that always descends into the
-// nearest remaining child block and drops every block whose box is farther
-// than the current k-th key.  A query far from every point reaches its
-// neighbours in a few hundred short steps, where a shell search visits
-// every cell of the shells in between.  The stack holds one entry per level
-// in LDS: block coordinates and the mask of children not yet visited.
+// The occupancy pyramid of the fine level, as a walk reads it
 struct PyrArgs {
     const uint8_t* mask;
     const int4* dim;
@@ -1246,18 +1077,6 @@ __device__ __forceinline__ float tight_box_d2(const float4 lo, const float4 hi, 
     return dist2(gx, gy, gz);
 }
 
-typedef float KnnFloat4 __attribute__((ext_vector_type(4)));
-// a wave-uniform box through the scalar data cache
-__device__ __forceinline__ float tight_box_d2_uniform(const float4* box, int64_t i, float qx, float qy, float qz) {
-    const auto* b = (const __attribute__((address_space(4))) KnnFloat4*)box;
-    const KnnFloat4 lo = b[2 * i], hi = b[2 * i + 1];
-    return tight_box_d2(make_float4(lo.x, lo.y, lo.z, 0.f), make_float4(hi.x, hi.y, hi.z, 0.f), qx, qy, qz);
-}
-
-__device__ __forceinline__ uint64_t pyr_entry(int x, int y, int z, uint32_t m) {
-    return uint64_t(uint32_t(x)) | (uint64_t(uint32_t(y)) << 16) | (uint64_t(uint32_t(z)) << 32) | (uint64_t(m) << 48);
-}
-
 // squared distance from q to the box of cells [b·2^l, (b+1)·2^l) along each
 // axis, each axis gap shrunk by the rounding margin
 __device__ __forceinline__ float pyr_box_d2(const KnnGridArgs& G, float w, float margin, float qx, float qy, float qz,
@@ -1270,19 +1089,58 @@ __device__ __forceinline__ float pyr_box_d2(const KnnGridArgs& G, float w, float
     return __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
 }
 
-constexpr int kPyrThreads = 64;  // one wave per block: a block frees its slot when its slowest walk ends
+// One wave per query over the occupancy pyramid, for queries that are few or
+// whose search is long: the lanes test the 8 children of up to 8 blocks in
+// one step, and scan 64 points in one.  The k best keys lie in ascending
+// order in lanes 0 .. k − 1 of one register pair, so the wave's exact k-th
+// key bounds every step, with no list per lane to fill first, and few
+// registers leave room for many waves.  Blocks wait on a stack in LDS with
+// their box distance; until k points are known one block is opened a step,
+// its nearest child on top, then 8.  Bound by the latency of a step (a child
+// load, then a point load), so by waves in flight.
+// The stack never overflows: opening a block leaves at most 7 entries more
+// than it took, a step takes several only while that leaves kDescReserve
+// entries free, and a single depth-first descent needs no more than these.
+constexpr int kDescWaves = 4;
+constexpr int kDescStack = 320;
+constexpr int kDescReserve = 7 * kMaxPyr + 8;
+constexpr int kDescGreedy = 64;  // steps of one block at most while no k points are known
+constexpr int kDescPoints = 8;   // points a cell hands out a round
 
-template <int K>
-__global__ __launch_bounds__(kPyrThreads) void knn_pyramid_kernel(KnnGridArgs G, PyrArgs Y,
-                                                                  const int64_t* __restrict__ cell_start,
-                                                                  const float4* __restrict__ pts,
-                                                                  const float* __restrict__ q, int64_t nq,
-                                                                  const int* __restrict__ qlist, int k,
-                                                                  const uint8_t* __restrict__ skip,
-                                                                  const float* __restrict__ init_kth,
-                                                                  int32_t* __restrict__ out_idx,
-                                                                  float* __restrict__ out_d2) {
-    extern __shared__ uint64_t stk[];  // Y.levels × kPyrThreads entries
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ int dpp_or_zero(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+
+// inclusive prefix sum over the wave
+__device__ __forceinline__ int wave_scan_add(int v) {
+    v += dpp_or_zero<0x111>(v);  // row_shr 1, 2, 4, 8: within rows of 16 lanes
+    v += dpp_or_zero<0x112>(v);
+    v += dpp_or_zero<0x114>(v);
+    v += dpp_or_zero<0x118>(v);
+    v += dpp_or_zero<0x142, 0xA>(v);  // row_bcast 15: rows 1 and 3 take the row before
+    v += dpp_or_zero<0x143, 0xC>(v);  // row_bcast 31: the upper half takes lane 31
+    return v;
+}
+
+__device__ __forceinline__ uint32_t read_lane(uint32_t v, int l) {
+    return uint32_t(__builtin_amdgcn_readlane(int(v), l));
+}
+__device__ __forceinline__ uint64_t read_lane64(uint64_t v, int l) {
+    return (uint64_t(read_lane(uint32_t(v >> 32), l)) << 32) | read_lane(uint32_t(v), l);
+}
+
+// qlist (nullable) holds the queries, `count` (nullable) their number on the
+// device (else nq); init_kth[t] bounds the k-th d² of list entry t
+template <bool BOXES>
+__global__ __launch_bounds__(kDescWaves * 64) void knn_descent_kernel(
+    KnnGridArgs G, PyrArgs Y, const int64_t* __restrict__ cell_start, const float4* __restrict__ pts,
+    const float* __restrict__ q, int64_t nq, const int64_t* __restrict__ count, const int* __restrict__ qlist, int k,
+    const uint8_t* __restrict__ skip, const uint8_t* __restrict__ qmask, const float* __restrict__ init_kth,
+    int32_t* __restrict__ out_idx, float* __restrict__ out_d2) {
+    __shared__ uint64_t s_ent[kDescWaves][kDescStack];  // x | y << 16 | z << 32 | occupancy << 48 | level << 56
+    __shared__ float s_ed2[kDescWaves][kDescStack];     // box distance
+    __shared__ int s_pt[kDescWaves][64 * kDescPoints];
     __shared__ int4 s_dim[kMaxPyr];
     __shared__ int64_t s_off[kMaxPyr];
     if (threadIdx.x < Y.levels) {
@@ -1290,63 +1148,130 @@ __global__ __launch_bounds__(kPyrThreads) void knn_pyramid_kernel(KnnGridArgs G,
         s_off[threadIdx.x] = Y.off[threadIdx.x];
     }
     __syncthreads();
-    const int64_t t = int64_t(blockIdx.x) * kPyrThreads + threadIdx.x;
-    if (t >= nq) return;
-    const int64_t i = qlist ? int64_t(qlist[t]) : t;
-    const float qx = q[3 * i], qy = q[3 * i + 1], qz = q[3 * i + 2];
-    uint64_t best[K];
-    knn_reset<K>(best, k);
-    // an upper bound of the k-th d² known beforehand (k points at most that
-    // far exist): blocks beyond it are never opened.  A point at exactly the
-    // bound has a box distance ≤ it, so ties are still seen.
-    const float cap = init_kth ? init_kth[t] : INFINITY;
-    uint64_t* st = stk + threadIdx.x;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint64_t below = (1ull << lane) - 1ull;
+    uint64_t* ent = s_ent[wave];
+    float* ed2 = s_ed2[wave];
+    int* pt = s_pt[wave];
+    const int64_t n = count ? int64_t(uniform64(uint64_t(*count))) : nq;
     const int top = Y.levels - 1;
-    st[top * kPyrThreads] = pyr_entry(0, 0, 0, Y.mask[s_off[top]]);
-    int l = top;
-    while (l <= top) {
-        const uint64_t e = st[l * kPyrThreads];
-        const int bx = int(e & 0xFFFF), by = int((e >> 16) & 0xFFFF), bz = int((e >> 32) & 0xFFFF);
-        uint32_t m = uint32_t(e >> 48);
-        // the nearest child block not yet visited
-        const float w = G.cell * float(1 << (l - 1));
-        float bd = INFINITY;
-        int bc = -1;
-        for (uint32_t r = m; r; r &= r - 1) {
-            const int c = __builtin_ctz(r);
-            const float d = pyr_box_d2(G, w, Y.margin, qx, qy, qz, 2 * bx + (c & 1), 2 * by + ((c >> 1) & 1),
-                                       2 * bz + (c >> 2));
-            if (d < bd) {
-                bd = d;
-                bc = c;
+    const uint64_t root = (uint64_t(uint32_t(uniform(int(Y.mask[s_off[top]])))) << 48) | (uint64_t(uint32_t(top)) << 56);
+    for (int64_t t = int64_t(blockIdx.x) * kDescWaves + wave; t < n; t += int64_t(gridDim.x) * kDescWaves) {
+        const int64_t i = qlist ? int64_t(uniform(qlist[t])) : t;
+        if (qmask && !uniform(int(qmask[i]))) continue;
+        const float qx = q[3 * i], qy = q[3 * i + 1], qz = q[3 * i + 2];
+        const float cap = init_kth ? init_kth[t] : INFINITY;
+        uint64_t list = kNoKey, kth = kNoKey;
+        float bound = cap;
+        int sp = 1, steps = 0;
+        ent[0] = root;
+        ed2[0] = 0.f;
+        __builtin_amdgcn_wave_barrier();
+        while (sp > 0) {
+            int nb = 1;
+            if (bound < INFINITY || steps >= kDescGreedy)
+                nb = min(8, max(1, (kDescStack - kDescReserve - sp) / 7));
+            nb = min(nb, sp);
+            ++steps;
+            // lane 8g + c: child c of the g-th entry from the top
+            const int g = lane >> 3, c = lane & 7;
+            uint64_t e = 0;
+            bool on = g < nb;
+            if (on) {
+                e = ent[sp - 1 - g];
+                on = ed2[sp - 1 - g] <= bound && ((e >> (48 + c)) & 1ull);
             }
-        }
-        const float kth = best[0] == kNoKey ? cap : fminf(cap, __uint_as_float(uint32_t(best[0] >> 32)));
-        if (bc < 0 || !(bd <= kth)) {  // nothing left here can hold a closer point
-            ++l;
-            continue;
-        }
-        m &= ~(1u << bc);
-        st[l * kPyrThreads] = pyr_entry(bx, by, bz, m);
-        const int x = 2 * bx + (bc & 1), y = 2 * by + ((bc >> 1) & 1), z = 2 * bz + (bc >> 2);
-        if (l == 1) {  // a cell: its points
-            const int64_t c = x + int64_t(G.dim[0]) * (y + int64_t(G.dim[1]) * z);
-            const int64_t se = cell_start[c + 1];
-            for (int64_t s = cell_start[c]; s < se; ++s) {
-                const float4 p = pts[s];
-                const int idx = __float_as_int(p.w);
-                const float d2 = dist2(qx - p.x, qy - p.y, qz - p.z);
-                const uint64_t key = (uint64_t(__float_as_uint(d2)) << 32) | uint32_t(idx);
-                // the skip byte only for a point that would enter the list
-                if (key < best[0] && !(skip && skip[idx])) knn_insert<K>(best, key);
+            sp -= nb;
+            const int l = int(e >> 56) & 0xF;
+            const int x = 2 * int(e & 0xFFFF) + (c & 1), y = 2 * int((e >> 16) & 0xFFFF) + ((c >> 1) & 1),
+                      z = 2 * int((e >> 32) & 0xFFFF) + (c >> 2);
+            int64_t ci = 0;
+            float d = INFINITY;
+            if (on) {
+                const int4 cd = s_dim[l - 1];
+                ci = x + int64_t(cd.x) * (y + int64_t(cd.y) * z);
+                if (BOXES) {
+                    const int64_t bi = 2 * ((l == 1 ? 0 : Y.ncells + s_off[l - 1]) + ci);
+                    d = tight_box_d2(Y.box[bi], Y.box[bi + 1], qx, qy, qz);
+                } else {
+                    d = pyr_box_d2(G, G.cell * float(1 << (l - 1)), Y.margin, qx, qy, qz, x, y, z);
+                }
+                on = d <= bound;
             }
-        } else {
-            const int4 cd = s_dim[l - 1];
-            --l;
-            st[l * kPyrThreads] = pyr_entry(x, y, z, Y.mask[s_off[l] + x + int64_t(cd.x) * (y + int64_t(cd.y) * z)]);
+            const bool push = on && l > 1, cell = on && l == 1;
+            __builtin_amdgcn_wave_barrier();
+            const uint64_t pm = __builtin_amdgcn_ballot_w64(push);
+            if (pm) {
+                const int occ = push ? int(Y.mask[s_off[l - 1] + ci]) : 0;
+                int at = sp + __builtin_popcountll(pm & below);
+                sp = uniform(sp + __builtin_popcountll(pm));
+                // the nearest child of the top entry that pushes goes on top
+                // (of the wave's first 8 lanes where these push any)
+                const uint32_t db = push && g == 0 ? __float_as_uint(d) : 0xFFFFFFFFu;
+                uint32_t mn = min(db, uint32_t(dpp_or_zero<0xB1>(int(db))));     // quad_perm: lane ^ 1
+                mn = min(mn, uint32_t(dpp_or_zero<0x4E>(int(mn))));              // lane ^ 2
+                mn = min(mn, uint32_t(dpp_or_zero<0x141>(int(mn))));             // row_half_mirror: the other quad
+                const uint64_t lead = __builtin_amdgcn_ballot_w64(push && g == 0 && db == mn);
+                if (lead) {
+                    const int ll = __builtin_ctzll(lead);
+                    const int was = __builtin_amdgcn_readlane(at, ll);
+                    at = lane == ll ? sp - 1 : (at == sp - 1 ? was : at);
+                }
+                if (push) {
+                    ent[at] = uint64_t(uint32_t(x)) | (uint64_t(uint32_t(y)) << 16) | (uint64_t(uint32_t(z)) << 32) |
+                              (uint64_t(uint32_t(occ)) << 48) | (uint64_t(uint32_t(l - 1)) << 56);
+                    ed2[at] = d;
+                }
+            }
+            if (__builtin_amdgcn_ballot_w64(cell)) {
+                int64_t b = 0, be = 0;
+                if (cell) {
+                    b = cell_start[ci];
+                    be = cell_start[ci + 1];
+                }
+                // the cells' points, up to kDescPoints of each a round, laid
+                // out one after the other and scanned 64 a step
+                while (__builtin_amdgcn_ballot_w64(b < be)) {
+                    const int m = int(min(be - b, int64_t(kDescPoints)));
+                    const int incl = wave_scan_add(m);
+                    const int total = __builtin_amdgcn_readlane(incl, 63);
+                    for (int j = 0; j < m; ++j) pt[incl - m + j] = int(b + j);
+                    b += m;
+                    __builtin_amdgcn_wave_barrier();
+                    for (int cb = 0; cb < total; cb += 64) {
+                        uint64_t key = ~0ull;
+                        if (cb + lane < total) {
+                            const float4 p = pts[pt[cb + lane]];
+                            const int idx = __float_as_int(p.w);
+                            key = (uint64_t(__float_as_uint(dist2(qx - p.x, qy - p.y, qz - p.z))) << 32) | uint32_t(idx);
+                            // the skip byte only for a point that would enter the list
+                            if (key < kth && skip && skip[idx]) key = ~0ull;
+                        }
+                        for (uint64_t m2 = __builtin_amdgcn_ballot_w64(key < kth); m2; m2 &= m2 - 1) {
+                            const uint64_t c2 = read_lane64(key, __builtin_ctzll(m2));
+                            if (!(c2 < kth)) continue;
+                            // c2 enters at p: the lanes from p on take their
+                            // lower neighbour's key
+                            const int p = __builtin_popcountll(__builtin_amdgcn_ballot_w64(list < c2));
+                            const uint32_t plo = uint32_t(dpp_or_zero<0x138>(int(uint32_t(list))));  // wave_shr 1
+                            const uint32_t phi = uint32_t(dpp_or_zero<0x138>(int(uint32_t(list >> 32))));
+                            const uint64_t prev = (uint64_t(phi) << 32) | plo;
+                            list = lane == p ? c2 : (lane > p ? prev : list);
+                            list = lane < k ? list : kNoKey;
+                            kth = read_lane64(list, k - 1);
+                        }
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                }
+                if (kth != kNoKey) bound = fminf(cap, __uint_as_float(uint32_t(kth >> 32)));
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        if (lane < k) {
+            out_idx[i * k + lane] = list == kNoKey ? -1 : int32_t(uint32_t(list));
+            if (out_d2) out_d2[i * k + lane] = list == kNoKey ? INFINITY : __uint_as_float(uint32_t(list >> 32));
         }
     }
-    knn_store<K>(best, k, i, out_idx, out_d2);
 }
 
 // The same pyramid walk shared by a wave: 64 neighbouring queries (the far
@@ -1368,17 +1293,36 @@ __global__ __launch_bounds__(kPyrThreads) void knn_pyramid_kernel(KnnGridArgs G,
 // cell's points come in one vector load (64 at a time) staged in LDS.
 constexpr int kPwWaves = 2;  // small blocks free their slots sooner: the walks end at very different times
 constexpr int kPwStack = 128;  // ≥ 7 · kMaxPyr + 1 entries
+// A walk's length varies tenfold and more, and the launch lasts as long as
+// its longest walks, on an otherwise idle chip: a wave stops after this many
+// pops and hands its open queries, with the bounds they have, to a search of
+// their own (knn_descent_kernel).  Sharing pays while the waves fill the
+// chip, so the more queries, the more pops: below 32,768 queries none at all
+// (20,000 far centroids: 0.8 ms shared, 0.3 alone), at 180,000 of 3M
+// centroids 12.5 → 2.1 ms with about 350 pops, at 900,000 10 → 4.6 ms with
+// 1,024 (6.5 ms with 400)
+constexpr int64_t kShareMin = 32768;
+__device__ __forceinline__ int shared_walk_budget(int64_t nq) {
+    return nq < kShareMin ? 0 : int(min(max(nq / 512, int64_t(64)), int64_t(1024)));
+}
 
 template <int K>
 __global__ __launch_bounds__(kPwWaves * 64) void knn_pyramid_wave_kernel(KnnGridArgs G, PyrArgs Y,
                                                                         const int64_t* __restrict__ cell_start,
                                                                         const float4* __restrict__ pts,
-                                                                        const float* __restrict__ q, int64_t nq,
+                                                                        const float* __restrict__ q,
+                                                                        const int64_t* __restrict__ count,
                                                                         const int* __restrict__ qlist, int k,
                                                                         const uint8_t* __restrict__ skip,
                                                                         const float* __restrict__ init_kth,
                                                                         int32_t* __restrict__ out_idx,
-                                                                        float* __restrict__ out_d2) {
+                                                                        float* __restrict__ out_d2,
+                                                                        int* __restrict__ open_q,
+                                                                        float* __restrict__ open_kth,
+                                                                        unsigned long long* __restrict__ n_open) {
+    const int64_t nq = *count;  // launched for every query
+    if (int64_t(blockIdx.x) * kPwWaves * 64 >= nq) return;
+    const int budget = shared_walk_budget(nq);
     // stack entry: (x | y << 16, z | level << 16 | occupancy << 20, lanes lo, lanes hi)
     __shared__ int4 s_stk[kPwWaves][kPwStack];
     __shared__ float4 s_box[kPwWaves][16];    // box of child c: lo at 2c, hi at 2c + 1
@@ -1420,7 +1364,7 @@ __global__ __launch_bounds__(kPwWaves * 64) void knn_pyramid_wave_kernel(KnnGrid
     stk[0] = make_int4(0, (top << 16) | (occ_top << 20), int(uint32_t(all)), int(uint32_t(all >> 32)));
     __builtin_amdgcn_wave_barrier();
     int sp = 1;
-    while (sp > 0) {
+    for (int pops = 0; sp > 0 && pops < budget; ++pops) {
         --sp;
         const int4 e = stk[sp];
         const uint32_t e0 = uint32_t(uniform(e.x)), e1 = uint32_t(uniform(e.y));
@@ -1528,97 +1472,130 @@ __global__ __launch_bounds__(kPwWaves * 64) void knn_pyramid_wave_kernel(KnnGrid
         }
         __builtin_amdgcn_wave_barrier();
     }
-    if (valid) knn_store<K>(best, k, i, out_idx, out_d2);
+    // out of pops: the lanes that blocks on the stack still wait for are
+    // listed with the bound they have, for a search of their own
+    uint64_t open = 0;
+    for (int j = 0; j < sp; ++j)
+        open |= (uint64_t(uint32_t(uniform(stk[j].w))) << 32) | uint32_t(uniform(stk[j].z));
+    if (open) {
+        unsigned int base = 0;
+        if (lane == 0) base = (unsigned int)(atomicAdd(n_open, (unsigned long long)__builtin_popcountll(open)));
+        base = uint32_t(uniform(int(base)));
+        if ((open >> lane) & 1ull) {
+            const unsigned int slot = base + unsigned(__builtin_popcountll(open & ((1ull << lane) - 1ull)));
+            open_q[slot] = int(i);
+            open_kth[slot] = kth_of();
+        }
+    }
+    if (valid && !((open >> lane) & 1ull)) knn_store<K>(best, k, i, out_idx, out_d2);
 }
 
-// far queries: the pyramid walk when there are enough of them to fill the
-// lanes, else (or without a pyramid) one wave per query on the coarse level
-constexpr int64_t kPyrMinQueries = 2048;
-// below this many queries (and fewer than one per 8 indexed points) a query
-// set skips the tiled passes for the pyramid walk
-constexpr int64_t kSparseMaxQueries = 65536;
+// Query sets answered by one search per query from the start: below
+// kDescAlways the tiles' bucketing costs more than it saves also for queries
+// on the surface (10,000 queries over as many points: 137 → 67 µs); up to
+// kDescFew where they are fewer than the points, as then few share a tile
+// (20,000 over 30,000: 286 → 198 µs; at 90,000 self queries the tiles win,
+// 190 against 328 µs); up to kDescSparse where they are under one per 8
+// points (30,000 over 1M: 3.3 ms by coarse-cell shells, 1.2 ms)
+constexpr int64_t kDescAlways = 16384, kDescFew = 32768, kDescSparse = 65536;
 
-static void launch_far(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const int* qlist, int k,
-                       const uint8_t* skip, int32_t* out_idx, float* out_d2, const float* init_kth = nullptr,
-                       bool shared = false, const uint8_t* pyr_mask = nullptr) {
-    if (nq == 0) return;
+static PyrArgs pyr_args(const dwg_knn_index::Level& L, const uint8_t* mask) {
+    return PyrArgs{mask ? mask : L.pyr, L.pyr_dim, L.pyr_off, L.pyr_levels, L.pyr_margin, L.pbox, L.ncells};
+}
+
+// nq queries (of which *count, when given), one wave each
+static void launch_wave(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const int64_t* count,
+                        const int* qlist, int k, const uint8_t* skip, const uint8_t* qmask, int32_t* out_idx,
+                        float* out_d2) {
+    dim3 grid(grid_for(nq, 4)), block(256);
+    const auto& L = I->lvl[1];
+#define DWG_KNNW(KK)                                                                                               \
+    hipLaunchKernelGGL(knn_wave_kernel<KK>, grid, block, 0, ctx->stream, L.G, L.cell_start, L.pts, L.empty, q, nq, \
+                       count, qlist, k, skip, qmask, out_idx, out_d2)
+    if (k <= 10) DWG_KNNW(10);
+    else if (k <= 17) DWG_KNNW(17);
+    else DWG_KNNW(32);
+#undef DWG_KNNW
+    check_launch();
+}
+
+static void launch_descent(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const int64_t* count,
+                           const int* qlist, int k, const uint8_t* skip, const uint8_t* qmask, const float* init_kth,
+                           int32_t* out_idx, float* out_d2, const uint8_t* pyr_mask = nullptr) {
     const auto& L = I->lvl[0];
-    if (L.pyr_levels < 2 || nq < kPyrMinQueries) {
-        launch_wave(ctx, I, q, nq, qlist, k, skip, out_idx, out_d2);
+    if (L.pyr_levels < 2) {
+        launch_wave(ctx, I, q, nq, count, qlist, k, skip, qmask, out_idx, out_d2);
+        return;
+    }
+    const PyrArgs Y = pyr_args(L, pyr_mask);
+    // enough blocks to fill the chip; the waves take further queries in turn
+    dim3 grid(unsigned(std::min<int64_t>(grid_for(nq, kDescWaves), 4096))), block(kDescWaves * 64);
+    if (L.pbox)
+        hipLaunchKernelGGL(knn_descent_kernel<true>, grid, block, 0, ctx->stream, L.G, Y, L.cell_start, L.pts, q, nq,
+                           count, qlist, k, skip, qmask, init_kth, out_idx, out_d2);
+    else
+        hipLaunchKernelGGL(knn_descent_kernel<false>, grid, block, 0, ctx->stream, L.G, Y, L.cell_start, L.pts, q, nq,
+                           count, qlist, k, skip, qmask, init_kth, out_idx, out_d2);
+    check_launch();
+}
+
+// the queries qlist[0..*count) that the tiled pass left open (of nq) with
+// their bounds; `shared`: 64 neighbours share a walk first
+static void launch_far(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const int64_t* count,
+                       const int* qlist, int k, const uint8_t* skip, int32_t* out_idx, float* out_d2,
+                       const float* init_kth, bool shared, const uint8_t* pyr_mask) {
+    const auto& L = I->lvl[0];
+    // an index without boxes (its first such query) builds them, a dozen
+    // launches, only if there are enough far queries to share a walk
+    if (shared && L.pyr_levels >= 2 && !L.pbox && read_scalar<int64_t>(ctx, count) < kShareMin) shared = false;
+    if (!shared || L.pyr_levels < 2) {
+        launch_descent(ctx, I, q, nq, count, qlist, k, skip, nullptr, init_kth, out_idx, out_d2, pyr_mask);
         return;
     }
     // the boxes are a cache of the index's own points: building them
     // leaves the index unchanged
-    if (shared) ensure_boxes(ctx, const_cast<dwg_knn_index::Level&>(L));
-    const PyrArgs Y{pyr_mask ? pyr_mask : L.pyr, L.pyr_dim, L.pyr_off, L.pyr_levels, L.pyr_margin, L.pbox, L.ncells};
-    if (shared) {
-        DWG_REQUIRE(L.pyr_levels <= kMaxPyr && 7 * L.pyr_levels + 1 <= kPwStack, "pyramid deeper than the wave stack");
-        dim3 grid(grid_for(nq, kPwWaves * 64)), block(kPwWaves * 64);
-#define DWG_KNNPW(KK)                                                                                              \
-    hipLaunchKernelGGL(knn_pyramid_wave_kernel<KK>, grid, block, 0, ctx->stream, L.G, Y, L.cell_start, L.pts, q, nq, \
-                       qlist, k, skip, init_kth, out_idx, out_d2)
-        if (k <= 8) DWG_KNNPW(8);
-        else if (k <= 10) DWG_KNNPW(10);
-        else if (k == 15) DWG_KNNPW(15);  // the diffusion's 15 neighbours: no spare slot to sink through
-        else if (k <= 16) DWG_KNNPW(16);
-        else if (k <= 17) DWG_KNNPW(17);  // the learned start's 16-point patches with the point itself
-        else DWG_KNNPW(32);
+    ensure_boxes(ctx, const_cast<dwg_knn_index::Level&>(L));
+    const PyrArgs Y = pyr_args(L, pyr_mask);
+    DWG_REQUIRE(L.pyr_levels <= kMaxPyr && 7 * L.pyr_levels + 1 <= kPwStack, "pyramid deeper than the wave stack");
+    int* open_q = static_cast<int*>(ctx->buf("knn_open_q", sizeof(int) * nq));
+    float* open_kth = static_cast<float*>(ctx->buf("knn_open_kth", sizeof(float) * nq));
+    auto* n_open = static_cast<unsigned long long*>(ctx->buf("knn_n_open", 64));
+    fill_u32(ctx, n_open, 0, 2);
+    dim3 grid(grid_for(nq, kPwWaves * 64)), block(kPwWaves * 64);
+#define DWG_KNNPW(KK)                                                                                           \
+    hipLaunchKernelGGL(knn_pyramid_wave_kernel<KK>, grid, block, 0, ctx->stream, L.G, Y, L.cell_start, L.pts, q, \
+                       count, qlist, k, skip, init_kth, out_idx, out_d2, open_q, open_kth, n_open)
+    if (k <= 8) DWG_KNNPW(8);
+    else if (k <= 10) DWG_KNNPW(10);
+    else if (k == 15) DWG_KNNPW(15);  // the diffusion's 15 neighbours: no spare slot to sink through
+    else if (k <= 16) DWG_KNNPW(16);
+    else if (k <= 17) DWG_KNNPW(17);  // the learned start's 16-point patches with the point itself
+    else DWG_KNNPW(32);
 #undef DWG_KNNPW
-        check_launch();
-        return;
-    }
-    dim3 grid(grid_for(nq, kPyrThreads)), block(kPyrThreads);
-    const size_t lds = sizeof(uint64_t) * size_t(L.pyr_levels) * kPyrThreads;
-#define DWG_KNNP(KK)                                                                                             \
-    hipLaunchKernelGGL(knn_pyramid_kernel<KK>, grid, block, lds, ctx->stream, L.G, Y, L.cell_start, L.pts, q, nq, \
-                       qlist, k, skip, init_kth, out_idx, out_d2)
-    if (k <= 8) DWG_KNNP(8);
-    else if (k <= 10) DWG_KNNP(10);
-    else if (k <= 16) DWG_KNNP(16);
-    else if (k <= 17) DWG_KNNP(17);  // the learned start's 16-point patches with the point itself
-    else DWG_KNNP(32);
-#undef DWG_KNNP
     check_launch();
+    launch_descent(ctx, I, q, nq, reinterpret_cast<const int64_t*>(n_open), open_q, k, skip, nullptr, open_kth, out_idx,
+                   out_d2, pyr_mask);
 }
 
-static void launch_per_lane(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const int* qlist, int k,
-                            const uint8_t* skip, const uint8_t* qmask, int32_t* out_idx, float* out_d2) {
-    if (nq == 0) return;
-    dim3 grid(grid_for(nq, 256)), block(256);
-#define DWG_KNN(KK)                                                                                                  \
-    hipLaunchKernelGGL(knn_query_kernel<KK>, grid, block, 0, ctx->stream, I->lvl[0].G, I->lvl[0].cell_start,        \
-                       I->lvl[0].pts, I->lvl[1].G, I->lvl[1].cell_start, I->lvl[1].pts, I->lvl[1].empty, q, nq, qlist, \
-                       k, skip, qmask,                                                                            \
-                       out_idx, out_d2)
-    if (k <= 8) DWG_KNN(8);
-    else if (k <= 10) DWG_KNN(10);
-    else if (k <= 16) DWG_KNN(16);
-    else if (k <= 17) DWG_KNN(17);  // the learned start's 16-point patches with the point itself
-    else DWG_KNN(32);
-#undef DWG_KNN
-    check_launch();
-}
-
-// The queries qlist[0..nq) (or 0..nq−1, masked by qmask) bucketed by tile
-// of kTile³ fine cells (and by eighth of it when sub is 8): order[start[sub·t]
-// ..start[sub·(t+1))) are tile t's queries, list[0..nlist) the tiles that
-// have any
+// The queries 0..nq−1 (masked by qmask) bucketed by tile of kTile³ fine cells
+// and eighth of it: order[start[sub·t]..start[sub·(t+1))) are tile t's
+// queries, list[0..*nlist) the tiles that have any
 struct TileBuckets {
     TileArgs T;
-    int64_t ntiles = 0, nlist = 0;
+    int64_t ntiles = 0;
+    int64_t* nlist = nullptr;
     int64_t* start = nullptr;
     int* order = nullptr;
     int* list = nullptr;
 };
 
-static TileBuckets tile_buckets(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const int* qlist,
-                                const uint8_t* qmask, int sub, bool want_list = true) {
+static TileBuckets tile_buckets(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq,
+                                const uint8_t* qmask) {
     const KnnGridArgs& G = I->lvl[0].G;
     TileBuckets B;
+    constexpr int sub = kSubTiled;
     TileArgs& T = B.T;
     for (int d = 0; d < 3; ++d) T.tdim[d] = (G.dim[d] + kTile - 1) / kTile;
-    T.margin = cell_margin(G);
-    T.sub = sub;
     const int64_t ntiles = int64_t(T.tdim[0]) * T.tdim[1] * T.tdim[2], nb = ntiles * sub;
     DWG_REQUIRE(nb < (int64_t(1) << 31), "too many query buckets");
     B.ntiles = ntiles;
@@ -1629,29 +1606,24 @@ static TileBuckets tile_buckets(dwg_ctx* ctx, const dwg_knn_index* I, const floa
     int64_t* flags = static_cast<int64_t*>(ctx->buf("knnt_flags", sizeof(int64_t) * (ntiles + 1)));
     int* list = static_cast<int*>(ctx->buf("knnt_list", sizeof(int) * ntiles));
     fill_u32(ctx, start, 0, 2 * (nb + 1));
-    hipLaunchKernelGGL(tile_count_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, q, nq, qlist, qmask, G, T,
+    hipLaunchKernelGGL(tile_count_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, q, nq, qmask, G, T,
                        tile_of, reinterpret_cast<unsigned long long*>(start));
     check_launch();
     exclusive_scan<int64_t>(ctx, start, nb);
     hipLaunchKernelGGL(copy_i64_kernel, dim3(grid_for(nb, 256)), dim3(256), 0, ctx->stream, start, cursor, nb);
     check_launch();
-    hipLaunchKernelGGL(tile_scatter_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, tile_of, nq, qlist,
-                       cursor, order);
+    hipLaunchKernelGGL(tile_scatter_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, tile_of, nq, cursor,
+                       order);
     check_launch();
     B.start = start;
     B.order = order;
-    if (!want_list) {  // the caller takes the queries in tile order only: no list, no host read
-        B.nlist = 0;
-        B.list = nullptr;
-        return B;
-    }
     hipLaunchKernelGGL(tile_flags_kernel, dim3(grid_for(ntiles + 1, 256)), dim3(256), 0, ctx->stream, start, ntiles,
-                       sub, flags);
+                       flags);
     check_launch();
     exclusive_scan<int64_t>(ctx, flags, ntiles);
     hipLaunchKernelGGL(tile_list_kernel, dim3(grid_for(ntiles, 256)), dim3(256), 0, ctx->stream, flags, ntiles, list);
     check_launch();
-    B.nlist = read_scalar<int64_t>(ctx, flags + ntiles);
+    B.nlist = flags + ntiles;
     B.list = list;
     return B;
 }
@@ -1663,54 +1635,48 @@ __global__ void redo_compact_kernel(const int64_t* __restrict__ pos, const int* 
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (t >= n || pos[t + 1] == pos[t]) return;
     redo[pos[t]] = tmp_q[t];
-    if (redo_kth) redo_kth[pos[t]] = tmp_kth[t];
+    redo_kth[pos[t]] = tmp_kth[t];
 }
 
-// One tiled pass over the queries qlist[0..nq) (or 0..nq−1, masked by
-// qmask); the queries it cannot close are listed in redo (with their k-th
-// bound in redo_kth), in tile order when `ordered`, else in the order the
-// waves end.  Returns their count.
-template <int HALO>
-static int64_t tiled_pass(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const int* qlist,
-                          const uint8_t* qmask, int k, const uint8_t* skip, int32_t* out_idx, float* out_d2,
-                          int* redo, const std::string& name, const KnnScatter* sc = nullptr,
-                          float* redo_kth = nullptr, bool ordered = false) {
+// up to this many tile blocks are launched without reading how many have
+// queries: the surplus blocks return at once, for less than the read costs
+constexpr int64_t kTileBlind = 16384;
+
+// The tiled pass over the queries 0..nq−1 (masked by qmask); the queries it
+// cannot close are listed in redo with their k-th bound in redo_kth, in tile
+// order.  Returns the device address of their count.
+static const int64_t* tiled_pass(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const uint8_t* qmask,
+                                 int k, const uint8_t* skip, int32_t* out_idx, float* out_d2, int* redo,
+                                 float* redo_kth, const std::string& name, const KnnScatter* sc) {
     const KnnGridArgs& G = I->lvl[0].G;
-    const TileBuckets B = tile_buckets(ctx, I, q, nq, qlist, qmask, kSubTiled);
+    const TileBuckets B = tile_buckets(ctx, I, q, nq, qmask);
     const TileArgs& T = B.T;
-    const int64_t ntiles = B.ntiles, nlist = B.nlist;
-    const int64_t* start = B.start;
-    const int* order = B.order;
-    const int* list = B.list;
-    unsigned int* n_redo = static_cast<unsigned int*>(ctx->buf("knnt_nredo", 64));
-    fill_u32(ctx, n_redo, 0, 1);
-    if (ctx->profile) ctx->count(name + ":queries", read_scalar<int64_t>(ctx, start + ntiles * T.sub));
-    // ordered: each query's place t in tile order gets its flag (and, when
-    // open, its index and bound) in scratch arrays, compacted below
-    int64_t* rflag = nullptr;
-    int* tmp_q = nullptr;
-    float* tmp_kth = nullptr;
-    if (ordered) {
-        rflag = static_cast<int64_t*>(ctx->buf("knnt_rflag", sizeof(int64_t) * (nq + 1)));
-        tmp_q = static_cast<int*>(ctx->buf("knnt_rtmp", sizeof(int) * nq + 64));
-        if (redo_kth) tmp_kth = static_cast<float*>(ctx->buf("knnt_rkth", sizeof(float) * nq + 64));
-        fill_u32(ctx, rflag, 0, 2 * (nq + 1));
+    if (ctx->profile) ctx->count(name + ":queries", read_scalar<int64_t>(ctx, B.start + B.ntiles * kSubTiled));
+    // each query's place t in tile order gets its flag (and, when open, its
+    // index and bound) in scratch arrays, compacted below
+    int64_t* rflag = static_cast<int64_t*>(ctx->buf("knnt_rflag", sizeof(int64_t) * (nq + 1)));
+    int* tmp_q = static_cast<int*>(ctx->buf("knnt_rtmp", sizeof(int) * nq + 64));
+    float* tmp_kth = static_cast<float*>(ctx->buf("knnt_rkth", sizeof(float) * nq + 64));
+    fill_u32(ctx, rflag, 0, 2 * (nq + 1));
+    int64_t blocks = std::min(B.ntiles, nq);
+    const int64_t* exact = B.nlist;
+    if (blocks > kTileBlind) {
+        blocks = read_scalar<int64_t>(ctx, B.nlist);
+        exact = nullptr;
     }
-    int* redo_out = ordered ? tmp_q : redo;
-    float* kth_out = ordered ? tmp_kth : redo_kth;
-    if (nlist > 0) {
+    if (blocks > 0) {
         ProfileScope pt(ctx, name.c_str());
         const KnnScatter scv = sc ? *sc : KnnScatter{nullptr, nullptr};
-#define DWG_KNNT(KK)                                                                                                   \
-    do {                                                                                                               \
-        if (sc)                                                                                                        \
-            hipLaunchKernelGGL((knn_tile_kernel<KK, HALO, true>), dim3(unsigned(nlist)), dim3(kTileThreads), 0,        \
-                               ctx->stream, G, T, I->lvl[0].cell_start, I->lvl[0].pts, list, start, order, q, k, skip, \
-                               out_idx, out_d2, redo_out, kth_out, n_redo, rflag, scv);                                \
-        else                                                                                                           \
-            hipLaunchKernelGGL((knn_tile_kernel<KK, HALO, false>), dim3(unsigned(nlist)), dim3(kTileThreads), 0,       \
-                               ctx->stream, G, T, I->lvl[0].cell_start, I->lvl[0].pts, list, start, order, q, k, skip, \
-                               out_idx, out_d2, redo_out, kth_out, n_redo, rflag, scv);                                \
+#define DWG_KNNT(KK)                                                                                                \
+    do {                                                                                                            \
+        if (sc)                                                                                                     \
+            hipLaunchKernelGGL((knn_tile_kernel<KK, true>), dim3(unsigned(blocks)), dim3(kTileThreads), 0,          \
+                               ctx->stream, G, T, I->lvl[0].cell_start, I->lvl[0].pts, B.list, B.start, B.order, q, \
+                               k, skip, out_idx, out_d2, tmp_q, tmp_kth, rflag, exact, scv);                        \
+        else                                                                                                        \
+            hipLaunchKernelGGL((knn_tile_kernel<KK, false>), dim3(unsigned(blocks)), dim3(kTileThreads), 0,         \
+                               ctx->stream, G, T, I->lvl[0].cell_start, I->lvl[0].pts, B.list, B.start, B.order, q, \
+                               k, skip, out_idx, out_d2, tmp_q, tmp_kth, rflag, exact, scv);                        \
     } while (0)
         if (k <= 8) DWG_KNNT(8);
         else if (k <= 10) DWG_KNNT(10);
@@ -1721,18 +1687,11 @@ static int64_t tiled_pass(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, 
 #undef DWG_KNNT
         check_launch();
     }
-    int64_t nredo;
-    if (ordered) {
-        exclusive_scan<int64_t>(ctx, rflag, nq);
-        hipLaunchKernelGGL(redo_compact_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, rflag, tmp_q,
-                           tmp_kth, nq, redo, redo_kth);
-        check_launch();
-        nredo = read_scalar<int64_t>(ctx, rflag + nq);
-    } else {
-        nredo = int64_t(read_scalar<unsigned int>(ctx, n_redo));
-    }
-    ctx->count(name + ":redo", nredo);
-    return nredo;
+    exclusive_scan<int64_t>(ctx, rflag, nq);
+    hipLaunchKernelGGL(redo_compact_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, rflag, tmp_q, tmp_kth, nq,
+                       redo, redo_kth);
+    check_launch();
+    return rflag + nq;
 }
 
 void knn_query(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, int k, const uint8_t* skip,
@@ -1745,81 +1704,41 @@ void knn_query(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq,
     if (nq == 0) return;
     ProfileScope ps(ctx, tag ? tag : "knn_query");
     const std::string base = tag ? tag : "knn_query";
-    if (nq < 4096) {  // too few to pay for the bucketing
-        launch_per_lane(ctx, I, q, nq, nullptr, k, skip, qmask, out_idx, out_d2);
+    const bool sparse = nq * 8 < I->n;
+    if (nq < kDescAlways || (nq < kDescFew && nq < I->n) || (nq < kDescSparse && sparse)) {
+        ctx->count(base + (sparse ? ":sparse" : ":tiles3:redo"), nq);
+        launch_descent(ctx, I, q, nq, nullptr, nullptr, k, skip, qmask, nullptr, out_idx, out_d2);
         if (sc) {
             hipLaunchKernelGGL(scatter_pairs_kernel, dim3(grid_for(nq * k, 256)), dim3(256), 0, ctx->stream, out_idx, k,
-                               nullptr, nq, *sc);
+                               nq, *sc);
             check_launch();
         }
         return;
     }
-    if (!qmask && nq < kSparseMaxQueries && nq * 8 < I->n && I->lvl[0].pyr_levels >= 2) {
-        // a few tens of thousands of queries spread thin over a large index
-        // (the zero fill's) leave the tiles nearly empty, so staging a tile's
-        // points serves one or two queries: a search per query costs less
-        // (1.2 vs 2.1 ms for 35k queries over 950k points).  One wave per
-        // query, its 64 lanes scanning the points of the coarse grid's
-        // shells, beats one query per lane walking the occupancy pyramid
-        // (0.63 vs 0.79 ms for the zero fill's ~30k queries, skipped points
-        // included): the per-lane walks are few and long, the wave searches
-        // many and short
-        ctx->count(base + ":sparse", nq);
-        // the queries in tile order: neighbouring waves read the same cells
-        const TileBuckets B = tile_buckets(ctx, I, q, nq, nullptr, nullptr, 1, false);
-        launch_wave(ctx, I, q, nq, B.order, k, skip, out_idx, out_d2);
-        if (sc) {
-            hipLaunchKernelGGL(scatter_pairs_kernel, dim3(grid_for(nq * k, 256)), dim3(256), 0, ctx->stream, out_idx, k,
-                               nullptr, nq, *sc);
-            check_launch();
-        }
-        return;
-    }
-    int* redo3 = static_cast<int*>(ctx->buf("knnt_redo3", sizeof(int) * nq + 64));
-    float* kth3 = static_cast<float*>(ctx->buf("knnt_kth3", sizeof(float) * nq + 64));
+    int* redo = static_cast<int*>(ctx->buf("knnt_redo", sizeof(int) * nq + 64));
+    float* kth = static_cast<float*>(ctx->buf("knnt_kth", sizeof(float) * nq + 64));
     // at least as many queries as indexed points (triangle centroids): the
     // far ones come in dense patches (spurious surface pieces) and in tile
     // order, so a wave's 64 share most of their search and take the
-    // wave-shared walk (6.4 vs 7.2 ms per centroid query at 1M points);
-    // sparser far queries are spread apart and walk per lane
+    // wave-shared walk; sparser far queries are spread apart and search alone
     const bool shared = nq >= I->n;
-    int64_t n3 = 0;
-    if (shared) {
-        // the queries the first pass leaves open go straight to the shared
-        // walk: its time is set by its longest walks (far queries deep
-        // inside large closed pieces), not by how many queries it gets, so
-        // wider tiled passes before it cost more than they save (4.41
-        // instead of 5.20 ms per centroid query at 1M points)
-        n3 = tiled_pass<kHalo1>(ctx, I, q, nq, nullptr, qmask, k, skip, out_idx, out_d2, redo3, base + ":tiles", sc,
-                                kth3, true);
-    } else {
-        int* redo1 = static_cast<int*>(ctx->buf("knnt_redo1", sizeof(int) * nq + 64));
-        int* redo2 = static_cast<int*>(ctx->buf("knnt_redo2", sizeof(int) * nq + 64));
-        const int64_t n1 = tiled_pass<kHalo1>(ctx, I, q, nq, nullptr, qmask, k, skip, out_idx, out_d2, redo1,
-                                              base + ":tiles", sc);
-        // every tiled pass scatters the queries it closes (summed per tile
-        // in LDS first); the far queries scatter after the last search
-        const int64_t n2 = n1 > 0 ? tiled_pass<kHalo2>(ctx, I, q, n1, redo1, nullptr, k, skip, out_idx, out_d2,
-                                                       redo2, base + ":tiles2", sc)
-                                  : 0;
-        n3 = n2 > 0 ? tiled_pass<kHalo3>(ctx, I, q, n2, redo2, nullptr, k, skip, out_idx, out_d2, redo3,
-                                         base + ":tiles3", sc, kth3, true)
-                    : 0;
+    const int64_t* nfar = tiled_pass(ctx, I, q, nq, qmask, k, skip, out_idx, out_d2, redo, kth, base + ":tiles", sc);
+    if (ctx->profile) {  // the queries that no tiled pass closes
+        const int64_t n = read_scalar<int64_t>(ctx, nfar);
+        ctx->count(base + ":tiles:redo", n);
+        ctx->count(base + (shared ? ":far_shared" : ":tiles3:redo"), n);
     }
     {
         const std::string name = base + ":redo";
         ProfileScope pr(ctx, name.c_str());
-        if (shared) ctx->count(base + ":far_shared", n3);
-        const uint8_t* pm = (skip && n3 >= kPyrMinQueries && I->lvl[0].pyr_levels >= 2)
-                                ? masked_pyramid(ctx, I->lvl[0], skip)
-                                : nullptr;
-        launch_far(ctx, I, q, n3, redo3, k, skip, out_idx, out_d2, kth3, shared, pm);
+        const uint8_t* pm = (skip && I->lvl[0].pyr_levels >= 2) ? masked_pyramid(ctx, I->lvl[0], skip) : nullptr;
+        launch_far(ctx, I, q, nq, nfar, redo, k, skip, out_idx, out_d2, kth, shared, pm);
     }
-    if (sc && n3 > 0) {
+    if (sc) {
         const std::string name = base + ":scatter";
         ProfileScope pr(ctx, name.c_str());
-        hipLaunchKernelGGL(scatter_pairs_hashed_kernel, dim3(grid_for(n3, 256)), dim3(256), 0, ctx->stream, out_idx,
-                           k, redo3, n3, *sc);
+        hipLaunchKernelGGL(scatter_pairs_hashed_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, out_idx, k,
+                           redo, nfar, *sc);
         check_launch();
     }
 }

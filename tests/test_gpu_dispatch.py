@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+import oracle as O
 from dwg_amd import gpu, shapes
 
 pytestmark = pytest.mark.gpu
@@ -87,3 +88,44 @@ def test_grid_walk_equals_the_point_walk(ctx, res, h, shift, screened, bf16, rad
     got = tree.eval_grid(grid, 2.3, **kw).cpu().numpy()
     want = tree.eval(Q, 2.3, **kw).cpu().numpy()
     np.testing.assert_array_equal(got, want)
+
+
+# (points, queries): fewer points than k, one query, one cell's worth, a
+# query set at each end of the sizes searched one query at a time and of the
+# tiled ones (dense and not)
+@pytest.mark.parametrize("n,nq,k", [(1, 3, 4), (5, 1, 10), (40, 64, 32), (3000, 1, 1), (3000, 257, 32),
+                                    (20_000, 16_383, 15), (2500, 16_384, 15), (33_000, 32_767, 8),
+                                    (33_000, 32_768, 10), (2000, 40_000, 17)])
+@pytest.mark.parametrize("skipped", [0.0, 0.5, 0.999])
+def test_knn_by_query_count(ctx, n, nq, k, skipped):
+    rng = np.random.default_rng(n + nq)
+    P, _ = shapes.sphere(n, 3)
+    P = (P + rng.normal(0, 0.002, P.shape)).astype(np.float32)
+    P[: n // 8] = P[0]  # one cell holds an eighth of the points, all at one place
+    Q = np.concatenate([P[rng.integers(0, n, nq - nq // 2)] + rng.normal(0, 0.01, (nq - nq // 2, 3)),
+                        rng.uniform(-1.6, 1.6, (nq // 2, 3))]).astype(np.float32)
+    skip = (rng.uniform(size=n) < skipped).astype(np.uint8)
+    skip[-1] = 0
+    idx = gpu.KnnIndex(ctx, P, k_hint=k)
+    got, d2 = idx.query(Q, k, d2=True, skip=torch.from_numpy(skip) if skipped else None)
+    sub = rng.permutation(nq)[:3000]  # the reference is brute force
+    ref, rd2 = O.knn_brute(P, Q[sub], k, skip=skip if skipped else None, return_d2=True)
+    np.testing.assert_array_equal(got.cpu().numpy()[sub], ref)
+    # the oracle gives no distance where there is no neighbour, the library ∞
+    np.testing.assert_array_equal(d2.cpu().numpy()[sub], np.where(ref < 0, np.inf, rd2))
+
+
+def test_knn_far_walk_hands_over(ctx):
+    # 60,000 far queries near the centre of a sphere of 30,000 points: every
+    # point is about as near as any other, so the shared walks run out of pops
+    # and their queries search alone
+    rng = np.random.default_rng(5)
+    P, _ = shapes.sphere(30_000, 4)
+    P = (0.5 * P + rng.normal(0, 1e-4, P.shape)).astype(np.float32)
+    Q = rng.normal(0, 0.02, (60_000, 3)).astype(np.float32)
+    idx = gpu.KnnIndex(ctx, P, k_hint=15)
+    got, d2 = idx.query(Q, 15, d2=True)
+    sub = rng.permutation(len(Q))[:3000]
+    ref, rd2 = O.knn_brute(P, Q[sub], 15, return_d2=True)
+    np.testing.assert_array_equal(got.cpu().numpy()[sub], ref)
+    np.testing.assert_array_equal(d2.cpu().numpy()[sub], rd2)
