@@ -169,6 +169,29 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
     return (uint64_t(hi) << 32) | lo;
 }
 
+// Points and queries often arrive in runs that share a cell or bucket (sources
+// in tree order, triangle centroids in brick order): each wave adds one run
+// with one atomic.  A run starts at lane 0 and wherever the key changes; its
+// first lane (the head) reserves the run's slots, the others take theirs
+// from the head in lane order.
+__device__ __forceinline__ uint64_t run_starts(int tl) {
+    const int lane = threadIdx.x & 63;
+    const int prev = __shfl_up(tl, 1, 64);
+    return __ballot(lane == 0 || tl != prev);
+}
+
+// lanes from `lane` up to the next run start (or the end of the wave)
+__device__ __forceinline__ int run_length(uint64_t starts, int lane) {
+    const uint64_t after = lane == 63 ? 0ull : starts >> (lane + 1);
+    return after ? __builtin_ctzll(after) + 1 : 64 - lane;
+}
+
+// the run start at or before `lane`
+__device__ __forceinline__ int run_head(uint64_t starts, int lane) {
+    const uint64_t upto = lane == 63 ? starts : starts & ((2ull << lane) - 1ull);
+    return 63 - __builtin_clzll(upto);
+}
+
 __device__ __forceinline__ void kahan_add(float& sum, float& comp, float x) {
     float y = x - comp;
     float t = sum + y;

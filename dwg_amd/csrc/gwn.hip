@@ -611,7 +611,7 @@ constexpr int kMaxTreeLevel = 21;
 // stack entries a walk of a tree of max_level levels needs at most: 7 left
 // over per level and the 8 children of the deepest node opened
 __host__ __device__ constexpr int tree_stack_entries(int max_level) { return 7 * max_level + 8; }
-constexpr int kStack = tree_stack_entries(kMaxTreeLevel);  // the gradient walk's fixed stack
+constexpr int kStack = tree_stack_entries(kMaxTreeLevel);  // the shared gradient walk's fixed stack
 // grid walks: each lane evaluates kGridParts points, one in each 4×4×4 part
 // of a brick of kPartsX × kPartsY × kPartsZ parts (parts that differ in z
 // share a child's x and y products)
@@ -658,8 +658,20 @@ __device__ __forceinline__ float bf16_round(float f) {
     return __uint_as_float(u & 0xFFFF0000u);
 }
 
+// The order in which explicit queries share walks: order[slot] where the
+// sampled extent of their runs (query_order) is over `limit`, else the
+// caller's own
+struct QueryOrder {
+    const int* order;
+    const unsigned int* extent;  // nullptr: the caller's order
+    unsigned int limit;
+    __device__ __forceinline__ bool sorted() const { return extent && *extent > limit; }
+    __device__ __forceinline__ int64_t query(int64_t slot) const { return sorted() ? int64_t(order[slot]) : slot; }
+};
+
 struct QueryArgs {
     const float* q;          // explicit points
+    QueryOrder order;        // and their order
     const int* self_perm;    // the tree's own points in tree order, results to out[perm[slot]]
     bool grid;               // implicit grid (q and self_perm unused)
     int64_t nq;
@@ -706,6 +718,7 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
                 qz[h] = a.z;
                 qi[h] = valid[h] ? int64_t(Q.self_perm[qi[h]]) : 0;
             } else {
+                if (valid[h]) qi[h] = Q.order.query(qi[h]);
                 qx[h] = valid[h] ? Q.q[3 * qi[h]] : 0.f;
                 qy[h] = valid[h] ? Q.q[3 * qi[h] + 1] : 0.f;
                 qz[h] = valid[h] ? Q.q[3 * qi[h] + 2] : 0.f;
@@ -765,8 +778,15 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
         if (BF16) return __builtin_fmaf((on && ok) ? x : 0.f, inv, part);  // last product fused into the sum
         return part + ((on && ok) ? x * inv : 0.f);
     };
-    auto add = [&](float part, int h) {
-        if (kahan) kahan_add(sum[h], comp[h], part); else sum[h] += part;
+    // (one part: only the lanes that opened the node, as adding a zero would
+    // move bits between the sum and its compensation, and an explicit query's
+    // value must not depend on the queries it shares the wave with)
+    auto add = [&](float part, int h, uint64_t m) {
+        if (!kahan) {
+            sum[h] += part;
+        } else if (H > 1 || __builtin_amdgcn_inverse_ballot_w64(m)) {
+            kahan_add(sum[h], comp[h], part);
+        }
     };
     // a leaf of several points, summed point by point for the parts whose
     // lanes opened it
@@ -783,7 +803,7 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
 #pragma unroll
         for (int h = 0; h < H; ++h) {
             if (COUNT && __builtin_amdgcn_inverse_ballot_w64(m[h])) nterms[h] += e - b;
-            if (H == 1 || m[h]) add(part[h], h);
+            if (H == 1 || m[h]) add(part[h], h, m[h]);
         }
     };
 
@@ -982,7 +1002,7 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
         }
 #pragma unroll
         for (int h = 0; h < H; ++h)
-            if (H == 1 || mask[h]) add(part[h], h);
+            if (H == 1 || mask[h]) add(part[h], h, mask[h]);
     }
 #pragma unroll
     for (int h = 0; h < H; ++h) {
@@ -993,21 +1013,320 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
     }
 }
 
-// Barnes-Hut value and gradient at query points (new; the reference has no
-// gradient): the walk and far test of gwn_tree_kernel (FP32 path: far
-// dipoles at (CM_f − q) + residual), each lane accumulating w and ∇w of its
-// own term set.
+// Barnes-Hut sums at explicit query points, and (GRAD; new, the reference has
+// no gradient) their gradient.  The points come in the caller's order, so 64
+// consecutive ones need not have anything in common, and one walk for the
+// union of their traversals opens many times the nodes each needs.  Here L
+// lanes walk for one query alone: lane 8g + c of them tests child c of the
+// g-th node from the top of the query's stack, so L / 8 nodes are opened a
+// step.  Each query takes exactly its own term set (the far test of
+// gwn_tree_kernel; far dipoles at (CM_f − q) + residual, without the residual
+// for BF16 moments); a lane sums its terms in FP64 and the lanes are added in
+// a fixed order.
+// Bound by the L2 reads of the node records (56 B a child, about 20 KB a
+// query) and, for few queries, by the latency of a step (records, then
+// payloads): few queries take 64 lanes each, many 8.
+// A query's stack holds first-child indices (leaves of several points: the
+// complement of the leaf's own index) and never overflows: opening a node
+// leaves at most 7 entries more than it took, a step takes several nodes only
+// while at most kWalkDeep entries wait, and above what that leaves there is
+// room for a depth-first descent.
+constexpr int kWalkWaves = 4, kWalkDeep = 64;
+__host__ __device__ constexpr int walk_stack_entries(int max_level, int lanes) {
+    return tree_stack_entries(max_level) + (lanes > 8 ? kWalkDeep + 7 * (lanes / 8) : 0);
+}
+
+// value and gradient of tree_term_split's term; 0 unless `on` and beyond the
+// guard
+template <bool SCREENED>
+__device__ __forceinline__ void tree_term_grad(float dx, float dy, float dz, float s2, const float4 b, float sigma,
+                                               float sigma_l2e, float& w, float& gx, float& gy, float& gz) {
+    const float r2 = dist2(dx, dy, dz);
+    const float dot = __builtin_fmaf(dz, b.z, __builtin_fmaf(dy, b.y, dx * b.x));
+    if constexpr (!SCREENED) {
+        const float r = fast_sqrt(r2);
+        const float inv = fast_rcp(__builtin_fmaf(r2, r, kEpsPlain * kInv4Pi));
+        w = dot * inv;
+        const float c = 3.0f * r * w * inv;
+        gx = __builtin_fmaf(c, dx, -b.x * inv);
+        gy = __builtin_fmaf(c, dy, -b.y * inv);
+        gz = __builtin_fmaf(c, dz, -b.z * inv);
+    } else {
+        const bool ok = r2 > 1e-20f, inside = s2 > r2;  // inside: ρ = s, no dependence on q through ρ
+        const float rho = fast_sqrt(max_nonneg(r2, s2));
+        const float er2 = fast_exp2(sigma_l2e * rho) * (rho * rho);
+        const float eps = kEpsScreened * kInv4Pi;
+        const float inv = fast_rcp(__builtin_fmaf(er2, rho, eps));
+        const float sr = sigma * rho;
+        const float g = ok ? __builtin_fmaf(sigma, rho, 1.0f) * inv : 0.0f;
+        const float gp = (sigma * eps - er2 * __builtin_fmaf(sr, sr + 3.0f, 3.0f)) * inv * inv;
+        const float c = (inside || !ok) ? 0.0f : -dot * gp * fast_rcp(rho);
+        w = g * dot;
+        gx = __builtin_fmaf(c, dx, -g * b.x);
+        gy = __builtin_fmaf(c, dy, -g * b.y);
+        gz = __builtin_fmaf(c, dz, -g * b.z);
+    }
+}
+
+template <bool SCREENED, bool BF16, bool GRAD, int L>
+__global__ __launch_bounds__(kWalkWaves * 64) void gwn_walk_kernel(TreeArgs T, const float* __restrict__ q, int64_t nq,
+                                                                    int stack, float sigma, float* __restrict__ out_w,
+                                                                    float* __restrict__ out_g) {
+    constexpr int kQueries = 64 / L, kNodes = L / 8;
+    extern __shared__ int s_stacks[];  // kWalkWaves × kQueries stacks of `stack` entries
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int sub = lane / L, sl = lane % L, g = sl >> 3, c = lane & 7;
+    int* ent = s_stacks + (wave * kQueries + sub) * stack;
+    const int64_t qi = (int64_t(blockIdx.x) * kWalkWaves + wave) * kQueries + sub;
+    const bool valid = qi < nq;
+    if (!__builtin_amdgcn_ballot_w64(valid)) return;
+    const float qx = valid ? q[3 * qi] : 0.f, qy = valid ? q[3 * qi + 1] : 0.f, qz = valid ? q[3 * qi + 2] : 0.f;
+    const float sl2e = sigma * kLog2e;
+    double sum[GRAD ? 4 : 1];
+#pragma unroll
+    for (int k = 0; k < (GRAD ? 4 : 1); ++k) sum[k] = 0.0;
+    auto add = [&](float dx, float dy, float dz, float s2, const float4 b) {
+        if constexpr (GRAD) {
+            float w, gx, gy, gz;
+            tree_term_grad<SCREENED>(dx, dy, dz, s2, b, sigma, sl2e, w, gx, gy, gz);
+            sum[0] += double(w);
+            sum[1] += double(gx);
+            sum[2] += double(gy);
+            sum[3] += double(gz);
+        } else {
+            float inv;
+            bool ok;
+            const float x = tree_term_split<SCREENED>(dx, dy, dz, dist2(dx, dy, dz), s2, b, sigma, sl2e, inv, ok);
+            sum[0] += double(ok ? x * inv : 0.f);
+        }
+    };
+    // the points of a leaf, 8 lanes of the query a step
+    auto leaf = [&](int b, int e) {
+        for (int j = b + c; j < e; j += 8) {
+            const float4 pa = T.sa[j];
+            add(pa.x - qx, pa.y - qy, pa.z - qz, pa.w * pa.w, T.sb[j]);
+        }
+    };
+    const int4 root = T.info[0];
+    int sp = 0;
+    if (root.x < 0) {
+        if (valid && g == 0) leaf(root.y, root.z);
+    } else if (valid) {
+        ent[0] = root.x;
+        sp = 1;
+    }
+    __builtin_amdgcn_wave_barrier();
+    while (__builtin_amdgcn_ballot_w64(sp > 0)) {
+        const int nb = min(sp, sp <= kWalkDeep ? kNodes : 1);
+        const bool on = g < nb;
+        const int top = on ? ent[sp - 1 - g] : 0;
+        sp -= nb;
+        bool push = false;
+        int next = 0;
+        if (on && top < 0) {
+            const int2 lf = T.kid[~top];
+            leaf(lf.y, lf.y - lf.x);
+        } else if (on) {
+            const int64_t ch = int64_t(top) + c;
+            const int2 nk = T.kid[ch];
+            const float4 cr = T.cm_r[ch];
+            if (nk.x != 0) {
+                const float dx = cr.x - qx, dy = cr.y - qy, dz = cr.z - qz;
+                // an internal node is far when d² > (β·R)² (cm_r.w), a one-point
+                // leaf's record makes the test its term's guard, a leaf of
+                // several points is never far (∞)
+                if (dist2(dx, dy, dz) > cr.w) {
+                    const float4* pay = reinterpret_cast<const float4*>(T.payload) + 2 * ch;
+                    const float4 e4 = pay[0];
+                    const float4 lo = BF16 ? make_float4(0.f, 0.f, 0.f, 0.f) : pay[1];
+                    add(dx + lo.x, dy + lo.y, dz + lo.z, e4.w, e4);
+                } else if (nk.x != -1) {
+                    push = true;
+                    next = nk.x > 0 ? nk.x : ~int(ch);
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        const uint64_t pm = __builtin_amdgcn_ballot_w64(push) >> (sub * L);  // bit sl: this query's lane
+        const uint64_t mine = L == 64 ? pm : pm & ((1ull << (L & 63)) - 1ull);
+        if (push) ent[sp + __builtin_popcountll(mine & ((1ull << sl) - 1ull))] = next;
+        sp += __builtin_popcountll(mine);
+        __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int off = 1; off < L; off <<= 1)
+#pragma unroll
+        for (int k = 0; k < (GRAD ? 4 : 1); ++k) sum[k] += __shfl_xor(sum[k], off, 64);
+    if (valid && sl == 0) {
+        out_w[qi] = float(sum[0]);
+        if constexpr (GRAD) {
+            if (out_g) {
+                out_g[3 * qi] = float(sum[1]);
+                out_g[3 * qi + 1] = float(sum[2]);
+                out_g[3 * qi + 2] = float(sum[3]);
+            }
+        }
+    }
+}
+
+// Which walk explicit queries take.  Alone (gwn_walk_kernel), 64 lanes a query
+// below kWalkFew, where the waves do not fill the chip (1,000 of 100k sources:
+// 17 µs, with 8 lanes 48, shared 1,190), else 8 (32,000: 57 and 75 against
+// 1,380 µs; 100,000 with gradient: 0.17 against 2.5 ms).  From kShareValue on
+// (kShareGrad with the gradient) 64 to a shared walk, in spatial order: the
+// node records are then read once for 64 queries, which for 1M queries on the
+// surface takes half the time, while unordered ones (2M: 12.8 ms shared, 3.3 ms
+// alone) are put in order first
+constexpr int64_t kWalkFew = 40000, kShareValue = 196608, kShareGrad = 786432;
+
+// The order: a counting sort by the Morton code of a 64³ grid over the tree's
+// cube.  Queries that come in order already are left as they are, which a
+// sample of runs of 64 decides: they come unsorted when such runs extend, on
+// average, over twice the side that 64 of nq uniform points fill
+constexpr int kOrderBits = 6, kOrderBuckets = 1 << (3 * kOrderBits);
+constexpr int kOrderSamples = 256;
+
+__device__ __forceinline__ float wave_min(float v) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) v = fminf(v, __shfl_xor(v, off, 64));
+    return v;
+}
+
+// extent of sampled runs relative to the cube, in 2^-16, summed into *total
+__global__ __launch_bounds__(64) void order_sample_kernel(const float* __restrict__ q, int64_t nq,
+                                                          const double4* __restrict__ cell,
+                                                          unsigned int* __restrict__ total) {
+    const int64_t runs = nq / 64;
+    const int64_t i = int64_t(blockIdx.x) * runs / gridDim.x * 64 + threadIdx.x;  // nq ≥ 64
+    float e = 0.f;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const float v = q[3 * i + d];
+        e = fmaxf(e, -wave_min(-v) - wave_min(v));
+    }
+    const float w = float(cell[0].w);
+    if (threadIdx.x == 0) atomicAdd(total, (unsigned int)(65536.f * fminf(fmaxf(e / w, 0.f), 1.f)));
+}
+
+__device__ __forceinline__ int order_bucket(const float* __restrict__ q, int64_t i, const double4 c) {
+    const float inv = float(double(1 << kOrderBits) / c.w);
+    const float lo[3] = {float(c.x - 0.5 * c.w), float(c.y - 0.5 * c.w), float(c.z - 0.5 * c.w)};
+    int m = 0;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        // (a NaN, also of a cube of no width, becomes 0)
+        const int v = int(fminf(fmaxf((q[3 * i + d] - lo[d]) * inv, 0.f), float((1 << kOrderBits) - 1)));
+#pragma unroll
+        for (int b = 0; b < kOrderBits; ++b) m |= ((v >> b) & 1) << (3 * b + d);
+    }
+    return m;
+}
+
+__global__ void order_count_kernel(const float* __restrict__ q, int64_t nq, const double4* __restrict__ cell,
+                                   QueryOrder O, int* __restrict__ bucket_of,
+                                   unsigned long long* __restrict__ count) {
+    if (!O.sorted()) return;
+    const double4 root = cell[0];
+    const int lane = threadIdx.x & 63;
+    for (int64_t i0 = int64_t(blockIdx.x) * blockDim.x; i0 < nq; i0 += int64_t(gridDim.x) * blockDim.x) {
+        const int64_t i = i0 + threadIdx.x;
+        const int b = i < nq ? order_bucket(q, i, root) : -1;
+        if (i < nq) bucket_of[i] = b;
+        const uint64_t starts = run_starts(b);
+        if (b >= 0 && ((starts >> lane) & 1ull)) atomicAdd(&count[b], (unsigned long long)run_length(starts, lane));
+    }
+}
+
+__global__ void order_scatter_kernel(const int* __restrict__ bucket_of, int64_t nq, QueryOrder O,
+                                     unsigned long long* __restrict__ cursor, int* __restrict__ order) {
+    if (!O.sorted()) return;
+    const int lane = threadIdx.x & 63;
+    for (int64_t i0 = int64_t(blockIdx.x) * blockDim.x; i0 < nq; i0 += int64_t(gridDim.x) * blockDim.x) {
+        const int64_t i = i0 + threadIdx.x;
+        const int b = i < nq ? bucket_of[i] : -1;
+        const uint64_t starts = run_starts(b);
+        int at = 0;
+        if (b >= 0 && ((starts >> lane) & 1ull))
+            at = int(atomicAdd(&cursor[b], (unsigned long long)run_length(starts, lane)));
+        const int head = run_head(starts, lane);
+        at = __shfl(at, head, 64) + (lane - head);
+        if (b >= 0) order[at] = int(i);
+    }
+}
+
+static QueryOrder query_order(dwg_ctx* ctx, const dwg_octree* T, const float* q, int64_t nq) {
+    DWG_REQUIRE(nq < (int64_t(1) << 31) - 1, "too many queries");
+    auto* start = static_cast<unsigned long long*>(ctx->buf("order_start", sizeof(uint64_t) * (kOrderBuckets + 2)));
+    int* bucket_of = static_cast<int*>(ctx->buf("order_bucket_of", sizeof(int) * size_t(nq)));
+    int* order = static_cast<int*>(ctx->buf("order", sizeof(int) * size_t(nq)));
+    auto* extent = reinterpret_cast<unsigned int*>(start + kOrderBuckets + 1);
+    ProfileScope ps(ctx, "gwn_query_order");
+    fill_u32(ctx, start, 0, 2 * (kOrderBuckets + 2));
+    const int samples = int(std::min<int64_t>(nq / 64, kOrderSamples));
+    hipLaunchKernelGGL(order_sample_kernel, dim3(samples), dim3(64), 0, ctx->stream, q, nq, T->cell, extent);
+    check_launch();
+    const QueryOrder O{order, extent, unsigned(65536.f * 2.f * std::cbrt(64.f / float(nq)) * float(samples))};
+    const unsigned blocks = std::min(grid_for(nq, 256), 2048u);
+    hipLaunchKernelGGL(order_count_kernel, dim3(blocks), dim3(256), 0, ctx->stream, q, nq, T->cell, O, bucket_of,
+                       start);
+    check_launch();
+    exclusive_scan_i64(ctx, reinterpret_cast<int64_t*>(start), kOrderBuckets);
+    hipLaunchKernelGGL(order_scatter_kernel, dim3(blocks), dim3(256), 0, ctx->stream, bucket_of, nq, O, start,
+                       order);
+    check_launch();
+    return O;
+}
+
+template <bool GRAD>
+static void launch_walk(dwg_ctx* ctx, const dwg_octree* T, const float* q, int64_t nq, float sigma, uint32_t flags,
+                        float* out_w, float* out_g) {
+    const TreeArgs A{T->info, T->kid, T->cm_r, reinterpret_cast<const float*>(T->payload), T->sa, T->sb};
+    const int lanes = nq < kWalkFew ? 64 : 8;
+    const int stack = walk_stack_entries(std::max(T->max_level, 1), lanes);
+    const int64_t per = int64_t(kWalkWaves) * (64 / lanes);
+    const size_t lds = sizeof(int) * size_t(stack) * size_t(per);
+    dim3 grid(grid_for(nq, int(per))), block(kWalkWaves * 64);
+#define DWG_WALK(S, B)                                                                                                  \
+    do {                                                                                                                \
+        if (lanes == 64)                                                                                                \
+            hipLaunchKernelGGL((gwn_walk_kernel<S, B, GRAD, 64>), grid, block, lds, ctx->stream, A, q, nq, stack, sigma, \
+                               out_w, out_g);                                                                           \
+        else                                                                                                            \
+            hipLaunchKernelGGL((gwn_walk_kernel<S, B, GRAD, 8>), grid, block, lds, ctx->stream, A, q, nq, stack, sigma, \
+                               out_w, out_g);                                                                           \
+    } while (0)
+    const bool scr = flags & DWG_SCREENED;
+    bool done = false;
+    if constexpr (!GRAD) {
+        if (flags & DWG_FAR_BF16) {
+            if (scr) DWG_WALK(true, true);
+            else DWG_WALK(false, true);
+            done = true;
+        }
+    }
+    if (!done) {
+        if (scr) DWG_WALK(true, false);
+        else DWG_WALK(false, false);
+    }
+#undef DWG_WALK
+    check_launch();
+}
+
+// Value and gradient at many query points: the shared walk and far test of
+// gwn_tree_kernel (FP32 path: far dipoles at (CM_f − q) + residual), each
+// lane accumulating w and ∇w of its own term set.
 template <bool SCREENED>
 __global__ __launch_bounds__(kTreeThreads) void gwn_tree_grad_kernel(TreeArgs T, const float* __restrict__ q,
-                                                                      int64_t nq, float sigma,
+                                                                      int64_t nq, QueryOrder order, float sigma,
                                                                       float* __restrict__ out_w,
                                                                       float* __restrict__ out_g) {
     __shared__ int s_node[kTreeWaves][kStack];
     __shared__ uint64_t s_mask[kTreeWaves][kStack];
     __shared__ float4 s_pay[kTreeWaves][16];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int64_t qi = (int64_t(blockIdx.x) * kTreeWaves + wave) * 64 + lane;
-    const bool valid = qi < nq;
+    const int64_t slot = (int64_t(blockIdx.x) * kTreeWaves + wave) * 64 + lane;
+    const bool valid = slot < nq;
+    const int64_t qi = valid ? order.query(slot) : slot;
     const float qx = valid ? q[3 * qi] : 0.f, qy = valid ? q[3 * qi + 1] : 0.f, qz = valid ? q[3 * qi + 2] : 0.f;
     const uint64_t all = __builtin_amdgcn_ballot_w64(valid);
     if (all == 0) return;
@@ -1024,10 +1343,12 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_grad_kernel(TreeArgs T,
         part[2] += on ? gy : 0.f;
         part[3] += on ? gz : 0.f;
     };
-    auto fold = [&]() {
+    // (for the lanes that took part: adding a zero would move bits between the
+    // sum and its compensation)
+    auto fold = [&](bool on) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            kahan_add(acc[k], comp[k], part[k]);
+            if (on) kahan_add(acc[k], comp[k], part[k]);
             part[k] = 0.f;
         }
     };
@@ -1041,7 +1362,7 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_grad_kernel(TreeArgs T,
     const int4 root = T.info[0];
     if (root.x < 0) {
         leaf(root.y, root.z, valid);
-        fold();
+        fold(valid);
     } else {
         if (lane == 0) {
             s_node[wave][0] = root.x;
@@ -1080,7 +1401,7 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_grad_kernel(TreeArgs T,
                 ++sp;
             }
         }
-        fold();
+        fold(act);
         __builtin_amdgcn_wave_barrier();
     }
     if (valid) {
@@ -1181,6 +1502,13 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
         check_launch();
         T->payload_bf16 = want_bf16;
     }
+    const bool near64 = (flags & DWG_SCREENED) && (flags & DWG_NEAR_FP64);
+    if (Q.q && !count && !near64 && Q.nq < kShareValue) {
+        if (Q.nq == 0) return;
+        ProfileScope ps(ctx, (flags & DWG_SCREENED) ? "gwn_tree_screened" : "gwn_tree_plain");
+        launch_walk<false>(ctx, T, Q.q, Q.nq, sigma, flags, out, nullptr);
+        return;
+    }
     const int64_t waves = Q.grid ? Q.n_bricks : (Q.nq + 64 * kPointPts - 1) / (64 * kPointPts);
     if (waves == 0) return;
     TreeArgs A{T->info, T->kid, T->cm_r, reinterpret_cast<const float*>(T->payload), T->sa, T->sb};
@@ -1188,12 +1516,12 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
     // the walk's stack: one record and one lane mask per part for each entry
     QueryArgs Qs = Q;
     Qs.stack = tree_stack_entries(std::max(T->max_level, 1));
+    if (Q.q && Q.nq >= kShareValue) Qs.order = query_order(ctx, T, Q.q, Q.nq);
     const size_t lds = sizeof(uint64_t) * size_t(Qs.stack) * size_t(1 + (Q.grid ? kGridParts : kPointPts));
     const bool scr = flags & DWG_SCREENED, bf = flags & DWG_FAR_BF16;
     const char* name = count ? "gwn_tree_terms" : (!Q.grid ? (scr ? "gwn_tree_screened" : "gwn_tree_plain")
                                                            : (scr ? "gwn_tree_grid_screened" : "gwn_tree_grid_plain"));
     ProfileScope ps(ctx, name);
-    const bool near64 = scr && (flags & DWG_NEAR_FP64);
 #define DWG_TREE_LAUNCH(S, C, B, G, N) \
     hipLaunchKernelGGL((gwn_tree_kernel<S, C, B, G, N>), grid, block, lds, ctx->stream, A, Qs, beta, sigma, flags, out, terms)
 #define DWG_TREE_LAUNCH_Q(S, C, B, N)       \
@@ -1254,13 +1582,20 @@ void gwn_tree_grad(dwg_ctx* ctx, const dwg_octree* Tc, const float* q, int64_t n
         T->payload_bf16 = false;
     }
     if (nq == 0) return;
+    if (nq < kShareGrad) {
+        ProfileScope ps(ctx, "gwn_tree_grad");
+        launch_walk<true>(ctx, T, q, nq, sigma, flags, out_w, out_g);
+        return;
+    }
+    const QueryOrder order = query_order(ctx, T, q, nq);
     TreeArgs A{T->info, T->kid, T->cm_r, reinterpret_cast<const float*>(T->payload), T->sa, T->sb};
     dim3 grid(grid_for((nq + 63) / 64, kTreeWaves)), block(kTreeThreads);
     ProfileScope ps(ctx, "gwn_tree_grad");
     if (flags & DWG_SCREENED)
-        hipLaunchKernelGGL(gwn_tree_grad_kernel<true>, grid, block, 0, ctx->stream, A, q, nq, sigma, out_w, out_g);
+        hipLaunchKernelGGL(gwn_tree_grad_kernel<true>, grid, block, 0, ctx->stream, A, q, nq, order, sigma, out_w, out_g);
     else
-        hipLaunchKernelGGL(gwn_tree_grad_kernel<false>, grid, block, 0, ctx->stream, A, q, nq, sigma, out_w, out_g);
+        hipLaunchKernelGGL(gwn_tree_grad_kernel<false>, grid, block, 0, ctx->stream, A, q, nq, order, sigma, out_w,
+                           out_g);
     check_launch();
 }
 

@@ -34,29 +34,6 @@ __device__ __forceinline__ int cell_coord(float v, float lo, float inv_cell, int
     return min(max(c, 0), dim - 1);
 }
 
-// Points and queries arrive in runs that share a cell or tile (sources in
-// tree order, triangle centroids in brick order): each wave adds one run
-// with one atomic.  A run starts at lane 0 and wherever the key changes; its
-// first lane (the head) reserves the run's slots, the others take theirs
-// from the head in lane order.
-__device__ __forceinline__ uint64_t run_starts(int tl) {
-    const int lane = threadIdx.x & 63;
-    const int prev = __shfl_up(tl, 1, 64);
-    return __ballot(lane == 0 || tl != prev);
-}
-
-// lanes from `lane` up to the next run start (or the end of the wave)
-__device__ __forceinline__ int run_length(uint64_t starts, int lane) {
-    const uint64_t after = lane == 63 ? 0ull : starts >> (lane + 1);
-    return after ? __builtin_ctzll(after) + 1 : 64 - lane;
-}
-
-// the run start at or before `lane`
-__device__ __forceinline__ int run_head(uint64_t starts, int lane) {
-    const uint64_t upto = lane == 63 ? starts : starts & ((2ull << lane) - 1ull);
-    return 63 - __builtin_clzll(upto);
-}
-
 __global__ void knn_count_kernel(const float* __restrict__ p, int64_t n, KnnGridArgs G,
                                  unsigned long long* __restrict__ counts, int* __restrict__ cell_of) {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;

@@ -71,7 +71,8 @@ def test_direct_sums_split_over_sources(ctx, n, nq, screened, kahan):
                                                  (False, True, False)])
 def test_grid_walk_equals_the_point_walk(ctx, res, h, shift, screened, bf16, radii):
     # the brick's whole-box decisions are each point's own, so a grid value is
-    # the explicit point's bit for bit (the same terms in the same order)
+    # the explicit point's bit for bit where that takes the same terms in the
+    # same order: in the shared walk of many points (here the grid's, repeated)
     P, N = shapes.union(3000, 8, 11)
     P = np.concatenate([P, P[:40], P[:3] + 1e-6]).astype(np.float64) + shift  # leaves of several points
     N = np.concatenate([N, N[:40], N[:3]]).astype(np.float32)
@@ -86,7 +87,7 @@ def test_grid_walk_equals_the_point_walk(ctx, res, h, shift, screened, bf16, rad
     Q = torch.from_numpy(np.stack([x, y, z], -1).reshape(-1, 3).astype(np.float32)).cuda()
     kw = dict(sigma=SIGMA, screened=screened, bf16=bf16)
     got = tree.eval_grid(grid, 2.3, **kw).cpu().numpy()
-    want = tree.eval(Q, 2.3, **kw).cpu().numpy()
+    want = tree.eval(Q.repeat(200_000 // len(Q) + 1, 1), 2.3, **kw).cpu().numpy()[:len(Q)]
     np.testing.assert_array_equal(got, want)
 
 
@@ -129,3 +130,46 @@ def test_knn_far_walk_hands_over(ctx):
     ref, rd2 = O.knn_brute(P, Q[sub], 15, return_d2=True)
     np.testing.assert_array_equal(got.cpu().numpy()[sub], ref)
     np.testing.assert_array_equal(d2.cpu().numpy()[sub], rd2)
+
+
+# one query, the last set searched with 64 lanes a query, the first with 8, the
+# first that share walks in order (unordered and ordered), and trees of one
+# leaf, of one level and with leaves of several points
+@pytest.mark.parametrize("n,nq,ordered", [(1, 5, False), (2, 1, False), (3000, 1, False), (3000, 39_999, False),
+                                          (3000, 40_001, False), (3000, 196_607, False), (3000, 196_611, False),
+                                          (3000, 196_611, True), (3000, 786_435, False)])
+@pytest.mark.parametrize("screened,radii,bf16", [(True, False, False), (True, True, False), (False, False, False),
+                                                 (True, False, True), (False, False, True)])
+def test_tree_sums_by_query_count(ctx, n, nq, ordered, screened, radii, bf16):
+    P, N = shapes.sphere(n, 7)
+    rng = np.random.default_rng(n + nq)
+    P = (0.5 * P + rng.normal(0, 0.002, P.shape)).astype(np.float32).astype(np.float64)
+    P[: n // 10] = P[0]  # a leaf of several points
+    A = rng.uniform(1e-6, 4e-6, n).astype(np.float32)
+    R = rng.uniform(0.0015, 0.015, n).astype(np.float32) if radii else None
+    Q = np.concatenate([P[rng.integers(0, n, nq // 2)] + rng.normal(0, 0.01, (nq // 2, 3)),
+                        rng.uniform(-0.8, 0.8, (nq - nq // 2, 3))]).astype(np.float32)
+    if ordered:
+        Q = Q[np.lexsort((Q * 40).astype(int).T)]
+    tree = gpu.Octree(ctx, P, A.astype(np.float64), max_depth=10)
+    tree.update(N, A, R)
+    o = O.Octree(P, 10, 1)
+    o.precompute(N.astype(np.float64), A.astype(np.float64))
+    sub = rng.permutation(nq)[:1500]
+    kind = "screened" if screened else "plain"
+    rad = None if R is None else R.astype(np.float64)
+    ref = o.eval(Q[sub].astype(np.float64), 2.3, kind=kind, sigma=SIGMA, radii=rad)
+    w = tree.eval(Q, 2.3, sigma=SIGMA, screened=screened, bf16=bf16).cpu().numpy()[sub]
+    if bf16:
+        # the rounded moments are the same for every walk: against the shared
+        # walk of many points (the queries compared, repeated)
+        many = torch.from_numpy(np.tile(Q[sub], (200_000 // len(sub) + 1, 1)))
+        ref = tree.eval(many, 2.3, sigma=SIGMA, screened=screened, bf16=True).cpu().numpy()[:len(sub)]
+    # FP32 terms: 1e-5 of max|w|, the bound the precision sweep holds
+    assert np.abs(w - ref).max() <= 1e-5 * np.abs(ref).max()
+    if bf16:
+        return
+    wg, g = (t.cpu().numpy()[sub] for t in tree.eval_grad(Q, 2.3, sigma=SIGMA, screened=screened))
+    assert np.abs(wg - ref).max() <= 1e-5 * np.abs(ref).max()
+    rw, rg = o.eval_grad(Q[sub].astype(np.float64), 2.3, kind=kind, sigma=SIGMA, radii=rad)
+    assert np.abs(g - rg).max() <= 1e-4 * np.abs(rg).max()  # the tree gradient's bound
