@@ -24,7 +24,7 @@ constexpr int64_t kTrainPoints = 50000;
 
 struct dwg_mlp {
     float* params = nullptr;     // FP32 master weights (kParams)
-    uint16_t* bf16 = nullptr;    // BF16 copy used by the kernels (kParams)
+    uint16_t* bf16 = nullptr;    // BF16 copy used by the kernels (kParams), then W2 transposed
     float* grad = nullptr;       // FP32 gradient (kParams)
     float* adam_m = nullptr;
     float* adam_v = nullptr;

@@ -18,6 +18,7 @@
 // free), ŷ = y/|y|, t the unit target normal.  The initialisation orients
 // the predicted line away from the bounding-box centre, as the Gauss map
 // does (TurboNormalInit.cu:3-44).
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -194,86 +195,16 @@ __device__ __forceinline__ float gelu(float x, float* dgelu) {
     return 0.5f * x * (1.0f + t);
 }
 
-// z += bias; h = bf16(gelu(z)); z keeps the pre-activation for the backward pass
-__global__ void bias_gelu_kernel(float* __restrict__ z, const float* __restrict__ bias, int64_t rows, int cols,
-                                 uint16_t* __restrict__ h) {
-    const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= rows * cols) return;
-    const float v = z[t] + bias[t % cols];
-    z[t] = v;
-    h[t] = to_bf16(gelu(v, nullptr));
-}
-
-// grad of the pre-activation: dz = bf16(dh · gelu'(z))
-__global__ void gelu_back_kernel(const float* __restrict__ dh, const float* __restrict__ z, int64_t count,
-                                 uint16_t* __restrict__ dz, float* __restrict__ dz32) {
-    const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= count) return;
-    float g;
-    (void)gelu(z[t], &g);
-    const float v = dh[t] * g;
-    dz[t] = to_bf16(v);
-    if (dz32) dz32[t] = v;
-}
-
-__global__ void add_bias_normalize_kernel(float* __restrict__ y, const float* __restrict__ b3, int64_t rows,
-                                          int normalize) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= rows) return;
-    float v[3];
-    for (int c = 0; c < 3; ++c) v[c] = y[3 * i + c] + b3[c];
-    if (normalize) {
-        const float s = 1.0f / (sqrtf(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]) + 1e-12f);
-        for (int c = 0; c < 3; ++c) v[c] *= s;
+// the BF16 copy of parameter i, and W2's transposed one after all parameters
+// (the backward product reads W2 by columns), at a 16-byte boundary
+constexpr int64_t kOffW2T = (kParams + 7) / 8 * 8;
+__device__ __forceinline__ void store_bf16_param(uint16_t* __restrict__ b16, int64_t i, float v) {
+    const uint16_t b = to_bf16(v);
+    b16[i] = b;
+    if (i >= kOffW2 && i < kOffB2) {
+        const int64_t e = i - kOffW2;
+        b16[kOffW2T + (e % kHid) * kHid + e / kHid] = b;
     }
-    for (int c = 0; c < 3; ++c) y[3 * i + c] = v[c];
-}
-
-// oriented:  loss = mean(1 − c),  dL/dy = −(t − c ŷ)/(|y|·B)
-// line:      loss = mean(1 − c²), dL/dy = −2c (t − c ŷ)/(|y|·B),   c = ŷ·t
-__global__ void loss_kernel(const float* __restrict__ y, const float* __restrict__ t, int64_t rows, int mode,
-                            float* __restrict__ dy, uint16_t* __restrict__ dy16, double* __restrict__ loss_part) {
-    __shared__ double lds[256];
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    double l = 0;
-    if (i < rows) {
-        const float y0 = y[3 * i], y1 = y[3 * i + 1], y2 = y[3 * i + 2];
-        const float ny = sqrtf(y0 * y0 + y1 * y1 + y2 * y2) + 1e-12f;
-        const float h0 = y0 / ny, h1 = y1 / ny, h2 = y2 / ny;
-        const float t0 = t[3 * i], t1 = t[3 * i + 1], t2 = t[3 * i + 2];
-        const float c = h0 * t0 + h1 * t1 + h2 * t2;
-        l = mode ? 1.0 - double(c) * double(c) : 1.0 - double(c);
-        const float s = (mode ? -2.0f * c : -1.0f) / (ny * float(rows));
-        const float g[3] = {s * (t0 - c * h0), s * (t1 - c * h1), s * (t2 - c * h2)};
-        for (int k = 0; k < 3; ++k) {
-            dy[3 * i + k] = g[k];
-            dy16[3 * i + k] = to_bf16(g[k]);
-        }
-    }
-    lds[threadIdx.x] = l;
-    __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) lds[threadIdx.x] += lds[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) loss_part[blockIdx.x] = lds[0];
-}
-
-// column sums of a rows×cols FP32 matrix into out[cols]: one block per
-// column, fixed-order tree reduction (deterministic)
-__global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ m, int64_t rows, int cols,
-                                                     float* __restrict__ out) {
-    __shared__ double lds[256];
-    const int c = blockIdx.x;
-    double s = 0;
-    for (int64_t r = threadIdx.x; r < rows; r += 256) s += m[r * cols + c];
-    lds[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) lds[threadIdx.x] += lds[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[c] = float(lds[0]);
 }
 
 __global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
@@ -288,12 +219,12 @@ __global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ g, 
     v[i] = vi;
     const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
     p[i] = pi;
-    b16[i] = to_bf16(pi);
+    store_bf16_param(b16, i, pi);
 }
 
-__global__ void to_bf16_kernel(const float* __restrict__ a, uint16_t* __restrict__ b, int64_t n) {
+__global__ void params_bf16_kernel(const float* __restrict__ a, uint16_t* __restrict__ b16) {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) b[i] = to_bf16(a[i]);
+    if (i < kParams) store_bf16_param(b16, i, a[i]);
 }
 
 // batch gather with one rotation R (row-major 3×3) applied to every patch
@@ -328,7 +259,7 @@ static dwg_mlp* mlp_alloc() {
     auto* m = new dwg_mlp();
     try {
         m->params = static_cast<decltype(m->params)>(dev_malloc(sizeof(float) * kParams));
-        m->bf16 = static_cast<decltype(m->bf16)>(dev_malloc(sizeof(uint16_t) * kParams));
+        m->bf16 = static_cast<decltype(m->bf16)>(dev_malloc(sizeof(uint16_t) * (kOffW2T + kHid * kHid)));
         m->grad = static_cast<decltype(m->grad)>(dev_malloc(sizeof(float) * kParams));
         m->adam_m = static_cast<decltype(m->adam_m)>(dev_malloc(sizeof(float) * kParams));
         m->adam_v = static_cast<decltype(m->adam_v)>(dev_malloc(sizeof(float) * kParams));
@@ -341,8 +272,7 @@ static dwg_mlp* mlp_alloc() {
 
 static void mlp_set(dwg_ctx* ctx, dwg_mlp* m, const float* h) {
     DWG_HIP_CHECK(hipMemcpyAsync(m->params, h, sizeof(float) * kParams, hipMemcpyHostToDevice, ctx->stream));
-    hipLaunchKernelGGL(to_bf16_kernel, dim3(grid_for(kParams, 256)), dim3(256), 0, ctx->stream, m->params, m->bf16,
-                       kParams);
+    hipLaunchKernelGGL(params_bf16_kernel, dim3(grid_for(kParams, 256)), dim3(256), 0, ctx->stream, m->params, m->bf16);
     check_launch();
     fill_u32(ctx, m->adam_m, 0, kParams);
     fill_u32(ctx, m->adam_v, 0, kParams);
@@ -428,35 +358,6 @@ void mlp_patches_from(dwg_ctx* ctx, const dwg_knn_index* I, const float* src, in
 
 void mlp_patches(dwg_ctx* ctx, const dwg_knn_index* I, const float* p, int64_t n, uint16_t* out) {
     mlp_patches_from(ctx, I, p, n, p, n, out);
-}
-
-struct Acts {
-    float *z1, *z2, *y;
-    uint16_t *h1, *h2;
-};
-
-static Acts acts(dwg_ctx* ctx, int64_t rows) {
-    Acts a;
-    a.z1 = static_cast<float*>(ctx->buf("mlp_z1", sizeof(float) * rows * kHid));
-    a.z2 = static_cast<float*>(ctx->buf("mlp_z2", sizeof(float) * rows * kHid));
-    a.y = static_cast<float*>(ctx->buf("mlp_y", sizeof(float) * rows * kOut));
-    a.h1 = static_cast<uint16_t*>(ctx->buf("mlp_h1", sizeof(uint16_t) * rows * kHid));
-    a.h2 = static_cast<uint16_t*>(ctx->buf("mlp_h2", sizeof(uint16_t) * rows * kHid));
-    return a;
-}
-
-// y = W3·gelu(W2·gelu(W1·x + b1) + b2) + b3 for `rows` patches (raw y in a.y)
-static void forward(dwg_ctx* ctx, const dwg_mlp* m, const uint16_t* x, int64_t rows, const Acts& a) {
-    const uint16_t* W = m->bf16;
-    gemm(ctx, {x, kIn, 1, W + kOffW1, 1, kIn, a.z1, kHid, 1, rows, kHid, kIn, 0});
-    hipLaunchKernelGGL(bias_gelu_kernel, dim3(grid_for(rows * kHid, 256)), dim3(256), 0, ctx->stream, a.z1,
-                       m->params + kOffB1, rows, kHid, a.h1);
-    check_launch();
-    gemm(ctx, {a.h1, kHid, 1, W + kOffW2, 1, kHid, a.z2, kHid, 1, rows, kHid, kHid, 0});
-    hipLaunchKernelGGL(bias_gelu_kernel, dim3(grid_for(rows * kHid, 256)), dim3(256), 0, ctx->stream, a.z2,
-                       m->params + kOffB2, rows, kHid, a.h2);
-    check_launch();
-    gemm(ctx, {a.h2, kHid, 1, W + kOffW3, 1, kHid, a.y, kOut, 1, rows, kOut, kHid, 0});
 }
 
 // Inference of the whole network, 32 patches per wave: the three layers as
@@ -572,51 +473,305 @@ void mlp_forward(dwg_ctx* ctx, const dwg_mlp* m, const uint16_t* x, int64_t n, f
     check_launch();
 }
 
+// ---------------------------------------------------------------------------
+// training: loss and gradient of a batch in three launches
+//
+// 1. train_rows_kernel: a block takes 32 rows through the whole network and
+//    back, wave w owning columns 32w .. 32w + 31 of the hidden layers, so 8,192
+//    rows fill the 256 CUs.  Activations and their derivatives stay in
+//    registers and LDS; what the weight gradients need (X, H1, H2, dY, dZ1,
+//    dZ2 in BF16) goes to memory transposed in blocks of 32 rows, so that the
+//    products over the rows read 16 B a lane.  Bias gradients and the loss
+//    are summed over the block's rows in FP64.
+// 2. train_weights_kernel: dW = dZᵀ·H over the batch, the rows split: a wave
+//    takes one 32×32 tile of one weight matrix over 256 rows
+//    (the whole batch in one wave per tile left 4 blocks on the chip).
+// 3. train_sum_kernel: the splits' sums added in a fixed order in FP64.
+// The layer products are the MFMA sequences of mlp_infer_kernel, so the
+// activations are the same bit for bit.  Bound by launches and latencies at
+// the trainer's 8,192 rows (1 GFLOP): 1,240 → 60 µs a step with the read-back
+// of the loss and the gradient.
+// ---------------------------------------------------------------------------
+constexpr int kRows = 32;          // rows of a block
+constexpr int kSplitBlocks = 8;    // blocks of rows a weight-gradient wave sums over, at least
+constexpr int kMaxSplits = 256;    // (more for batches over 65,536 rows: bounds the partial sums' memory)
+constexpr int kYPad = 4;           // dY's columns in memory
+// a block's transposed tiles, in BF16 values: column-major [column][32 rows]
+constexpr int kTX = 0, kTH1 = kTX + kIn * kRows, kTH2 = kTH1 + kHid * kRows, kTD1 = kTH2 + kHid * kRows,
+              kTD2 = kTD1 + kHid * kRows, kTDY = kTD2 + kHid * kRows, kTBlock = kTDY + kYPad * kRows;
+constexpr int kSums = 2 * kHid + kOut + 1;  // FP64 sums of every block: db1, db2, db3, loss, by column
+
+__device__ __forceinline__ void clear(f32x16& a) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) a[q] = 0.f;
+}
+
+// row of accumulator register q in lane `lane`
+__device__ __forceinline__ int acc_row(int q, int lane) { return 8 * (q / 4) + 4 * (lane >> 5) + (q % 4); }
+
+// 8 consecutive BF16 values at a 16-byte boundary (LDS rows, the weights'
+// matrices and the tiles all keep to it)
+__device__ __forceinline__ bf16x8 load8(const uint16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
+static_assert(kOffW2 % 8 == 0 && kOffW3 % 8 == 0 && kIn % 8 == 0 && kHPad % 8 == 0, "16-byte rows");
+
+// a 32-row column of a tile in BF16: this lane's 16 rows of column `c`, to LDS
+// (row-major, when `lds`) and transposed to memory
+__device__ __forceinline__ void store_column(const uint16_t (&v)[16], int c, int lane, uint16_t (*lds)[kHPad],
+                                             uint16_t* __restrict__ tile) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const int r = acc_row(4 * g, lane);
+        if (lds) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) lds[r + j][c] = v[4 * g + j];
+        }
+        const uint2 w = make_uint2(uint32_t(v[4 * g]) | (uint32_t(v[4 * g + 1]) << 16),
+                                   uint32_t(v[4 * g + 2]) | (uint32_t(v[4 * g + 3]) << 16));
+        *reinterpret_cast<uint2*>(tile + c * kRows + r) = w;  // 8-byte aligned: r is a multiple of 4
+    }
+}
+
+// the sum of the tile's column over its 32 rows, in lanes 0 .. 31
+__device__ __forceinline__ double column_sum(const float (&v)[16]) {
+    double s = 0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) s += double(v[q]);
+    return s + __shfl_xor(s, 32, 64);
+}
+
+__global__ __launch_bounds__(256) void train_rows_kernel(const uint16_t* __restrict__ x, const float* __restrict__ target,
+                                                         int64_t rows, int mode, const uint16_t* __restrict__ W,
+                                                         const float* __restrict__ P, uint16_t* __restrict__ tiles,
+                                                         double* __restrict__ sums) {
+    __shared__ __align__(16) uint16_t s_x[kRows][kIn + 8];
+    __shared__ __align__(16) uint16_t s_a[kRows][kHPad];  // H1, then dZ2
+    __shared__ __align__(16) uint16_t s_b[kRows][kHPad];  // H2
+    __shared__ float s_y[kRows][kOut];
+    __shared__ uint16_t s_dy[kRows][kOut];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 31, kq = 8 * (lane >> 5), c = 32 * wave + r;  // c: this lane's hidden column
+    const int64_t row0 = int64_t(blockIdx.x) * kRows;
+    uint16_t* tile = tiles + int64_t(blockIdx.x) * kTBlock;
+    double* sum = sums + blockIdx.x;
+    const int64_t nb = gridDim.x;
+    for (int e = threadIdx.x; e < kRows * kIn; e += 256)
+        s_x[e / kIn][e % kIn] = row0 + e / kIn < rows ? x[row0 * kIn + e] : uint16_t(0);
+    __syncthreads();
+    for (int e = threadIdx.x; e < kIn * kRows / 2; e += 256) {  // X transposed, two rows a store
+        const int col = e / (kRows / 2), rr = 2 * (e % (kRows / 2));
+        reinterpret_cast<uint32_t*>(tile + kTX)[e] = uint32_t(s_x[rr][col]) | (uint32_t(s_x[rr + 1][col]) << 16);
+    }
+    f32x16 acc;
+    float d1[16], d2[16];  // gelu'(z1), gelu'(z2)
+    uint16_t v16[16];
+    // layer 1
+    clear(acc);
+#pragma unroll
+    for (int k0 = 0; k0 < kIn; k0 += 16)
+        acc = mfma_32x32x16(load8(&s_x[r][k0 + kq]), load8(W + kOffW1 + int64_t(c) * kIn + k0 + kq), acc);
+    const float b1 = P[kOffB1 + c], b2 = P[kOffB2 + c];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        v16[q] = to_bf16(gelu(acc[q] + b1, &d1[q]));
+    }
+    store_column(v16, c, lane, s_a, tile + kTH1);
+    __syncthreads();
+    // layer 2
+    clear(acc);
+#pragma unroll
+    for (int k0 = 0; k0 < kHid; k0 += 16)
+        acc = mfma_32x32x16(load8(&s_a[r][k0 + kq]), load8(W + kOffW2 + int64_t(c) * kHid + k0 + kq), acc);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        v16[q] = to_bf16(gelu(acc[q] + b2, &d2[q]));
+    }
+    store_column(v16, c, lane, s_b, tile + kTH2);
+    __syncthreads();
+    // layer 3 and the loss of each row, in one wave
+    if (wave == 0) {
+        clear(acc);
+#pragma unroll
+        for (int k0 = 0; k0 < kHid; k0 += 16) {
+            bf16x8 b;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) b[j] = 0;
+            if (r < kOut) b = load8(W + kOffW3 + int64_t(r) * kHid + k0 + kq);
+            acc = mfma_32x32x16(load8(&s_b[r][k0 + kq]), b, acc);
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            if (r < kOut) s_y[acc_row(q, lane)][r] = acc[q];
+        __builtin_amdgcn_wave_barrier();
+        // oriented:  loss = mean(1 − c),  dL/dy = −(t − c ŷ)/(|y|·B)
+        // line:      loss = mean(1 − c²), dL/dy = −2c (t − c ŷ)/(|y|·B),   c = ŷ·t
+        double l = 0;
+        float g[kOut] = {0.f, 0.f, 0.f};
+        const int64_t row = row0 + r;
+        if (lane < kRows && row < rows) {
+            const float y0 = s_y[r][0] + P[kOffB3], y1 = s_y[r][1] + P[kOffB3 + 1], y2 = s_y[r][2] + P[kOffB3 + 2];
+            const float ny = sqrtf(y0 * y0 + y1 * y1 + y2 * y2) + 1e-12f;
+            const float h0 = y0 / ny, h1 = y1 / ny, h2 = y2 / ny;
+            const float t0 = target[3 * row], t1 = target[3 * row + 1], t2 = target[3 * row + 2];
+            const float cs = h0 * t0 + h1 * t1 + h2 * t2;
+            l = mode ? 1.0 - double(cs) * double(cs) : 1.0 - double(cs);
+            const float s = (mode ? -2.0f * cs : -1.0f) / (ny * float(rows));
+            g[0] = s * (t0 - cs * h0);
+            g[1] = s * (t1 - cs * h1);
+            g[2] = s * (t2 - cs * h2);
+        }
+        if (lane < kRows) {
+#pragma unroll
+            for (int k = 0; k < kOut; ++k) {
+                s_dy[r][k] = to_bf16(g[k]);
+                tile[kTDY + k * kRows + r] = to_bf16(g[k]);
+            }
+        }
+        double v[kOut + 1] = {double(g[0]), double(g[1]), double(g[2]), l};
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1)
+#pragma unroll
+            for (int k = 0; k <= kOut; ++k) v[k] += __shfl_xor(v[k], off, 64);
+        if (lane == 0)
+#pragma unroll
+            for (int k = 0; k <= kOut; ++k) sum[(2 * kHid + k) * nb] = v[k];
+    }
+    __syncthreads();
+    // dH2 = dY·W3 (K = 3 of 16), dZ2 = dH2 · gelu'(z2)
+    float d[16];
+    {
+        bf16x8 a, b;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            a[j] = (lane < 32 && j < kOut) ? short(s_dy[r][j < kOut ? j : 0]) : short(0);
+            b[j] = (lane < 32 && j < kOut) ? short(W[kOffW3 + (j < kOut ? j : 0) * kHid + c]) : short(0);
+        }
+        clear(acc);
+        acc = mfma_32x32x16(a, b, acc);
+    }
+    // (H1 in s_a was last read before two barriers)
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        d[q] = acc[q] * d2[q];
+        v16[q] = to_bf16(d[q]);
+    }
+    store_column(v16, c, lane, s_a, tile + kTD2);
+    double cs = column_sum(d);
+    if (lane < 32) sum[(kHid + c) * nb] = cs;
+    __syncthreads();
+    // dH1 = dZ2·W2, dZ1 = dH1 · gelu'(z1)
+    clear(acc);
+#pragma unroll
+    for (int k0 = 0; k0 < kHid; k0 += 16)
+        acc = mfma_32x32x16(load8(&s_a[r][k0 + kq]), load8(W + kOffW2T + c * kHid + k0 + kq), acc);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        d[q] = acc[q] * d1[q];
+        v16[q] = to_bf16(d[q]);
+    }
+    store_column(v16, c, lane, nullptr, tile + kTD1);
+    cs = column_sum(d);
+    if (lane < 32) sum[c * nb] = cs;
+}
+
+// tiles of the weight gradients: dW1 4 × 2 (48 columns), dW2 4 × 4, dW3 1 × 4
+constexpr int kTilesW1 = 8, kTilesW2 = 16, kTilesW3 = 4, kWeightTiles = kTilesW1 + kTilesW2 + kTilesW3;
+
+__global__ __launch_bounds__(256) void train_weights_kernel(const uint16_t* __restrict__ tiles, int blocks, int per,
+                                                            float* __restrict__ part) {
+    static_assert(kWeightTiles % 4 == 0, "whole blocks of four tiles");
+    const int split = blockIdx.y;
+    const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int r = lane & 31, kq = 8 * (lane >> 5);
+    int at, bt, i0, j0, ni, nj;
+    int64_t out;
+    if (t < kTilesW1) {
+        at = kTD1, bt = kTX, i0 = 32 * (t / 2), j0 = 32 * (t % 2), ni = kHid, nj = kIn, out = kOffW1;
+    } else if (t < kTilesW1 + kTilesW2) {
+        const int u = t - kTilesW1;
+        at = kTD2, bt = kTH1, i0 = 32 * (u / 4), j0 = 32 * (u % 4), ni = kHid, nj = kHid, out = kOffW2;
+    } else {
+        at = kTDY, bt = kTH2, i0 = 0, j0 = 32 * (t - kTilesW1 - kTilesW2), ni = kOut, nj = kHid, out = kOffW3;
+    }
+    // rows and columns past the matrix repeat its last one: they end in
+    // entries of the product that are not stored
+    const uint16_t* pa = tiles + at + min(i0 + r, ni - 1) * kRows + kq;
+    const uint16_t* pb = tiles + bt + min(j0 + r, nj - 1) * kRows + kq;
+    const int b0 = split * per, b1 = min(b0 + per, blocks);
+    f32x16 acc;
+    clear(acc);
+    int b = b0;
+    for (; b + 4 <= b1; b += 4) {  // the loads of four blocks of rows in flight
+        bf16x8 a[8], w[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int64_t o = int64_t(b + u / 2) * kTBlock + 16 * (u % 2);
+            a[u] = load8(pa + o);
+            w[u] = load8(pb + o);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc = mfma_32x32x16(a[u], w[u], acc);
+    }
+    for (; b < b1; ++b)
+#pragma unroll
+        for (int k0 = 0; k0 < kRows; k0 += 16)
+            acc = mfma_32x32x16(load8(pa + int64_t(b) * kTBlock + k0), load8(pb + int64_t(b) * kTBlock + k0), acc);
+    float* o = part + int64_t(split) * kParams + out;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const int i = i0 + acc_row(q, lane), j = j0 + r;
+        if (i < ni && j < nj) o[int64_t(i) * nj + j] = acc[q];
+    }
+}
+
+// The first kSums waves: a bias's gradient, or the loss, each from its column
+// of the blocks' sums; then the weights' gradients, one a thread, from the
+// splits' sums
+constexpr int kSumBlocks = (kSums + 3) / 4;
+__global__ __launch_bounds__(256) void train_sum_kernel(const float* __restrict__ part, int splits,
+                                                        const double* __restrict__ sums, int blocks,
+                                                        float* __restrict__ grad, double* __restrict__ loss) {
+    if (blockIdx.x < kSumBlocks) {
+        const int col = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+        if (col >= kSums) return;
+        double s = 0;
+        for (int b = lane; b < blocks; b += 64) s += sums[int64_t(col) * blocks + b];
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) s += __shfl_xor(s, off, 64);
+        if (lane != 0) return;
+        if (col < kHid) grad[kOffB1 + col] = float(s);
+        else if (col < 2 * kHid) grad[kOffB2 + col - kHid] = float(s);
+        else if (col < kSums - 1) grad[kOffB3 + col - 2 * kHid] = float(s);
+        else *loss = s;
+        return;
+    }
+    const int64_t i = int64_t(blockIdx.x - kSumBlocks) * 256 + threadIdx.x;
+    const bool bias = (i >= kOffB1 && i < kOffW2) || (i >= kOffB2 && i < kOffW3) || i >= kOffB3;
+    if (bias) return;
+    double s = 0;
+#pragma unroll 8
+    for (int k = 0; k < splits; ++k) s += double(part[int64_t(k) * kParams + i]);
+    grad[i] = float(s);
+}
+
 double mlp_loss_grad(dwg_ctx* ctx, dwg_mlp* m, const uint16_t* x, const float* target, int64_t B, int mode) {
     DWG_REQUIRE(B > 0, "empty batch");
     ProfileScope ps(ctx, "mlp_train");
-    Acts a = acts(ctx, B);
-    forward(ctx, m, x, B, a);
-    hipLaunchKernelGGL(add_bias_normalize_kernel, dim3(grid_for(B, 256)), dim3(256), 0, ctx->stream, a.y,
-                       m->params + kOffB3, B, 0);
+    const int blocks = int(grid_for(B, kRows));
+    const int per = std::max(kSplitBlocks, (blocks + kMaxSplits - 1) / kMaxSplits), splits = (blocks + per - 1) / per;
+    uint16_t* tiles = static_cast<uint16_t*>(ctx->buf("mlp_tiles", sizeof(uint16_t) * size_t(blocks) * kTBlock));
+    double* sums = static_cast<double*>(ctx->buf("mlp_sums", sizeof(double) * (size_t(blocks) * kSums + 1)));
+    float* part = static_cast<float*>(ctx->buf("mlp_part", sizeof(float) * size_t(splits) * kParams));
+    double* loss = sums + size_t(blocks) * kSums;
+    hipLaunchKernelGGL(train_rows_kernel, dim3(blocks), dim3(256), 0, ctx->stream, x, target, B, mode, m->bf16, m->params,
+                       tiles, sums);
     check_launch();
-    float* dy = static_cast<float*>(ctx->buf("mlp_dy", sizeof(float) * B * kOut));
-    uint16_t* dy16 = static_cast<uint16_t*>(ctx->buf("mlp_dy16", sizeof(uint16_t) * B * kOut));
-    const unsigned lb = grid_for(B, 256);
-    double* lpart = static_cast<double*>(ctx->buf("mlp_loss", sizeof(double) * (lb + 1)));
-    hipLaunchKernelGGL(loss_kernel, dim3(lb), dim3(256), 0, ctx->stream, a.y, target, B, mode, dy, dy16, lpart);
+    hipLaunchKernelGGL(train_weights_kernel, dim3(kWeightTiles / 4, splits), dim3(256), 0, ctx->stream, tiles, blocks, per,
+                       part);
     check_launch();
-    float* G = m->grad;
-    const uint16_t* W = m->bf16;
-    // layer 3: dW3 = dYᵀ·H2, db3 = Σ dY, dH2 = dY·W3
-    gemm(ctx, {dy16, 1, kOut, a.h2, kHid, 1, G + kOffW3, kHid, 1, kOut, kHid, B, 0});
-    hipLaunchKernelGGL(colsum_kernel, dim3(kOut), dim3(256), 0, ctx->stream, dy, B, kOut, G + kOffB3);
+    hipLaunchKernelGGL(train_sum_kernel, dim3(kSumBlocks + grid_for(kParams, 256)), dim3(256), 0, ctx->stream, part, splits, sums,
+                       blocks, m->grad, loss);
     check_launch();
-    float* dh = static_cast<float*>(ctx->buf("mlp_dh", sizeof(float) * B * kHid));
-    float* dz32 = static_cast<float*>(ctx->buf("mlp_dz32", sizeof(float) * B * kHid));
-    uint16_t* dz = static_cast<uint16_t*>(ctx->buf("mlp_dz", sizeof(uint16_t) * B * kHid));
-    gemm(ctx, {dy16, kOut, 1, W + kOffW3, kHid, 1, dh, kHid, 1, B, kHid, kOut, 0});
-    hipLaunchKernelGGL(gelu_back_kernel, dim3(grid_for(B * kHid, 256)), dim3(256), 0, ctx->stream, dh, a.z2, B * kHid,
-                       dz, dz32);
-    check_launch();
-    // layer 2: dW2 = dZ2ᵀ·H1, db2 = Σ dZ2, dH1 = dZ2·W2
-    gemm(ctx, {dz, 1, kHid, a.h1, kHid, 1, G + kOffW2, kHid, 1, kHid, kHid, B, 0});
-    hipLaunchKernelGGL(colsum_kernel, dim3(kHid), dim3(256), 0, ctx->stream, dz32, B, kHid, G + kOffB2);
-    check_launch();
-    gemm(ctx, {dz, kHid, 1, W + kOffW2, kHid, 1, dh, kHid, 1, B, kHid, kHid, 0});
-    hipLaunchKernelGGL(gelu_back_kernel, dim3(grid_for(B * kHid, 256)), dim3(256), 0, ctx->stream, dh, a.z1, B * kHid,
-                       dz, dz32);
-    check_launch();
-    // layer 1: dW1 = dZ1ᵀ·X, db1 = Σ dZ1
-    gemm(ctx, {dz, 1, kHid, x, kIn, 1, G + kOffW1, kIn, 1, kHid, kIn, B, 0});
-    hipLaunchKernelGGL(colsum_kernel, dim3(kHid), dim3(256), 0, ctx->stream, dz32, B, kHid, G + kOffB1);
-    check_launch();
-    std::vector<double> h(lb);
-    DWG_HIP_CHECK(hipMemcpyAsync(h.data(), lpart, sizeof(double) * lb, hipMemcpyDeviceToHost, ctx->stream));
-    DWG_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-    double l = 0;
-    for (double v : h) l += v;
-    return l / double(B);
+    return read_scalar<double>(ctx, loss) / double(B);
 }
 
 void mlp_adam(dwg_ctx* ctx, dwg_mlp* m, float lr, float b1, float b2, float eps) {

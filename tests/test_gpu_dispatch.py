@@ -6,6 +6,7 @@ import torch
 
 import oracle as O
 from dwg_amd import gpu, shapes
+from oracle import mlp as M
 
 pytestmark = pytest.mark.gpu
 
@@ -173,3 +174,34 @@ def test_tree_sums_by_query_count(ctx, n, nq, ordered, screened, radii, bf16):
     assert np.abs(wg - ref).max() <= 1e-5 * np.abs(ref).max()
     rw, rg = o.eval_grad(Q[sub].astype(np.float64), 2.3, kind=kind, sigma=SIGMA, radii=rad)
     assert np.abs(g - rg).max() <= 1e-4 * np.abs(rg).max()  # the tree gradient's bound
+
+
+# one row, a block of rows but one, one past it, past one split of the rows,
+# past a multiple of it, and enough splits to take more rows each
+@pytest.mark.parametrize("batch", [1, 31, 33, 257, 2049, 70_001])
+@pytest.mark.parametrize("line", [False, True])
+def test_training_gradient_by_batch(ctx, batch, line):
+    rng = np.random.default_rng(batch)
+    theta = np.concatenate([(rng.uniform(-1, 1, s) / np.sqrt(s[1] if len(s) == 2 else 64)).ravel()
+                            for s in M.SIZES]).astype(np.float32)
+    net = gpu.Mlp(ctx, 0)
+    net.set_params(theta)
+    X = M.to_bf16(rng.normal(size=(batch, 48)).astype(np.float32))
+    T = rng.normal(size=(batch, 3)) + [1.0, 0.5, 0.0]
+    T /= np.linalg.norm(T, axis=1, keepdims=True)
+    xb = torch.from_numpy(M.bf16_bits(X).view(np.int16)).cuda()
+    loss = net.loss_grad(xb, torch.from_numpy(T.astype(np.float32)), line=line)
+    g = net.grad().astype(np.float64)
+    W = [torch.from_numpy(M.to_bf16(a.astype(np.float32)).astype(np.float64) if a.ndim == 2 else a.astype(np.float64))
+         .requires_grad_(True) for a in M.unpack(theta)]
+    h = torch.from_numpy(X.astype(np.float64))
+    for w, b in ((W[0], W[1]), (W[2], W[3])):
+        h = torch.nn.functional.gelu(h @ w.T + b, approximate="tanh")
+    y = h @ W[4].T + W[5]
+    c = (y / y.norm(dim=1, keepdim=True) * torch.from_numpy(T)).sum(1)
+    ref = (1 - c * c if line else 1 - c).mean()
+    ref.backward()
+    rg = torch.cat([w.grad.reshape(-1) for w in W]).numpy()
+    # the bounds of the 512-row gradient: BF16 activations and their gradients
+    assert loss == pytest.approx(float(ref.detach()), abs=1e-2 if batch < 32 else 1e-3)
+    assert np.linalg.norm(g - rg) < 0.03 * np.linalg.norm(rg)
