@@ -677,19 +677,23 @@ struct QueryArgs {
     int64_t nq;
     float ox, oy, oz, h;
     int rx, ry, rz;
-    int bx, by, bz;  // bricks per axis (kPartsX·4 × kPartsY·4 × kPartsZ·4 points per brick)
+    int parts;       // 4×4×4 parts of a brick (grid walks): kGridParts or 1
+    int lanes;       // points of a part, or explicit queries, a wave takes: 16, 32 or 64
+    int bx, by, bz;  // bricks per axis
     int64_t n_bricks;
     int stack;  // walk stack entries (tree_stack_entries of the tree's depth)
 };
 
 
-template <bool SCREENED, bool COUNT, bool BF16, bool GRID, bool NEAR64 = false>
+template <bool SCREENED, bool COUNT, bool BF16, int GRID, bool NEAR64 = false>
 __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, QueryArgs Q, float beta, float sigma,
                                                                  uint32_t flags, float* __restrict__ out,
                                                                  int64_t* __restrict__ terms_out) {
     // grid walks: each lane evaluates kGridParts points (one per 4×4×4 part
     // of the brick), so that a pop, its loads and its pushes serve them all
-    constexpr int H = GRID ? kGridParts : kPointPts;
+    constexpr int H = GRID ? GRID : kPointPts;
+    constexpr int PX = GRID == kGridParts ? kPartsX : 1, PY = GRID == kGridParts ? kPartsY : 1,
+                  PZ = GRID == kGridParts ? kPartsZ : 1;
     static_assert(kTreeWaves == 1, "one wave per block: the stack lives in the block's dynamic LDS");
     // the stack: Q.stack entries of (record, H lane masks), in dynamic LDS
     // sized by the tree's depth (a shallow tree leaves room for more blocks)
@@ -709,8 +713,8 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
         // H consecutive runs of 64 queries
 #pragma unroll
         for (int h = 0; h < H; ++h) {
-            qi[h] = (wid * H + h) * 64 + lane;
-            valid[h] = qi[h] < Q.nq;
+            qi[h] = (wid * H + h) * Q.lanes + lane;
+            valid[h] = lane < Q.lanes && qi[h] < Q.nq;
             if (Q.self_perm) {  // consecutive tree slots: spatially coherent waves
                 const float4 a = valid[h] ? T.sa[qi[h]] : make_float4(0.f, 0.f, 0.f, 0.f);
                 qx[h] = a.x;
@@ -732,10 +736,10 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
         bzi = int(br / (int64_t(Q.bx) * Q.by));
 #pragma unroll
         for (int h = 0; h < H; ++h) {
-            const int x = (bxi * kPartsX + h % kPartsX) * 4 + (lane & 3);
-            const int y = (byi * kPartsY + (h / kPartsX) % kPartsY) * 4 + ((lane >> 2) & 3);
-            const int z = (bzi * kPartsZ + h / (kPartsX * kPartsY)) * 4 + (lane >> 4);
-            valid[h] = br < Q.n_bricks && x < Q.rx && y < Q.ry && z < Q.rz;
+            const int x = (bxi * PX + h % PX) * 4 + (lane & 3);
+            const int y = (byi * PY + (h / PX) % PY) * 4 + ((lane >> 2) & 3);
+            const int z = H > 1 ? (bzi * PZ + h / (PX * PY)) * 4 + (lane >> 4) : bzi * (Q.lanes >> 4) + (lane >> 4);
+            valid[h] = lane < Q.lanes && br < Q.n_bricks && x < Q.rx && y < Q.ry && z < Q.rz;
             qi[h] = int64_t(x) + int64_t(Q.rx) * (int64_t(y) + int64_t(Q.ry) * z);
             qx[h] = __builtin_fmaf(float(x), Q.h, Q.ox);
             qy[h] = __builtin_fmaf(float(y), Q.h, Q.oy);
@@ -812,13 +816,14 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
     constexpr bool BOX = GRID && !COUNT && !NEAR64;
     float blx = 0.f, bly = 0.f, blz = 0.f, bhx = 0.f, bhy = 0.f, bhz = 0.f;
     if (BOX) {
-        const int x0 = bxi * kPartsX * 4, y0 = byi * kPartsY * 4, z0 = bzi * kPartsZ * 4;
+        const int zn = H > 1 ? kPartsZ * 4 : Q.lanes >> 4;
+        const int x0 = bxi * PX * 4, y0 = byi * PY * 4, z0 = bzi * zn;
         blx = __builtin_fmaf(float(x0), Q.h, Q.ox);
         bly = __builtin_fmaf(float(y0), Q.h, Q.oy);
         blz = __builtin_fmaf(float(z0), Q.h, Q.oz);
-        bhx = __builtin_fmaf(float(x0 + 4 * kPartsX - 1), Q.h, Q.ox);
-        bhy = __builtin_fmaf(float(y0 + 4 * kPartsY - 1), Q.h, Q.oy);
-        bhz = __builtin_fmaf(float(z0 + 4 * kPartsZ - 1), Q.h, Q.oz);
+        bhx = __builtin_fmaf(float(x0 + 4 * PX - 1), Q.h, Q.ox);
+        bhy = __builtin_fmaf(float(y0 + 4 * PY - 1), Q.h, Q.oy);
+        bhz = __builtin_fmaf(float(z0 + zn - 1), Q.h, Q.oz);
     }
 
     // the stack holds (traversal record of a node to open, lanes that open
@@ -1418,6 +1423,7 @@ static QueryArgs make_points(const float* q, int64_t nq) {
     QueryArgs Q{};
     Q.q = q;
     Q.nq = nq;
+    Q.lanes = 64;
     return Q;
 }
 
@@ -1425,10 +1431,21 @@ static QueryArgs make_self(const dwg_octree* T) {
     QueryArgs Q{};
     Q.self_perm = T->perm;
     Q.nq = T->n_points;
+    Q.lanes = 64;
     return Q;
 }
 
-static QueryArgs make_grid(const dwg_grid* g) {
+// Grids of fewer whole bricks than this leave the chip short of waves, and
+// the launch lasts as long as its longest walks: they take one 4×4×4 part a
+// wave, whose walk opens fewer nodes and lasts a quarter as long (64³ over 100k
+// sources 628 → 250 µs, 160³ over 500k 1,106 → 916 µs; at 256³, 65,536 bricks,
+// whole ones win, 1,776 against 2,204 µs), and grids of very few parts half a
+// part (33×29×31 over 2,000 sources 181 → 72 µs, whole parts 77 µs).  The
+// values are the same: each point takes its own terms in the same order
+constexpr int64_t kWholeBricks = 24576, kHalfParts = 1536;
+
+// `whole_bricks`: for the walks that take no others
+static QueryArgs make_grid(const dwg_grid* g, bool whole_bricks) {
     QueryArgs Q{};
     Q.grid = true;
     Q.ox = g->origin[0];
@@ -1438,10 +1455,21 @@ static QueryArgs make_grid(const dwg_grid* g) {
     Q.rx = g->res[0];
     Q.ry = g->res[1];
     Q.rz = g->res[2];
-    Q.bx = (Q.rx + 4 * kPartsX - 1) / (4 * kPartsX);
-    Q.by = (Q.ry + 4 * kPartsY - 1) / (4 * kPartsY);
-    Q.bz = (Q.rz + 4 * kPartsZ - 1) / (4 * kPartsZ);
-    Q.n_bricks = int64_t(Q.bx) * Q.by * Q.bz;
+    auto bricks = [&](int parts, int lanes) {
+        const bool many = parts == kGridParts;
+        const int nx = many ? 4 * kPartsX : 4, ny = many ? 4 * kPartsY : 4, nz = many ? 4 * kPartsZ : lanes / 16;
+        Q.parts = parts;
+        Q.lanes = lanes;
+        Q.bx = (Q.rx + nx - 1) / nx;
+        Q.by = (Q.ry + ny - 1) / ny;
+        Q.bz = (Q.rz + nz - 1) / nz;
+        Q.n_bricks = int64_t(Q.bx) * Q.by * Q.bz;
+    };
+    bricks(kGridParts, 64);
+    if (!whole_bricks && Q.n_bricks < kWholeBricks) {
+        bricks(1, 64);
+        if (Q.n_bricks < kHalfParts) bricks(1, 32);
+    }
     Q.nq = int64_t(Q.rx) * Q.ry * Q.rz;
     return Q;
 }
@@ -1509,7 +1537,7 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
         launch_walk<false>(ctx, T, Q.q, Q.nq, sigma, flags, out, nullptr);
         return;
     }
-    const int64_t waves = Q.grid ? Q.n_bricks : (Q.nq + 64 * kPointPts - 1) / (64 * kPointPts);
+    const int64_t waves = Q.grid ? Q.n_bricks : (Q.nq + Q.lanes * kPointPts - 1) / (Q.lanes * kPointPts);
     if (waves == 0) return;
     TreeArgs A{T->info, T->kid, T->cm_r, reinterpret_cast<const float*>(T->payload), T->sa, T->sb};
     dim3 grid(grid_for(waves, kTreeWaves)), block(kTreeThreads);
@@ -1517,27 +1545,36 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
     QueryArgs Qs = Q;
     Qs.stack = tree_stack_entries(std::max(T->max_level, 1));
     if (Q.q && Q.nq >= kShareValue) Qs.order = query_order(ctx, T, Q.q, Q.nq);
-    const size_t lds = sizeof(uint64_t) * size_t(Qs.stack) * size_t(1 + (Q.grid ? kGridParts : kPointPts));
+    const size_t lds = sizeof(uint64_t) * size_t(Qs.stack) * size_t(1 + (Q.grid ? Q.parts : kPointPts));
     const bool scr = flags & DWG_SCREENED, bf = flags & DWG_FAR_BF16;
     const char* name = count ? "gwn_tree_terms" : (!Q.grid ? (scr ? "gwn_tree_screened" : "gwn_tree_plain")
                                                            : (scr ? "gwn_tree_grid_screened" : "gwn_tree_grid_plain"));
     ProfileScope ps(ctx, name);
 #define DWG_TREE_LAUNCH(S, C, B, G, N) \
     hipLaunchKernelGGL((gwn_tree_kernel<S, C, B, G, N>), grid, block, lds, ctx->stream, A, Qs, beta, sigma, flags, out, terms)
-#define DWG_TREE_LAUNCH_Q(S, C, B, N)       \
-    do {                                    \
-        if (!Q.grid)                        \
-            DWG_TREE_LAUNCH(S, C, B, false, N); \
-        else                                \
-            DWG_TREE_LAUNCH(S, C, B, true, N);  \
+#define DWG_TREE_LAUNCH_Q(S, C, B, N)                \
+    do {                                             \
+        if (!Q.grid)                                 \
+            DWG_TREE_LAUNCH(S, C, B, 0, N);          \
+        else                                         \
+            DWG_TREE_LAUNCH(S, C, B, kGridParts, N); \
+    } while (0)
+// (the counting and the FP64 near-field walks take whole bricks only)
+#define DWG_TREE_LAUNCH_P(S, B)                 \
+    do {                                        \
+        if (Q.grid && Q.parts == 1)             \
+            DWG_TREE_LAUNCH(S, false, B, 1, false); \
+        else                                    \
+            DWG_TREE_LAUNCH_Q(S, false, B, false);  \
     } while (0)
     if (count) DWG_TREE_LAUNCH_Q(false, true, false, false);
     else if (near64 && bf) DWG_TREE_LAUNCH_Q(true, false, true, true);
     else if (near64) DWG_TREE_LAUNCH_Q(true, false, false, true);
-    else if (scr && bf) DWG_TREE_LAUNCH_Q(true, false, true, false);
-    else if (scr) DWG_TREE_LAUNCH_Q(true, false, false, false);
-    else if (bf) DWG_TREE_LAUNCH_Q(false, false, true, false);
-    else DWG_TREE_LAUNCH_Q(false, false, false, false);
+    else if (scr && bf) DWG_TREE_LAUNCH_P(true, true);
+    else if (scr) DWG_TREE_LAUNCH_P(true, false);
+    else if (bf) DWG_TREE_LAUNCH_P(false, true);
+    else DWG_TREE_LAUNCH_P(false, false);
+#undef DWG_TREE_LAUNCH_P
 #undef DWG_TREE_LAUNCH_Q
 #undef DWG_TREE_LAUNCH
     check_launch();
@@ -1557,7 +1594,8 @@ void gwn_tree_self(dwg_ctx* ctx, const dwg_octree* T, float beta, float sigma, u
 void gwn_tree_grid(dwg_ctx* ctx, const dwg_octree* T, const dwg_grid* g, float beta, float sigma, uint32_t flags,
                    float* out) {
     DWG_REQUIRE(g && g->res[0] > 0 && g->res[1] > 0 && g->res[2] > 0 && g->h > 0, "bad grid");
-    launch_tree(ctx, T, make_grid(g), beta, sigma, flags, out, nullptr, false);
+    launch_tree(ctx, T, make_grid(g, (flags & DWG_SCREENED) && (flags & DWG_NEAR_FP64)), beta, sigma, flags, out, nullptr,
+                false);
 }
 
 void gwn_tree_grad(dwg_ctx* ctx, const dwg_octree* Tc, const float* q, int64_t nq, float beta, float sigma,
@@ -1617,7 +1655,7 @@ __global__ void sum_i64_kernel(const int64_t* __restrict__ v, int64_t n, unsigne
 }
 
 int64_t gwn_tree_grid_terms(dwg_ctx* ctx, const dwg_octree* T, const dwg_grid* g, float beta) {
-    QueryArgs Q = make_grid(g);
+    QueryArgs Q = make_grid(g, true);
     int64_t* terms = static_cast<int64_t*>(ctx->buf("grid_terms", sizeof(int64_t) * (Q.nq + 1)));
     unsigned long long* tot = reinterpret_cast<unsigned long long*>(terms + Q.nq);
     fill_u32(ctx, tot, 0, 2);

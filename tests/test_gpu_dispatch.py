@@ -62,12 +62,13 @@ def test_direct_sums_split_over_sources(ctx, n, nq, screened, kahan):
     assert (np.abs(g - rg) <= 2 * tol * mg + 1e-30).all()
 
 
-# bricks cut by every face of the grid, a grid inside one brick, grids far
-# from and across the cloud, and a cloud far from the origin (large residuals
-# of the rounded centres)
+# half parts, whole parts and whole bricks cut by every face of the grid, a grid
+# inside one, grids far from and across the cloud, and a cloud far from the
+# origin (large residuals of the rounded centres)
 @pytest.mark.parametrize("res,h,shift", [((8, 4, 8), 0.05, 0.0), ((9, 5, 7), 0.002, 0.0), ((1, 1, 1), 0.1, 0.0),
                                          ((33, 29, 31), 0.08, 0.0), ((23, 3, 17), 0.3, 0.0),
-                                         ((25, 26, 9), 0.05, 100.0)])
+                                         ((25, 26, 9), 0.05, 100.0), ((45, 47, 50), 0.02, 0.0),
+                                         ((190, 181, 183), 0.005, 0.0), ((193, 189, 185), 0.005, 0.0)])
 @pytest.mark.parametrize("screened,bf16,radii", [(True, False, False), (True, True, True), (False, False, False),
                                                  (False, True, False)])
 def test_grid_walk_equals_the_point_walk(ctx, res, h, shift, screened, bf16, radii):
@@ -83,12 +84,13 @@ def test_grid_walk_equals_the_point_walk(ctx, res, h, shift, screened, bf16, rad
     tree.update(N, A, R)
     c = P.mean(0)
     grid = gpu.make_grid([c[d] - 0.5 * h * (res[d] - 1) for d in range(3)], h, res)
-    ax = [np.array([np.float32(np.float64(i) * grid.h + grid.origin[d]) for i in range(res[d])]) for d in range(3)]
+    ax = [(np.arange(res[d]) * np.float64(grid.h) + grid.origin[d]).astype(np.float32) for d in range(3)]
     z, y, x = np.meshgrid(ax[2], ax[1], ax[0], indexing="ij")
     Q = torch.from_numpy(np.stack([x, y, z], -1).reshape(-1, 3).astype(np.float32)).cuda()
     kw = dict(sigma=SIGMA, screened=screened, bf16=bf16)
     got = tree.eval_grid(grid, 2.3, **kw).cpu().numpy()
-    want = tree.eval(Q.repeat(200_000 // len(Q) + 1, 1), 2.3, **kw).cpu().numpy()[:len(Q)]
+    many = Q if len(Q) > 200_000 else Q.repeat(200_000 // len(Q) + 1, 1)
+    want = tree.eval(many, 2.3, **kw).cpu().numpy()[:len(Q)]
     np.testing.assert_array_equal(got, want)
 
 
