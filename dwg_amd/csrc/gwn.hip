@@ -678,7 +678,6 @@ struct QueryArgs {
     float ox, oy, oz, h;
     int rx, ry, rz;
     int parts;       // 4×4×4 parts of a brick (grid walks): kGridParts or 1
-    int lanes;       // points of a part, or explicit queries, a wave takes: 16, 32 or 64
     int bx, by, bz;  // bricks per axis
     int64_t n_bricks;
     int stack;  // walk stack entries (tree_stack_entries of the tree's depth)
@@ -713,8 +712,8 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
         // H consecutive runs of 64 queries
 #pragma unroll
         for (int h = 0; h < H; ++h) {
-            qi[h] = (wid * H + h) * Q.lanes + lane;
-            valid[h] = lane < Q.lanes && qi[h] < Q.nq;
+            qi[h] = (wid * H + h) * 64 + lane;
+            valid[h] = qi[h] < Q.nq;
             if (Q.self_perm) {  // consecutive tree slots: spatially coherent waves
                 const float4 a = valid[h] ? T.sa[qi[h]] : make_float4(0.f, 0.f, 0.f, 0.f);
                 qx[h] = a.x;
@@ -738,8 +737,8 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
         for (int h = 0; h < H; ++h) {
             const int x = (bxi * PX + h % PX) * 4 + (lane & 3);
             const int y = (byi * PY + (h / PX) % PY) * 4 + ((lane >> 2) & 3);
-            const int z = H > 1 ? (bzi * PZ + h / (PX * PY)) * 4 + (lane >> 4) : bzi * (Q.lanes >> 4) + (lane >> 4);
-            valid[h] = lane < Q.lanes && br < Q.n_bricks && x < Q.rx && y < Q.ry && z < Q.rz;
+            const int z = (bzi * PZ + h / (PX * PY)) * 4 + (lane >> 4);
+            valid[h] = br < Q.n_bricks && x < Q.rx && y < Q.ry && z < Q.rz;
             qi[h] = int64_t(x) + int64_t(Q.rx) * (int64_t(y) + int64_t(Q.ry) * z);
             qx[h] = __builtin_fmaf(float(x), Q.h, Q.ox);
             qy[h] = __builtin_fmaf(float(y), Q.h, Q.oy);
@@ -816,14 +815,13 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
     constexpr bool BOX = GRID && !COUNT && !NEAR64;
     float blx = 0.f, bly = 0.f, blz = 0.f, bhx = 0.f, bhy = 0.f, bhz = 0.f;
     if (BOX) {
-        const int zn = H > 1 ? kPartsZ * 4 : Q.lanes >> 4;
-        const int x0 = bxi * PX * 4, y0 = byi * PY * 4, z0 = bzi * zn;
+        const int x0 = bxi * PX * 4, y0 = byi * PY * 4, z0 = bzi * PZ * 4;
         blx = __builtin_fmaf(float(x0), Q.h, Q.ox);
         bly = __builtin_fmaf(float(y0), Q.h, Q.oy);
         blz = __builtin_fmaf(float(z0), Q.h, Q.oz);
         bhx = __builtin_fmaf(float(x0 + 4 * PX - 1), Q.h, Q.ox);
         bhy = __builtin_fmaf(float(y0 + 4 * PY - 1), Q.h, Q.oy);
-        bhz = __builtin_fmaf(float(z0 + zn - 1), Q.h, Q.oz);
+        bhz = __builtin_fmaf(float(z0 + 4 * PZ - 1), Q.h, Q.oz);
     }
 
     // the stack holds (traversal record of a node to open, lanes that open
@@ -1174,6 +1172,141 @@ __global__ __launch_bounds__(kWalkWaves * 64) void gwn_walk_kernel(TreeArgs T, c
     }
 }
 
+// The sums at the tree's own points (Q.self_perm) or at the points of a grid,
+// 8 lanes a point as gwn_walk_kernel walks, but with each point's terms summed exactly as a lane of the shared walk sums
+// them: the 8 children's terms of an opened node are computed side by side and
+// added from child 0 to child 7, node by node in the same depth-first order, so
+// the values are the shared walk's bit for bit.  For clouds and grids whose
+// shared walks (up to 64 points a wave) leave most of the chip idle: bound by
+// the latency of a node's records along one point's walk.
+template <int CTRL>
+__device__ __forceinline__ float dpp_row(float v) {  // lanes without a source keep v
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+
+template <bool SCREENED, bool BF16>
+__global__ __launch_bounds__(kWalkWaves * 64) void gwn_ordered_walk_kernel(TreeArgs T, QueryArgs Q, float sigma,
+                                                                            uint32_t flags,
+                                                                            float* __restrict__ out) {
+    extern __shared__ int s_stacks[];  // kWalkWaves × 8 stacks of `stack` entries
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sub = lane >> 3, c = lane & 7;
+    int* ent = s_stacks + (wave * 8 + sub) * Q.stack;
+    const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
+    const int64_t slot = (blk * kWalkWaves + wave) * 8 + sub;
+    const bool valid = slot < Q.nq;
+    if (!__builtin_amdgcn_ballot_w64(valid)) return;
+    float qx = 0.f, qy = 0.f, qz = 0.f;
+    if (Q.grid) {
+        qx = __builtin_fmaf(float(int(slot % Q.rx)), Q.h, Q.ox);
+        qy = __builtin_fmaf(float(int(slot / Q.rx % Q.ry)), Q.h, Q.oy);
+        qz = __builtin_fmaf(float(int(slot / (int64_t(Q.rx) * Q.ry))), Q.h, Q.oz);
+    } else if (valid) {
+        const float4 a = T.sa[slot];
+        qx = a.x;
+        qy = a.y;
+        qz = a.z;
+    }
+    const float sl2e = sigma * kLog2e;
+    const bool kahan = flags & DWG_KAHAN;
+    float sum = 0.f, comp = 0.f;  // in lane 7 of the point
+    // the terms x·inv of lanes 0 .. 7 added to `part` in that order (rounded
+    // product by product, or fused, as the shared walk's sums are); the total
+    // in lane 7.  Lanes without a term pass the sum on
+    auto ordered = [&](float part, bool on, float x, float inv) {
+        float t;
+        {
+#pragma clang fp contract(off)
+            t = x * inv;
+        }
+        auto with = [&](float p) { return !on ? p : BF16 ? __builtin_fmaf(x, inv, p) : p + t; };
+        float v = with(part);  // right in lane 0
+#pragma unroll
+        for (int k = 1; k < 8; ++k) {
+            const float before = dpp_row<0x111>(v);  // row_shr 1: lane k takes lane k − 1
+            v = c == k ? with(before) : v;
+        }
+        return v;
+    };
+    auto fold = [&](float part, bool on) {
+        if (!on) return;
+        if (kahan) kahan_add(sum, comp, part); else sum += part;
+    };
+    // a leaf of several points, 8 a step, for the points of the wave that
+    // opened one (b .. e; an empty range for the others)
+    auto leaf = [&](int b, int e, bool on) {
+        float part = 0.f;
+        for (int j0 = 0; __builtin_amdgcn_ballot_w64(on && b + j0 < e); j0 += 8) {
+            const int j = b + j0 + c;
+            const bool have = on && j < e;
+            float inv = 0.f, x = 0.f;
+            bool ok = false;
+            if (have) {
+                const float4 pa = T.sa[j];
+                const float dx = pa.x - qx, dy = pa.y - qy, dz = pa.z - qz;
+                x = tree_term_split<SCREENED>(dx, dy, dz, dist2(dx, dy, dz), pa.w * pa.w, T.sb[j], sigma, sl2e, inv, ok);
+            }
+            // (a guarded term adds a zero in the shared walk, which leaves the sum)
+            const float v = ordered(part, have && ok, x, inv);
+            part = __shfl(v, lane | 7, 64);
+        }
+        fold(part, on);
+    };
+    const int4 root = T.info[0];
+    int sp = 0;
+    if (root.x < 0) {
+        leaf(root.y, root.z, valid);
+    } else if (valid) {
+        ent[0] = root.x;
+        sp = 1;
+    }
+    __builtin_amdgcn_wave_barrier();
+    while (__builtin_amdgcn_ballot_w64(sp > 0)) {
+        const bool on = sp > 0;
+        const int top = on ? ent[sp - 1] : 0;
+        if (on) --sp;
+        const bool node = on && top >= 0;
+        bool push = false, term = false;
+        int next = 0;
+        float x = 0.f, inv = 0.f;
+        if (node) {
+            const int64_t ch = int64_t(top) + c;
+            const int2 nk = T.kid[ch];
+            const float4 cr = T.cm_r[ch];
+            const float4* pay = reinterpret_cast<const float4*>(T.payload) + 2 * ch;
+            const float4 e4 = pay[0];
+            const float4 lo = BF16 ? make_float4(0.f, 0.f, 0.f, 0.f) : pay[1];
+            const float dx = cr.x - qx, dy = cr.y - qy, dz = cr.z - qz;
+            const float r2 = dist2(dx, dy, dz);
+            if (nk.x != 0 && r2 > cr.w) {
+                bool ok;
+                if (BF16) {
+                    x = tree_term_split<SCREENED>(dx, dy, dz, r2, e4.w, e4, sigma, sl2e, inv, ok);
+                    term = true;
+                } else {
+                    const float ex = dx + lo.x, ey = dy + lo.y, ez = dz + lo.z;
+                    x = tree_term_split<SCREENED>(ex, ey, ez, dist2(ex, ey, ez), e4.w, e4, sigma, sl2e, inv, ok);
+                    term = ok;
+                }
+            } else if (nk.x != 0 && nk.x != -1) {
+                push = true;
+                next = nk.x > 0 ? nk.x : ~int(ch);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t mine = uint32_t(__builtin_amdgcn_ballot_w64(push) >> (8 * sub)) & 0xFFu;
+        if (push) ent[sp + __builtin_popcount(mine & ((1u << c) - 1u))] = next;
+        sp += __builtin_popcount(mine);
+        __builtin_amdgcn_wave_barrier();
+        fold(ordered(0.f, term, x, inv), node);
+        if (__builtin_amdgcn_ballot_w64(on && top < 0)) {
+            int2 lf = make_int2(0, 0);
+            if (on && top < 0) lf = T.kid[~top];
+            leaf(lf.y, lf.y - lf.x, on && top < 0);
+        }
+    }
+    if (valid && c == 7) out[Q.grid ? slot : int64_t(Q.self_perm[slot])] = sum - comp;
+}
+
 // Which walk explicit queries take.  Alone (gwn_walk_kernel), 64 lanes a query
 // below kWalkFew, where the waves do not fill the chip (1,000 of 100k sources:
 // 17 µs, with 8 lanes 48, shared 1,190), else 8 (32,000: 57 and 75 against
@@ -1423,7 +1556,6 @@ static QueryArgs make_points(const float* q, int64_t nq) {
     QueryArgs Q{};
     Q.q = q;
     Q.nq = nq;
-    Q.lanes = 64;
     return Q;
 }
 
@@ -1431,18 +1563,25 @@ static QueryArgs make_self(const dwg_octree* T) {
     QueryArgs Q{};
     Q.self_perm = T->perm;
     Q.nq = T->n_points;
-    Q.lanes = 64;
     return Q;
 }
 
 // Grids of fewer whole bricks than this leave the chip short of waves, and
 // the launch lasts as long as its longest walks: they take one 4×4×4 part a
-// wave, whose walk opens fewer nodes and lasts a quarter as long (64³ over 100k
-// sources 628 → 250 µs, 160³ over 500k 1,106 → 916 µs; at 256³, 65,536 bricks,
-// whole ones win, 1,776 against 2,204 µs), and grids of very few parts half a
-// part (33×29×31 over 2,000 sources 181 → 72 µs, whole parts 77 µs).  The
-// values are the same: each point takes its own terms in the same order
-constexpr int64_t kWholeBricks = 24576, kHalfParts = 1536;
+// wave, whose walk opens fewer nodes and lasts a quarter as long (96³ over 30k
+// sources 315 → 216 µs, 160³ over 500k 1,106 → 916 µs; at 256³, 65,536 bricks,
+// whole ones win, 1,776 against 2,204 µs).  The values are the same: each
+// point takes its own terms in the same order
+constexpr int64_t kWholeBricks = 24576;
+
+// And below kGridAlone points (kGridAloneDense where the sources are a third of
+// them or more, as then a part's walks have little in common), or kSelfAlone of
+// the tree's own, 8 lanes walk for each point (gwn_ordered_walk_kernel):
+// 33×29×31 over 2,000 sources 181 µs by whole bricks, 77 by parts, 33 alone;
+// 48³ over 2,000 66 by either; 64³ over 10,000 101 and 151, over 100,000 253 and
+// 216; 80³ over 1M 531 and 449.  Own points: 30,000 208 → 52 µs, 200,000 350 →
+// 270, 1M 0.91 and 1.56 ms
+constexpr int64_t kGridAlone = 131072, kGridAloneDense = 524288, kSelfAlone = 250000;
 
 // `whole_bricks`: for the walks that take no others
 static QueryArgs make_grid(const dwg_grid* g, bool whole_bricks) {
@@ -1455,21 +1594,15 @@ static QueryArgs make_grid(const dwg_grid* g, bool whole_bricks) {
     Q.rx = g->res[0];
     Q.ry = g->res[1];
     Q.rz = g->res[2];
-    auto bricks = [&](int parts, int lanes) {
-        const bool many = parts == kGridParts;
-        const int nx = many ? 4 * kPartsX : 4, ny = many ? 4 * kPartsY : 4, nz = many ? 4 * kPartsZ : lanes / 16;
+    auto bricks = [&](int parts, int px, int py, int pz) {
         Q.parts = parts;
-        Q.lanes = lanes;
-        Q.bx = (Q.rx + nx - 1) / nx;
-        Q.by = (Q.ry + ny - 1) / ny;
-        Q.bz = (Q.rz + nz - 1) / nz;
+        Q.bx = (Q.rx + 4 * px - 1) / (4 * px);
+        Q.by = (Q.ry + 4 * py - 1) / (4 * py);
+        Q.bz = (Q.rz + 4 * pz - 1) / (4 * pz);
         Q.n_bricks = int64_t(Q.bx) * Q.by * Q.bz;
     };
-    bricks(kGridParts, 64);
-    if (!whole_bricks && Q.n_bricks < kWholeBricks) {
-        bricks(1, 64);
-        if (Q.n_bricks < kHalfParts) bricks(1, 32);
-    }
+    bricks(kGridParts, kPartsX, kPartsY, kPartsZ);
+    if (!whole_bricks && Q.n_bricks < kWholeBricks) bricks(1, 1, 1, 1);
     Q.nq = int64_t(Q.rx) * Q.ry * Q.rz;
     return Q;
 }
@@ -1537,7 +1670,28 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
         launch_walk<false>(ctx, T, Q.q, Q.nq, sigma, flags, out, nullptr);
         return;
     }
-    const int64_t waves = Q.grid ? Q.n_bricks : (Q.nq + Q.lanes * kPointPts - 1) / (Q.lanes * kPointPts);
+    const bool alone = Q.grid ? Q.nq < kGridAlone || (Q.nq < kGridAloneDense && 3 * T->n_points >= Q.nq)
+                              : Q.self_perm && Q.nq < kSelfAlone;
+    if (alone && !count && !near64) {
+        const bool scr = flags & DWG_SCREENED, bf = flags & DWG_FAR_BF16;
+        const TreeArgs A{T->info, T->kid, T->cm_r, reinterpret_cast<const float*>(T->payload), T->sa, T->sb};
+        QueryArgs Qs = Q;
+        Qs.stack = tree_stack_entries(std::max(T->max_level, 1));
+        dim3 grid(grid_for(Q.nq, kWalkWaves * 8)), block(kWalkWaves * 64);
+        const size_t lds = sizeof(int) * size_t(Qs.stack) * kWalkWaves * 8;
+        ProfileScope ps(ctx, Q.grid ? (scr ? "gwn_tree_grid_screened" : "gwn_tree_grid_plain")
+                                    : (scr ? "gwn_tree_screened" : "gwn_tree_plain"));
+#define DWG_ORDERED(S, B) \
+    hipLaunchKernelGGL((gwn_ordered_walk_kernel<S, B>), grid, block, lds, ctx->stream, A, Qs, sigma, flags, out)
+        if (scr && bf) DWG_ORDERED(true, true);
+        else if (scr) DWG_ORDERED(true, false);
+        else if (bf) DWG_ORDERED(false, true);
+        else DWG_ORDERED(false, false);
+#undef DWG_ORDERED
+        check_launch();
+        return;
+    }
+    const int64_t waves = Q.grid ? Q.n_bricks : (Q.nq + 64 * kPointPts - 1) / (64 * kPointPts);
     if (waves == 0) return;
     TreeArgs A{T->info, T->kid, T->cm_r, reinterpret_cast<const float*>(T->payload), T->sa, T->sb};
     dim3 grid(grid_for(waves, kTreeWaves)), block(kTreeThreads);

@@ -1,5 +1,7 @@
 """The variants a call is dispatched to by its sizes, each at the edges of its
 range, against the FP64 references."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -62,13 +64,14 @@ def test_direct_sums_split_over_sources(ctx, n, nq, screened, kahan):
     assert (np.abs(g - rg) <= 2 * tol * mg + 1e-30).all()
 
 
-# half parts, whole parts and whole bricks cut by every face of the grid, a grid
-# inside one, grids far from and across the cloud, and a cloud far from the
-# origin (large residuals of the rounded centres)
+# each point alone, parts and whole bricks cut by every face of the grid, a
+# single point, a flat grid, grids far from and across the cloud, and a cloud far
+# from the origin (large residuals of the rounded centres)
 @pytest.mark.parametrize("res,h,shift", [((8, 4, 8), 0.05, 0.0), ((9, 5, 7), 0.002, 0.0), ((1, 1, 1), 0.1, 0.0),
                                          ((33, 29, 31), 0.08, 0.0), ((23, 3, 17), 0.3, 0.0),
-                                         ((25, 26, 9), 0.05, 100.0), ((45, 47, 50), 0.02, 0.0),
-                                         ((190, 181, 183), 0.005, 0.0), ((193, 189, 185), 0.005, 0.0)])
+                                         ((25, 26, 9), 0.05, 100.0), ((51, 53, 55), 0.02, 0.0),
+                                         ((401, 399, 1), 0.003, 0.0), ((65, 66, 67), 0.02, 100.0),
+                                         ((190, 181, 183), 0.005, 0.0), ((195, 191, 185), 0.005, 0.0)])
 @pytest.mark.parametrize("screened,bf16,radii", [(True, False, False), (True, True, True), (False, False, False),
                                                  (False, True, False)])
 def test_grid_walk_equals_the_point_walk(ctx, res, h, shift, screened, bf16, radii):
@@ -207,3 +210,25 @@ def test_training_gradient_by_batch(ctx, batch, line):
     # the bounds of the 512-row gradient: BF16 activations and their gradients
     assert loss == pytest.approx(float(ref.detach()), abs=1e-2 if batch < 32 else 1e-3)
     assert np.linalg.norm(g - rg) < 0.03 * np.linalg.norm(rg)
+
+
+@pytest.mark.parametrize("n", [1, 2, 9, 3000, 30_011])
+@pytest.mark.parametrize("screened,bf16,kahan,radii", [(True, False, False, False), (True, True, True, True),
+                                                       (False, False, True, False), (False, True, False, False)])
+def test_own_points_equal_the_shared_walk(ctx, n, screened, bf16, kahan, radii):
+    # the sums at the tree's own points, 8 lanes a point, against the shared walk
+    # of as many explicit points as take it: the same terms in the same order
+    P, N = shapes.sphere(n, 9)
+    P = P.astype(np.float32)
+    P[: n // 20] = P[0]  # a leaf of several points
+    A = np.full(n, 2e-6, np.float32)
+    R = np.linspace(0.0, 0.05, n, dtype=np.float32) if radii else None
+    tree = gpu.Octree(ctx, P.astype(np.float64), None, max_depth=10)
+    tree.update(N, A, R)
+    out = torch.full((n,), float("nan"), device="cuda")
+    flags = tree._flags(screened, None, kahan, bf16)
+    ctx.check(ctx.L.dwg_gwn_tree_self(ctx.h, tree.h, ctypes.c_float(2.3), ctypes.c_float(SIGMA), flags,
+                                      ctypes.c_void_p(out.data_ptr())))
+    many = torch.from_numpy(np.tile(P, (200_000 // n + 1, 1)))
+    want = tree.eval(many, 2.3, sigma=SIGMA, screened=screened, bf16=bf16, kahan=kahan)[:n]
+    np.testing.assert_array_equal(out.cpu().numpy(), want.cpu().numpy())
