@@ -594,16 +594,18 @@ __global__ void tile_scatter_kernel(const int* __restrict__ tile_of, int64_t nq,
     if (tl >= 0) order[hb + (lane - head)] = int(t);
 }
 
-__global__ void tile_flags_kernel(const int64_t* __restrict__ start, int64_t ntiles, int64_t* __restrict__ flags) {
+// blocks a tile's queries take, kTileChunk each
+__global__ void tile_flags_kernel(const int64_t* __restrict__ start, int64_t ntiles, int chunk,
+                                  int64_t* __restrict__ flags) {
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (t > ntiles) return;
-    flags[t] = (t < ntiles && start[kSubTiled * (t + 1)] > start[kSubTiled * t]) ? 1 : 0;
+    flags[t] = t < ntiles ? (start[kSubTiled * (t + 1)] - start[kSubTiled * t] + chunk - 1) / chunk : 0;
 }
 
-__global__ void tile_list_kernel(const int64_t* __restrict__ flags, int64_t ntiles, int* __restrict__ list) {
+__global__ void tile_list_kernel(const int64_t* __restrict__ flags, int64_t ntiles, int2* __restrict__ list) {
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= ntiles || flags[t + 1] == flags[t]) return;
-    list[flags[t]] = int(t);
+    if (t >= ntiles) return;
+    for (int64_t b = flags[t], e = flags[t + 1], c = 0; b + c < e; ++c) list[b + c] = make_int2(int(t), int(c));
 }
 
 // Staged candidates are ordered by ring: the rows of cells that cross the
@@ -618,7 +620,7 @@ __global__ void tile_list_kernel(const int64_t* __restrict__ flags, int64_t ntil
 template <int K, bool SCATTER>
 __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     KnnGridArgs G, TileArgs T, const int64_t* __restrict__ cell_start, const float4* __restrict__ pts,
-    const int* __restrict__ tiles, const int64_t* __restrict__ tile_start, const int* __restrict__ order,
+    const int2* __restrict__ tiles, int chunk, const int64_t* __restrict__ tile_start, const int* __restrict__ order,
     const float* __restrict__ q, int k, const uint8_t* __restrict__ skip, int32_t* __restrict__ out_idx,
     float* __restrict__ out_d2, int* __restrict__ redo, float* __restrict__ redo_kth, int64_t* __restrict__ redo_flag,
     const int64_t* __restrict__ ntiles, KnnScatter sc) {
@@ -644,7 +646,7 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     __shared__ int s_pref[kRows + 1];
     __shared__ int s_wsum[kTileThreads / 64];
     __shared__ int s_ring[kHalo + 2];
-    const int tile = tiles[blockIdx.x];
+    const int tile = tiles[blockIdx.x].x;
     const int tx = tile % T.tdim[0], ty = (tile / T.tdim[0]) % T.tdim[1], tz = tile / (T.tdim[0] * T.tdim[1]);
     const int x0 = max(tx * kTile - kHalo, 0), x1 = min(tx * kTile + kTile - 1 + kHalo, G.dim[0] - 1);
     const int y0 = max(ty * kTile - kHalo, 0), y1 = min(ty * kTile + kTile - 1 + kHalo, G.dim[1] - 1);
@@ -724,7 +726,8 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     const float fhy = y1 + 1 < G.dim[1] ? G.lo[1] + float(y1 + 1) * G.cell : INFINITY;
     const float flz = z0 > 0 ? G.lo[2] + float(z0) * G.cell : -INFINITY;
     const float fhz = z1 + 1 < G.dim[2] ? G.lo[2] + float(z1 + 1) * G.cell : INFINITY;
-    const int64_t qs = tile_start[int64_t(tile) * kSubTiled], qe = tile_start[int64_t(tile + 1) * kSubTiled];
+    const int64_t qs = tile_start[int64_t(tile) * kSubTiled] + int64_t(tiles[blockIdx.x].y) * chunk;
+    const int64_t qe = min(tile_start[int64_t(tile + 1) * kSubTiled], qs + chunk);
     for (int64_t qb = qs; qb < qe; qb += kTileThreads) {
         const int64_t t = qb + threadIdx.x;
         const bool active = t < qe;
@@ -1274,11 +1277,12 @@ constexpr int kPwStack = 128;  // ≥ 7 · kMaxPyr + 1 entries
 // its longest walks, on an otherwise idle chip: a wave stops after this many
 // pops and hands its open queries, with the bounds they have, to a search of
 // their own (knn_descent_kernel).  Sharing pays while the waves fill the
-// chip, so the more queries, the more pops: below 32,768 queries none at all
-// (20,000 far centroids: 0.8 ms shared, 0.3 alone), at 180,000 of 3M
+// chip, so the more queries, the more pops: below 65,536 queries none at all
+// (53,000 far centroids of a 30,000-point cloud: 0.41 ms with 100 pops, 0.35
+// alone), at 180,000 of 3M
 // centroids 12.5 → 2.1 ms with about 350 pops, at 900,000 10 → 4.6 ms with
 // 1,024 (6.5 ms with 400)
-constexpr int64_t kShareMin = 32768;
+constexpr int64_t kShareMin = 65536;
 __device__ __forceinline__ int shared_walk_budget(int64_t nq) {
     return nq < kShareMin ? 0 : int(min(max(nq / 512, int64_t(64)), int64_t(1024)));
 }
@@ -1556,14 +1560,17 @@ static void launch_far(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int
 
 // The queries 0..nq−1 (masked by qmask) bucketed by tile of kTile³ fine cells
 // and eighth of it: order[start[sub·t]..start[sub·(t+1))) are tile t's
-// queries, list[0..*nlist) the tiles that have any
+// queries, list[0..*nlist) the tiles that have any, once for each `chunk` of
+// them (tile, chunk)
+constexpr int64_t kTileBlocks = 4096;
 struct TileBuckets {
     TileArgs T;
-    int64_t ntiles = 0;
+    int64_t ntiles = 0, max_list = 0;
+    int chunk = 0;
     int64_t* nlist = nullptr;
     int64_t* start = nullptr;
     int* order = nullptr;
-    int* list = nullptr;
+    int2* list = nullptr;
 };
 
 static TileBuckets tile_buckets(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq,
@@ -1581,7 +1588,12 @@ static TileBuckets tile_buckets(dwg_ctx* ctx, const dwg_knn_index* I, const floa
     unsigned long long* cursor = static_cast<unsigned long long*>(ctx->buf("knnt_cursor", sizeof(uint64_t) * nb));
     int* order = static_cast<int*>(ctx->buf("knnt_order", sizeof(int) * nq));
     int64_t* flags = static_cast<int64_t*>(ctx->buf("knnt_flags", sizeof(int64_t) * (ntiles + 1)));
-    int* list = static_cast<int*>(ctx->buf("knnt_list", sizeof(int) * ntiles));
+    // a tile's queries are split over blocks so that there are a few thousand:
+    // 230,000 centroids over 3,375 points fill 300 tiles, each a thousand
+    // queries long (tiled pass 1.3 → 0.2 ms)
+    B.chunk = kTileThreads * int(std::max<int64_t>(1, nq / (kTileBlocks * kTileThreads)));
+    B.max_list = std::min(ntiles, nq) + nq / B.chunk;
+    int2* list = static_cast<int2*>(ctx->buf("knnt_list", sizeof(int2) * size_t(B.max_list)));
     fill_u32(ctx, start, 0, 2 * (nb + 1));
     hipLaunchKernelGGL(tile_count_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, q, nq, qmask, G, T,
                        tile_of, reinterpret_cast<unsigned long long*>(start));
@@ -1595,7 +1607,7 @@ static TileBuckets tile_buckets(dwg_ctx* ctx, const dwg_knn_index* I, const floa
     B.start = start;
     B.order = order;
     hipLaunchKernelGGL(tile_flags_kernel, dim3(grid_for(ntiles + 1, 256)), dim3(256), 0, ctx->stream, start, ntiles,
-                       flags);
+                       B.chunk, flags);
     check_launch();
     exclusive_scan<int64_t>(ctx, flags, ntiles);
     hipLaunchKernelGGL(tile_list_kernel, dim3(grid_for(ntiles, 256)), dim3(256), 0, ctx->stream, flags, ntiles, list);
@@ -1635,7 +1647,7 @@ static const int64_t* tiled_pass(dwg_ctx* ctx, const dwg_knn_index* I, const flo
     int* tmp_q = static_cast<int*>(ctx->buf("knnt_rtmp", sizeof(int) * nq + 64));
     float* tmp_kth = static_cast<float*>(ctx->buf("knnt_rkth", sizeof(float) * nq + 64));
     fill_u32(ctx, rflag, 0, 2 * (nq + 1));
-    int64_t blocks = std::min(B.ntiles, nq);
+    int64_t blocks = B.max_list;
     const int64_t* exact = B.nlist;
     if (blocks > kTileBlind) {
         blocks = read_scalar<int64_t>(ctx, B.nlist);
@@ -1648,12 +1660,12 @@ static const int64_t* tiled_pass(dwg_ctx* ctx, const dwg_knn_index* I, const flo
     do {                                                                                                            \
         if (sc)                                                                                                     \
             hipLaunchKernelGGL((knn_tile_kernel<KK, true>), dim3(unsigned(blocks)), dim3(kTileThreads), 0,          \
-                               ctx->stream, G, T, I->lvl[0].cell_start, I->lvl[0].pts, B.list, B.start, B.order, q, \
-                               k, skip, out_idx, out_d2, tmp_q, tmp_kth, rflag, exact, scv);                        \
+                               ctx->stream, G, T, I->lvl[0].cell_start, I->lvl[0].pts, B.list, B.chunk, B.start, B.order, \
+                               q, k, skip, out_idx, out_d2, tmp_q, tmp_kth, rflag, exact, scv);                        \
         else                                                                                                        \
             hipLaunchKernelGGL((knn_tile_kernel<KK, false>), dim3(unsigned(blocks)), dim3(kTileThreads), 0,         \
-                               ctx->stream, G, T, I->lvl[0].cell_start, I->lvl[0].pts, B.list, B.start, B.order, q, \
-                               k, skip, out_idx, out_d2, tmp_q, tmp_kth, rflag, exact, scv);                        \
+                               ctx->stream, G, T, I->lvl[0].cell_start, I->lvl[0].pts, B.list, B.chunk, B.start, B.order, \
+                               q, k, skip, out_idx, out_d2, tmp_q, tmp_kth, rflag, exact, scv);                        \
     } while (0)
         if (k <= 8) DWG_KNNT(8);
         else if (k <= 10) DWG_KNNT(10);

@@ -232,3 +232,27 @@ def test_own_points_equal_the_shared_walk(ctx, n, screened, bf16, kahan, radii):
     many = torch.from_numpy(np.tile(P, (200_000 // n + 1, 1)))
     want = tree.eval(many, 2.3, sigma=SIGMA, screened=screened, bf16=bf16, kahan=kahan)[:n]
     np.testing.assert_array_equal(out.cpu().numpy(), want.cpu().numpy())
+
+
+@pytest.mark.parametrize("n,ntri", [(300, 20_000), (2500, 90_000), (40_000, 41_000)])
+def test_diffusion_of_crowded_tiles(ctx, n, ntri):
+    # tiles of up to thousands of centroids, split over blocks: every face normal
+    # reaches its 15 nearest sources once, in the same fixed-point sums
+    rng = np.random.default_rng(n)
+    P, N = shapes.sphere(n, 6)
+    P = (0.5 * P).astype(np.float32)
+    C = (P[rng.integers(0, n, ntri)] + rng.normal(0, 0.01, (ntri, 3))).astype(np.float32)
+    T = rng.normal(size=(ntri, 3)).astype(np.float32)
+    T /= np.linalg.norm(T, axis=1, keepdims=True)
+    nrm = torch.from_numpy(N.astype(np.float32)).cuda()
+    gpu.diffuse_normals(ctx, gpu.KnnIndex(ctx, P, 15), C, T, nrm, zero_threshold=n)
+    idx = O.knn_brute(P, C, 15) if n * ntri < 1e9 else O.knn_grid(P, C, 15)
+    acc = np.zeros((n, 3), np.int64)
+    fixed = np.rint(T.astype(np.float64) * 2.0 ** 40).astype(np.int64)
+    for k in range(15):
+        np.add.at(acc, idx[:, k], fixed)
+    a = acc * 2.0 ** -40
+    length = np.linalg.norm(a, axis=1, keepdims=True)
+    want = np.where(length < 1e-10, N, a / (length + 1e-8))
+    # FP64 until the last rounding on both sides
+    np.testing.assert_allclose(nrm.cpu().numpy(), want, rtol=2.0 ** -23, atol=1e-12)
