@@ -8,6 +8,7 @@ import torch
 
 import oracle as O
 from dwg_amd import gpu, shapes
+from mc_order import to_brick_order
 from oracle import mlp as M
 
 pytestmark = pytest.mark.gpu
@@ -256,3 +257,41 @@ def test_diffusion_of_crowded_tiles(ctx, n, ntri):
     want = np.where(length < 1e-10, N, a / (length + 1e-8))
     # FP64 until the last rounding on both sides
     np.testing.assert_allclose(nrm.cpu().numpy(), want, rtol=2.0 ** -23, atol=1e-12)
+
+
+@pytest.mark.parametrize("res,crossed", [((2, 2, 2), "all"), ((65, 9, 17), "all"), ((66, 10, 19), "all"),
+                                         ((130, 19, 35), "all"), ((9, 1030, 1030), "few")])
+def test_marching_cubes_by_runs(ctx, res, crossed):
+    """Runs of 64 cubes that end on, before and past the grid's end, by a block
+    and by a wave (the last size), with every cube crossed or few, and samples
+    that are infinite or not a number (above no level): the ordered mesh is the
+    oracle's in brick order, and the any-order pass has its rows bit for bit."""
+    rng = np.random.default_rng(sum(res))
+    n = res[0] * res[1] * res[2]
+    if crossed == "all":
+        f = rng.normal(size=n).astype(np.float32)
+        if n > 8:
+            f[rng.integers(0, n, 20)] = np.repeat(np.float32([np.nan, np.inf, -np.inf, 0.0]), 5)
+        f[:2] = 1.0, -1.0  # a triangle at least
+    else:
+        z, y, x = np.meshgrid(*(np.arange(r, dtype=np.float32) for r in res[::-1]), indexing="ij")
+        f = (np.hypot(y - 512, z - 500) - 480 + np.sin(x)).astype(np.float32).ravel()
+    origin, h = np.float32([-1.1, -0.9, -1.0]), np.float32(0.05)
+    grid = gpu.make_grid(origin, h, np.int32(res))
+    ft = torch.from_numpy(f).cuda()
+    tris, cent, nrm = gpu.marching_cubes(ctx, ft, grid, 0.0, tris=True)
+    with np.errstate(all="ignore"):
+        rt, rc, _ = O.marching_cubes(f.astype(np.float64), np.int32(res), origin.astype(float), float(h), 0.0)
+    order = to_brick_order(f, res, np.float32(0))
+    assert len(rt) == tris.shape[0] > 0
+    # a vertex: two rounded corners, their difference, its multiple and the sum,
+    # each half a unit of the largest coordinate; a centroid: three more
+    ulp = 2.0 ** -23 * (1.1 + float(h) * max(res))
+    for got, want, tol in ((tris, rt, 4 * ulp), (cent, rc, 8 * ulp)):
+        got, want = got.cpu().numpy(), want[order]
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        ok = ~np.isnan(want)
+        assert np.abs(got[ok] - want[ok]).max() <= tol
+    c1, n1 = gpu.marching_cubes_any_order(ctx, ft, grid, 0.0, capacity=len(rt))
+    rows = [np.concatenate([c.cpu().numpy(), m.cpu().numpy()], 1).view(np.uint32) for c, m in ((cent, nrm), (c1, n1))]
+    assert np.array_equal(*(r[np.lexsort(r.T[::-1])] for r in rows))
