@@ -1077,7 +1077,8 @@ __device__ __forceinline__ float pyr_box_d2(const KnnGridArgs& G, float w, float
 // registers leave room for many waves.  Blocks wait on a stack in LDS with
 // their box distance; until k points are known one block is opened a step,
 // its nearest child on top, then 8.  Bound by the latency of a step (a child
-// load, then a point load), so by waves in flight.
+// load, then a point load) where queries are few (1,500 over 100,000 points:
+// 0.12 ms), by instructions where they fill the card.
 // The stack never overflows: opening a block leaves at most 7 entries more
 // than it took, a step takes several only while that leaves kDescReserve
 // entries free, and a single depth-first descent needs no more than these.
@@ -1103,11 +1104,109 @@ __device__ __forceinline__ int wave_scan_add(int v) {
     return v;
 }
 
+// maximum over the wave
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    v = max(v, uint32_t(dpp_or_zero<0x111>(int(v))));
+    v = max(v, uint32_t(dpp_or_zero<0x112>(int(v))));
+    v = max(v, uint32_t(dpp_or_zero<0x114>(int(v))));
+    v = max(v, uint32_t(dpp_or_zero<0x118>(int(v))));
+    v = max(v, uint32_t(dpp_or_zero<0x142, 0xA>(int(v))));
+    v = max(v, uint32_t(dpp_or_zero<0x143, 0xC>(int(v))));
+    return uint32_t(__builtin_amdgcn_readlane(int(v), 63));
+}
+
 __device__ __forceinline__ uint32_t read_lane(uint32_t v, int l) {
     return uint32_t(__builtin_amdgcn_readlane(int(v), l));
 }
 __device__ __forceinline__ uint64_t read_lane64(uint64_t v, int l) {
     return (uint64_t(read_lane(uint32_t(v >> 32), l)) << 32) | read_lane(uint32_t(v), l);
+}
+
+// The keys `key` of the lanes `cand` (all < kth) join the wave's best keys,
+// ascending in the lanes 0 .. k − 1 of `list` (kNoKey where there is none), of
+// which the least k stay; kth is the k-th then.  Up to kDescOneByOne keys enter
+// one after the other, each shifting the list.  Where there are more, a
+// bisection finds a bound with k keys below it, in the bits of the squared
+// distance and, if several points lie at the k-th distance, of the index: two
+// compares and some scalar work a step, whatever the number of keys; the keys
+// that stay are then placed by the number of smaller ones.  A cell's first
+// points are 20 to 60 keys, and one by one they were half of the kernel's work;
+// a long walk's later cells add a few each, which the bisection's serial steps
+// only delay (1,500 queries over 100,000 points: all by bisection 188 µs, all
+// one by one 173, mixed 2 % below that; a reconstruction of 30,000 points on a
+// 128³ grid with 50,000 far centroids an iteration 7.27 → 7.04 ms).
+constexpr int kDescOneByOne = 12;
+
+__device__ __forceinline__ void desc_take(uint64_t& list, uint64_t& kth, uint64_t key, uint64_t cand, int k,
+                                          uint64_t* sel) {
+    const int lane = threadIdx.x & 63;
+    const int many = __builtin_popcountll(cand);
+    if (many <= kDescOneByOne) {
+        for (; cand; cand &= cand - 1) {
+            const uint64_t c = read_lane64(key, __builtin_ctzll(cand));
+            if (!(c < kth)) continue;
+            // c enters at p: the lanes from p on take their lower neighbour's key
+            const int p = __builtin_popcountll(__builtin_amdgcn_ballot_w64(list < c));
+            const uint32_t plo = uint32_t(dpp_or_zero<0x138>(int(uint32_t(list))));  // wave_shr 1
+            const uint32_t phi = uint32_t(dpp_or_zero<0x138>(int(uint32_t(list >> 32))));
+            const uint64_t prev = (uint64_t(phi) << 32) | plo;
+            list = lane == p ? c : (lane > p ? prev : list);
+            list = lane < k ? list : kNoKey;
+            kth = read_lane64(list, k - 1);
+        }
+        return;
+    }
+    const bool is = (cand >> lane) & 1ull;
+    key = is ? key : ~0ull;
+    const uint32_t ld = uint32_t(list >> 32), kd = uint32_t(key >> 32);
+    const int total = __builtin_popcountll(__builtin_amdgcn_ballot_w64(list < kNoKey)) + many;
+    uint64_t limit = kNoKey;  // the keys below it stay
+    if (total > k) {
+        // count(d < lo) < k < count(d < hi) in the distance's bits
+        uint32_t lo = 0, hi = uint32_t(kth >> 32) + 1u;
+        if (kth == kNoKey) hi = wave_max_u32(max(is ? kd : 0u, list < kNoKey ? ld : 0u)) + 1u;
+        // first a quarter of the largest squared distance: on a surface a
+        // quarter of the points
+        uint32_t mid = hi > (2u << 24) ? hi - (2u << 23) : hi >> 1;
+        bool found = false;
+        while (hi - lo > 1) {
+            const int c = __builtin_popcountll(__builtin_amdgcn_ballot_w64(ld < mid)) +
+                          __builtin_popcountll(__builtin_amdgcn_ballot_w64(kd < mid));
+            if (c == k) {
+                found = true;
+                break;
+            }
+            (c > k ? hi : lo) = mid;
+            mid = lo + ((hi - lo) >> 1);
+        }
+        limit = uint64_t(mid) << 32;
+        if (!found) {  // some of the points at distance lo stay
+            uint64_t l = uint64_t(lo) << 32, h = l + (1ull << 32);
+            for (;;) {  // keys differ, so some bound has k keys below it
+                limit = l + ((h - l) >> 1);
+                const int c = __builtin_popcountll(__builtin_amdgcn_ballot_w64(list < limit)) +
+                              __builtin_popcountll(__builtin_amdgcn_ballot_w64(key < limit));
+                if (c == k || h - l <= 1) break;
+                (c > k ? h : l) = limit;
+            }
+        }
+    }
+    // the new keys that stay, then the old ones
+    const uint64_t below = (1ull << lane) - 1ull;
+    const uint64_t in = __builtin_amdgcn_ballot_w64(key < limit), old = __builtin_amdgcn_ballot_w64(list < limit);
+    const int nin = __builtin_popcountll(in), n = min(total, k);
+    if ((in >> lane) & 1ull) sel[__builtin_popcountll(in & below)] = key;
+    if ((old >> lane) & 1ull) sel[nin + __builtin_popcountll(old & below)] = list;
+    __builtin_amdgcn_wave_barrier();
+    const uint64_t mine = lane < n ? sel[lane] : kNoKey;
+    __builtin_amdgcn_wave_barrier();
+    int place = lane < n ? 0 : lane;
+    for (int j = 0; j < n; ++j) place += lane < n && read_lane64(mine, j) < mine ? 1 : 0;
+    sel[place] = mine;
+    __builtin_amdgcn_wave_barrier();
+    list = sel[lane];
+    __builtin_amdgcn_wave_barrier();
+    kth = read_lane64(list, k - 1);
 }
 
 // qlist (nullable) holds the queries, `count` (nullable) their number on the
@@ -1121,6 +1220,7 @@ __global__ __launch_bounds__(kDescWaves * 64) void knn_descent_kernel(
     __shared__ uint64_t s_ent[kDescWaves][kDescStack];  // x | y << 16 | z << 32 | occupancy << 48 | level << 56
     __shared__ float s_ed2[kDescWaves][kDescStack];     // box distance
     __shared__ int s_pt[kDescWaves][64 * kDescPoints];
+    __shared__ uint64_t s_sel[kDescWaves][64];
     __shared__ int4 s_dim[kMaxPyr];
     __shared__ int64_t s_off[kMaxPyr];
     if (threadIdx.x < Y.levels) {
@@ -1133,6 +1233,7 @@ __global__ __launch_bounds__(kDescWaves * 64) void knn_descent_kernel(
     uint64_t* ent = s_ent[wave];
     float* ed2 = s_ed2[wave];
     int* pt = s_pt[wave];
+    uint64_t* sel = s_sel[wave];
     const int64_t n = count ? int64_t(uniform64(uint64_t(*count))) : nq;
     const int top = Y.levels - 1;
     const uint64_t root = (uint64_t(uint32_t(uniform(int(Y.mask[s_off[top]])))) << 48) | (uint64_t(uint32_t(top)) << 56);
@@ -1227,19 +1328,8 @@ __global__ __launch_bounds__(kDescWaves * 64) void knn_descent_kernel(
                             // the skip byte only for a point that would enter the list
                             if (key < kth && skip && skip[idx]) key = ~0ull;
                         }
-                        for (uint64_t m2 = __builtin_amdgcn_ballot_w64(key < kth); m2; m2 &= m2 - 1) {
-                            const uint64_t c2 = read_lane64(key, __builtin_ctzll(m2));
-                            if (!(c2 < kth)) continue;
-                            // c2 enters at p: the lanes from p on take their
-                            // lower neighbour's key
-                            const int p = __builtin_popcountll(__builtin_amdgcn_ballot_w64(list < c2));
-                            const uint32_t plo = uint32_t(dpp_or_zero<0x138>(int(uint32_t(list))));  // wave_shr 1
-                            const uint32_t phi = uint32_t(dpp_or_zero<0x138>(int(uint32_t(list >> 32))));
-                            const uint64_t prev = (uint64_t(phi) << 32) | plo;
-                            list = lane == p ? c2 : (lane > p ? prev : list);
-                            list = lane < k ? list : kNoKey;
-                            kth = read_lane64(list, k - 1);
-                        }
+                        if (const uint64_t cand = __builtin_amdgcn_ballot_w64(key < kth))
+                            desc_take(list, kth, key, cand, k, sel);
                     }
                     __builtin_amdgcn_wave_barrier();
                 }
@@ -1527,8 +1617,11 @@ static void launch_far(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int
                        const float* init_kth, bool shared, const uint8_t* pyr_mask) {
     const auto& L = I->lvl[0];
     // an index without boxes (its first such query) builds them, a dozen
-    // launches, only if there are enough far queries to share a walk
-    if (shared && L.pyr_levels >= 2 && !L.pbox && read_scalar<int64_t>(ctx, count) < kShareMin) shared = false;
+    // launches and 70 µs for 30,000 points, only if there are enough far
+    // queries that these gain as much at once: 48,000 of a cloud of 30,000
+    // points 445 µs by cell boxes, 345 by the points' boxes
+    constexpr int64_t kBoxMin = 32768;
+    if (shared && L.pyr_levels >= 2 && !L.pbox && read_scalar<int64_t>(ctx, count) < kBoxMin) shared = false;
     if (!shared || L.pyr_levels < 2) {
         launch_descent(ctx, I, q, nq, count, qlist, k, skip, nullptr, init_kth, out_idx, out_d2, pyr_mask);
         return;

@@ -123,14 +123,32 @@ def test_knn_by_query_count(ctx, n, nq, k, skipped):
     np.testing.assert_array_equal(d2.cpu().numpy()[sub], np.where(ref < 0, np.inf, rd2))
 
 
-def test_knn_far_walk_hands_over(ctx):
-    # 60,000 far queries near the centre of a sphere of 30,000 points: every
-    # point is about as near as any other, so the shared walks run out of pops
-    # and their queries search alone
+@pytest.mark.parametrize("n,k", [(20, 32), (1331, 1), (1331, 7), (9261, 15), (9261, 32)])
+def test_knn_ties_at_the_last_neighbour(ctx, n, k):
+    # points of a lattice, the queries on them, between them and far off: the
+    # k-th distance is that of several points, of which those of least index
+    # stay (and all points where there are fewer than k)
+    side = round(n ** (1 / 3)) if n > 20 else 3
+    z, y, x = np.meshgrid(*(np.arange(side),) * 3, indexing="ij")
+    P = np.stack([x, y, z], -1).reshape(-1, 3)[:n].astype(np.float32) / 16
+    rng = np.random.default_rng(n + k)
+    P = P[rng.permutation(n)]
+    Q = np.concatenate([P, P + np.float32(1 / 32), P * np.float32([1, 1, 0]) + np.float32([0, 0, 8])])
+    got, d2 = gpu.KnnIndex(ctx, P, k_hint=k).query(Q[:6000], k, d2=True)
+    ref, rd2 = O.knn_brute(P, Q[:6000], k, return_d2=True)
+    np.testing.assert_array_equal(got.cpu().numpy(), ref)
+    np.testing.assert_array_equal(d2.cpu().numpy(), np.where(ref < 0, np.inf, rd2))
+
+
+@pytest.mark.parametrize("nq", [31_000, 60_000, 70_000])
+def test_knn_far_walk_hands_over(ctx, nq):
+    # far queries near the centre of a sphere of 30,000 points: every point is
+    # about as near as any other, so shared walks (of the last size) run out of
+    # pops and their queries search alone
     rng = np.random.default_rng(5)
     P, _ = shapes.sphere(30_000, 4)
     P = (0.5 * P + rng.normal(0, 1e-4, P.shape)).astype(np.float32)
-    Q = rng.normal(0, 0.02, (60_000, 3)).astype(np.float32)
+    Q = rng.normal(0, 0.02, (nq, 3)).astype(np.float32)
     idx = gpu.KnnIndex(ctx, P, k_hint=15)
     got, d2 = idx.query(Q, 15, d2=True)
     sub = rng.permutation(len(Q))[:3000]
