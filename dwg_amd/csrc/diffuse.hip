@@ -21,12 +21,18 @@ namespace dwg {
 constexpr double kInvFix = 1.0 / 1099511627776.0;  // 2^-40, the scatter's fixed point
 
 // NormalizeNormals (TurboDWG.cu:238-266): |acc| < 1e-10 keeps the old normal
-// and counts as zero; otherwise n = acc / (|acc| + 1e-8).
-__global__ __launch_bounds__(256) void normalize_kernel(const unsigned long long* __restrict__ acc, int64_t n,
-                                                        float* __restrict__ nrm, uint8_t* __restrict__ zero,
+// and counts as zero; otherwise n = acc / (|acc| + 1e-8).  The zero sources'
+// indices and positions are listed, a block's with one atomic add and in no
+// order between the blocks (each fills its own normal later).
+constexpr int kNormThreads = 1024;
+__global__ __launch_bounds__(kNormThreads) void normalize_kernel(const unsigned long long* __restrict__ acc, int64_t n,
+                                                        const float* __restrict__ p, float* __restrict__ nrm,
+                                                        uint8_t* __restrict__ zero, float* __restrict__ zq,
+                                                        int32_t* __restrict__ zlist,
                                                         unsigned long long* __restrict__ nzero) {
-    __shared__ int cnt[256];
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    __shared__ int s_cnt[kNormThreads / 64];
+    __shared__ int s_first;
+    const int64_t i = int64_t(blockIdx.x) * kNormThreads + threadIdx.x;
     int z = 0;
     if (i < n) {
         const double ax = double((long long)acc[3 * i]) * kInvFix;
@@ -43,30 +49,22 @@ __global__ __launch_bounds__(256) void normalize_kernel(const unsigned long long
         }
         zero[i] = uint8_t(z);
     }
-    cnt[threadIdx.x] = z;
+    const uint64_t zeros = __builtin_amdgcn_ballot_w64(z);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) s_cnt[wave] = __builtin_popcountll(zeros);
     __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) cnt[threadIdx.x] += cnt[threadIdx.x + off];
-        __syncthreads();
+    int before = 0, total = 0;
+    for (int w = 0; w < kNormThreads / 64; ++w) {
+        before += w < wave ? s_cnt[w] : 0;
+        total += s_cnt[w];
     }
-    if (threadIdx.x == 0 && cnt[0]) atomicAdd(nzero, (unsigned long long)cnt[0]);
-}
-
-__global__ void nonzero_flags_kernel(const uint8_t* __restrict__ zero, int64_t n, int64_t* __restrict__ slot) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i > n) return;
-    slot[i] = (i < n && !zero[i]) ? 1 : 0;
-}
-
-// the zero sources, compacted: their indices and positions (slot[i] counts
-// the non-zero sources before i, so i − slot[i] counts the zero ones)
-__global__ void zero_gather_kernel(const int64_t* __restrict__ slot, const float* __restrict__ p, int64_t n,
-                                   float* __restrict__ zq, int32_t* __restrict__ zlist) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n || slot[i + 1] != slot[i]) return;
-    const int64_t j = i - slot[i];
-    for (int d = 0; d < 3; ++d) zq[3 * j + d] = p[3 * i + d];
-    zlist[j] = int32_t(i);
+    if (total == 0) return;
+    if (threadIdx.x == 0) s_first = int(atomicAdd(nzero, (unsigned long long)total));
+    __syncthreads();
+    if (!z) return;
+    const int at = s_first + before + __builtin_popcountll(zeros & ((1ull << lane) - 1ull));
+    for (int d = 0; d < 3; ++d) zq[3 * int64_t(at) + d] = p[3 * i + d];
+    zlist[at] = int32_t(i);
 }
 
 // SimpleUpdateNonzeroNormals (TurboDWG.cu:322-359): a zero source takes the
@@ -107,23 +105,14 @@ void diffuse_normals(dwg_ctx* ctx, const dwg_knn_index* I, const float* src, int
         const KnnScatter sc{tri_nrm, acc};
         knn_query(ctx, I, cent, ntri, k, nullptr, nullptr, knn, nullptr, "knn_query_centroids", &sc);
     }
-    {
-        ProfileScope ps(ctx, "diffuse_normalize");
-        hipLaunchKernelGGL(normalize_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, acc, n, nrm, zero, nz);
-        check_launch();
-    }
-    // the zero sources' positions and indices, compacted (room for n): queued
-    // before their count is read back, as the zero fill nearly always runs
-    int64_t* slot = static_cast<int64_t*>(ctx->buf("diff_nz_slot", sizeof(int64_t) * (n + 1)));
+    // the zero sources' positions and indices (room for n), queued before their
+    // count is read back, as the zero fill nearly always runs
     float* zq = static_cast<float*>(ctx->buf("diff_z_pts", sizeof(float) * 3 * n));
     int32_t* zlist = static_cast<int32_t*>(ctx->buf("diff_z_list", sizeof(int32_t) * n));
     {
-        ProfileScope ps(ctx, "diffuse_nonzero_index");
-        hipLaunchKernelGGL(nonzero_flags_kernel, dim3(grid_for(n + 1, 256)), dim3(256), 0, ctx->stream, zero, n, slot);
-        check_launch();
-        exclusive_scan<int64_t>(ctx, slot, n);
-        hipLaunchKernelGGL(zero_gather_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, slot, src, n, zq,
-                           zlist);
+        ProfileScope ps(ctx, "diffuse_normalize");
+        hipLaunchKernelGGL(normalize_kernel, dim3(grid_for(n, kNormThreads)), dim3(kNormThreads), 0, ctx->stream, acc, n, src, nrm, zero,
+                           zq, zlist, nz);
         check_launch();
     }
     const int64_t nzero = int64_t(read_scalar<unsigned long long>(ctx, nz));

@@ -34,40 +34,48 @@ __device__ __forceinline__ int cell_coord(float v, float lo, float inv_cell, int
     return min(max(c, 0), dim - 1);
 }
 
+// Adds this thread's item to its bucket (−1: none) and returns its place there:
+// a run of lanes with one bucket takes its places with one atomic add.  The
+// second pass then needs no atomics (3M triangle centroids: count and scatter
+// 248 → 140 µs).
+__device__ __forceinline__ int take_place(int bucket, unsigned long long* __restrict__ counts) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t starts = run_starts(bucket);
+    int base = 0;
+    if (bucket >= 0 && ((starts >> lane) & 1ull))
+        base = int(atomicAdd(&counts[bucket], (unsigned long long)run_length(starts, lane)));
+    const int head = run_head(starts, lane);
+    return __shfl(base, head, 64) + (lane - head);
+}
+
+__device__ __forceinline__ int cell_of_point(const KnnGridArgs& G, const float* __restrict__ p, int64_t i) {
+    const int cx = cell_coord(p[3 * i], G.lo[0], G.inv_cell, G.dim[0]);
+    const int cy = cell_coord(p[3 * i + 1], G.lo[1], G.inv_cell, G.dim[1]);
+    const int cz = cell_coord(p[3 * i + 2], G.lo[2], G.inv_cell, G.dim[2]);
+    return int(cx + int64_t(G.dim[0]) * (cy + int64_t(G.dim[1]) * cz));
+}
+
+// place (nullable): (cell, place in it) of every point
 __global__ void knn_count_kernel(const float* __restrict__ p, int64_t n, KnnGridArgs G,
-                                 unsigned long long* __restrict__ counts, int* __restrict__ cell_of) {
+                                 unsigned long long* __restrict__ counts, int2* __restrict__ place) {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    int c = -1;  // every lane takes part in the run detection
-    if (i < n) {
-        const int cx = cell_coord(p[3 * i], G.lo[0], G.inv_cell, G.dim[0]);
-        const int cy = cell_coord(p[3 * i + 1], G.lo[1], G.inv_cell, G.dim[1]);
-        const int cz = cell_coord(p[3 * i + 2], G.lo[2], G.inv_cell, G.dim[2]);
-        c = int(cx + int64_t(G.dim[0]) * (cy + int64_t(G.dim[1]) * cz));
-        cell_of[i] = c;
+    const int c = i < n ? cell_of_point(G, p, i) : -1;  // every lane takes part in the run detection
+    if (place) {
+        const int at = take_place(c, counts);
+        if (i < n) place[i] = make_int2(c, at);
+        return;
     }
     const int lane = threadIdx.x & 63;
     const uint64_t starts = run_starts(c);
     if (c >= 0 && ((starts >> lane) & 1ull)) atomicAdd(&counts[c], (unsigned long long)run_length(starts, lane));
 }
 
-__global__ void knn_scatter_kernel(const float* __restrict__ p, int64_t n, const int* __restrict__ cell_of,
-                                   unsigned long long* __restrict__ cursor, float4* __restrict__ out) {
+__global__ void knn_scatter_kernel(const float* __restrict__ p, int64_t n, const int2* __restrict__ place,
+                                   const int64_t* __restrict__ cell_start, float4* __restrict__ out) {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const int c = i < n ? cell_of[i] : -1;
-    const int lane = threadIdx.x & 63;
-    const uint64_t starts = run_starts(c);
-    int64_t base = 0;
-    if (c >= 0 && ((starts >> lane) & 1ull))
-        base = int64_t(atomicAdd(&cursor[c], (unsigned long long)run_length(starts, lane)));
-    const int head = run_head(starts, lane);
-    const int64_t hb = (int64_t(__shfl(int(uint32_t(base >> 32)), head, 64)) << 32) |
-                       int64_t(uint32_t(__shfl(int(uint32_t(base)), head, 64)));
-    if (c >= 0) out[hb + (lane - head)] = make_float4(p[3 * i], p[3 * i + 1], p[3 * i + 2], __int_as_float(int(i)));
-}
-
-__global__ void copy_i64_kernel(const int64_t* __restrict__ a, unsigned long long* __restrict__ b, int64_t n) {
-    int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) b[i] = (unsigned long long)a[i];
+    if (i >= n) return;
+    const int2 c = place[i];
+    out[cell_start[c.x] + c.y] = make_float4(p[3 * i], p[3 * i + 1], p[3 * i + 2], __int_as_float(int(i)));
 }
 
 __global__ __launch_bounds__(256) void bounds_kernel(const float* __restrict__ p, int64_t n, float* __restrict__ partial) {
@@ -145,25 +153,22 @@ static double cells_of(const float* lo, const float* hi, double cell) {
     return nc;
 }
 
-// histogram + scan (+ scatter when out != nullptr) of the points into level L
+// histogram + scan + scatter of the points into level L; without `scatter`
+// only the histogram
 static void bucket(dwg_ctx* ctx, const float* p, int64_t n, dwg_knn_index::Level& L, bool scatter) {
     L.ncells = int64_t(L.G.dim[0]) * L.G.dim[1] * L.G.dim[2];
     dwg::dev_free(L.cell_start);
     L.cell_start = nullptr;
     L.cell_start = static_cast<decltype(L.cell_start)>(dev_malloc(sizeof(int64_t) * (L.ncells + 1)));
-    int* cell_of = static_cast<int*>(ctx->buf("knn_cell_of", sizeof(int) * n));
+    int2* place = scatter ? static_cast<int2*>(ctx->buf("knn_place", sizeof(int2) * n)) : nullptr;
     fill_u32(ctx, L.cell_start, 0, 2 * (L.ncells + 1));
     hipLaunchKernelGGL(knn_count_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, p, n, L.G,
-                       reinterpret_cast<unsigned long long*>(L.cell_start), cell_of);
+                       reinterpret_cast<unsigned long long*>(L.cell_start), place);
     check_launch();
     if (!scatter) return;
-    unsigned long long* cursor = static_cast<unsigned long long*>(ctx->buf("knn_cursor", sizeof(uint64_t) * L.ncells));
     exclusive_scan<int64_t>(ctx, L.cell_start, L.ncells);
-    hipLaunchKernelGGL(copy_i64_kernel, dim3(grid_for(L.ncells, 256)), dim3(256), 0, ctx->stream, L.cell_start,
-                       cursor, L.ncells);
-    check_launch();
     L.pts = static_cast<decltype(L.pts)>(dev_malloc(sizeof(float4) * n));
-    hipLaunchKernelGGL(knn_scatter_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, p, n, cell_of, cursor,
+    hipLaunchKernelGGL(knn_scatter_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, p, n, place, L.cell_start,
                        L.pts);
     check_launch();
 }
@@ -439,10 +444,12 @@ dwg_knn_index* knn_build(dwg_ctx* ctx, const float* p, int64_t n, int k_hint) {
         while (cells_of(lo, hi, cell) > max_cells) cell *= 1.25;
         I->lvl[0].G = grid_args(lo, hi, cell);
         bucket(ctx, p, n, I->lvl[0], true);
-        I->lvl[1].G = grid_args(lo, hi, cell * 8.0);
-        bucket(ctx, p, n, I->lvl[1], true);
-        empty_distance(ctx, I->lvl[1]);
         pyramid(ctx, I->lvl[0]);
+        if (I->lvl[0].pyr_levels < 2) {  // its queries take the coarse level's shells
+            I->lvl[1].G = grid_args(lo, hi, cell * 8.0);
+            bucket(ctx, p, n, I->lvl[1], true);
+            empty_distance(ctx, I->lvl[1]);
+        }
     } catch (...) {
         delete I;
         throw;
@@ -568,44 +575,39 @@ __device__ __forceinline__ int bucket_of_point(const KnnGridArgs& G, const TileA
 
 // masked queries are left out
 __global__ void tile_count_kernel(const float* __restrict__ q, int64_t nq, const uint8_t* __restrict__ qmask, KnnGridArgs G, TileArgs T,
-                                  int* __restrict__ tile_of, unsigned long long* __restrict__ count) {
+                                  int2* __restrict__ place, unsigned long long* __restrict__ count) {
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     int tl = -1;  // every lane takes part in the run detection
-    if (t < nq) {
-        if (!qmask || qmask[t]) tl = bucket_of_point(G, T, q[3 * t], q[3 * t + 1], q[3 * t + 2]);
-        tile_of[t] = tl;
-    }
-    const int lane = threadIdx.x & 63;
-    const uint64_t starts = run_starts(tl);
-    if (tl >= 0 && ((starts >> lane) & 1ull)) atomicAdd(&count[tl], (unsigned long long)run_length(starts, lane));
+    if (t < nq && (!qmask || qmask[t])) tl = bucket_of_point(G, T, q[3 * t], q[3 * t + 1], q[3 * t + 2]);
+    const int at = take_place(tl, count);
+    if (t < nq) place[t] = make_int2(tl, at);
 }
 
-__global__ void tile_scatter_kernel(const int* __restrict__ tile_of, int64_t nq,
-                                    unsigned long long* __restrict__ cursor, int* __restrict__ order) {
+__global__ void tile_scatter_kernel(const int2* __restrict__ place, int64_t nq, const int64_t* __restrict__ start,
+                                    int* __restrict__ order) {
     const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    const int tl = t < nq ? tile_of[t] : -1;
-    const int lane = threadIdx.x & 63;
-    const uint64_t starts = run_starts(tl);
-    int base = 0;
-    if (tl >= 0 && ((starts >> lane) & 1ull))
-        base = int(atomicAdd(&cursor[tl], (unsigned long long)run_length(starts, lane)));
-    const int head = run_head(starts, lane);
-    const int hb = __shfl(base, head, 64);
-    if (tl >= 0) order[hb + (lane - head)] = int(t);
+    if (t >= nq) return;
+    const int2 b = place[t];
+    if (b.x >= 0) order[start[b.x] + b.y] = int(t);
 }
 
-// blocks a tile's queries take, kTileChunk each
-__global__ void tile_flags_kernel(const int64_t* __restrict__ start, int64_t ntiles, int chunk,
-                                  int64_t* __restrict__ flags) {
-    const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t > ntiles) return;
-    flags[t] = t < ntiles ? (start[kSubTiled * (t + 1)] - start[kSubTiled * t] + chunk - 1) / chunk : 0;
-}
-
-__global__ void tile_list_kernel(const int64_t* __restrict__ flags, int64_t ntiles, int2* __restrict__ list) {
-    const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= ntiles) return;
-    for (int64_t b = flags[t], e = flags[t + 1], c = 0; b + c < e; ++c) list[b + c] = make_int2(int(t), int(c));
+// The blocks that the tiles' queries take, `chunk` each, listed by (tile,
+// chunk): a block's tiles take their places with one atomic add, so the list
+// is in order but for the order of the blocks, on which no result depends.
+constexpr int kListThreads = 1024;
+__global__ __launch_bounds__(kListThreads) void tile_list_kernel(const int64_t* __restrict__ start, int64_t ntiles,
+                                                                 int chunk, int2* __restrict__ list,
+                                                                 unsigned long long* __restrict__ nlist) {
+    __shared__ int s_wsum[kListThreads / 64];
+    __shared__ int s_first;
+    const int64_t t = int64_t(blockIdx.x) * kListThreads + threadIdx.x;
+    const int64_t len = t < ntiles ? start[kSubTiled * (t + 1)] - start[kSubTiled * t] : 0;
+    const int blocks = int((len + chunk - 1) / chunk);
+    const int before = block_exclusive_sum<kListThreads>(blocks, s_wsum);
+    if (threadIdx.x == kListThreads - 1)
+        s_first = before + blocks > 0 ? int(atomicAdd(nlist, (unsigned long long)(before + blocks))) : 0;
+    __syncthreads();
+    for (int c = 0; c < blocks; ++c) list[s_first + before + c] = make_int2(int(t), c);
 }
 
 // Staged candidates are ordered by ring: the rows of cells that cross the
@@ -622,9 +624,13 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     KnnGridArgs G, TileArgs T, const int64_t* __restrict__ cell_start, const float4* __restrict__ pts,
     const int2* __restrict__ tiles, int chunk, const int64_t* __restrict__ tile_start, const int* __restrict__ order,
     const float* __restrict__ q, int k, const uint8_t* __restrict__ skip, int32_t* __restrict__ out_idx,
-    float* __restrict__ out_d2, int* __restrict__ redo, float* __restrict__ redo_kth, int64_t* __restrict__ redo_flag,
-    const int64_t* __restrict__ ntiles, KnnScatter sc) {
-    if (ntiles && int64_t(blockIdx.x) >= *ntiles) return;  // launched for the most tiles there can be
+    float* __restrict__ out_d2, int* __restrict__ redo, float* __restrict__ redo_kth,
+    unsigned long long* __restrict__ nredo, int64_t* __restrict__ tile_open, const int64_t* __restrict__ ntiles,
+    KnnScatter sc) {
+    if (ntiles && int64_t(blockIdx.x) >= *ntiles) {  // launched for the most tiles there can be
+        if (tile_open && threadIdx.x == 0) tile_open[blockIdx.x] = 0;
+        return;
+    }
     constexpr int kRegion = kTile + 2 * kHalo;
     // each row is split into the tile's own cells and the halo cells at x
     // distance 1 and 2 on either side, so that the staging order (by
@@ -646,6 +652,8 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     __shared__ int s_pref[kRows + 1];
     __shared__ int s_wsum[kTileThreads / 64];
     __shared__ int s_ring[kHalo + 2];
+    __shared__ int s_open;
+    if (threadIdx.x == 0) s_open = 0;
     const int tile = tiles[blockIdx.x].x;
     const int tx = tile % T.tdim[0], ty = (tile / T.tdim[0]) % T.tdim[1], tz = tile / (T.tdim[0] * T.tdim[1]);
     const int x0 = max(tx * kTile - kHalo, 0), x1 = min(tx * kTile + kTile - 1 + kHalo, G.dim[0] - 1);
@@ -775,12 +783,19 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
             exact = safe > 0.f && kd2 < safe * safe;
         }
         if (!exact) {
-            // the query keeps its place in tile order (compacted afterwards),
-            // so the far walk's waves get spatially coherent runs; the k
-            // candidates it has bound its k-th distance
-            redo_flag[t] = 1;
-            redo[t] = qi;
-            redo_kth[t] = kd2;
+            // a wave lists its open queries side by side: with the tile's
+            // others at the start of its range of places (tile_open), or after
+            // those of any tile; the k candidates a query has bound its k-th
+            // distance
+            const uint64_t open = __builtin_amdgcn_ballot_w64(true);
+            const int lane = threadIdx.x & 63, head = __builtin_ctzll(open);
+            int at = 0;
+            if (lane == head)
+                at = tile_open ? int(qs) + atomicAdd(&s_open, __builtin_popcountll(open))
+                               : int(atomicAdd(nredo, (unsigned long long)__builtin_popcountll(open)));
+            at = __shfl(at, head, 64) + __builtin_popcountll(open & ((1ull << lane) - 1ull));
+            redo[at] = qi;
+            redo_kth[at] = kd2;
             continue;
         }
         knn_store<K>(best, k, qi, out_idx, out_d2);
@@ -809,14 +824,32 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
             }
         }
     }
+    if (SCATTER || tile_open) __syncthreads();
+    if (tile_open && threadIdx.x == 0) tile_open[blockIdx.x] = s_open;
     if (SCATTER) {
-        __syncthreads();
         for (int h = threadIdx.x; h < kHash; h += kTileThreads) {
             const int key = s_hkey[h];
             if (key >= 0)
 #pragma unroll
                 for (int d = 0; d < 3; ++d) atomicAdd(&sc.acc[3 * int64_t(key) + d], s_hacc[h][d]);
         }
+    }
+}
+
+// The open queries of the tiles, each tile's at the start of its range of
+// places, one after the other in the list's order (pos: the scan of tile_open)
+__global__ __launch_bounds__(64) void tile_open_kernel(const int2* __restrict__ tiles, int chunk,
+                                                       const int64_t* __restrict__ tile_start,
+                                                       const int64_t* __restrict__ pos, const int* __restrict__ tmp_q,
+                                                       const float* __restrict__ tmp_kth, int* __restrict__ redo,
+                                                       float* __restrict__ redo_kth) {
+    const int64_t b = pos[blockIdx.x], n = pos[blockIdx.x + 1] - b;
+    if (n == 0) return;
+    const int2 e = tiles[blockIdx.x];
+    const int64_t qs = tile_start[int64_t(e.x) * kSubTiled] + int64_t(e.y) * chunk;
+    for (int64_t j = threadIdx.x; j < n; j += 64) {
+        redo[b + j] = tmp_q[qs + j];
+        redo_kth[b + j] = tmp_kth[qs + j];
     }
 }
 
@@ -1266,11 +1299,11 @@ __global__ __launch_bounds__(kDescWaves * 64) void knn_descent_kernel(
             const int l = int(e >> 56) & 0xF;
             const int x = 2 * int(e & 0xFFFF) + (c & 1), y = 2 * int((e >> 16) & 0xFFFF) + ((c >> 1) & 1),
                       z = 2 * int((e >> 32) & 0xFFFF) + (c >> 2);
-            int64_t ci = 0;
+            uint32_t ci = 0;  // an index has at most 2^27 cells
             float d = INFINITY;
             if (on) {
                 const int4 cd = s_dim[l - 1];
-                ci = x + int64_t(cd.x) * (y + int64_t(cd.y) * z);
+                ci = uint32_t(x) + uint32_t(cd.x) * (uint32_t(y) + uint32_t(cd.y) * uint32_t(z));
                 if (BOXES) {
                     const int64_t bi = 2 * ((l == 1 ? 0 : Y.ncells + s_off[l - 1]) + ci);
                     d = tight_box_d2(Y.box[bi], Y.box[bi + 1], qx, qy, qz);
@@ -1345,7 +1378,7 @@ __global__ __launch_bounds__(kDescWaves * 64) void knn_descent_kernel(
 }
 
 // The same pyramid walk shared by a wave: 64 neighbouring queries (the far
-// queries arrive in tile order) walk the union of their searches with one
+// queries arrive tile by tile) walk the union of their searches with one
 // wave-uniform stack of (block, lanes that need it) in LDS, the way the
 // Barnes-Hut walk shares its tree.  Every block and every point is then one
 // load for the wave instead of 64 scattered ones, and the lanes stay in
@@ -1654,13 +1687,14 @@ static void launch_far(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int
 // The queries 0..nq−1 (masked by qmask) bucketed by tile of kTile³ fine cells
 // and eighth of it: order[start[sub·t]..start[sub·(t+1))) are tile t's
 // queries, list[0..*nlist) the tiles that have any, once for each `chunk` of
-// them (tile, chunk)
+// them (tile, chunk); *nopen is 0
 constexpr int64_t kTileBlocks = 4096;
 struct TileBuckets {
     TileArgs T;
     int64_t ntiles = 0, max_list = 0;
     int chunk = 0;
     int64_t* nlist = nullptr;
+    int64_t* nopen = nullptr;
     int64_t* start = nullptr;
     int* order = nullptr;
     int2* list = nullptr;
@@ -1676,57 +1710,48 @@ static TileBuckets tile_buckets(dwg_ctx* ctx, const dwg_knn_index* I, const floa
     const int64_t ntiles = int64_t(T.tdim[0]) * T.tdim[1] * T.tdim[2], nb = ntiles * sub;
     DWG_REQUIRE(nb < (int64_t(1) << 31), "too many query buckets");
     B.ntiles = ntiles;
-    int* tile_of = static_cast<int*>(ctx->buf("knnt_tile_of", sizeof(int) * nq));
-    int64_t* start = static_cast<int64_t*>(ctx->buf("knnt_start", sizeof(int64_t) * (nb + 1)));
-    unsigned long long* cursor = static_cast<unsigned long long*>(ctx->buf("knnt_cursor", sizeof(uint64_t) * nb));
+    int2* place = static_cast<int2*>(ctx->buf("knnt_place", sizeof(int2) * nq));
+    // the buckets' starts, then the two counts
+    int64_t* start = static_cast<int64_t*>(ctx->buf("knnt_start", sizeof(int64_t) * (nb + 3)));
+    B.nlist = start + nb + 1;
+    B.nopen = start + nb + 2;
     int* order = static_cast<int*>(ctx->buf("knnt_order", sizeof(int) * nq));
-    int64_t* flags = static_cast<int64_t*>(ctx->buf("knnt_flags", sizeof(int64_t) * (ntiles + 1)));
     // a tile's queries are split over blocks so that there are a few thousand:
     // 230,000 centroids over 3,375 points fill 300 tiles, each a thousand
     // queries long (tiled pass 1.3 → 0.2 ms)
     B.chunk = kTileThreads * int(std::max<int64_t>(1, nq / (kTileBlocks * kTileThreads)));
     B.max_list = std::min(ntiles, nq) + nq / B.chunk;
     int2* list = static_cast<int2*>(ctx->buf("knnt_list", sizeof(int2) * size_t(B.max_list)));
-    fill_u32(ctx, start, 0, 2 * (nb + 1));
+    fill_u32(ctx, start, 0, 2 * (nb + 3));
     hipLaunchKernelGGL(tile_count_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, q, nq, qmask, G, T,
-                       tile_of, reinterpret_cast<unsigned long long*>(start));
+                       place, reinterpret_cast<unsigned long long*>(start));
     check_launch();
     exclusive_scan<int64_t>(ctx, start, nb);
-    hipLaunchKernelGGL(copy_i64_kernel, dim3(grid_for(nb, 256)), dim3(256), 0, ctx->stream, start, cursor, nb);
-    check_launch();
-    hipLaunchKernelGGL(tile_scatter_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, tile_of, nq, cursor,
+    hipLaunchKernelGGL(tile_scatter_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, place, nq, start,
                        order);
     check_launch();
     B.start = start;
     B.order = order;
-    hipLaunchKernelGGL(tile_flags_kernel, dim3(grid_for(ntiles + 1, 256)), dim3(256), 0, ctx->stream, start, ntiles,
-                       B.chunk, flags);
+    hipLaunchKernelGGL(tile_list_kernel, dim3(grid_for(ntiles, kListThreads)), dim3(kListThreads), 0, ctx->stream, start,
+                       ntiles, B.chunk, list, reinterpret_cast<unsigned long long*>(B.nlist));
     check_launch();
-    exclusive_scan<int64_t>(ctx, flags, ntiles);
-    hipLaunchKernelGGL(tile_list_kernel, dim3(grid_for(ntiles, 256)), dim3(256), 0, ctx->stream, flags, ntiles, list);
-    check_launch();
-    B.nlist = flags + ntiles;
     B.list = list;
     return B;
-}
-
-// the queries a tiled pass leaves open, gathered in tile order
-__global__ void redo_compact_kernel(const int64_t* __restrict__ pos, const int* __restrict__ tmp_q,
-                                    const float* __restrict__ tmp_kth, int64_t n, int* __restrict__ redo,
-                                    float* __restrict__ redo_kth) {
-    const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= n || pos[t + 1] == pos[t]) return;
-    redo[pos[t]] = tmp_q[t];
-    redo_kth[pos[t]] = tmp_kth[t];
 }
 
 // up to this many tile blocks are launched without reading how many have
 // queries: the surplus blocks return at once, for less than the read costs
 constexpr int64_t kTileBlind = 16384;
 
+// From this many queries the open ones are brought into the order of their
+// tiles (three launches): there may then be enough of them to share walks,
+// which need 64 neighbours.  180,000 of 3M centroids without it: walks and
+// their left-over searches 1.80 → 2.43 ms
+constexpr int64_t kOpenOrder = 262144;
+
 // The tiled pass over the queries 0..nq−1 (masked by qmask); the queries it
-// cannot close are listed in redo with their k-th bound in redo_kth, in tile
-// order.  Returns the device address of their count.
+// cannot close are listed in redo with their k-th bound in redo_kth, tile by
+// tile.  Returns the device address of their count.
 static const int64_t* tiled_pass(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const uint8_t* qmask,
                                  int k, const uint8_t* skip, int32_t* out_idx, float* out_d2, int* redo,
                                  float* redo_kth, const std::string& name, const KnnScatter* sc) {
@@ -1734,17 +1759,20 @@ static const int64_t* tiled_pass(dwg_ctx* ctx, const dwg_knn_index* I, const flo
     const TileBuckets B = tile_buckets(ctx, I, q, nq, qmask);
     const TileArgs& T = B.T;
     if (ctx->profile) ctx->count(name + ":queries", read_scalar<int64_t>(ctx, B.start + B.ntiles * kSubTiled));
-    // each query's place t in tile order gets its flag (and, when open, its
-    // index and bound) in scratch arrays, compacted below
-    int64_t* rflag = static_cast<int64_t*>(ctx->buf("knnt_rflag", sizeof(int64_t) * (nq + 1)));
-    int* tmp_q = static_cast<int*>(ctx->buf("knnt_rtmp", sizeof(int) * nq + 64));
-    float* tmp_kth = static_cast<float*>(ctx->buf("knnt_rkth", sizeof(float) * nq + 64));
-    fill_u32(ctx, rflag, 0, 2 * (nq + 1));
+    auto* nopen = reinterpret_cast<unsigned long long*>(B.nopen);
+    int* open_q = redo;
+    float* open_kth = redo_kth;
+    int64_t* tile_open = nullptr;
     int64_t blocks = B.max_list;
     const int64_t* exact = B.nlist;
     if (blocks > kTileBlind) {
         blocks = read_scalar<int64_t>(ctx, B.nlist);
         exact = nullptr;
+    }
+    if (nq >= kOpenOrder) {
+        open_q = static_cast<int*>(ctx->buf("knnt_rtmp", sizeof(int) * nq));
+        open_kth = static_cast<float*>(ctx->buf("knnt_rkth", sizeof(float) * nq));
+        tile_open = static_cast<int64_t*>(ctx->buf("knnt_topen", sizeof(int64_t) * (blocks + 1)));
     }
     if (blocks > 0) {
         ProfileScope pt(ctx, name.c_str());
@@ -1754,11 +1782,11 @@ static const int64_t* tiled_pass(dwg_ctx* ctx, const dwg_knn_index* I, const flo
         if (sc)                                                                                                     \
             hipLaunchKernelGGL((knn_tile_kernel<KK, true>), dim3(unsigned(blocks)), dim3(kTileThreads), 0,          \
                                ctx->stream, G, T, I->lvl[0].cell_start, I->lvl[0].pts, B.list, B.chunk, B.start, B.order, \
-                               q, k, skip, out_idx, out_d2, tmp_q, tmp_kth, rflag, exact, scv);                        \
+                               q, k, skip, out_idx, out_d2, open_q, open_kth, nopen, tile_open, exact, scv);              \
         else                                                                                                        \
             hipLaunchKernelGGL((knn_tile_kernel<KK, false>), dim3(unsigned(blocks)), dim3(kTileThreads), 0,         \
                                ctx->stream, G, T, I->lvl[0].cell_start, I->lvl[0].pts, B.list, B.chunk, B.start, B.order, \
-                               q, k, skip, out_idx, out_d2, tmp_q, tmp_kth, rflag, exact, scv);                        \
+                               q, k, skip, out_idx, out_d2, open_q, open_kth, nopen, tile_open, exact, scv);              \
     } while (0)
         if (k <= 8) DWG_KNNT(8);
         else if (k <= 10) DWG_KNNT(10);
@@ -1769,11 +1797,14 @@ static const int64_t* tiled_pass(dwg_ctx* ctx, const dwg_knn_index* I, const flo
 #undef DWG_KNNT
         check_launch();
     }
-    exclusive_scan<int64_t>(ctx, rflag, nq);
-    hipLaunchKernelGGL(redo_compact_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, rflag, tmp_q, tmp_kth, nq,
-                       redo, redo_kth);
-    check_launch();
-    return rflag + nq;
+    if (!tile_open) return B.nopen;
+    exclusive_scan<int64_t>(ctx, tile_open, blocks);
+    if (blocks > 0) {
+        hipLaunchKernelGGL(tile_open_kernel, dim3(unsigned(blocks)), dim3(64), 0, ctx->stream, B.list, B.chunk, B.start,
+                           tile_open, open_q, open_kth, redo, redo_kth);
+        check_launch();
+    }
+    return tile_open + blocks;
 }
 
 void knn_query(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, int k, const uint8_t* skip,

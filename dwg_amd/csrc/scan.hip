@@ -3,6 +3,7 @@
 #include "scan.h"
 
 #include <cstring>
+#include <type_traits>
 
 namespace dwg {
 
@@ -12,19 +13,27 @@ constexpr int kScanThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
 
+// v of the lane `off` below
 template <class T>
-__device__ T block_exclusive_scan(T v, T* lds, T& total) {
-    // wave-level inclusive scan via LDS (64 lanes), then across 4 waves
+__device__ __forceinline__ T from_lane_below(const T& v, int off) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    uint32_t w[sizeof(T) / 4];
+    __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / 4; ++i) w[i] = uint32_t(__shfl_up(int(w[i]), off, 64));
+    T r;
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
+}
+
+template <class T>
+__device__ T block_exclusive_scan(T v, T& total) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     T x = v;
-    lds[threadIdx.x] = x;
-    __syncthreads();
+#pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
-        T y = (lane >= off) ? lds[threadIdx.x - off] : T();
-        __syncthreads();
-        x = x + y;
-        lds[threadIdx.x] = x;
-        __syncthreads();
+        const T y = from_lane_below(x, off);
+        x = x + (lane >= off ? y : T());
     }
     __shared__ T wave_tot[kScanThreads / 64];
     if (lane == 63) wave_tot[wave] = x;
@@ -40,21 +49,29 @@ __device__ T block_exclusive_scan(T v, T* lds, T& total) {
 template <class T>
 __global__ __launch_bounds__(kScanThreads) void tile_reduce(const T* __restrict__ d, int64_t n,
                                                              T* __restrict__ partial) {
-    __shared__ T lds[kScanThreads];
     int64_t base = int64_t(blockIdx.x) * kScanTile + int64_t(threadIdx.x) * kScanItems;
     T s = T();
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k)
         if (base + k < n) s = s + d[base + k];
     T total;
-    (void)block_exclusive_scan(s, lds, total);
+    (void)block_exclusive_scan(s, total);
     if (threadIdx.x == 0) partial[blockIdx.x] = total;
 }
 
-template <class T>
+// SUMS: partial holds the tiles' sums, of which each block adds up those before
+// its own (whole numbers: the order does not matter); else their scan.
+template <class T, bool SUMS>
 __global__ __launch_bounds__(kScanThreads) void tile_scan(T* __restrict__ d, int64_t n,
                                                            const T* __restrict__ partial) {
-    __shared__ T lds[kScanThreads];
+    T before;
+    if constexpr (SUMS) {
+        T p = T();
+        for (unsigned j = threadIdx.x; j < blockIdx.x; j += kScanThreads) p = p + partial[j];
+        (void)block_exclusive_scan(p, before);
+    } else {
+        before = partial[blockIdx.x];
+    }
     int64_t base = int64_t(blockIdx.x) * kScanTile + int64_t(threadIdx.x) * kScanItems;
     T items[kScanItems];
     T s = T();
@@ -64,20 +81,19 @@ __global__ __launch_bounds__(kScanThreads) void tile_scan(T* __restrict__ d, int
         s = s + items[k];
     }
     T total;
-    T run = block_exclusive_scan(s, lds, total) + partial[blockIdx.x];
+    T run = block_exclusive_scan(s, total) + before;
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         if (base + k < n) d[base + k] = run;
         run = run + items[k];
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kScanThreads - 1) d[n] = partial[blockIdx.x] + total;
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kScanThreads - 1) d[n] = before + total;
 }
 
 template <class T>
 __global__ __launch_bounds__(kScanThreads) void single_scan(T* __restrict__ d, int64_t n) {
     // inputs of at most kScanTile elements (the top level of a scan): one
     // block, kScanItems consecutive elements a thread
-    __shared__ T lds[kScanThreads];
     const int64_t base = int64_t(threadIdx.x) * kScanItems;
     T items[kScanItems];
     T s = T();
@@ -87,7 +103,7 @@ __global__ __launch_bounds__(kScanThreads) void single_scan(T* __restrict__ d, i
         s = s + items[k];
     }
     T total;
-    T run = block_exclusive_scan(s, lds, total);
+    T run = block_exclusive_scan(s, total);
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         if (base + k < n) d[base + k] = run;
@@ -232,6 +248,12 @@ void radix_sort_pairs(dwg_ctx* ctx, const uint64_t* kin, const int* vin, uint64_
     }
 }
 
+// Up to this many tiles (8M numbers) a block adds up the tiles before its own
+// itself, 64 kB at most and from L2: one launch of three, 4.5 µs back to back,
+// is gone.  Beyond, these reads would grow with the square of the tiles.
+// Sums of FP64 keep the scan of the tiles, whose order of adding stays.
+constexpr int64_t kScanSums = 4096;
+
 template <class T>
 void exclusive_scan(dwg_ctx* ctx, T* d, int64_t n, int level) {
     if (n <= kScanTile) {
@@ -244,8 +266,16 @@ void exclusive_scan(dwg_ctx* ctx, T* d, int64_t n, int level) {
     T* partial = static_cast<T*>(ctx->buf(name, sizeof(T) * (tiles + 1)));
     hipLaunchKernelGGL(tile_reduce<T>, dim3(unsigned(tiles)), dim3(kScanThreads), 0, ctx->stream, d, n, partial);
     check_launch();
+    if constexpr (std::is_integral<T>::value) {
+        if (tiles <= kScanSums) {
+            hipLaunchKernelGGL((tile_scan<T, true>), dim3(unsigned(tiles)), dim3(kScanThreads), 0, ctx->stream, d, n,
+                               partial);
+            check_launch();
+            return;
+        }
+    }
     exclusive_scan<T>(ctx, partial, tiles, level + 1);
-    hipLaunchKernelGGL(tile_scan<T>, dim3(unsigned(tiles)), dim3(kScanThreads), 0, ctx->stream, d, n, partial);
+    hipLaunchKernelGGL((tile_scan<T, false>), dim3(unsigned(tiles)), dim3(kScanThreads), 0, ctx->stream, d, n, partial);
     check_launch();
 }
 
