@@ -466,52 +466,39 @@ dwg_knn_index* knn_build(dwg_ctx* ctx, const float* p, int64_t n, int k_hint) {
 constexpr uint64_t kNoKey = 0x7FF0000000000000ull;
 
 template <int K>
-__device__ __forceinline__ void knn_reset(uint64_t (&best)[K], int k) {
+__device__ __forceinline__ void knn_reset(uint64_t (&best)[K], int k, uint64_t none = kNoKey) {
 #pragma unroll
-    for (int j = 0; j < K; ++j) best[j] = j < k ? kNoKey : 0ull;
+    for (int j = 0; j < K; ++j) best[j] = j < k ? none : 0ull;
 }
 
-// key < best[0]: it replaces the largest key and sinks to its place.  Every
-// key (and kNoKey, and the 0 of an unused slot) read as a double is a
-// non-negative number, never NaN, and non-negative doubles order as their
-// bit patterns do (the kernels keep FP64 denormals): each compare-exchange
-// is one FP64 max and one min, which return one of their operands bit for
-// bit, instead of a 64-bit compare and four selects.  Written as the two
-// instructions themselves: the compiler would first quiet possible
-// signalling NaNs of both operands, which these keys never are
-__device__ __forceinline__ uint64_t key_max(uint64_t a, uint64_t b) {
-    uint64_t r;
-    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ uint64_t key_min(uint64_t a, uint64_t b) {
-    uint64_t r;
-    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-
+// The key takes its place in the list and the largest key leaves it (the key
+// itself, if it is not below that).  Every key (and kNoKey, and the 0 of an
+// unused slot) read as a double is a non-negative number, never NaN, and
+// non-negative doubles order as their bit patterns do (the kernels keep FP64
+// denormals): slot i takes max(min(key, slot i), slot i + 1), one FP64 min and
+// one max which return one of their operands bit for bit.  Both in place, so
+// no slot waits for another and no register is copied; written as the
+// instructions themselves, as the compiler would first quiet possible
+// signalling NaNs of the operands, which these keys never are.
 template <int K>
 __device__ __forceinline__ void knn_insert(uint64_t (&best)[K], uint64_t key) {
-    best[0] = key;
 #pragma unroll
-    for (int i = 0; i < K - 1; ++i) {
-        const uint64_t a = best[i], b = best[i + 1];
-        best[i] = key_max(a, b);
-        best[i + 1] = key_min(a, b);
-    }
+    for (int i = 0; i + 1 < K; ++i)
+        asm("v_min_f64 %0, %1, %0\n\tv_max_f64 %0, %0, %2" : "+&v"(best[i]) : "v"(key), "v"(best[i + 1]));
+    asm("v_min_f64 %0, %1, %0" : "+v"(best[K - 1]) : "v"(key));
 }
 
 // writes the k keys in ascending order (index −1 / d² ∞ where fewer were found)
 template <int K>
 __device__ __forceinline__ void knn_store(const uint64_t (&best)[K], int k, int64_t row, int32_t* __restrict__ out_idx,
-                                          float* __restrict__ out_d2) {
+                                          float* __restrict__ out_d2, uint64_t none = kNoKey) {
 #pragma unroll
     for (int j = 0; j < K; ++j) {
         if (j < k) {
             const uint64_t b = best[j];
             const int64_t o = row * k + (k - 1 - j);
-            out_idx[o] = b == kNoKey ? -1 : int32_t(uint32_t(b));
-            if (out_d2) out_d2[o] = b == kNoKey ? INFINITY : __uint_as_float(uint32_t(b >> 32));
+            out_idx[o] = b == none ? -1 : int32_t(uint32_t(b));
+            if (out_d2) out_d2[o] = b == none ? INFINITY : __uint_as_float(uint32_t(b >> 32));
         }
     }
 }
@@ -530,6 +517,17 @@ constexpr double kScatterFix = 1099511627776.0;  // 2^40
 constexpr int kTile = 4;
 constexpr int kStage = 512;
 constexpr int kTileThreads = 256;
+// The candidates are tested kBatch at a time: half of the batches hold nothing
+// for any lane of a wave, which one compare then tells.  Of 300 candidates a
+// wave takes in about 100, as the union of its lanes' neighbours alone has 75:
+// these insertions and the distances bound the pass (3M centroids over 1M
+// points, 15 neighbours: 1.29 → 1.13 ms; 300,000 points, 17: 0.151 → 0.120).
+// Sorting a batch to join it at once spills (1.38 ms); boxes around the
+// batches, also with the nearest first, cost what they save.
+constexpr int kBatch = 16;
+static_assert(kStage % kBatch == 0 && kTileThreads >= kBatch, "whole batches, filled up by one thread a place");
+// An empty slot here: its high word is a d² of ∞, which any d² but NaN passes
+constexpr uint64_t kFar = 0x7F800000FFFFFFFFull;
 // most queries close within 2 cells of their tile.  Wider passes for the
 // others (5 and 9 cells) cost more than walking the pyramid at once: 200,000
 // queries over 1M points, half of them off the surface, 5.6 → 3.4 ms
@@ -620,7 +618,7 @@ __global__ __launch_bounds__(kListThreads) void tile_list_kernel(const int64_t* 
 // global atomics; integer sums are associative, so the result equals
 // per-pair atomics bit for bit.
 template <int K, bool SCATTER>
-__global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
+__global__ __launch_bounds__(kTileThreads, K <= 17 ? 4 : 2) void knn_tile_kernel(
     KnnGridArgs G, TileArgs T, const int64_t* __restrict__ cell_start, const float4* __restrict__ pts,
     const int2* __restrict__ tiles, int chunk, const int64_t* __restrict__ tile_start, const int* __restrict__ order,
     const float* __restrict__ q, int k, const uint8_t* __restrict__ skip, int32_t* __restrict__ out_idx,
@@ -647,9 +645,8 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
         }
     }
     __shared__ float4 s_pts[kStage];
-    __shared__ int64_t s_rb[kRows];
-    __shared__ int s_cnt[kRows];
-    __shared__ int s_pref[kRows + 1];
+    __shared__ int s_rb[kRows];
+    __shared__ int s_pref[kRows + 1];  // the rows' point counts, then their exclusive prefix
     __shared__ int s_wsum[kTileThreads / 64];
     __shared__ int s_ring[kHalo + 2];
     __shared__ int s_open;
@@ -667,7 +664,7 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     // h · kTileThreads, h < kRowIters
     constexpr int kRowIters = (kRows + kTileThreads - 1) / kTileThreads;
     int ring[kRowIters], rank[kRowIters], rc[kRowIters];
-    int64_t rb[kRowIters];
+    int rb[kRowIters];
 #pragma unroll
     for (int h = 0; h < kRowIters; ++h) {
         ring[h] = rank[h] = rc[h] = 0;
@@ -685,8 +682,8 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
             xa = max(xa, x0);
             xb = min(xb, x1);
             const int64_t c = xa + int64_t(G.dim[0]) * (y + int64_t(G.dim[1]) * z);
-            rb[h] = cell_start[c];
-            rc[h] = xb >= xa ? int(cell_start[c + (xb - xa) + 1] - rb[h]) : 0;
+            rb[h] = int(cell_start[c]);  // an index holds fewer than 2^31 points
+            rc[h] = xb >= xa ? int(cell_start[c + (xb - xa) + 1]) - rb[h] : 0;
             const int dy = max(max(ty * kTile - y, y - (ty * kTile + kTile - 1)), 0);
             const int dz = max(max(tz * kTile - z, z - (tz * kTile + kTile - 1)), 0);
             ring[h] = max(max(dy, dz), dx);
@@ -702,7 +699,7 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
         if (threadIdx.x + h * kTileThreads < nrows) {
             const int pos = s_ring[ring[h]] + rank[h];
             s_rb[pos] = rb[h];
-            s_cnt[pos] = rc[h];
+            s_pref[pos] = rc[h];
         }
     }
     __syncthreads();
@@ -713,7 +710,7 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
 #pragma unroll
         for (int i = 0; i < kRowIters; ++i) {
             const int r = threadIdx.x * kRowIters + i;
-            loc[i] = r < nrows ? s_cnt[r] : 0;
+            loc[i] = r < nrows ? s_pref[r] : 0;
             sum += loc[i];
         }
         int run = block_exclusive_sum<kTileThreads>(sum, s_wsum);
@@ -736,15 +733,23 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     const float fhz = z1 + 1 < G.dim[2] ? G.lo[2] + float(z1 + 1) * G.cell : INFINITY;
     const int64_t qs = tile_start[int64_t(tile) * kSubTiled] + int64_t(tiles[blockIdx.x].y) * chunk;
     const int64_t qe = min(tile_start[int64_t(tile + 1) * kSubTiled], qs + chunk);
+    // one staging serves all queries: the waves left over leave after it (a
+    // barrier waits for the waves that are there).  Half of them are, with 105
+    // queries a tile, and held the places of others (1.13 → 1.07 ms for 3M
+    // centroids)
+    const bool once = total <= kStage && qe - qs <= kTileThreads;
+    const int stay = once ? int(qe - qs + 63) / 64 * 64 : kTileThreads;
     for (int64_t qb = qs; qb < qe; qb += kTileThreads) {
         const int64_t t = qb + threadIdx.x;
         const bool active = t < qe;
         const int qi = active ? order[t] : 0;
-        const float qx = active ? q[3 * int64_t(qi)] : 0.f, qy = active ? q[3 * int64_t(qi) + 1] : 0.f,
-                    qz = active ? q[3 * int64_t(qi) + 2] : 0.f;
+        // (a lane without a query is at no distance from anything)
+        const float qx = active ? q[3 * int64_t(qi)] : NAN, qy = active ? q[3 * int64_t(qi) + 1] : NAN,
+                    qz = active ? q[3 * int64_t(qi) + 2] : NAN;
         uint64_t best[K];
-        knn_reset<K>(best, k);
-        float kd2 = INFINITY;  // float d² of the k-th key: a cheap first test
+        const uint64_t has = __builtin_amdgcn_ballot_w64(active);
+        knn_reset<K>(best, k, kFar);
+        auto kth = [&]() { return __uint_as_float(uint32_t(best[0] >> 32)); };  // the k-th d², or ∞
         for (int cb = 0; cb < total; cb += kStage) {
             const int cnt = min(kStage, total - cb);
             __syncthreads();
@@ -757,30 +762,38 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
                     else hi = mid - 1;
                 }
                 float4 p = pts[s_rb[lo] + (g - s_pref[lo])];
-                if (skip && skip[__float_as_int(p.w)]) p.w = __int_as_float(-1);
+                if (skip && skip[__float_as_int(p.w)]) p.x = NAN;  // at no distance
                 s_pts[j] = p;
             }
+            const int padded = (cnt + kBatch - 1) / kBatch * kBatch;
+            if (threadIdx.x < padded - cnt) s_pts[cnt + threadIdx.x] = make_float4(NAN, 0.f, 0.f, 0.f);
             __syncthreads();
-            auto candidate = [&](const float4 p) {
-                const float d2 = dist2(qx - p.x, qy - p.y, qz - p.z);
-                if (!(d2 <= kd2)) return;
-                const int idx = __float_as_int(p.w);
-                if (idx < 0) return;
-                const uint64_t key = (uint64_t(__float_as_uint(d2)) << 32) | uint32_t(idx);
-                if (key < best[0]) {
-                    knn_insert<K>(best, key);
-                    kd2 = best[0] == kNoKey ? INFINITY : __uint_as_float(uint32_t(best[0] >> 32));
+            // a wave without queries is done where nothing is staged after this
+            if (!has && once) return;
+            for (int j = 0; j < (has ? padded : 0); j += kBatch) {
+                float d2[kBatch], least = NAN;  // no number for a lane without a query
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    const float4 p = s_pts[j + u];
+                    d2[u] = dist2(qx - p.x, qy - p.y, qz - p.z);
+                    least = fminf(least, d2[u]);
                 }
-            };
-            if (active)
-                for (int j = 0; j < cnt; ++j) candidate(s_pts[j]);
+                if (!__builtin_amdgcn_ballot_w64(least <= kth())) continue;
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    const bool near = d2[u] <= kth();
+                    if (!__builtin_amdgcn_ballot_w64(near)) continue;
+                    knn_insert<K>(best, near ? (uint64_t(__float_as_uint(d2[u])) << 32) | __float_as_uint(s_pts[j + u].w)
+                                             : kFar);
+                }
+            }
         }
         if (!active) continue;
         const float dmin = fminf(fminf(fminf(qx - flx, fhx - qx), fminf(qy - fly, fhy - qy)), fminf(qz - flz, fhz - qz));
         bool exact = dmin == INFINITY;
-        if (!exact && best[0] != kNoKey) {
+        if (!exact && best[0] != kFar) {
             const float safe = dmin * (1.0f - 1e-5f) - 1e-6f * G.cell;
-            exact = safe > 0.f && kd2 < safe * safe;
+            exact = safe > 0.f && kth() < safe * safe;
         }
         if (!exact) {
             // a wave lists its open queries side by side: with the tile's
@@ -795,17 +808,17 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
                                : int(atomicAdd(nredo, (unsigned long long)__builtin_popcountll(open)));
             at = __shfl(at, head, 64) + __builtin_popcountll(open & ((1ull << lane) - 1ull));
             redo[at] = qi;
-            redo_kth[at] = kd2;
+            redo_kth[at] = kth();
             continue;
         }
-        knn_store<K>(best, k, qi, out_idx, out_d2);
+        knn_store<K>(best, k, qi, out_idx, out_d2, kFar);
         if (SCATTER) {
             long long v[3];
 #pragma unroll
             for (int d = 0; d < 3; ++d) v[d] = __double2ll_rn(double(sc.val[3 * int64_t(qi) + d]) * kScatterFix);
 #pragma unroll
             for (int j = 0; j < K; ++j) {
-                if (j >= k || best[j] == kNoKey) continue;
+                if (j >= k || best[j] == kFar) continue;
                 const int idx = int(uint32_t(best[j]));
                 int h = int((uint32_t(idx) * 0x9E3779B1u) >> 24);  // 8 bits
                 bool done = false;
@@ -827,7 +840,7 @@ __global__ __launch_bounds__(kTileThreads) void knn_tile_kernel(
     if (SCATTER || tile_open) __syncthreads();
     if (tile_open && threadIdx.x == 0) tile_open[blockIdx.x] = s_open;
     if (SCATTER) {
-        for (int h = threadIdx.x; h < kHash; h += kTileThreads) {
+        for (int h = threadIdx.x; h < kHash; h += stay) {
             const int key = s_hkey[h];
             if (key >= 0)
 #pragma unroll
