@@ -26,7 +26,7 @@ struct dwg_octree {
     float4* ec = nullptr;      // (EC/4π, 0), refreshed per iteration
 
     float4* sa = nullptr;      // packed sources in tree order (x, y, z, s)
-    float4* sb = nullptr;      // (A·n/4π, A)
+    float4* sb = nullptr;      // (A·n/4π, ·)
     int* perm = nullptr;       // tree slot → caller index
     dwg::Double3* an64 = nullptr;  // FP64 prefix sums of A·n (n+1)
     double4* cell = nullptr;       // cell centre and width (breadth-first node order)

@@ -29,26 +29,6 @@ namespace dwg {
 // ---------------------------------------------------------------------------
 // per-pair terms
 // ---------------------------------------------------------------------------
-// term from the offset d = p − q; s = screening radius of the source
-// term from the offset d and a squared distance r2 (normally |d|²)
-template <bool SCREENED>
-__device__ __forceinline__ float gwn_term_r2(float dx, float dy, float dz, float r2, float s, const float4 b,
-                                             float sigma, float sigma_l2e) {
-    const float dot = __builtin_fmaf(dz, b.z, __builtin_fmaf(dy, b.y, dx * b.x));
-    const float r = fast_sqrt(r2);
-    if constexpr (!SCREENED) {
-        const float den = __builtin_fmaf(r2, r, kEpsPlain * kInv4Pi);
-        return dot * fast_rcp(den);
-    } else {
-        const float rho = fmaxf(r, s);
-        const float e = fast_exp2(sigma_l2e * rho);
-        const float rho3 = rho * rho * rho;
-        const float den = __builtin_fmaf(e, rho3, kEpsScreened * kInv4Pi);
-        const float t = (__builtin_fmaf(sigma, rho, 1.0f) * dot) * fast_rcp(den);
-        return r > 1e-10f ? t : 0.0f;
-    }
-}
-
 // max of two non-negative floats on their bit patterns (the integer order is
 // the float order there): one instruction, no NaN quieting of the operands
 __device__ __forceinline__ float max_nonneg(float a, float b) {
@@ -100,16 +80,17 @@ __device__ __forceinline__ float add_rounded(float part, float x, float inv) {
     return part + t;
 }
 
+// The direct sums' point term as such factors, a = (p, ·), b = (A·n/4π, s²);
+// 0 at the guard.  With the product left to the sum's multiply-add it takes
+// 21 instructions screened (24 with ρ = max(r, s), ρ·ρ·ρ and a selected sum:
+// 10,000 sources at 2M queries 13.6 → 11.9 ms, the chip's whole issue rate).
 template <bool SCREENED>
-__device__ __forceinline__ float gwn_term_d(float dx, float dy, float dz, float s, const float4 b, float sigma,
-                                            float sigma_l2e) {
-    return gwn_term_r2<SCREENED>(dx, dy, dz, dist2(dx, dy, dz), s, b, sigma, sigma_l2e);
-}
-
-template <bool SCREENED>
-__device__ __forceinline__ float gwn_term(float qx, float qy, float qz, const float4 a, const float4 b,
-                                          float sigma, float sigma_l2e) {
-    return gwn_term_d<SCREENED>(a.x - qx, a.y - qy, a.z - qz, a.w, b, sigma, sigma_l2e);
+__device__ __forceinline__ float gwn_term_split(float qx, float qy, float qz, const float4 a, const float4 b,
+                                                float sigma, float sigma_l2e, float& inv) {
+    const float dx = a.x - qx, dy = a.y - qy, dz = a.z - qz;
+    bool ok;
+    const float x = tree_term_split<SCREENED>(dx, dy, dz, dist2(dx, dy, dz), b.w, b, sigma, sigma_l2e, inv, ok);
+    return ok ? x : 0.f;
 }
 
 // DWG_NEAR_FP64: a screened point term inside its source's screening radius
@@ -169,7 +150,8 @@ __device__ __forceinline__ void gwn_term_grad_d(float dx, float dy, float dz, fl
 }
 
 // ---------------------------------------------------------------------------
-// source packing: (x, y, z, s) and (A·n/4π, A)
+// source packing: (x, y, z, s) and (A·n/4π, s²), s² 0 for s ≤ 0 or NaN (ρ = r)
+// and kept finite with s
 // ---------------------------------------------------------------------------
 __global__ void pack_sources_kernel(const float* __restrict__ pts, const float* __restrict__ nrm,
                                     const float* __restrict__ area, const float* __restrict__ radii,
@@ -183,7 +165,8 @@ __global__ void pack_sources_kernel(const float* __restrict__ pts, const float* 
     const float s = use_radii ? radii[p] : kScreenDefault;
     if (sa) sa[i] = make_float4(pts[3 * p], pts[3 * p + 1], pts[3 * p + 2], s);
     const float nx = nrm[3 * p], ny = nrm[3 * p + 1], nz = nrm[3 * p + 2];
-    sb[i] = make_float4(A * nx * kInv4Pi, A * ny * kInv4Pi, A * nz * kInv4Pi, A);
+    const float s2 = s > 0.f ? (s < INFINITY ? fminf(s * s, 3.402823466e38f) : s) : 0.f;
+    sb[i] = make_float4(A * nx * kInv4Pi, A * ny * kInv4Pi, A * nz * kInv4Pi, s2);
     if (an64) an64[i] = Double3(double(A) * nx, double(A) * ny, double(A) * nz);
 }
 
@@ -202,25 +185,27 @@ __device__ __forceinline__ void direct_value(const float4* __restrict__ sa, cons
     const float sl2e = sigma * kLog2e;
     sum = comp = 0.f;
     near = 0.0;
-    auto term = [&](const float4 a, const float4 b) {
+    auto add = [&](float& part, const float4 a, const float4 b) {
+        float inv;
+        float x = gwn_term_split<SCREENED>(qx, qy, qz, a, b, sigma, sl2e, inv);
         if constexpr (NEAR64) {
             const float dx = a.x - qx, dy = a.y - qy, dz = a.z - qz;
             const bool nr = near_field(dist2(dx, dy, dz), a.w);
             if (__builtin_amdgcn_ballot_w64(nr)) {
                 if (nr) near += near_term64(a, b, qx, qy, qz, sigma);
             }
-            return nr ? 0.f : gwn_term<SCREENED>(qx, qy, qz, a, b, sigma, sl2e);
+            x = nr ? 0.f : x;
         }
-        return gwn_term<SCREENED>(qx, qy, qz, a, b, sigma, sl2e);
+        part = __builtin_fmaf(x, inv, part);
     };
     for (; j0 + kDirectTile <= j1; j0 += kDirectTile) {
         float part = 0.f;
 #pragma unroll 8
-        for (int j = 0; j < kDirectTile; ++j) part += term(sa[j0 + j], sb[j0 + j]);
+        for (int j = 0; j < kDirectTile; ++j) add(part, sa[j0 + j], sb[j0 + j]);
         if (KAHAN) kahan_add(sum, comp, part); else sum += part;
     }
     float part = 0.f;
-    for (int64_t j = j0; j < j1; ++j) part += term(sa[j], sb[j]);
+    for (int64_t j = j0; j < j1; ++j) add(part, sa[j], sb[j]);
     if (KAHAN) kahan_add(sum, comp, part); else sum += part;
 }
 
