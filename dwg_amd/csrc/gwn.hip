@@ -1551,13 +1551,15 @@ static QueryArgs make_self(const dwg_octree* T) {
     return Q;
 }
 
-// Grids of fewer whole bricks than this leave the chip short of waves, and
-// the launch lasts as long as its longest walks: they take one 4×4×4 part a
-// wave, whose walk opens fewer nodes and lasts a quarter as long (96³ over 30k
-// sources 315 → 216 µs, 160³ over 500k 1,106 → 916 µs; at 256³, 65,536 bricks,
-// whole ones win, 1,776 against 2,204 µs).  The values are the same: each
-// point takes its own terms in the same order
-constexpr int64_t kWholeBricks = 24576;
+// Grids of few whole bricks leave the chip short of waves, and the launch lasts
+// as long as its longest walks: they take one 4×4×4 part a wave, whose walk
+// opens fewer nodes and lasts a quarter as long.  The longer the walks, the
+// more bricks it takes to hide the longest: whole ones win from about
+// 420 · ∛n on (800 sources: 96³ 100 µs whole and 95 in parts, 112³ 125 and 131;
+// 30,000: 144³ 467 and 462, 160³ 560 and 594; 400,000: 160³ 1,011 and 849, 192³
+// 1,270 and 1,220, 256³ 1,776 and 2,204).  The values are the same: each point
+// takes its own terms in the same order
+constexpr double kWholeBricks = 420.0;
 
 // And below kGridAlone points (kGridAloneDense where the sources are a third of
 // them or more, as then a part's walks have little in common), or kSelfAlone of
@@ -1569,7 +1571,7 @@ constexpr int64_t kWholeBricks = 24576;
 constexpr int64_t kGridAlone = 131072, kGridAloneDense = 524288, kSelfAlone = 250000;
 
 // `whole_bricks`: for the walks that take no others
-static QueryArgs make_grid(const dwg_grid* g, bool whole_bricks) {
+static QueryArgs make_grid(const dwg_octree* T, const dwg_grid* g, bool whole_bricks) {
     QueryArgs Q{};
     Q.grid = true;
     Q.ox = g->origin[0];
@@ -1587,7 +1589,7 @@ static QueryArgs make_grid(const dwg_grid* g, bool whole_bricks) {
         Q.n_bricks = int64_t(Q.bx) * Q.by * Q.bz;
     };
     bricks(kGridParts, kPartsX, kPartsY, kPartsZ);
-    if (!whole_bricks && Q.n_bricks < kWholeBricks) bricks(1, 1, 1, 1);
+    if (!whole_bricks && double(Q.n_bricks) < kWholeBricks * std::cbrt(double(T->n_points))) bricks(1, 1, 1, 1);
     Q.nq = int64_t(Q.rx) * Q.ry * Q.rz;
     return Q;
 }
@@ -1732,9 +1734,10 @@ void gwn_tree_self(dwg_ctx* ctx, const dwg_octree* T, float beta, float sigma, u
 
 void gwn_tree_grid(dwg_ctx* ctx, const dwg_octree* T, const dwg_grid* g, float beta, float sigma, uint32_t flags,
                    float* out) {
+    DWG_REQUIRE(T, "null octree");
     DWG_REQUIRE(g && g->res[0] > 0 && g->res[1] > 0 && g->res[2] > 0 && g->h > 0, "bad grid");
-    launch_tree(ctx, T, make_grid(g, (flags & DWG_SCREENED) && (flags & DWG_NEAR_FP64)), beta, sigma, flags, out, nullptr,
-                false);
+    launch_tree(ctx, T, make_grid(T, g, (flags & DWG_SCREENED) && (flags & DWG_NEAR_FP64)), beta, sigma, flags, out,
+                nullptr, false);
 }
 
 void gwn_tree_grad(dwg_ctx* ctx, const dwg_octree* Tc, const float* q, int64_t nq, float beta, float sigma,
@@ -1794,7 +1797,7 @@ __global__ void sum_i64_kernel(const int64_t* __restrict__ v, int64_t n, unsigne
 }
 
 int64_t gwn_tree_grid_terms(dwg_ctx* ctx, const dwg_octree* T, const dwg_grid* g, float beta) {
-    QueryArgs Q = make_grid(g, true);
+    QueryArgs Q = make_grid(T, g, true);
     int64_t* terms = static_cast<int64_t*>(ctx->buf("grid_terms", sizeof(int64_t) * (Q.nq + 1)));
     unsigned long long* tot = reinterpret_cast<unsigned long long*>(terms + Q.nq);
     fill_u32(ctx, tot, 0, 2);
