@@ -532,21 +532,27 @@ __global__ void node_ec_kernel(const int4* __restrict__ info, const Double3* __r
     }
 }
 
-__global__ void set_radius_kernel(float4* __restrict__ sa, const float* __restrict__ radii, const int* __restrict__ perm,
-                                  int64_t n) {
+// the sources in tree order for new normals, areas and radii; their positions
+// are there
+__global__ void repack_sources_kernel(const float* __restrict__ nrm, const float* __restrict__ area,
+                                      const float* __restrict__ radii, const int* __restrict__ perm, int64_t n,
+                                      float4* __restrict__ sa, float4* __restrict__ sb, Double3* __restrict__ an64) {
     int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    sa[i].w = radii ? radii[perm[i]] : kScreenDefault;
+    const int64_t p = perm[i];
+    const float A = area ? area[p] : 2e-6f;
+    sa[i].w = radii ? radii[p] : kScreenDefault;
+    const float nx = nrm[3 * p], ny = nrm[3 * p + 1], nz = nrm[3 * p + 2];
+    sb[i] = make_float4(A * nx * kInv4Pi, A * ny * kInv4Pi, A * nz * kInv4Pi, 0.f);
+    an64[i] = Double3(double(A) * nx, double(A) * ny, double(A) * nz);
 }
 
 void octree_update(dwg_ctx* ctx, dwg_octree* T, const float* nrm, const float* area, const float* radii) {
     const int64_t n = T->n_points, m = T->n_nodes;
     {
         ProfileScope ps(ctx, "octree_pack");
-        hipLaunchKernelGGL(set_radius_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, T->sa, radii, T->perm, n);
-        check_launch();
-        hipLaunchKernelGGL(pack_sources_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, nullptr, nrm, area,
-                           nullptr, T->perm, n, 0, nullptr, T->sb, T->an64);
+        hipLaunchKernelGGL(repack_sources_kernel, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, nrm, area, radii,
+                           T->perm, n, T->sa, T->sb, T->an64);
         check_launch();
     }
     {

@@ -1255,14 +1255,28 @@ __device__ __forceinline__ void desc_take(uint64_t& list, uint64_t& kth, uint64_
     kth = read_lane64(list, k - 1);
 }
 
-// qlist (nullable) holds the queries, `count` (nullable) their number on the
-// device (else nq); init_kth[t] bounds the k-th d² of list entry t
+// far queries below which none share a walk (see shared_walk_budget)
+constexpr int64_t kShareMin = 65536;
+
+// The queries of a search: `list` (nullable) holds them, `count` (nullable)
+// their number on the device (else nq), kth[t] (nullable) bounds the k-th d² of
+// entry t.  From kShareMin queries on, what the shared walks left of them takes
+// their place, if there is a `rest`.
+struct DescQueries {
+    int64_t nq;
+    const int64_t* count;
+    const int* list;
+    const float* kth;
+    const int64_t* rest;
+    const int* rest_list;
+    const float* rest_kth;
+};
+
 template <bool BOXES>
 __global__ __launch_bounds__(kDescWaves * 64) void knn_descent_kernel(
     KnnGridArgs G, PyrArgs Y, const int64_t* __restrict__ cell_start, const float4* __restrict__ pts,
-    const float* __restrict__ q, int64_t nq, const int64_t* __restrict__ count, const int* __restrict__ qlist, int k,
-    const uint8_t* __restrict__ skip, const uint8_t* __restrict__ qmask, const float* __restrict__ init_kth,
-    int32_t* __restrict__ out_idx, float* __restrict__ out_d2) {
+    const float* __restrict__ q, DescQueries S, int k, const uint8_t* __restrict__ skip,
+    const uint8_t* __restrict__ qmask, int32_t* __restrict__ out_idx, float* __restrict__ out_d2) {
     __shared__ uint64_t s_ent[kDescWaves][kDescStack];  // x | y << 16 | z << 32 | occupancy << 48 | level << 56
     __shared__ float s_ed2[kDescWaves][kDescStack];     // box distance
     __shared__ int s_pt[kDescWaves][64 * kDescPoints];
@@ -1280,7 +1294,11 @@ __global__ __launch_bounds__(kDescWaves * 64) void knn_descent_kernel(
     float* ed2 = s_ed2[wave];
     int* pt = s_pt[wave];
     uint64_t* sel = s_sel[wave];
-    const int64_t n = count ? int64_t(uniform64(uint64_t(*count))) : nq;
+    int64_t n = S.count ? int64_t(uniform64(uint64_t(*S.count))) : S.nq;
+    const bool rest = S.rest && n >= kShareMin;
+    if (rest) n = int64_t(uniform64(uint64_t(*S.rest)));
+    const int* qlist = rest ? S.rest_list : S.list;
+    const float* init_kth = rest ? S.rest_kth : S.kth;
     const int top = Y.levels - 1;
     const uint64_t root = (uint64_t(uint32_t(uniform(int(Y.mask[s_off[top]])))) << 48) | (uint64_t(uint32_t(top)) << 56);
     for (int64_t t = int64_t(blockIdx.x) * kDescWaves + wave; t < n; t += int64_t(gridDim.x) * kDescWaves) {
@@ -1418,9 +1436,8 @@ constexpr int kPwStack = 128;  // ≥ 7 · kMaxPyr + 1 entries
 // alone), at 180,000 of 3M
 // centroids 12.5 → 2.1 ms with about 350 pops, at 900,000 10 → 4.6 ms with
 // 1,024 (6.5 ms with 400)
-constexpr int64_t kShareMin = 65536;
 __device__ __forceinline__ int shared_walk_budget(int64_t nq) {
-    return nq < kShareMin ? 0 : int(min(max(nq / 512, int64_t(64)), int64_t(1024)));
+    return int(min(max(nq / 512, int64_t(64)), int64_t(1024)));
 }
 
 template <int K>
@@ -1438,7 +1455,7 @@ __global__ __launch_bounds__(kPwWaves * 64) void knn_pyramid_wave_kernel(KnnGrid
                                                                         float* __restrict__ open_kth,
                                                                         unsigned long long* __restrict__ n_open) {
     const int64_t nq = *count;  // launched for every query
-    if (int64_t(blockIdx.x) * kPwWaves * 64 >= nq) return;
+    if (nq < kShareMin || int64_t(blockIdx.x) * kPwWaves * 64 >= nq) return;
     const int budget = shared_walk_budget(nq);
     // stack entry: (x | y << 16, z | level << 16 | occupancy << 20, lanes lo, lanes hi)
     __shared__ int4 s_stk[kPwWaves][kPwStack];
@@ -1636,31 +1653,32 @@ static void launch_wave(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, in
     check_launch();
 }
 
-static void launch_descent(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const int64_t* count,
-                           const int* qlist, int k, const uint8_t* skip, const uint8_t* qmask, const float* init_kth,
+static void launch_descent(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, const DescQueries& S, int k,
+                           const uint8_t* skip, const uint8_t* qmask,
                            int32_t* out_idx, float* out_d2, const uint8_t* pyr_mask = nullptr) {
     const auto& L = I->lvl[0];
     if (L.pyr_levels < 2) {
-        launch_wave(ctx, I, q, nq, count, qlist, k, skip, qmask, out_idx, out_d2);
+        launch_wave(ctx, I, q, S.nq, S.count, S.list, k, skip, qmask, out_idx, out_d2);
         return;
     }
     const PyrArgs Y = pyr_args(L, pyr_mask);
     // enough blocks to fill the chip; the waves take further queries in turn
-    dim3 grid(unsigned(std::min<int64_t>(grid_for(nq, kDescWaves), 4096))), block(kDescWaves * 64);
+    dim3 grid(unsigned(std::min<int64_t>(grid_for(S.nq, kDescWaves), 4096))), block(kDescWaves * 64);
     if (L.pbox)
-        hipLaunchKernelGGL(knn_descent_kernel<true>, grid, block, 0, ctx->stream, L.G, Y, L.cell_start, L.pts, q, nq,
-                           count, qlist, k, skip, qmask, init_kth, out_idx, out_d2);
+        hipLaunchKernelGGL(knn_descent_kernel<true>, grid, block, 0, ctx->stream, L.G, Y, L.cell_start, L.pts, q, S, k,
+                           skip, qmask, out_idx, out_d2);
     else
-        hipLaunchKernelGGL(knn_descent_kernel<false>, grid, block, 0, ctx->stream, L.G, Y, L.cell_start, L.pts, q, nq,
-                           count, qlist, k, skip, qmask, init_kth, out_idx, out_d2);
+        hipLaunchKernelGGL(knn_descent_kernel<false>, grid, block, 0, ctx->stream, L.G, Y, L.cell_start, L.pts, q, S, k,
+                           skip, qmask, out_idx, out_d2);
     check_launch();
 }
 
 // the queries qlist[0..*count) that the tiled pass left open (of nq) with
-// their bounds; `shared`: 64 neighbours share a walk first
+// their bounds; `shared`: 64 neighbours share a walk first, counting in *n_open
+// (0) what they leave
 static void launch_far(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const int64_t* count,
                        const int* qlist, int k, const uint8_t* skip, int32_t* out_idx, float* out_d2,
-                       const float* init_kth, bool shared, const uint8_t* pyr_mask) {
+                       const float* init_kth, bool shared, unsigned long long* n_open, const uint8_t* pyr_mask) {
     const auto& L = I->lvl[0];
     // an index without boxes (its first such query) builds them, a dozen
     // launches and 70 µs for 30,000 points, only if there are enough far
@@ -1668,8 +1686,9 @@ static void launch_far(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int
     // points 445 µs by cell boxes, 345 by the points' boxes
     constexpr int64_t kBoxMin = 32768;
     if (shared && L.pyr_levels >= 2 && !L.pbox && read_scalar<int64_t>(ctx, count) < kBoxMin) shared = false;
+    DescQueries S{nq, count, qlist, init_kth, nullptr, nullptr, nullptr};
     if (!shared || L.pyr_levels < 2) {
-        launch_descent(ctx, I, q, nq, count, qlist, k, skip, nullptr, init_kth, out_idx, out_d2, pyr_mask);
+        launch_descent(ctx, I, q, S, k, skip, nullptr, out_idx, out_d2, pyr_mask);
         return;
     }
     // the boxes are a cache of the index's own points: building them
@@ -1679,8 +1698,6 @@ static void launch_far(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int
     DWG_REQUIRE(L.pyr_levels <= kMaxPyr && 7 * L.pyr_levels + 1 <= kPwStack, "pyramid deeper than the wave stack");
     int* open_q = static_cast<int*>(ctx->buf("knn_open_q", sizeof(int) * nq));
     float* open_kth = static_cast<float*>(ctx->buf("knn_open_kth", sizeof(float) * nq));
-    auto* n_open = static_cast<unsigned long long*>(ctx->buf("knn_n_open", 64));
-    fill_u32(ctx, n_open, 0, 2);
     dim3 grid(grid_for(nq, kPwWaves * 64)), block(kPwWaves * 64);
 #define DWG_KNNPW(KK)                                                                                           \
     hipLaunchKernelGGL(knn_pyramid_wave_kernel<KK>, grid, block, 0, ctx->stream, L.G, Y, L.cell_start, L.pts, q, \
@@ -1693,14 +1710,16 @@ static void launch_far(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int
     else DWG_KNNPW(32);
 #undef DWG_KNNPW
     check_launch();
-    launch_descent(ctx, I, q, nq, reinterpret_cast<const int64_t*>(n_open), open_q, k, skip, nullptr, open_kth, out_idx,
-                   out_d2, pyr_mask);
+    S.rest = reinterpret_cast<const int64_t*>(n_open);
+    S.rest_list = open_q;
+    S.rest_kth = open_kth;
+    launch_descent(ctx, I, q, S, k, skip, nullptr, out_idx, out_d2, pyr_mask);
 }
 
 // The queries 0..nq−1 (masked by qmask) bucketed by tile of kTile³ fine cells
 // and eighth of it: order[start[sub·t]..start[sub·(t+1))) are tile t's
 // queries, list[0..*nlist) the tiles that have any, once for each `chunk` of
-// them (tile, chunk); *nopen is 0
+// them (tile, chunk); *nopen and the number after it are 0
 constexpr int64_t kTileBlocks = 4096;
 struct TileBuckets {
     TileArgs T;
@@ -1724,8 +1743,8 @@ static TileBuckets tile_buckets(dwg_ctx* ctx, const dwg_knn_index* I, const floa
     DWG_REQUIRE(nb < (int64_t(1) << 31), "too many query buckets");
     B.ntiles = ntiles;
     int2* place = static_cast<int2*>(ctx->buf("knnt_place", sizeof(int2) * nq));
-    // the buckets' starts, then the two counts
-    int64_t* start = static_cast<int64_t*>(ctx->buf("knnt_start", sizeof(int64_t) * (nb + 3)));
+    // the buckets' starts, then the counts
+    int64_t* start = static_cast<int64_t*>(ctx->buf("knnt_start", sizeof(int64_t) * (nb + 4)));
     B.nlist = start + nb + 1;
     B.nopen = start + nb + 2;
     int* order = static_cast<int*>(ctx->buf("knnt_order", sizeof(int) * nq));
@@ -1735,7 +1754,7 @@ static TileBuckets tile_buckets(dwg_ctx* ctx, const dwg_knn_index* I, const floa
     B.chunk = kTileThreads * int(std::max<int64_t>(1, nq / (kTileBlocks * kTileThreads)));
     B.max_list = std::min(ntiles, nq) + nq / B.chunk;
     int2* list = static_cast<int2*>(ctx->buf("knnt_list", sizeof(int2) * size_t(B.max_list)));
-    fill_u32(ctx, start, 0, 2 * (nb + 3));
+    fill_u32(ctx, start, 0, 2 * (nb + 4));
     hipLaunchKernelGGL(tile_count_kernel, dim3(grid_for(nq, 256)), dim3(256), 0, ctx->stream, q, nq, qmask, G, T,
                        place, reinterpret_cast<unsigned long long*>(start));
     check_launch();
@@ -1764,15 +1783,17 @@ constexpr int64_t kOpenOrder = 262144;
 
 // The tiled pass over the queries 0..nq−1 (masked by qmask); the queries it
 // cannot close are listed in redo with their k-th bound in redo_kth, tile by
-// tile.  Returns the device address of their count.
+// tile.  Returns the device address of their count; *left is that of a 0.
 static const int64_t* tiled_pass(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq, const uint8_t* qmask,
                                  int k, const uint8_t* skip, int32_t* out_idx, float* out_d2, int* redo,
-                                 float* redo_kth, const std::string& name, const KnnScatter* sc) {
+                                 float* redo_kth, const std::string& name, const KnnScatter* sc,
+                                 unsigned long long** left) {
     const KnnGridArgs& G = I->lvl[0].G;
     const TileBuckets B = tile_buckets(ctx, I, q, nq, qmask);
     const TileArgs& T = B.T;
     if (ctx->profile) ctx->count(name + ":queries", read_scalar<int64_t>(ctx, B.start + B.ntiles * kSubTiled));
     auto* nopen = reinterpret_cast<unsigned long long*>(B.nopen);
+    *left = nopen + 1;
     int* open_q = redo;
     float* open_kth = redo_kth;
     int64_t* tile_open = nullptr;
@@ -1833,7 +1854,7 @@ void knn_query(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq,
     const bool sparse = nq * 8 < I->n;
     if (nq < kDescAlways || (nq < kDescFew && nq < I->n) || (nq < kDescSparse && sparse)) {
         ctx->count(base + (sparse ? ":sparse" : ":tiles3:redo"), nq);
-        launch_descent(ctx, I, q, nq, nullptr, nullptr, k, skip, qmask, nullptr, out_idx, out_d2);
+        launch_descent(ctx, I, q, DescQueries{nq}, k, skip, qmask, out_idx, out_d2);
         if (sc) {
             hipLaunchKernelGGL(scatter_pairs_kernel, dim3(grid_for(nq * k, 256)), dim3(256), 0, ctx->stream, out_idx, k,
                                nq, *sc);
@@ -1848,7 +1869,8 @@ void knn_query(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq,
     // order, so a wave's 64 share most of their search and take the
     // wave-shared walk; sparser far queries are spread apart and search alone
     const bool shared = nq >= I->n;
-    const int64_t* nfar = tiled_pass(ctx, I, q, nq, qmask, k, skip, out_idx, out_d2, redo, kth, base + ":tiles", sc);
+    unsigned long long* left = nullptr;
+    const int64_t* nfar = tiled_pass(ctx, I, q, nq, qmask, k, skip, out_idx, out_d2, redo, kth, base + ":tiles", sc, &left);
     if (ctx->profile) {  // the queries that no tiled pass closes
         const int64_t n = read_scalar<int64_t>(ctx, nfar);
         ctx->count(base + ":tiles:redo", n);
@@ -1858,7 +1880,7 @@ void knn_query(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int64_t nq,
         const std::string name = base + ":redo";
         ProfileScope pr(ctx, name.c_str());
         const uint8_t* pm = (skip && I->lvl[0].pyr_levels >= 2) ? masked_pyramid(ctx, I->lvl[0], skip) : nullptr;
-        launch_far(ctx, I, q, nq, nfar, redo, k, skip, out_idx, out_d2, kth, shared, pm);
+        launch_far(ctx, I, q, nq, nfar, redo, k, skip, out_idx, out_d2, kth, shared, left, pm);
     }
     if (sc) {
         const std::string name = base + ":scatter";
