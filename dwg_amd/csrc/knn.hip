@@ -1431,13 +1431,13 @@ constexpr int kPwStack = 128;  // ≥ 7 · kMaxPyr + 1 entries
 // its longest walks, on an otherwise idle chip: a wave stops after this many
 // pops and hands its open queries, with the bounds they have, to a search of
 // their own (knn_descent_kernel).  Sharing pays while the waves fill the
-// chip, so the more queries, the more pops: below 65,536 queries none at all
-// (53,000 far centroids of a 30,000-point cloud: 0.41 ms with 100 pops, 0.35
-// alone), at 180,000 of 3M
-// centroids 12.5 → 2.1 ms with about 350 pops, at 900,000 10 → 4.6 ms with
-// 1,024 (6.5 ms with 400)
-__device__ __forceinline__ int shared_walk_budget(int64_t nq) {
-    return int(min(max(nq / 512, int64_t(64)), int64_t(1024)));
+// chip, so the more queries, the more pops, and walks are longer in a larger
+// cloud: 120,000 far of 30,000 points 880 µs with 470 pops, 644 with 117;
+// 270,000 of 300,000 3.3 ms with 1,024, 2.35 with 527, 2.12 with 264; 180,000 of
+// 1M 5.3 ms with 1,024, 3.78 with 350, 4.18 with 88.  Below kShareMin queries
+// none share (53,000 of 30,000 points: 0.41 ms with 100 pops, 0.35 alone).
+__device__ __forceinline__ int shared_walk_budget(int64_t nq, int64_t points) {
+    return int(min(max(nq / 1024 + points / 6144, int64_t(64)), int64_t(1024)));
 }
 
 template <int K>
@@ -1450,13 +1450,13 @@ __global__ __launch_bounds__(kPwWaves * 64) void knn_pyramid_wave_kernel(KnnGrid
                                                                         const uint8_t* __restrict__ skip,
                                                                         const float* __restrict__ init_kth,
                                                                         int32_t* __restrict__ out_idx,
-                                                                        float* __restrict__ out_d2,
+                                                                        float* __restrict__ out_d2, int64_t points,
                                                                         int* __restrict__ open_q,
                                                                         float* __restrict__ open_kth,
                                                                         unsigned long long* __restrict__ n_open) {
     const int64_t nq = *count;  // launched for every query
     if (nq < kShareMin || int64_t(blockIdx.x) * kPwWaves * 64 >= nq) return;
-    const int budget = shared_walk_budget(nq);
+    const int budget = shared_walk_budget(nq, points);
     // stack entry: (x | y << 16, z | level << 16 | occupancy << 20, lanes lo, lanes hi)
     __shared__ int4 s_stk[kPwWaves][kPwStack];
     __shared__ float4 s_box[kPwWaves][16];    // box of child c: lo at 2c, hi at 2c + 1
@@ -1701,7 +1701,7 @@ static void launch_far(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int
     dim3 grid(grid_for(nq, kPwWaves * 64)), block(kPwWaves * 64);
 #define DWG_KNNPW(KK)                                                                                           \
     hipLaunchKernelGGL(knn_pyramid_wave_kernel<KK>, grid, block, 0, ctx->stream, L.G, Y, L.cell_start, L.pts, q, \
-                       count, qlist, k, skip, init_kth, out_idx, out_d2, open_q, open_kth, n_open)
+                       count, qlist, k, skip, init_kth, out_idx, out_d2, I->n, open_q, open_kth, n_open)
     if (k <= 8) DWG_KNNPW(8);
     else if (k <= 10) DWG_KNNPW(10);
     else if (k == 15) DWG_KNNPW(15);  // the diffusion's 15 neighbours: no spare slot to sink through
