@@ -360,6 +360,18 @@ int dwg_marching_cubes(dwg_ctx* ctx, const float* d_field, const dwg_grid* grid,
     }
 }
 
+int dwg_marching_cubes_alloc(dwg_ctx* ctx, const float* d_field, const dwg_grid* grid, float iso, dwg_mc_alloc alloc,
+                             void* user, int64_t* h_count) {
+    if (!ctx) return DWG_ERR_ARG;
+    return guarded(ctx, [&] {
+        DWG_REQUIRE(d_field && grid, "null field/grid");
+        DWG_REQUIRE(alloc, "null allocator");
+        set_device(ctx);
+        const int64_t t = dwg::marching_cubes_alloc(ctx, d_field, grid, iso, alloc, user);
+        if (h_count) *h_count = t;
+    });
+}
+
 int dwg_marching_cubes_any_order(dwg_ctx* ctx, const float* d_field, const dwg_grid* grid, float iso,
                                  int64_t capacity, float* d_cent, float* d_nrm, int64_t* h_count) {
     if (!ctx) return DWG_ERR_ARG;

@@ -467,8 +467,10 @@ int64_t marching_cubes_any_order(dwg_ctx* ctx, const float* field, const dwg_gri
     return total;
 }
 
-int64_t marching_cubes(dwg_ctx* ctx, const float* field, const dwg_grid* g, float iso, int64_t capacity, float* tris,
-                       float* cent, float* nrm) {
+// 480×512×451 into exact-size buffers 300 µs with a call to count and one to
+// count and emit, 176 so
+int64_t marching_cubes_alloc(dwg_ctx* ctx, const float* field, const dwg_grid* g, float iso, dwg_mc_alloc alloc,
+                             void* user) {
     McBricks B;
     int64_t tiles;
     const McArgs A = mc_args(field, g, iso, B, tiles);
@@ -496,13 +498,36 @@ int64_t marching_cubes(dwg_ctx* ctx, const float* field, const dwg_grid* g, floa
     };
     const Totals tot = read_scalar<Totals>(ctx, reinterpret_cast<const Totals*>(offs + tiles));
     const int64_t total = tot.tris;
-    if (total > capacity) throw Error(DWG_ERR_CAPACITY, "marching cubes output exceeds capacity", total);
+    float *tris = nullptr, *cent = nullptr, *nrm = nullptr;
+    DWG_REQUIRE(alloc(user, total, &tris, &cent, &nrm) == 0, "marching cubes buffers refused");
     if (total > 0 && (tris || cent || nrm)) {
         ProfileScope ps(ctx, "mc_emit");
         hipLaunchKernelGGL(mc_emit_kernel, dim3(unsigned(tot.bricks)), dim3(kMcThreads), 0, ctx->stream, A, B, offs,
                            list, tris, cent, nrm);
         check_launch();
     }
+    return total;
+}
+
+int64_t marching_cubes(dwg_ctx* ctx, const float* field, const dwg_grid* g, float iso, int64_t capacity, float* tris,
+                       float* cent, float* nrm) {
+    struct Buffers {
+        int64_t capacity;
+        float *tris, *cent, *nrm;
+    } b{capacity, tris, cent, nrm};
+    const int64_t total = marching_cubes_alloc(
+        ctx, field, g, iso,
+        [](void* user, int64_t count, float** t, float** c, float** n) {
+            auto* u = static_cast<Buffers*>(user);
+            if (count <= u->capacity) {
+                *t = u->tris;
+                *c = u->cent;
+                *n = u->nrm;
+            }
+            return 0;
+        },
+        &b);
+    if (total > capacity) throw Error(DWG_ERR_CAPACITY, "marching cubes output exceeds capacity", total);
     return total;
 }
 

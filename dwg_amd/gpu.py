@@ -280,18 +280,25 @@ class KnnIndex:
 def marching_cubes(ctx: Context, field, grid: DwgGrid, iso, tris=False):
     """→ (tris or None, centroids, normals) as device tensors, cube order."""
     field = ctx.f32(field)
-    cnt = ctypes.c_int64()
-    rc = ctx.L.dwg_marching_cubes(ctx.h, _ptr(field), ctypes.byref(grid), float(iso), 0, None, None, None,
-                                  ctypes.byref(cnt))
-    if rc not in (0, _lib.DWG_ERR_CAPACITY):
-        ctx.check(rc)
-    T = cnt.value
-    t = torch.empty((T, 3, 3), device=ctx.device, dtype=torch.float32) if tris else None
-    c = torch.empty((T, 3), device=ctx.device, dtype=torch.float32)
-    n = torch.empty((T, 3), device=ctx.device, dtype=torch.float32)
-    ctx.check(ctx.L.dwg_marching_cubes(ctx.h, _ptr(field), ctypes.byref(grid), float(iso), T, _ptr(t), _ptr(c),
-                                       _ptr(n), ctypes.byref(cnt)))
-    return t, c, n
+    out, failed = [], []
+
+    def alloc(_, T, *where):
+        # called between the count and the emit; nothing may be raised through it
+        try:
+            for shape, w in zip(((T, 3, 3) if tris else None, (T, 3), (T, 3)), where):
+                out.append(None if shape is None else torch.empty(shape, device=ctx.device, dtype=torch.float32))
+                w[0] = None if shape is None else out[-1].data_ptr()
+            return 0
+        except BaseException as e:
+            failed.append(e)
+            return 1
+
+    rc = ctx.L.dwg_marching_cubes_alloc(ctx.h, _ptr(field), ctypes.byref(grid), float(iso), _lib.MC_ALLOC(alloc), None,
+                                        None)
+    if failed:
+        raise failed[0]
+    ctx.check(rc)
+    return tuple(out)
 
 
 def marching_cubes_any_order(ctx: Context, field, grid: DwgGrid, iso, capacity=1 << 16):

@@ -192,6 +192,13 @@ int dwg_knn_query(dwg_ctx* ctx, const dwg_knn_index* index, const float* d_q, in
 int dwg_marching_cubes(dwg_ctx* ctx, const float* d_field, const dwg_grid* grid, float iso,
                        int64_t capacity, float* d_tris, float* d_cent, float* d_nrm,
                        int64_t* h_count);
+/* The same for buffers of the exact size, without counting twice: alloc is
+ * called once, with the number of triangles, and sets the device buffers that
+ * are wanted (the others are NULL); it returns 0, or another number to give up
+ * (DWG_ERR_ARG).  It must not use the context. */
+typedef int (*dwg_mc_alloc)(void* user, int64_t count, float** d_tris, float** d_cent, float** d_nrm);
+int dwg_marching_cubes_alloc(dwg_ctx* ctx, const float* d_field, const dwg_grid* grid, float iso,
+                             dwg_mc_alloc alloc, void* user, int64_t* h_count);
 /* No counterpart in the reference: the same triangles' centroids and
  * normals (values as dwg_marching_cubes gives them) in one pass and in no
  * fixed order, for callers whose use does not depend on the order (the

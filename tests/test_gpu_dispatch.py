@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import oracle as O
-from dwg_amd import gpu, shapes
+from dwg_amd import _lib, gpu, shapes
 from mc_order import to_brick_order
 from oracle import mlp as M
 
@@ -313,3 +313,34 @@ def test_marching_cubes_by_runs(ctx, res, crossed):
     c1, n1 = gpu.marching_cubes_any_order(ctx, ft, grid, 0.0, capacity=len(rt))
     rows = [np.concatenate([c.cpu().numpy(), m.cpu().numpy()], 1).view(np.uint32) for c, m in ((cent, nrm), (c1, n1))]
     assert np.array_equal(*(r[np.lexsort(r.T[::-1])] for r in rows))
+
+
+@pytest.mark.parametrize("wanted", [(1, 1, 1), (1, 0, 0), (0, 0, 1), (0, 0, 0), None])
+def test_marching_cubes_into_given_buffers(ctx, wanted):
+    """The buffers that the allocator gives hold what the two calls with a
+    capacity write; an allocator that gives up leaves an error, not a result."""
+    rng = np.random.default_rng(8)
+    res = (40, 21, 33)
+    f = torch.from_numpy(rng.normal(size=res[0] * res[1] * res[2]).astype(np.float32)).cuda()
+    grid = gpu.make_grid([0.0, 0.0, 0.0], 0.1, np.int32(res))
+    want = gpu.marching_cubes(ctx, f, grid, 0.0, tris=True)
+    T, n = want[0].shape[0], ctypes.c_int64()
+    ref = [torch.empty_like(w) for w in want]
+    args = (ctx.h, ctypes.c_void_p(f.data_ptr()), ctypes.byref(grid), 0.0)
+    ctx.check(ctx.L.dwg_marching_cubes(*args, T, *(ctypes.c_void_p(r.data_ptr()) for r in ref), ctypes.byref(n)))
+    assert n.value == T > 1000 and all(torch.equal(a, b) for a, b in zip(want, ref))
+    got, calls = [torch.zeros_like(w) for w in want], []
+
+    def alloc(_, count, *where):
+        calls.append(count)
+        if wanted is None:
+            return 1
+        for b, use, w in zip(got, wanted, where):
+            w[0] = b.data_ptr() if use else None
+        return 0
+
+    rc = ctx.L.dwg_marching_cubes_alloc(*args, _lib.MC_ALLOC(alloc), None, ctypes.byref(n))
+    assert calls == [T] and rc == (0 if wanted else _lib.DWG_ERR_ARG)
+    torch.cuda.synchronize()
+    for b, use, w in zip(got, wanted or (0, 0, 0), want):
+        assert torch.equal(b, w) if use else not b.any()
