@@ -7,7 +7,8 @@
 //            a wave walks the union of its 64 lanes' traversals with one
 //            wave-uniform stack in LDS (node, lane mask), so every node and
 //            source load is wave-uniform and each lane still takes exactly
-//            the reference's per-query term set.
+//            the reference's per-query term set.  Few points, and points with
+//            little in common, walk alone, with 8 or 64 lanes each.
 //
 // Terms (reference semantics, d = p − q, r = |d|):
 //   plain     A(d·n) / (4π r³ + 1e-8)                         fast_winding_number.cpp:182-184

@@ -20,9 +20,9 @@ struct KnnGridArgs {
 constexpr int kMaxPyr = 16;
 }  // namespace dwg
 
-// Two cell grids over the same points: a fine one sized from the measured
-// occupancy and a coarse one (8× larger cells) for queries whose fine search
-// does not close within a few shells.
+// A cell grid over the points, sized from the measured occupancy, with an
+// occupancy pyramid; where there is none (one cell, or a grid too elongated) a
+// coarse grid of 8× larger cells as well, whose shells the queries search.
 struct dwg_knn_index {
     int64_t n = 0;
     struct Level {

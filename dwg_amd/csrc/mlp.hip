@@ -10,9 +10,9 @@
 // takes its patch points from a hashed subsample of that size, so patches
 // span the same fraction of the shape as in training.
 //
-// Every product is one launch of gemm_bf16: C = A·B with arbitrary element
-// strides for A (M×K), B (K×N) and C (M×N), BF16 operands, FP32
-// accumulation, one 32×32 output tile per wave on v_mfma_f32_32x32x16_bf16.
+// Every product runs on v_mfma_f32_32x32x16_bf16, BF16 operands and FP32
+// accumulation in 32×32 tiles: the whole network in one launch for inference,
+// in three for a training step.
 // GELU is the tanh form of Hendrycks & Gimpel (2016).  The loss is the mean
 // over the batch of 1 − ŷ·t (oriented) or 1 − (ŷ·t)² (normal line, sign
 // free), ŷ = y/|y|, t the unit target normal.  The initialisation orients

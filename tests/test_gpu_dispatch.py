@@ -100,10 +100,12 @@ def test_grid_walk_equals_the_point_walk(ctx, res, h, shift, screened, bf16, rad
 
 # (points, queries): fewer points than k, one query, one cell's worth, a
 # query set at each end of the sizes searched one query at a time and of the
-# tiled ones (dense and not)
+# tiled ones (dense and not), and of those whose open queries are put in order
+# (half of them, enough to share walks first)
 @pytest.mark.parametrize("n,nq,k", [(1, 3, 4), (5, 1, 10), (40, 64, 32), (3000, 1, 1), (3000, 257, 32),
                                     (20_000, 16_383, 15), (2500, 16_384, 15), (33_000, 32_767, 8),
-                                    (33_000, 32_768, 10), (2000, 40_000, 17)])
+                                    (33_000, 32_768, 10), (2000, 40_000, 17), (9000, 262_143, 15),
+                                    (9000, 262_144, 15)])
 @pytest.mark.parametrize("skipped", [0.0, 0.5, 0.999])
 def test_knn_by_query_count(ctx, n, nq, k, skipped):
     rng = np.random.default_rng(n + nq)
