@@ -120,7 +120,7 @@ __device__ __forceinline__ bool near_field(float r2, float s) { return r2 < s * 
 //             (∂ρ/∂q = −d/r), −g b for r < s;
 //             g' = (σε' − e^{σρ}ρ²(σ²ρ² + 3σρ + 3)) / D²  (no cancellation)
 // as the factors dot = d·b, g and c of w = g·dot, ∇w = c·d − g·b, with s2 the
-// squared screening radius (200,000 sources at 2,000 queries 540 → 484 µs:
+// squared screening radius (200,000 sources at 2,000 queries 540 → 460 µs:
 // selects on two factors instead of four results, and multiply-adds into the
 // sums.  ρ = ρ²·ρ^-1 would save another 5 %, for an error of w 8 to 13 % above
 // the root's).
@@ -236,7 +236,9 @@ __device__ __forceinline__ void direct_grad(const float4* __restrict__ sa, const
 #pragma unroll
     for (int k = 0; k < 4; ++k) p[k] = 0.f;
     for (; j0 + kDirectTile <= j1; j0 += kDirectTile) {
-#pragma unroll 4
+        // (857 sources at 1M queries, plain: 0.56 ms unrolled by 4, 0.53 by 2; 3,000
+        // at 300,000: 0.64 and 0.66; 200,000 at 2,000, screened: 0.52 and 0.51)
+#pragma unroll 2
         for (int j = 0; j < kDirectTile; ++j) term(sa[j0 + j], sb[j0 + j]);
         fold();
     }
