@@ -1353,42 +1353,32 @@ __device__ __forceinline__ int order_bucket(const float* __restrict__ q, int64_t
     return m;
 }
 
+// (bucket, place in it) of every query: the scatter then needs no atomics
 __global__ void order_count_kernel(const float* __restrict__ q, int64_t nq, const double4* __restrict__ cell,
-                                   QueryOrder O, int* __restrict__ bucket_of,
-                                   unsigned long long* __restrict__ count) {
+                                   QueryOrder O, int2* __restrict__ place, unsigned long long* __restrict__ count) {
     if (!O.sorted()) return;
     const double4 root = cell[0];
-    const int lane = threadIdx.x & 63;
     for (int64_t i0 = int64_t(blockIdx.x) * blockDim.x; i0 < nq; i0 += int64_t(gridDim.x) * blockDim.x) {
         const int64_t i = i0 + threadIdx.x;
         const int b = i < nq ? order_bucket(q, i, root) : -1;
-        if (i < nq) bucket_of[i] = b;
-        const uint64_t starts = run_starts(b);
-        if (b >= 0 && ((starts >> lane) & 1ull)) atomicAdd(&count[b], (unsigned long long)run_length(starts, lane));
+        const int at = take_place(b, count);
+        if (i < nq) place[i] = make_int2(b, at);
     }
 }
 
-__global__ void order_scatter_kernel(const int* __restrict__ bucket_of, int64_t nq, QueryOrder O,
-                                     unsigned long long* __restrict__ cursor, int* __restrict__ order) {
+__global__ void order_scatter_kernel(const int2* __restrict__ place, int64_t nq, QueryOrder O,
+                                     const unsigned long long* __restrict__ start, int* __restrict__ order) {
     if (!O.sorted()) return;
-    const int lane = threadIdx.x & 63;
-    for (int64_t i0 = int64_t(blockIdx.x) * blockDim.x; i0 < nq; i0 += int64_t(gridDim.x) * blockDim.x) {
-        const int64_t i = i0 + threadIdx.x;
-        const int b = i < nq ? bucket_of[i] : -1;
-        const uint64_t starts = run_starts(b);
-        int at = 0;
-        if (b >= 0 && ((starts >> lane) & 1ull))
-            at = int(atomicAdd(&cursor[b], (unsigned long long)run_length(starts, lane)));
-        const int head = run_head(starts, lane);
-        at = __shfl(at, head, 64) + (lane - head);
-        if (b >= 0) order[at] = int(i);
+    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < nq; i += int64_t(gridDim.x) * blockDim.x) {
+        const int2 b = place[i];
+        order[start[b.x] + b.y] = int(i);
     }
 }
 
 static QueryOrder query_order(dwg_ctx* ctx, const dwg_octree* T, const float* q, int64_t nq) {
     DWG_REQUIRE(nq < (int64_t(1) << 31) - 1, "too many queries");
     auto* start = static_cast<unsigned long long*>(ctx->buf("order_start", sizeof(uint64_t) * (kOrderBuckets + 2)));
-    int* bucket_of = static_cast<int*>(ctx->buf("order_bucket_of", sizeof(int) * size_t(nq)));
+    int2* place = static_cast<int2*>(ctx->buf("order_place", sizeof(int2) * size_t(nq)));
     int* order = static_cast<int*>(ctx->buf("order", sizeof(int) * size_t(nq)));
     auto* extent = reinterpret_cast<unsigned int*>(start + kOrderBuckets + 1);
     ProfileScope ps(ctx, "gwn_query_order");
@@ -1398,11 +1388,11 @@ static QueryOrder query_order(dwg_ctx* ctx, const dwg_octree* T, const float* q,
     check_launch();
     const QueryOrder O{order, extent, unsigned(65536.f * 2.f * std::cbrt(64.f / float(nq)) * float(samples))};
     const unsigned blocks = std::min(grid_for(nq, 256), 2048u);
-    hipLaunchKernelGGL(order_count_kernel, dim3(blocks), dim3(256), 0, ctx->stream, q, nq, T->cell, O, bucket_of,
+    hipLaunchKernelGGL(order_count_kernel, dim3(blocks), dim3(256), 0, ctx->stream, q, nq, T->cell, O, place,
                        start);
     check_launch();
     exclusive_scan_i64(ctx, reinterpret_cast<int64_t*>(start), kOrderBuckets);
-    hipLaunchKernelGGL(order_scatter_kernel, dim3(blocks), dim3(256), 0, ctx->stream, bucket_of, nq, O, start,
+    hipLaunchKernelGGL(order_scatter_kernel, dim3(blocks), dim3(256), 0, ctx->stream, place, nq, O, start,
                        order);
     check_launch();
     return O;

@@ -34,20 +34,6 @@ __device__ __forceinline__ int cell_coord(float v, float lo, float inv_cell, int
     return min(max(c, 0), dim - 1);
 }
 
-// Adds this thread's item to its bucket (−1: none) and returns its place there:
-// a run of lanes with one bucket takes its places with one atomic add.  The
-// second pass then needs no atomics (3M triangle centroids: count and scatter
-// 248 → 140 µs).
-__device__ __forceinline__ int take_place(int bucket, unsigned long long* __restrict__ counts) {
-    const int lane = threadIdx.x & 63;
-    const uint64_t starts = run_starts(bucket);
-    int base = 0;
-    if (bucket >= 0 && ((starts >> lane) & 1ull))
-        base = int(atomicAdd(&counts[bucket], (unsigned long long)run_length(starts, lane)));
-    const int head = run_head(starts, lane);
-    return __shfl(base, head, 64) + (lane - head);
-}
-
 __device__ __forceinline__ int cell_of_point(const KnnGridArgs& G, const float* __restrict__ p, int64_t i) {
     const int cx = cell_coord(p[3 * i], G.lo[0], G.inv_cell, G.dim[0]);
     const int cy = cell_coord(p[3 * i + 1], G.lo[1], G.inv_cell, G.dim[1]);
