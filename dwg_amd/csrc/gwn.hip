@@ -1313,7 +1313,10 @@ constexpr int64_t kWalkFew = 40000, kShareValue = 196608, kShareGrad = 786432;
 // The order: a counting sort by the Morton code of a 64³ grid over the tree's
 // cube.  Queries that come in order already are left as they are, which a
 // sample of runs of 64 decides: they come unsorted when such runs extend, on
-// average, over twice the side that 64 of nq uniform points fill
+// average, over twice the side that 64 of nq uniform points fill.  (32³ and 128³
+// cells: 300,000 points over 400,000 sources 417 and 427 µs against 394 with 64³,
+// 1M points 690 and 611 against 602.  Points in order pay 20 to 25 µs for the
+// passes that find it out: 500,000 over 500,000 sources 404 → 427.)
 constexpr int kOrderBits = 6, kOrderBuckets = 1 << (3 * kOrderBits);
 constexpr int kOrderSamples = 256;
 
