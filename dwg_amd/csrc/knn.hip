@@ -1090,12 +1090,15 @@ __device__ __forceinline__ float tight_box_d2(const float4 lo, const float4 hi, 
 }
 
 // squared distance from q to the box of cells [b·2^l, (b+1)·2^l) along each
-// axis, each axis gap shrunk by the rounding margin
+// axis, each axis gap shrunk by the rounding margin of the cells and, as the
+// differences to the box's side and to a point on the wrong side of it by less
+// than that margin may round apart by a unit in their last place (far larger
+// than the margin for a far query), by four units of its own
 __device__ __forceinline__ float pyr_box_d2(const KnnGridArgs& G, float w, float margin, float qx, float qy, float qz,
                                             int x, int y, int z) {
     auto gap = [&](float v, float lo, int b) {
         const float a = __builtin_fmaf(float(b), w, lo);
-        return fmaxf(fmaxf(a - v, v - (a + w)) - margin, 0.f);
+        return fmaxf(__builtin_fmaf(fmaxf(a - v, v - (a + w)), 1.f - 0x1p-22f, -margin), 0.f);
     };
     const float gx = gap(qx, G.lo[0], x), gy = gap(qy, G.lo[1], y), gz = gap(qz, G.lo[2], z);
     return __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
