@@ -120,10 +120,12 @@ __device__ __forceinline__ bool near_field(float r2, float s) { return r2 < s * 
 //             (∂ρ/∂q = −d/r), −g b for r < s;
 //             g' = (σε' − e^{σρ}ρ²(σ²ρ² + 3σρ + 3)) / D²  (no cancellation)
 // as the factors dot = d·b, g and c of w = g·dot, ∇w = c·d − g·b, with s2 the
-// squared screening radius (200,000 sources at 2,000 queries 540 → 460 µs:
-// selects on two factors instead of four results, and multiply-adds into the
-// sums.  ρ = ρ²·ρ^-1 would save another 5 %, for an error of w 8 to 13 % above
-// the root's).
+// squared screening radius (200,000 sources at 2,000 queries 540 → 480 µs with
+// selects on two factors instead of four results.  ρ = ρ²·ρ^-1 would save another
+// 5 %, for an error of w 8 to 13 % above the root's).  A component c·d − g·b is
+// formed before it joins its sum: its two products joined one by one, 460 µs,
+// round twice at the sum's size (half of 2,000 queries next to one of 20,000
+// sources: RMS error of ∇w 11 % and maximum 37 % more).
 template <bool SCREENED>
 __device__ __forceinline__ void gwn_term_grad(float dx, float dy, float dz, float s2, const float4 b, float sigma,
                                               float sigma_l2e, float& dot, float& g, float& c) {
@@ -222,9 +224,9 @@ __device__ __forceinline__ void direct_grad(const float4* __restrict__ sa, const
         float dot, g, c;
         gwn_term_grad<SCREENED>(dx, dy, dz, b.w, b, sigma, sl2e, dot, g, c);
         p[0] = __builtin_fmaf(g, dot, p[0]);
-        p[1] = __builtin_fmaf(c, dx, __builtin_fmaf(-g, b.x, p[1]));
-        p[2] = __builtin_fmaf(c, dy, __builtin_fmaf(-g, b.y, p[2]));
-        p[3] = __builtin_fmaf(c, dz, __builtin_fmaf(-g, b.z, p[3]));
+        p[1] += __builtin_fmaf(c, dx, -g * b.x);
+        p[2] += __builtin_fmaf(c, dy, -g * b.y);
+        p[3] += __builtin_fmaf(c, dz, -g * b.z);
     };
     auto fold = [&]() {
 #pragma unroll
@@ -1466,9 +1468,9 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_grad_kernel(TreeArgs T,
         g = on ? g : 0.f;
         c = on ? c : 0.f;
         part[0] = __builtin_fmaf(g, dot, part[0]);
-        part[1] = __builtin_fmaf(c, dx, __builtin_fmaf(-g, b.x, part[1]));
-        part[2] = __builtin_fmaf(c, dy, __builtin_fmaf(-g, b.y, part[2]));
-        part[3] = __builtin_fmaf(c, dz, __builtin_fmaf(-g, b.z, part[3]));
+        part[1] += __builtin_fmaf(c, dx, -g * b.x);
+        part[2] += __builtin_fmaf(c, dy, -g * b.y);
+        part[3] += __builtin_fmaf(c, dz, -g * b.z);
     };
     // (for the lanes that took part: adding a zero would move bits between the
     // sum and its compensation)

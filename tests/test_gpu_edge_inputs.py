@@ -3,11 +3,14 @@ to sources, values that are no numbers, radii below zero, more queries than 32
 bits count, calls recorded into a graph."""
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 from dwg_amd import gpu
 
 pytestmark = pytest.mark.gpu
+
+SIGMA = 10.0
 
 
 def test_knn_far_query_beside_a_cell_boundary(ctx):
@@ -32,3 +35,51 @@ def test_knn_far_query_beside_a_cell_boundary(ctx):
     assert sorted(ref[0]) == [0, 4, 5]
     np.testing.assert_array_equal(got.cpu().numpy(), ref)
     np.testing.assert_array_equal(d2.cpu().numpy(), rd2)
+
+
+def _factors(rho, screened):
+    """g and |g'| of w = g(ρ) d·b, b already divided by 4π, in FP64."""
+    s = SIGMA if screened else 0.0
+    eps = (1e-7 if screened else 1e-8) / (4 * np.pi)
+    e = np.exp(s * rho)
+    den = e * rho ** 3 + eps
+    return (s * rho + 1) / den, (e * rho ** 2 * (s * s * rho * rho + 3 * s * rho + 3) - s * eps) / den ** 2
+
+
+# one tile, several in one chain's place (split over waves), a leaf of the tree
+# in the walk of one query and of many (which share it)
+@pytest.mark.parametrize("where,n,nq", [("direct", 64, 1), ("direct", 1024, 1), ("tree", 64, 5), ("tree", 64, 786_432)])
+@pytest.mark.parametrize("screened", [False, True])
+def test_gradient_component_is_rounded_at_its_own_size(ctx, where, n, nq, screened):
+    # Each tile: one source whose component is the tile's sum P, then 63 whose
+    # two products are 0.55 and 0.45 units in the last place of P.  Formed first, a
+    # component is 0.1 units, and its addition rounds by half a unit at most; the
+    # products added one by one round to a whole unit and to none.
+    r = 0.5
+    g, gp = _factors(r, screened)
+    cos = np.sqrt(0.45 / 0.55 * g / (gp * r))
+    big = 1.25 / g  # P = 1.25
+    small = 0.55 * 2.0 ** -23 / g
+    tiles = n // 64
+    P = np.tile([r * cos, r * np.sqrt(1 - cos * cos), 0.0], (n, 1)).astype(np.float32)
+    A = np.full(n, small * 4 * np.pi, np.float32)
+    P[::64] = 0.0, -r, 0.0
+    A[::64] = big * 4 * np.pi
+    N = np.tile(np.float32([1, 0, 0]), (n, 1))
+    Q = torch.zeros((nq, 3), device="cuda")
+    if where == "direct":
+        _, got = ctx.gwn_direct(P, N, A, Q, sigma=SIGMA, screened=screened, kahan=True, grad=True)
+    else:
+        tree = gpu.Octree(ctx, P.astype(np.float64), A.astype(np.float64), max_depth=10, leaf_size=64)
+        assert tree.info()["nodes"] == 1
+        tree.update(N, A)
+        _, got = tree.eval_grad(Q, 2.3, sigma=SIGMA, screened=screened)
+    got = got.cpu().numpy()[:, 0].astype(np.float64)
+    d = P.astype(np.float64)
+    rr = np.linalg.norm(d, axis=1)
+    g, gp = _factors(rr, screened)
+    b = A.astype(np.float64) / (4 * np.pi)
+    want = (gp / rr * d[:, 0] * b * d[:, 0] - g * b).sum()
+    # units of 2^-23: the factors of P (32·2^-24 of it, as the sums' own test
+    # derives), half a unit an addition, one for the sums of the tiles
+    assert np.abs(got - want).max() <= tiles * (16 * 1.25 + 63 * 0.5 + 1) * 2.0 ** -23
