@@ -81,17 +81,31 @@ __device__ __forceinline__ float add_rounded(float part, float x, float inv) {
     return part + t;
 }
 
+// max(r², s²), and s² where r² is no number (an s² never is): written as the
+// instruction, as the compiler would first quiet a possible signalling NaN of s².
+// UNIFORM: s² is the same in every lane and in a scalar register
+template <bool UNIFORM>
+__device__ __forceinline__ float screened_r2(float r2, float s2) {
+    float m;
+    if constexpr (UNIFORM) asm("v_max_f32 %0, %1, %2" : "=v"(m) : "s"(s2), "v"(r2));
+    else asm("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(s2), "v"(r2));
+    return m;
+}
+
 // The direct sums' point term as such factors, a = (p, ·), b = (A·n/4π, s²);
-// 0 at the guard.  With the product left to the sum's multiply-add it takes
-// 21 instructions screened (24 with ρ = max(r, s), ρ·ρ·ρ and a selected sum:
+// 0 at the guard and where the distance is no number, by the factor x alone, as
+// the other is always one.  With the product left to the sum's multiply-add it
+// takes 21 instructions screened (24 with ρ = max(r, s), ρ·ρ·ρ and a selected sum:
 // 10,000 sources at 2M queries 13.6 → 11.9 ms, the chip's whole issue rate).
 template <bool SCREENED>
 __device__ __forceinline__ float gwn_term_split(float qx, float qy, float qz, const float4 a, const float4 b,
                                                 float sigma, float sigma_l2e, float& inv) {
     const float dx = a.x - qx, dy = a.y - qy, dz = a.z - qz;
+    const float r2 = dist2(dx, dy, dz);
     bool ok;
-    const float x = tree_term_split<SCREENED>(dx, dy, dz, dist2(dx, dy, dz), b.w, b, sigma, sigma_l2e, inv, ok);
-    return ok ? x : 0.f;
+    if constexpr (!SCREENED) return tree_term_split<false>(dx, dy, dz, r2, 0.f, b, sigma, sigma_l2e, inv, ok);
+    const float x = tree_term_split<true>(dx, dy, dz, screened_r2<true>(r2, b.w), 0.f, b, sigma, sigma_l2e, inv, ok);
+    return r2 > 1e-20f ? x : 0.f;
 }
 
 // DWG_NEAR_FP64: a screened point term inside its source's screening radius
@@ -120,13 +134,15 @@ __device__ __forceinline__ bool near_field(float r2, float s) { return r2 < s * 
 //             (∂ρ/∂q = −d/r), −g b for r < s;
 //             g' = (σε' − e^{σρ}ρ²(σ²ρ² + 3σρ + 3)) / D²  (no cancellation)
 // as the factors dot = d·b, g and c of w = g·dot, ∇w = c·d − g·b, with s2 the
-// squared screening radius (200,000 sources at 2,000 queries 540 → 480 µs with
+// squared screening radius (200,000 sources at 2,000 queries 540 → 487 µs with
 // selects on two factors instead of four results.  ρ = ρ²·ρ^-1 would save another
 // 5 %, for an error of w 8 to 13 % above the root's).  A component c·d − g·b is
 // formed before it joins its sum: its two products joined one by one, 460 µs,
 // round twice at the sum's size (half of 2,000 queries next to one of 20,000
 // sources: RMS error of ∇w 11 % and maximum 37 % more).
-template <bool SCREENED>
+// A screened term at the guard, or whose distance is no number, has only zeros
+// (d may still be no number).  UNIFORM as in screened_r2.
+template <bool SCREENED, bool UNIFORM>
 __device__ __forceinline__ void gwn_term_grad(float dx, float dy, float dz, float s2, const float4 b, float sigma,
                                               float sigma_l2e, float& dot, float& g, float& c) {
     const float r2 = dist2(dx, dy, dz);
@@ -137,7 +153,8 @@ __device__ __forceinline__ void gwn_term_grad(float dx, float dy, float dz, floa
         c = 3.0f * r * (dot * g) * g;
     } else {
         const bool ok = r2 > 1e-20f;
-        const float rho2 = max_nonneg(r2, s2);
+        dot = ok ? dot : 0.0f;
+        const float rho2 = screened_r2<UNIFORM>(r2, s2);
         const float rho = fast_sqrt(rho2), irho = fast_rsq(rho2);
         const float er2 = fast_exp2(sigma_l2e * rho) * rho2;
         const float eps = kEpsScreened * kInv4Pi;
@@ -148,6 +165,14 @@ __device__ __forceinline__ void gwn_term_grad(float dx, float dy, float dz, floa
         // inside (ρ = s) nothing depends on q through ρ
         c = ok && !(s2 > r2) ? (dot * irho) * (gp * inv) * inv : 0.0f;
     }
+}
+
+// a component c·d − g·b of the gradient: 0 · d is 0 by this multiplication, also
+// for a d that is no number
+__device__ __forceinline__ float grad_component(float c, float d, float g, float b) {
+    float cd;
+    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(cd) : "v"(c), "v"(d));
+    return __builtin_fmaf(-g, b, cd);
 }
 
 // ---------------------------------------------------------------------------
@@ -222,11 +247,11 @@ __device__ __forceinline__ void direct_grad(const float4* __restrict__ sa, const
     auto term = [&](const float4 a, const float4 b) {
         const float dx = a.x - qx, dy = a.y - qy, dz = a.z - qz;
         float dot, g, c;
-        gwn_term_grad<SCREENED>(dx, dy, dz, b.w, b, sigma, sl2e, dot, g, c);
+        gwn_term_grad<SCREENED, true>(dx, dy, dz, b.w, b, sigma, sl2e, dot, g, c);
         p[0] = __builtin_fmaf(g, dot, p[0]);
-        p[1] += __builtin_fmaf(c, dx, -g * b.x);
-        p[2] += __builtin_fmaf(c, dy, -g * b.y);
-        p[3] += __builtin_fmaf(c, dz, -g * b.z);
+        p[1] += grad_component(c, dx, g, b.x);
+        p[2] += grad_component(c, dy, g, b.y);
+        p[3] += grad_component(c, dz, g, b.z);
     };
     auto fold = [&]() {
 #pragma unroll
@@ -1034,38 +1059,6 @@ __host__ __device__ constexpr int walk_stack_entries(int max_level, int lanes) {
     return tree_stack_entries(max_level) + (lanes > 8 ? kWalkDeep + 7 * (lanes / 8) : 0);
 }
 
-// value and gradient of tree_term_split's term; 0 unless `on` and beyond the
-// guard
-template <bool SCREENED>
-__device__ __forceinline__ void tree_term_grad(float dx, float dy, float dz, float s2, const float4 b, float sigma,
-                                               float sigma_l2e, float& w, float& gx, float& gy, float& gz) {
-    const float r2 = dist2(dx, dy, dz);
-    const float dot = __builtin_fmaf(dz, b.z, __builtin_fmaf(dy, b.y, dx * b.x));
-    if constexpr (!SCREENED) {
-        const float r = fast_sqrt(r2);
-        const float inv = fast_rcp(__builtin_fmaf(r2, r, kEpsPlain * kInv4Pi));
-        w = dot * inv;
-        const float c = 3.0f * r * w * inv;
-        gx = __builtin_fmaf(c, dx, -b.x * inv);
-        gy = __builtin_fmaf(c, dy, -b.y * inv);
-        gz = __builtin_fmaf(c, dz, -b.z * inv);
-    } else {
-        const bool ok = r2 > 1e-20f, inside = s2 > r2;  // inside: ρ = s, no dependence on q through ρ
-        const float rho = fast_sqrt(max_nonneg(r2, s2));
-        const float er2 = fast_exp2(sigma_l2e * rho) * (rho * rho);
-        const float eps = kEpsScreened * kInv4Pi;
-        const float inv = fast_rcp(__builtin_fmaf(er2, rho, eps));
-        const float sr = sigma * rho;
-        const float g = ok ? __builtin_fmaf(sigma, rho, 1.0f) * inv : 0.0f;
-        const float gp = (sigma * eps - er2 * __builtin_fmaf(sr, sr + 3.0f, 3.0f)) * inv * inv;
-        const float c = (inside || !ok) ? 0.0f : -dot * gp * fast_rcp(rho);
-        w = g * dot;
-        gx = __builtin_fmaf(c, dx, -g * b.x);
-        gy = __builtin_fmaf(c, dy, -g * b.y);
-        gz = __builtin_fmaf(c, dz, -g * b.z);
-    }
-}
-
 template <bool SCREENED, bool BF16, bool GRAD, int L>
 __global__ __launch_bounds__(kWalkWaves * 64) void gwn_walk_kernel(TreeArgs T, const float* __restrict__ q, int64_t nq,
                                                                     int stack, float sigma, float* __restrict__ out_w,
@@ -1085,12 +1078,12 @@ __global__ __launch_bounds__(kWalkWaves * 64) void gwn_walk_kernel(TreeArgs T, c
     for (int k = 0; k < (GRAD ? 4 : 1); ++k) sum[k] = 0.0;
     auto add = [&](float dx, float dy, float dz, float s2, const float4 b) {
         if constexpr (GRAD) {
-            float w, gx, gy, gz;
-            tree_term_grad<SCREENED>(dx, dy, dz, s2, b, sigma, sl2e, w, gx, gy, gz);
-            sum[0] += double(w);
-            sum[1] += double(gx);
-            sum[2] += double(gy);
-            sum[3] += double(gz);
+            float dot, g, c;
+            gwn_term_grad<SCREENED, false>(dx, dy, dz, s2, b, sigma, sl2e, dot, g, c);
+            sum[0] += double(g * dot);
+            sum[1] += double(grad_component(c, dx, g, b.x));
+            sum[2] += double(grad_component(c, dy, g, b.y));
+            sum[3] += double(grad_component(c, dz, g, b.z));
         } else {
             float inv;
             bool ok;
@@ -1464,13 +1457,13 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_grad_kernel(TreeArgs T,
     auto add = [&](float dx, float dy, float dz, float sr, const float4 b, bool on) {
         float dot, g, c;
         const float s = fmaxf(sr, 0.f);
-        gwn_term_grad<SCREENED>(dx, dy, dz, s * s, b, sigma, sl2e, dot, g, c);
+        gwn_term_grad<SCREENED, false>(dx, dy, dz, s * s, b, sigma, sl2e, dot, g, c);
         g = on ? g : 0.f;
         c = on ? c : 0.f;
         part[0] = __builtin_fmaf(g, dot, part[0]);
-        part[1] += __builtin_fmaf(c, dx, -g * b.x);
-        part[2] += __builtin_fmaf(c, dy, -g * b.y);
-        part[3] += __builtin_fmaf(c, dz, -g * b.z);
+        part[1] += grad_component(c, dx, g, b.x);
+        part[2] += grad_component(c, dy, g, b.y);
+        part[3] += grad_component(c, dz, g, b.z);
     };
     // (for the lanes that took part: adding a zero would move bits between the
     // sum and its compensation)

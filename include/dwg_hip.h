@@ -80,7 +80,8 @@ int dwg_ctx_counter_get(dwg_ctx* ctx, const char* name, int64_t* value);
  * d_radii may be NULL unless DWG_USE_RADII.  d_out_grad (nullable, nq×3)
  * receives ∇_q w (new; the reference has no gradient), of the plain or the
  * screened term; a screened term inside its screening radius (ρ = s) has
- * ∇w = −g(s)·A·n. */
+ * ∇w = −g(s)·A·n.  A screened term whose distance is not above 1e-10, or is
+ * no number (a NaN in the source's or the query's position), is 0. */
 int dwg_gwn_direct(dwg_ctx* ctx, const float* d_pts, const float* d_nrm, const float* d_area,
                    const float* d_radii, int64_t n, const float* d_q, int64_t nq, float sigma,
                    uint32_t flags, float* d_out_w, float* d_out_grad);

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import oracle as O
-from dwg_amd import gpu
+from dwg_amd import gpu, shapes
 
 pytestmark = pytest.mark.gpu
 
@@ -83,3 +83,48 @@ def test_gradient_component_is_rounded_at_its_own_size(ctx, where, n, nq, screen
     # units of 2^-23: the factors of P (32·2^-24 of it, as the sums' own test
     # derives), half a unit an addition, one for the sums of the tiles
     assert np.abs(got - want).max() <= tiles * (16 * 1.25 + 63 * 0.5 + 1) * 2.0 ** -23
+
+
+# one chain and split over the sources
+@pytest.mark.parametrize("n,nq", [(100, 7), (700, 300)])
+@pytest.mark.parametrize("kahan,near64", [(False, False), (True, False), (True, True)])
+def test_screened_direct_sums_leave_out_what_is_no_number(ctx, n, nq, kahan, near64):
+    # a term whose distance is no number is 0, as one at the query itself: the
+    # sums are those of sources without it, and a query that is no number gets 0
+    P, N = shapes.sphere(n, 5)
+    rng = np.random.default_rng(n)
+    A = rng.uniform(1e-4, 3e-3, n).astype(np.float32)
+    Q = np.concatenate([rng.uniform(-1.3, 1.3, (nq - nq // 4, 3)), P[: nq // 4]]).astype(np.float32)
+    P, N, bad = P.astype(np.float32), N.astype(np.float32), np.arange(3, n, 41)
+    P0, N0 = P.copy(), N.copy()
+    P0[bad], N0[bad] = 0.25, 0.0  # the same places in the chain, no contribution
+    P[bad, rng.integers(0, 3, len(bad))] = np.nan
+    Qn = Q.copy()
+    Qn[::5, 1] = np.nan
+    kw = dict(sigma=SIGMA, screened=True, kahan=kahan, near64=near64)
+    for grad in (False, True):
+        want = ctx.gwn_direct(P0, N0, A, Q, grad=grad, **kw)
+        got = ctx.gwn_direct(P, N, A, Qn, grad=grad, **kw)
+        for w, v in zip(want if grad else (want,), got if grad else (got,)):
+            w = w.cpu().numpy().copy()
+            w[::5] = 0.0
+            np.testing.assert_array_equal(v.cpu().numpy(), w)
+
+
+# a walk a query (64 and 8 lanes) and walks shared by 64
+@pytest.mark.parametrize("nq", [500, 50_000, 786_500])
+def test_screened_tree_gradient_of_a_query_that_is_no_number(ctx, nq):
+    n = 2000
+    P, N = shapes.sphere(n, 5)
+    rng = np.random.default_rng(nq)
+    tree = gpu.Octree(ctx, P.astype(np.float64), None, max_depth=10)
+    A = np.full(n, 2e-6, np.float32)
+    tree.update(N, A)
+    Q = rng.uniform(-1.3, 1.3, (nq, 3)).astype(np.float32)
+    Q = torch.from_numpy(Q[np.lexsort((Q * 20).astype(int).T)]).cuda()  # in order, with or without the others
+    w0, g0 = tree.eval_grad(Q, 2.3, sigma=SIGMA)
+    Q[100:200:7, 2] = float("nan")
+    w, g = tree.eval_grad(Q, 2.3, sigma=SIGMA)
+    w0[100:200:7] = 0.0
+    g0[100:200:7] = 0.0
+    assert torch.equal(w, w0) and torch.equal(g, g0)
