@@ -801,13 +801,13 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
         if (BF16) return __builtin_fmaf((on && ok) ? x : 0.f, inv, part);  // last product fused into the sum
         return part + ((on && ok) ? x * inv : 0.f);
     };
-    // (one part: only the lanes that opened the node, as adding a zero would
-    // move bits between the sum and its compensation, and an explicit query's
-    // value must not depend on the queries it shares the wave with)
+    // (with compensation only the lanes that opened the node, as adding a zero
+    // would move bits between the sum and its compensation, and a point's value
+    // must not depend on the points it shares the wave with)
     auto add = [&](float part, int h, uint64_t m) {
         if (!kahan) {
             sum[h] += part;
-        } else if (H > 1 || __builtin_amdgcn_inverse_ballot_w64(m)) {
+        } else if (__builtin_amdgcn_inverse_ballot_w64(m)) {
             kahan_add(sum[h], comp[h], part);
         }
     };

@@ -128,3 +128,29 @@ def test_screened_tree_gradient_of_a_query_that_is_no_number(ctx, nq):
     w0[100:200:7] = 0.0
     g0[100:200:7] = 0.0
     assert torch.equal(w, w0) and torch.equal(g, g0)
+
+
+@pytest.mark.parametrize("res,h", [((8, 4, 8), 0.05), ((33, 29, 31), 0.08), ((51, 53, 55), 0.02), ((401, 399, 1), 0.003),
+                                   ((190, 181, 183), 0.005), ((195, 191, 185), 0.005)])
+@pytest.mark.parametrize("screened,bf16,radii", [(True, False, False), (True, True, True), (False, False, False),
+                                                 (False, True, False)])
+def test_compensated_grid_walk_equals_the_point_walk(ctx, res, h, screened, bf16, radii):
+    # with compensation too a grid value is the explicit point's bit for bit, by
+    # whichever walk the grid's size picks
+    P, N = shapes.union(3000, 8, 11)
+    P = np.concatenate([P, P[:40], P[:3] + 1e-6]).astype(np.float64)
+    N = np.concatenate([N, N[:40], N[:3]]).astype(np.float32)
+    A = np.full(len(P), 2e-6, np.float32)
+    R = np.linspace(0.0, 0.05, len(P), dtype=np.float32) if radii else None
+    tree = gpu.Octree(ctx, P, None, max_depth=10)
+    tree.update(N, A, R)
+    c = P.mean(0)
+    grid = gpu.make_grid([c[d] - 0.5 * h * (res[d] - 1) for d in range(3)], h, res)
+    ax = [(np.arange(res[d]) * np.float64(grid.h) + grid.origin[d]).astype(np.float32) for d in range(3)]
+    z, y, x = np.meshgrid(ax[2], ax[1], ax[0], indexing="ij")
+    Q = torch.from_numpy(np.stack([x, y, z], -1).reshape(-1, 3).astype(np.float32)).cuda()
+    kw = dict(sigma=SIGMA, screened=screened, bf16=bf16, kahan=True)
+    got = tree.eval_grid(grid, 2.3, **kw).cpu().numpy()
+    many = Q if len(Q) > 200_000 else Q.repeat(200_000 // len(Q) + 1, 1)
+    want = tree.eval(many, 2.3, **kw).cpu().numpy()[:len(Q)]
+    np.testing.assert_array_equal(got, want)
