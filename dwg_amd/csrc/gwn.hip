@@ -176,9 +176,14 @@ __device__ __forceinline__ float grad_component(float c, float d, float g, float
 }
 
 // ---------------------------------------------------------------------------
-// source packing: (x, y, z, s) and (A·n/4π, s²), s² 0 for s ≤ 0 or NaN (ρ = r)
-// and kept finite with s
+// source packing: (x, y, z, s) and (A·n/4π, s²)
 // ---------------------------------------------------------------------------
+// the screening radius of every sum: 0 for s ≤ 0 or NaN (ρ = max(s, r) = r), and a
+// finite one kept to where its square is finite
+__device__ __forceinline__ float screening_radius(float s) {
+    return s > 0.f ? (s < INFINITY ? fminf(s, 1.84467429e19f) : s) : 0.f;
+}
+
 __global__ void pack_sources_kernel(const float* __restrict__ pts, const float* __restrict__ nrm,
                                     const float* __restrict__ area, const float* __restrict__ radii,
                                     const int* __restrict__ perm, int64_t n, int use_radii,
@@ -188,11 +193,10 @@ __global__ void pack_sources_kernel(const float* __restrict__ pts, const float* 
     if (i >= n) return;
     const int64_t p = perm ? perm[i] : i;
     const float A = area ? area[p] : 2e-6f;
-    const float s = use_radii ? radii[p] : kScreenDefault;
+    const float s = use_radii ? screening_radius(radii[p]) : kScreenDefault;
     if (sa) sa[i] = make_float4(pts[3 * p], pts[3 * p + 1], pts[3 * p + 2], s);
     const float nx = nrm[3 * p], ny = nrm[3 * p + 1], nz = nrm[3 * p + 2];
-    const float s2 = s > 0.f ? (s < INFINITY ? fminf(s * s, 3.402823466e38f) : s) : 0.f;
-    sb[i] = make_float4(A * nx * kInv4Pi, A * ny * kInv4Pi, A * nz * kInv4Pi, s2);
+    sb[i] = make_float4(A * nx * kInv4Pi, A * ny * kInv4Pi, A * nz * kInv4Pi, s * s);
     if (an64) an64[i] = Double3(double(A) * nx, double(A) * ny, double(A) * nz);
 }
 
@@ -573,7 +577,7 @@ __global__ void repack_sources_kernel(const float* __restrict__ nrm, const float
     if (i >= n) return;
     const int64_t p = perm[i];
     const float A = area ? area[p] : 2e-6f;
-    sa[i].w = radii ? radii[p] : kScreenDefault;
+    sa[i].w = radii ? screening_radius(radii[p]) : kScreenDefault;
     const float nx = nrm[3 * p], ny = nrm[3 * p + 1], nz = nrm[3 * p + 2];
     sb[i] = make_float4(A * nx * kInv4Pi, A * ny * kInv4Pi, A * nz * kInv4Pi, 0.f);
     an64[i] = Double3(double(A) * nx, double(A) * ny, double(A) * nz);
@@ -1454,10 +1458,9 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_grad_kernel(TreeArgs T,
     // with Kahan compensation: the gradient's near terms are large and
     // cancel, so plain FP32 accumulation over many nodes would lose digits
     float acc[4] = {0.f, 0.f, 0.f, 0.f}, comp[4] = {0.f, 0.f, 0.f, 0.f}, part[4] = {0.f, 0.f, 0.f, 0.f};
-    auto add = [&](float dx, float dy, float dz, float sr, const float4 b, bool on) {
+    auto add = [&](float dx, float dy, float dz, float s2, const float4 b, bool on) {
         float dot, g, c;
-        const float s = fmaxf(sr, 0.f);
-        gwn_term_grad<SCREENED, false>(dx, dy, dz, s * s, b, sigma, sl2e, dot, g, c);
+        gwn_term_grad<SCREENED, false>(dx, dy, dz, s2, b, sigma, sl2e, dot, g, c);
         g = on ? g : 0.f;
         c = on ? c : 0.f;
         part[0] = __builtin_fmaf(g, dot, part[0]);
@@ -1477,7 +1480,7 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_grad_kernel(TreeArgs T,
     auto leaf = [&](int b, int e, bool on) {
         for (int j = b; j < e; ++j) {
             const float4 a = scalar_load(T.sa, j);
-            add(a.x - qx, a.y - qy, a.z - qz, a.w, scalar_load(T.sb, j), on);
+            add(a.x - qx, a.y - qy, a.z - qz, a.w * a.w, scalar_load(T.sb, j), on);
         }
     };
     int sp = 0;
@@ -1512,7 +1515,7 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_grad_kernel(TreeArgs T,
             const uint64_t farm = __builtin_amdgcn_ballot_w64(far);
             if (mask & farm) {
                 const float4 lo = s_pay[wave][2 * c + 1];
-                add(dx + lo.x, dy + lo.y, dz + lo.z, kScreenDefault, s_pay[wave][2 * c], act && far);
+                add(dx + lo.x, dy + lo.y, dz + lo.z, kDipoleS2, s_pay[wave][2 * c], act && far);
             }
             const uint64_t nm = mask & ~farm;
             if (nm) {

@@ -32,7 +32,8 @@ extern "C" {
 
 /* flags for the winding-number sums */
 #define DWG_SCREENED 1u   /* screened kernel (TurboLibiGWN.cu:552-585); else plain libigl kernel */
-#define DWG_USE_RADII 2u  /* screening radius per source; else 0.0015 for every source */
+#define DWG_USE_RADII 2u  /* screening radius per source (one not above 0 screens nothing); else 0.0015
+                             for every source */
 #define DWG_KAHAN 4u      /* compensated (Kahan) accumulation of per-tile partial sums */
 #define DWG_FAR_BF16 8u   /* far-field dipole moments stored and read as bf16 (tree only) */
 #define DWG_NEAR_FP64 16u /* screened point terms inside the source's screening radius (r < s)

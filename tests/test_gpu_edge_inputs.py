@@ -154,3 +154,34 @@ def test_compensated_grid_walk_equals_the_point_walk(ctx, res, h, screened, bf16
     many = Q if len(Q) > 200_000 else Q.repeat(200_000 // len(Q) + 1, 1)
     want = tree.eval(many, 2.3, **kw).cpu().numpy()[:len(Q)]
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("leaf_size", [1, 8])
+def test_radii_below_zero_screen_nothing(ctx, leaf_size):
+    # ρ = max(s, r) is r for a radius of 0, below 0 and no number alike, in every
+    # walk and the direct sums
+    n = 3000
+    P, N = shapes.sphere(n, 4)
+    rng = np.random.default_rng(n)
+    A = rng.uniform(1e-6, 4e-6, n).astype(np.float32)
+    R = rng.uniform(0.001, 0.05, n).astype(np.float32)
+    off = rng.uniform(size=n) < 0.5
+    P = P.astype(np.float32)
+    Q = (P[rng.integers(0, n, 786_500)] + rng.normal(0, 0.01, (786_500, 3))).astype(np.float32)
+    grid = gpu.make_grid([-1.1] * 3, 0.05, [45] * 3)
+
+    def results(bad):
+        r = R.copy()
+        r[off] = np.where(np.arange(off.sum()) % 3 == 0, np.float32(bad), r[off] * np.float32(0 if bad == 0 else -1))
+        tree = gpu.Octree(ctx, P.astype(np.float64), None, max_depth=6, leaf_size=leaf_size)
+        tree.update(N, A, r)
+        for near64 in (False, True):
+            yield tree.eval(Q[:500], 2.3, sigma=SIGMA, near64=near64)
+            yield tree.eval(Q[:200_000], 2.3, sigma=SIGMA, near64=near64)
+            yield ctx.gwn_direct(P, N, A, Q[:3000], sigma=SIGMA, screened=True, radii=r, near64=near64)
+        yield tree.eval_grid(grid, 2.3, sigma=SIGMA)
+        for nq in (500, 50_000, 786_500):
+            yield from tree.eval_grad(Q[:nq], 2.3, sigma=SIGMA)
+
+    for want, got in zip(results(0.0), results(float("nan"))):
+        assert bool(torch.isfinite(want).all()) and torch.equal(got, want)
