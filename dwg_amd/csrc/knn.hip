@@ -447,14 +447,15 @@ dwg_knn_index* knn_build(dwg_ctx* ctx, const float* p, int64_t n, int k_hint) {
 // best[0] is the k-th smallest key so far (the insertion threshold), the
 // slots k..K−1 hold 0 and never move (every key is ≥ 0).  Every access uses
 // a constant index, so the list is never demoted to scratch memory.
-// An empty slot: the bits of +∞ as a double, above every key (the high
-// word of a key is the float bits of a d² ≥ 0, at most 0x7F800000)
-constexpr uint64_t kNoKey = 0x7FF0000000000000ull;
+// An empty slot: above every key with a d² up to ∞ (the high word of a key is the
+// float bits of its d²) and below those of a d² that is no number, so that a point
+// or a query with a NaN has no neighbours and is none
+constexpr uint64_t kNoKey = 0x7F800000FFFFFFFFull;
 
 template <int K>
-__device__ __forceinline__ void knn_reset(uint64_t (&best)[K], int k, uint64_t none = kNoKey) {
+__device__ __forceinline__ void knn_reset(uint64_t (&best)[K], int k) {
 #pragma unroll
-    for (int j = 0; j < K; ++j) best[j] = j < k ? none : 0ull;
+    for (int j = 0; j < K; ++j) best[j] = j < k ? kNoKey : 0ull;
 }
 
 // The key takes its place in the list and the largest key leaves it (the key
@@ -477,14 +478,14 @@ __device__ __forceinline__ void knn_insert(uint64_t (&best)[K], uint64_t key) {
 // writes the k keys in ascending order (index −1 / d² ∞ where fewer were found)
 template <int K>
 __device__ __forceinline__ void knn_store(const uint64_t (&best)[K], int k, int64_t row, int32_t* __restrict__ out_idx,
-                                          float* __restrict__ out_d2, uint64_t none = kNoKey) {
+                                          float* __restrict__ out_d2) {
 #pragma unroll
     for (int j = 0; j < K; ++j) {
         if (j < k) {
             const uint64_t b = best[j];
             const int64_t o = row * k + (k - 1 - j);
-            out_idx[o] = b == none ? -1 : int32_t(uint32_t(b));
-            if (out_d2) out_d2[o] = b == none ? INFINITY : __uint_as_float(uint32_t(b >> 32));
+            out_idx[o] = b == kNoKey ? -1 : int32_t(uint32_t(b));
+            if (out_d2) out_d2[o] = b == kNoKey ? INFINITY : __uint_as_float(uint32_t(b >> 32));
         }
     }
 }
@@ -512,8 +513,6 @@ constexpr int kTileThreads = 256;
 // batches, also with the nearest first, cost what they save.
 constexpr int kBatch = 16;
 static_assert(kStage % kBatch == 0 && kTileThreads >= kBatch, "whole batches, filled up by one thread a place");
-// An empty slot here: its high word is a d² of ∞, which any d² but NaN passes
-constexpr uint64_t kFar = 0x7F800000FFFFFFFFull;
 // most queries close within 2 cells of their tile.  Wider passes for the
 // others (5 and 9 cells) cost more than walking the pyramid at once: 200,000
 // queries over 1M points, half of them off the surface, 5.6 → 3.4 ms
@@ -734,7 +733,7 @@ __global__ __launch_bounds__(kTileThreads, K <= 17 ? 4 : 2) void knn_tile_kernel
                     qz = active ? q[3 * int64_t(qi) + 2] : NAN;
         uint64_t best[K];
         const uint64_t has = __builtin_amdgcn_ballot_w64(active);
-        knn_reset<K>(best, k, kFar);
+        knn_reset<K>(best, k);
         auto kth = [&]() { return __uint_as_float(uint32_t(best[0] >> 32)); };  // the k-th d², or ∞
         for (int cb = 0; cb < total; cb += kStage) {
             const int cnt = min(kStage, total - cb);
@@ -770,14 +769,14 @@ __global__ __launch_bounds__(kTileThreads, K <= 17 ? 4 : 2) void knn_tile_kernel
                     const bool near = d2[u] <= kth();
                     if (!__builtin_amdgcn_ballot_w64(near)) continue;
                     knn_insert<K>(best, near ? (uint64_t(__float_as_uint(d2[u])) << 32) | __float_as_uint(s_pts[j + u].w)
-                                             : kFar);
+                                             : kNoKey);
                 }
             }
         }
         if (!active) continue;
         const float dmin = fminf(fminf(fminf(qx - flx, fhx - qx), fminf(qy - fly, fhy - qy)), fminf(qz - flz, fhz - qz));
         bool exact = dmin == INFINITY;
-        if (!exact && best[0] != kFar) {
+        if (!exact && best[0] != kNoKey) {
             const float safe = dmin * (1.0f - 1e-5f) - 1e-6f * G.cell;
             exact = safe > 0.f && kth() < safe * safe;
         }
@@ -797,14 +796,14 @@ __global__ __launch_bounds__(kTileThreads, K <= 17 ? 4 : 2) void knn_tile_kernel
             redo_kth[at] = kth();
             continue;
         }
-        knn_store<K>(best, k, qi, out_idx, out_d2, kFar);
+        knn_store<K>(best, k, qi, out_idx, out_d2);
         if (SCATTER) {
             long long v[3];
 #pragma unroll
             for (int d = 0; d < 3; ++d) v[d] = __double2ll_rn(double(sc.val[3 * int64_t(qi) + d]) * kScatterFix);
 #pragma unroll
             for (int j = 0; j < K; ++j) {
-                if (j >= k || best[j] == kFar) continue;
+                if (j >= k || best[j] == kNoKey) continue;
                 const int idx = int(uint32_t(best[j]));
                 int h = int((uint32_t(idx) * 0x9E3779B1u) >> 24);  // 8 bits
                 bool done = false;
@@ -1297,7 +1296,8 @@ __global__ __launch_bounds__(kDescWaves * 64) void knn_descent_kernel(
         const float cap = init_kth ? init_kth[t] : INFINITY;
         uint64_t list = kNoKey, kth = kNoKey;
         float bound = cap;
-        int sp = 1, steps = 0;
+        // (a query that is no number walks nowhere)
+        int sp = uniform(qx == qx && qy == qy && qz == qz ? 1 : 0), steps = 0;
         ent[0] = root;
         ed2[0] = 0.f;
         __builtin_amdgcn_wave_barrier();

@@ -182,7 +182,8 @@ int dwg_knn_build(dwg_ctx* ctx, const float* d_pts, int64_t n, int k_hint, dwg_k
 void dwg_knn_destroy(dwg_knn_index* index);
 /* k ≤ 32.  d_skip (nullable): points with d_skip[j] != 0 are not candidates.
  * d_qmask (nullable): queries with d_qmask[i] == 0 are not computed.
- * d_d2 (nullable) receives the distances.  Missing neighbours are -1. */
+ * d_d2 (nullable) receives the distances.  Missing neighbours are -1 (at ∞);
+ * a point with a NaN is nobody's neighbour, a query with one has none. */
 int dwg_knn_query(dwg_ctx* ctx, const dwg_knn_index* index, const float* d_q, int64_t nq, int k,
                   const uint8_t* d_skip, const uint8_t* d_qmask, int32_t* d_idx, float* d_d2);
 

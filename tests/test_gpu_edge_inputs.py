@@ -185,3 +185,27 @@ def test_radii_below_zero_screen_nothing(ctx, leaf_size):
 
     for want, got in zip(results(0.0), results(float("nan"))):
         assert bool(torch.isfinite(want).all()) and torch.equal(got, want)
+
+
+def test_knn_query_that_is_no_number(ctx):
+    # at no distance from any point, it has no neighbours, in a small query set as
+    # in a tiled one
+    P, _ = shapes.sphere(40_000, 3)
+    P = P.astype(np.float32)
+    idx = gpu.KnnIndex(ctx, P, k_hint=8)
+    rng = np.random.default_rng(1)
+    for nq in (100, 60_000):
+        Q = rng.uniform(-1.2, 1.2, (nq, 3)).astype(np.float32)
+        Q[5::7, rng.integers(0, 3)] = np.nan
+        got, d2 = (t.cpu().numpy() for t in idx.query(Q, 8, d2=True))
+        assert (got[5::7] == -1).all() and np.isinf(d2[5::7]).all()
+        sub = [0, 1, 2, 3, 4, 6, 7, 8, 9, 10, 11, 13]
+        np.testing.assert_array_equal(got[sub], O.knn_brute(P, Q[sub], 8))
+    # nor is a point that is no number anyone's neighbour, one cell or several
+    for scale in (0.0, 1.0):
+        P = np.float32(scale) * rng.uniform(-1, 1, (40, 3)).astype(np.float32)
+        P[::4, 1] = np.nan
+        for nq in (5, 20_000):
+            got = gpu.KnnIndex(ctx, P, k_hint=8).query(rng.uniform(-1, 1, (nq, 3)).astype(np.float32), 32)
+            got = np.sort(got.cpu().numpy(), axis=1)
+            assert (got[:, :2] == -1).all() and (got[:, 2:] == np.flatnonzero(np.arange(40) % 4)).all()
