@@ -1,5 +1,8 @@
 // Exact kNN on a uniform cell grid.
 #pragma once
+#include <atomic>
+#include <mutex>
+
 #include "common.h"
 
 namespace dwg {
@@ -42,8 +45,11 @@ struct dwg_knn_index {
         int pyr_levels = 0;             // 0: no pyramid (grid too elongated)
         float pyr_margin = 0.f;         // rounding allowance of cell boundaries
         // bounding box of the points of every cell (at 2·cell) and pyramid
-        // block (at 2·(ncells + byte offset)): (lo, 0), (hi, 0); (∞, −∞) empty
-        float4* pbox = nullptr;
+        // block (at 2·(ncells + byte offset)): (lo, 0), (hi, 0); (∞, −∞) empty.
+        // Null until a query builds them; set once they are whole, as queries
+        // on other streams and threads may read them from then on
+        std::atomic<float4*> pbox{nullptr};
+        std::mutex building;            // of the boxes
     } lvl[2];
     ~dwg_knn_index();
 };

@@ -278,27 +278,35 @@ __global__ void box_up_kernel(const float4* __restrict__ lower, int dx, int dy, 
     out[2 * b + 1] = hi;
 }
 
-// the points' bounding boxes of every cell and pyramid block, built the
-// first time a walk needs them (only the wave-shared walk does)
-static void ensure_boxes(dwg_ctx* ctx, dwg_knn_index::Level& L) {
-    if (L.pbox) return;
+// the points' bounding boxes of every cell and pyramid block, built the first
+// time a walk needs them (only the wave-shared walk does).  One caller builds
+// them, and waits until they are there: searches on other streams take them as
+// soon as they see them
+static const float4* ensure_boxes(dwg_ctx* ctx, dwg_knn_index::Level& L) {
+    std::lock_guard<std::mutex> lock(L.building);
+    if (const float4* there = L.pbox) return there;
     const int levels = L.pyr_levels;
     const int4* dims = L.pyr_dim_h;
     const int64_t* off = L.pyr_off_h;
     int64_t total = 0;
     for (int l = 1; l < levels; ++l) total += int64_t(dims[l].x) * dims[l].y * dims[l].z;
-    L.pbox = static_cast<decltype(L.pbox)>(dev_malloc(sizeof(float4) * 2 * size_t(L.ncells + total)));
+    DevBuf mem;
+    float4* box = static_cast<float4*>(mem.ensure(sizeof(float4) * 2 * size_t(L.ncells + total)));
     hipLaunchKernelGGL(cell_box_kernel, dim3(grid_for(L.ncells, 256)), dim3(256), 0, ctx->stream, L.cell_start, L.pts,
-                       L.ncells, L.pbox);
+                       L.ncells, box);
     check_launch();
     for (int l = 1; l < levels; ++l) {
         const int4 lo = dims[l - 1], up = dims[l];
         const int64_t nb = int64_t(up.x) * up.y * up.z;
-        const float4* lower = L.pbox + 2 * (l == 1 ? 0 : L.ncells + off[l - 1]);
+        const float4* lower = box + 2 * (l == 1 ? 0 : L.ncells + off[l - 1]);
         hipLaunchKernelGGL(box_up_kernel, dim3(grid_for(nb, 256)), dim3(256), 0, ctx->stream, lower, lo.x, lo.y, lo.z,
-                           up.x, up.y, up.z, L.pbox + 2 * (L.ncells + off[l]));
+                           up.x, up.y, up.z, box + 2 * (L.ncells + off[l]));
         check_launch();
     }
+    DWG_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+    mem.ptr = nullptr;  // the index's from here on
+    L.pbox = box;
+    return box;
 }
 
 // cell boundaries are computed as lo + b·w in float and points are
@@ -1622,8 +1630,9 @@ __global__ __launch_bounds__(kPwWaves * 64) void knn_pyramid_wave_kernel(KnnGrid
 // points (30,000 over 1M: 3.3 ms by coarse-cell shells, 1.2 ms)
 constexpr int64_t kDescAlways = 16384, kDescFew = 32768, kDescSparse = 65536;
 
-static PyrArgs pyr_args(const dwg_knn_index::Level& L, const uint8_t* mask) {
-    return PyrArgs{mask ? mask : L.pyr, L.pyr_dim, L.pyr_off, L.pyr_levels, L.pyr_margin, L.pbox, L.ncells};
+// (box: null for the boxes of the cells)
+static PyrArgs pyr_args(const dwg_knn_index::Level& L, const uint8_t* mask, const float4* box) {
+    return PyrArgs{mask ? mask : L.pyr, L.pyr_dim, L.pyr_off, L.pyr_levels, L.pyr_margin, box, L.ncells};
 }
 
 // nq queries (of which *count, when given), one wave each
@@ -1650,7 +1659,7 @@ static void launch_descent(dwg_ctx* ctx, const dwg_knn_index* I, const float* q,
         launch_wave(ctx, I, q, S.nq, S.count, S.list, k, skip, qmask, out_idx, out_d2);
         return;
     }
-    const PyrArgs Y = pyr_args(L, pyr_mask);
+    const PyrArgs Y = pyr_args(L, pyr_mask, L.pbox);
     // enough blocks to fill the chip; the waves take further queries in turn.
     // Far queries' walks differ most in length and get two waves where others
     // have one (75,000 left of 180,000 far ones: 3.88 ms the diffusion with 4096
@@ -1658,7 +1667,7 @@ static void launch_descent(dwg_ctx* ctx, const dwg_knn_index* I, const float* q,
     // 1.41, 1.43 and 1.53)
     const int64_t blocks = S.count ? 8192 : 4096;
     dim3 grid(unsigned(std::min<int64_t>(grid_for(S.nq, kDescWaves), blocks))), block(kDescWaves * 64);
-    if (L.pbox)
+    if (Y.box)
         hipLaunchKernelGGL(knn_descent_kernel<true>, grid, block, 0, ctx->stream, L.G, Y, L.cell_start, L.pts, q, S, k,
                            skip, qmask, out_idx, out_d2);
     else
@@ -1687,8 +1696,7 @@ static void launch_far(dwg_ctx* ctx, const dwg_knn_index* I, const float* q, int
     }
     // the boxes are a cache of the index's own points: building them
     // leaves the index unchanged
-    ensure_boxes(ctx, const_cast<dwg_knn_index::Level&>(L));
-    const PyrArgs Y = pyr_args(L, pyr_mask);
+    const PyrArgs Y = pyr_args(L, pyr_mask, ensure_boxes(ctx, const_cast<dwg_knn_index::Level&>(L)));
     DWG_REQUIRE(L.pyr_levels <= kMaxPyr && 7 * L.pyr_levels + 1 <= kPwStack, "pyramid deeper than the wave stack");
     int* open_q = static_cast<int*>(ctx->buf("knn_open_q", sizeof(int) * nq));
     float* open_kth = static_cast<float*>(ctx->buf("knn_open_kth", sizeof(float) * nq));

@@ -1,6 +1,8 @@
 """Inputs at the edges of what the entry points take: far queries, queries next
 to sources, values that are no numbers, radii below zero, more queries than 32
 bits count, calls recorded into a graph."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -209,3 +211,35 @@ def test_knn_query_that_is_no_number(ctx):
             got = gpu.KnnIndex(ctx, P, k_hint=8).query(rng.uniform(-1, 1, (nq, 3)).astype(np.float32), 32)
             got = np.sort(got.cpu().numpy(), axis=1)
             assert (got[:, :2] == -1).all() and (got[:, 2:] == np.flatnonzero(np.arange(40) % 4)).all()
+
+
+def test_index_whose_boxes_another_stream_builds(ctx):
+    # the first far walk of many queries builds the boxes that small query sets
+    # then take too, here on another stream and thread
+    rng = np.random.default_rng(2)
+    P, _ = shapes.sphere(30_000, 4)
+    P = (0.5 * P).astype(np.float32)
+    far = rng.uniform(-1, 1, (100_000, 3)).astype(np.float32)
+    Q = rng.uniform(-1, 1, (500, 3)).astype(np.float32)
+    want, want_far = O.knn_brute(P, Q, 15), O.knn_brute(P, far[:300], 15)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        other = gpu.Context(0)
+        q = torch.from_numpy(Q).cuda()
+    for _ in range(5):
+        index = gpu.KnnIndex(ctx, P, k_hint=15)
+        here = gpu.KnnIndex.__new__(gpu.KnnIndex)  # the same index by the other context
+        here.ctx, here.pts, here.n, here.h = other, index.pts, index.n, index.h
+        torch.cuda.synchronize()
+        got = []
+        walk = threading.Thread(target=lambda: got.append(index.query(far, 15)))
+        walk.start()
+        with torch.cuda.stream(stream):
+            small = [here.query(q, 15) for _ in range(20)]
+        walk.join()
+        torch.cuda.synchronize()
+        here.h = None
+        for s in small:
+            np.testing.assert_array_equal(s.cpu().numpy(), want)
+        np.testing.assert_array_equal(got[0].cpu().numpy()[:300], want_far)
+    other.close()
