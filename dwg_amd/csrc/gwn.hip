@@ -1377,11 +1377,29 @@ __global__ void order_scatter_kernel(const int2* __restrict__ place, int64_t nq,
     }
 }
 
+// Up to so many queries are put in order at a time, 12 B of scratch each: more are
+// taken in equal parts, so that what a context keeps for this stays below 204 MB
+// and a query's number in 32 bits
+constexpr int64_t kOrderMost = int64_t(1) << 24;
+
+static int64_t order_part(int64_t nq) {
+    const int64_t parts = (nq + kOrderMost - 1) / kOrderMost;
+    return ((nq + parts - 1) / parts + 63) / 64 * 64;
+}
+
+// the caller's order where there is no memory for another
 static QueryOrder query_order(dwg_ctx* ctx, const dwg_octree* T, const float* q, int64_t nq) {
-    DWG_REQUIRE(nq < (int64_t(1) << 31) - 1, "too many queries");
-    auto* start = static_cast<unsigned long long*>(ctx->buf("order_start", sizeof(uint64_t) * (kOrderBuckets + 2)));
-    int2* place = static_cast<int2*>(ctx->buf("order_place", sizeof(int2) * size_t(nq)));
-    int* order = static_cast<int*>(ctx->buf("order", sizeof(int) * size_t(nq)));
+    unsigned long long* start = nullptr;
+    int2* place = nullptr;
+    int* order = nullptr;
+    try {
+        start = static_cast<unsigned long long*>(ctx->buf("order_start", sizeof(uint64_t) * (kOrderBuckets + 2)));
+        place = static_cast<int2*>(ctx->buf("order_place", sizeof(int2) * size_t(nq)));
+        order = static_cast<int*>(ctx->buf("order", sizeof(int) * size_t(nq)));
+    } catch (const Error&) {
+        (void)hipGetLastError();
+        return QueryOrder{};
+    }
     auto* extent = reinterpret_cast<unsigned int*>(start + kOrderBuckets + 1);
     ProfileScope ps(ctx, "gwn_query_order");
     fill_u32(ctx, start, 0, 2 * (kOrderBuckets + 2));
@@ -1680,21 +1698,30 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
         check_launch();
         return;
     }
-    const int64_t waves = Q.grid ? Q.n_bricks : (Q.nq + 64 * kPointPts - 1) / (64 * kPointPts);
-    if (waves == 0) return;
     TreeArgs A{T->info, T->kid, T->cm_r, reinterpret_cast<const float*>(T->payload), T->sa, T->sb};
-    dim3 grid(grid_for(waves, kTreeWaves)), block(kTreeThreads);
-    // the walk's stack: one record and one lane mask per part for each entry
-    QueryArgs Qs = Q;
-    Qs.stack = tree_stack_entries(std::max(T->max_level, 1));
-    if (Q.q && Q.nq >= kShareValue) Qs.order = query_order(ctx, T, Q.q, Q.nq);
-    const size_t lds = sizeof(uint64_t) * size_t(Qs.stack) * size_t(1 + (Q.grid ? Q.parts : kPointPts));
     const bool scr = flags & DWG_SCREENED, bf = flags & DWG_FAR_BF16;
     const char* name = count ? "gwn_tree_terms" : (!Q.grid ? (scr ? "gwn_tree_screened" : "gwn_tree_plain")
                                                            : (scr ? "gwn_tree_grid_screened" : "gwn_tree_grid_plain"));
-    ProfileScope ps(ctx, name);
+    // explicit points are put in order first, a part of them at a time
+    const bool in_order = Q.q && Q.nq >= kShareValue;
+    const int64_t part = in_order ? order_part(Q.nq) : Q.nq;
+    for (int64_t first = 0; first < Q.nq; first += part) {
+        QueryArgs Qs = Q;
+        float* o = out ? out + first : nullptr;
+        int64_t* t = terms ? terms + first : nullptr;
+        if (in_order) {
+            Qs.q = Q.q + 3 * first;
+            Qs.nq = std::min(part, Q.nq - first);
+            Qs.order = query_order(ctx, T, Qs.q, Qs.nq);
+        }
+        const int64_t waves = Q.grid ? Q.n_bricks : (Qs.nq + 64 * kPointPts - 1) / (64 * kPointPts);
+        dim3 grid(grid_for(waves, kTreeWaves)), block(kTreeThreads);
+        // the walk's stack: one record and one lane mask per part for each entry
+        Qs.stack = tree_stack_entries(std::max(T->max_level, 1));
+        const size_t lds = sizeof(uint64_t) * size_t(Qs.stack) * size_t(1 + (Q.grid ? Q.parts : kPointPts));
+        ProfileScope ps(ctx, name);
 #define DWG_TREE_LAUNCH(S, C, B, G, N) \
-    hipLaunchKernelGGL((gwn_tree_kernel<S, C, B, G, N>), grid, block, lds, ctx->stream, A, Qs, beta, sigma, flags, out, terms)
+    hipLaunchKernelGGL((gwn_tree_kernel<S, C, B, G, N>), grid, block, lds, ctx->stream, A, Qs, beta, sigma, flags, o, t)
 #define DWG_TREE_LAUNCH_Q(S, C, B, N)                \
     do {                                             \
         if (!Q.grid)                                 \
@@ -1710,17 +1737,18 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
         else                                    \
             DWG_TREE_LAUNCH_Q(S, false, B, false);  \
     } while (0)
-    if (count) DWG_TREE_LAUNCH_Q(false, true, false, false);
-    else if (near64 && bf) DWG_TREE_LAUNCH_Q(true, false, true, true);
-    else if (near64) DWG_TREE_LAUNCH_Q(true, false, false, true);
-    else if (scr && bf) DWG_TREE_LAUNCH_P(true, true);
-    else if (scr) DWG_TREE_LAUNCH_P(true, false);
-    else if (bf) DWG_TREE_LAUNCH_P(false, true);
-    else DWG_TREE_LAUNCH_P(false, false);
+        if (count) DWG_TREE_LAUNCH_Q(false, true, false, false);
+        else if (near64 && bf) DWG_TREE_LAUNCH_Q(true, false, true, true);
+        else if (near64) DWG_TREE_LAUNCH_Q(true, false, false, true);
+        else if (scr && bf) DWG_TREE_LAUNCH_P(true, true);
+        else if (scr) DWG_TREE_LAUNCH_P(true, false);
+        else if (bf) DWG_TREE_LAUNCH_P(false, true);
+        else DWG_TREE_LAUNCH_P(false, false);
 #undef DWG_TREE_LAUNCH_P
 #undef DWG_TREE_LAUNCH_Q
 #undef DWG_TREE_LAUNCH
-    check_launch();
+        check_launch();
+    }
 }
 
 void gwn_tree(dwg_ctx* ctx, const dwg_octree* T, const float* q, int64_t nq, float beta, float sigma, uint32_t flags,
@@ -1769,16 +1797,21 @@ void gwn_tree_grad(dwg_ctx* ctx, const dwg_octree* Tc, const float* q, int64_t n
         launch_walk<true>(ctx, T, q, nq, sigma, flags, out_w, out_g);
         return;
     }
-    const QueryOrder order = query_order(ctx, T, q, nq);
     TreeArgs A{T->info, T->kid, T->cm_r, reinterpret_cast<const float*>(T->payload), T->sa, T->sb};
-    dim3 grid(grid_for((nq + 63) / 64, kTreeWaves)), block(kTreeThreads);
-    ProfileScope ps(ctx, "gwn_tree_grad");
-    if (flags & DWG_SCREENED)
-        hipLaunchKernelGGL(gwn_tree_grad_kernel<true>, grid, block, 0, ctx->stream, A, q, nq, order, sigma, out_w, out_g);
-    else
-        hipLaunchKernelGGL(gwn_tree_grad_kernel<false>, grid, block, 0, ctx->stream, A, q, nq, order, sigma, out_w,
-                           out_g);
-    check_launch();
+    const int64_t part = order_part(nq);
+    for (int64_t first = 0; first < nq; first += part) {
+        const int64_t n = std::min(part, nq - first);
+        const float* qs = q + 3 * first;
+        float *w = out_w + first, *g = out_g ? out_g + 3 * first : nullptr;
+        const QueryOrder order = query_order(ctx, T, qs, n);
+        dim3 grid(grid_for((n + 63) / 64, kTreeWaves)), block(kTreeThreads);
+        ProfileScope ps(ctx, "gwn_tree_grad");
+        if (flags & DWG_SCREENED)
+            hipLaunchKernelGGL(gwn_tree_grad_kernel<true>, grid, block, 0, ctx->stream, A, qs, n, order, sigma, w, g);
+        else
+            hipLaunchKernelGGL(gwn_tree_grad_kernel<false>, grid, block, 0, ctx->stream, A, qs, n, order, sigma, w, g);
+        check_launch();
+    }
 }
 
 void gwn_tree_terms(dwg_ctx* ctx, const dwg_octree* T, const float* q, int64_t nq, float beta, int64_t* terms) {

@@ -1,6 +1,7 @@
 """Inputs at the edges of what the entry points take: far queries, queries next
 to sources, values that are no numbers, radii below zero, more queries than 32
 bits count, calls recorded into a graph."""
+import ctypes
 import threading
 
 import numpy as np
@@ -243,3 +244,50 @@ def test_index_whose_boxes_another_stream_builds(ctx):
             np.testing.assert_array_equal(s.cpu().numpy(), want)
         np.testing.assert_array_equal(got[0].cpu().numpy()[:300], want_far)
     other.close()
+
+
+def test_more_queries_than_32_bits_count(ctx):
+    # all but a few at one place; the sums at the others, and beside them, are
+    # those of a call with few queries
+    nq = 2 ** 31 + 77
+    if torch.cuda.mem_get_info()[0] < 16 * nq + 2 ** 32:
+        pytest.skip("the queries and their sums take 35 GB")
+    P, N = shapes.sphere(3, 4)
+    tree = gpu.Octree(ctx, P.astype(np.float64), None, max_depth=4)
+    tree.update(N, np.full(3, 1e-3, np.float32))
+    Q = torch.zeros((nq, 3), device="cuda")
+    at = torch.tensor([0, 5, 2 ** 24 - 1, 2 ** 24, 2 ** 31 - 1, 2 ** 31, nq - 1], device="cuda")
+    Q[at] = torch.rand((len(at), 3), device="cuda")
+    at = torch.cat([at, at[1:] - 2])
+    few = Q[at].repeat(30_000, 1)  # enough to share walks as the many do
+    want = tree.eval(few, 2.3, sigma=SIGMA)[:len(at)].clone()
+    got = tree.eval(Q, 2.3, sigma=SIGMA)
+    assert torch.equal(got[at], want)
+    del got
+    want, wantg = (t[:len(at)].clone() for t in tree.eval_grad(few[:786_500], 2.3, sigma=SIGMA))
+    w = torch.empty(nq, device="cuda")
+    ctx.check(ctx.L.dwg_gwn_tree_grad(ctx.h, tree.h, ctypes.c_void_p(Q.data_ptr()), nq, 2.3, SIGMA, 1,
+                                      ctypes.c_void_p(w.data_ptr()), None))
+    ok = (w[at] - want).abs() <= 1e-5 * want.abs().max()
+    assert bool(ok.all())
+    del w, Q, few
+    torch.cuda.empty_cache()
+
+
+def test_scratch_of_many_queries_is_bounded():
+    c = gpu.Context(0)
+    P, N = shapes.sphere(100, 4)
+    tree = gpu.Octree(c, P.astype(np.float64), None, max_depth=6)
+    tree.update(N, np.full(100, 1e-3, np.float32))
+    Q = torch.rand((40_000_000, 3), device="cuda")
+    out = torch.empty(len(Q), device="cuda")
+    tree.eval(Q[:300_000], 2.3, sigma=SIGMA, out=out)
+    gpu.cache_release()
+    before = torch.cuda.mem_get_info()[0]
+    tree.eval(Q, 2.3, sigma=SIGMA, out=out)
+    torch.cuda.synchronize()
+    assert before - torch.cuda.mem_get_info()[0] <= 256 << 20
+    want = tree.eval(Q[-200_000:], 2.3, sigma=SIGMA)
+    assert torch.equal(out[-200_000:], want)
+    del tree
+    c.close()
