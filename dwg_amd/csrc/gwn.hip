@@ -1314,10 +1314,28 @@ constexpr int64_t kWalkFew = 40000, kShareValue = 196608, kShareGrad = 786432;
 // sample of runs of 64 decides: they come unsorted when such runs extend, on
 // average, over twice the side that 64 of nq uniform points fill.  (32³ and 128³
 // cells: 300,000 points over 400,000 sources 417 and 427 µs against 394 with 64³,
-// 1M points 690 and 611 against 602.  Points in order pay 20 to 25 µs for the
-// passes that find it out: 500,000 over 500,000 sources 404 → 427.)
+// 1M points 690 and 611 against 602.)  Queries in order pay for the launches that
+// find it out, which are four for that reason: 8 to 10 µs (200,000 over 3,000 sources 66
+// → 75, 800,000 over 400,000 446 → 455; with six launches 84 and 464).  The extent of
+// each wave's own queries would cost them nothing, but then unordered ones could
+// only walk alone
 constexpr int kOrderBits = 6, kOrderBuckets = 1 << (3 * kOrderBits);
-constexpr int kOrderSamples = 256;
+constexpr int kOrderSamples = 256;  // runs, one a block of the first launch
+constexpr int kOrderThreads = 256;
+static_assert(kOrderSamples == kOrderThreads, "a block adds up the samples, one a thread");
+
+// 12 B of scratch a query, and up to so many queries at a time: more are taken in
+// equal parts, so that the scratch a context keeps for this stays below 204 MB
+// and a query's number in 32 bits
+constexpr int64_t kOrderMost = int64_t(1) << 24;
+
+struct OrderCells {
+    uint32_t count[kOrderBuckets];  // queries of a bucket
+    uint32_t start[kOrderBuckets];  // queries before a bucket
+    uint32_t sample[kOrderSamples]; // extent of a run relative to the cube, in 2^-16
+    uint32_t extent;                // their sum
+};
+constexpr int kOrderZero = kOrderBuckets / kOrderSamples;  // counts that a block of the first launch clears
 
 __device__ __forceinline__ float wave_min(float v) {
 #pragma unroll
@@ -1325,12 +1343,12 @@ __device__ __forceinline__ float wave_min(float v) {
     return v;
 }
 
-// extent of sampled runs relative to the cube, in 2^-16, summed into *total
-__global__ __launch_bounds__(64) void order_sample_kernel(const float* __restrict__ q, int64_t nq,
-                                                          const double4* __restrict__ cell,
-                                                          unsigned int* __restrict__ total) {
-    const int64_t runs = nq / 64;
-    const int64_t i = int64_t(blockIdx.x) * runs / gridDim.x * 64 + threadIdx.x;  // nq ≥ 64
+__global__ __launch_bounds__(kOrderThreads) void order_sample_kernel(const float* __restrict__ q, int64_t nq,
+                                                                     const double4* __restrict__ cell,
+                                                                     OrderCells* __restrict__ C) {
+    for (int k = threadIdx.x; k < kOrderZero; k += kOrderThreads) C->count[blockIdx.x * kOrderZero + k] = 0;
+    if (threadIdx.x >= 64) return;
+    const int64_t i = int64_t(blockIdx.x) * (nq / 64) / kOrderSamples * 64 + threadIdx.x;  // nq ≥ 64
     float e = 0.f;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -1338,7 +1356,7 @@ __global__ __launch_bounds__(64) void order_sample_kernel(const float* __restric
         e = fmaxf(e, -wave_min(-v) - wave_min(v));
     }
     const float w = float(cell[0].w);
-    if (threadIdx.x == 0) atomicAdd(total, (unsigned int)(65536.f * fminf(fmaxf(e / w, 0.f), 1.f)));
+    if (threadIdx.x == 0) C->sample[blockIdx.x] = uint32_t(65536.f * fminf(fmaxf(e / w, 0.f), 1.f));
 }
 
 __device__ __forceinline__ int order_bucket(const float* __restrict__ q, int64_t i, const double4 c) {
@@ -1355,65 +1373,110 @@ __device__ __forceinline__ int order_bucket(const float* __restrict__ q, int64_t
     return m;
 }
 
+// the sum of v over the block's NT threads
+template <int NT>
+__device__ __forceinline__ uint32_t block_sum(uint32_t v) {
+    __shared__ uint32_t s_wave[NT / 64];
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) v += uint32_t(__shfl_xor(int(v), off, 64));
+    if ((threadIdx.x & 63) == 0) s_wave[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = 0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) v += s_wave[w];
+    return v;
+}
+
 // (bucket, place in it) of every query: the scatter then needs no atomics
-__global__ void order_count_kernel(const float* __restrict__ q, int64_t nq, const double4* __restrict__ cell,
-                                   QueryOrder O, int2* __restrict__ place, unsigned long long* __restrict__ count) {
-    if (!O.sorted()) return;
+__global__ __launch_bounds__(kOrderThreads) void order_count_kernel(const float* __restrict__ q, int64_t nq,
+                                                                    const double4* __restrict__ cell, unsigned limit,
+                                                                    OrderCells* __restrict__ C,
+                                                                    int2* __restrict__ place) {
+    const uint32_t extent = block_sum<kOrderThreads>(C->sample[threadIdx.x]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) C->extent = extent;
+    if (extent <= limit) return;
     const double4 root = cell[0];
-    for (int64_t i0 = int64_t(blockIdx.x) * blockDim.x; i0 < nq; i0 += int64_t(gridDim.x) * blockDim.x) {
+    for (int64_t i0 = int64_t(blockIdx.x) * kOrderThreads; i0 < nq; i0 += int64_t(gridDim.x) * kOrderThreads) {
         const int64_t i = i0 + threadIdx.x;
         const int b = i < nq ? order_bucket(q, i, root) : -1;
-        const int at = take_place(b, count);
+        const int at = take_place(b, C->count);
         if (i < nq) place[i] = make_int2(b, at);
     }
 }
 
-__global__ void order_scatter_kernel(const int2* __restrict__ place, int64_t nq, QueryOrder O,
-                                     const unsigned long long* __restrict__ start, int* __restrict__ order) {
+// The buckets' starts: a block takes a tile of them, four a thread, and adds up all
+// counts before its own, 1 MB at most and from L2, in place of a launch that does
+constexpr int kStartThreads = 1024, kStartTile = 4 * kStartThreads;
+__global__ __launch_bounds__(kStartThreads) void order_start_kernel(QueryOrder O, OrderCells* __restrict__ C) {
     if (!O.sorted()) return;
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < nq; i += int64_t(gridDim.x) * blockDim.x) {
+    const uint4* count = reinterpret_cast<const uint4*>(C->count);
+    const int tile = blockIdx.x * kStartThreads;  // in fours
+    uint32_t before = 0;
+#pragma unroll 8
+    for (int k = threadIdx.x; k < tile; k += kStartThreads) {
+        const uint4 c = count[k];
+        before += (c.x + c.y) + (c.z + c.w);
+    }
+    before = block_sum<kStartThreads>(before);
+    const uint4 c = count[tile + threadIdx.x];
+    const uint32_t sum = (c.x + c.y) + (c.z + c.w);
+    __shared__ uint32_t s_scan[kStartThreads / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t incl = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = uint32_t(__shfl_up(int(incl), off, 64));
+        incl += lane >= off ? y : 0;
+    }
+    if (lane == 63) s_scan[wave] = incl;
+    __syncthreads();
+    uint32_t at = before + incl - sum;
+#pragma unroll
+    for (int w = 0; w < kStartThreads / 64; ++w) at += w < wave ? s_scan[w] : 0;
+    reinterpret_cast<uint4*>(C->start)[tile + threadIdx.x] = make_uint4(at, at + c.x, at + c.x + c.y, at + c.x + c.y + c.z);
+}
+
+__global__ __launch_bounds__(kOrderThreads) void order_scatter_kernel(const int2* __restrict__ place, int64_t nq,
+                                                                      QueryOrder O, const OrderCells* __restrict__ C,
+                                                                      int* __restrict__ order) {
+    if (!O.sorted()) return;
+    for (int64_t i = int64_t(blockIdx.x) * kOrderThreads + threadIdx.x; i < nq;
+         i += int64_t(gridDim.x) * kOrderThreads) {
         const int2 b = place[i];
-        order[start[b.x] + b.y] = int(i);
+        order[C->start[b.x] + b.y] = int(i);
     }
 }
 
-// Up to so many queries are put in order at a time, 12 B of scratch each: more are
-// taken in equal parts, so that what a context keeps for this stays below 204 MB
-// and a query's number in 32 bits
-constexpr int64_t kOrderMost = int64_t(1) << 24;
-
+// The queries of one launch that shares walks, and where there is no memory to
+// order them the caller's order
 static int64_t order_part(int64_t nq) {
     const int64_t parts = (nq + kOrderMost - 1) / kOrderMost;
     return ((nq + parts - 1) / parts + 63) / 64 * 64;
 }
 
-// the caller's order where there is no memory for another
 static QueryOrder query_order(dwg_ctx* ctx, const dwg_octree* T, const float* q, int64_t nq) {
-    unsigned long long* start = nullptr;
+    OrderCells* C = nullptr;
     int2* place = nullptr;
     int* order = nullptr;
     try {
-        start = static_cast<unsigned long long*>(ctx->buf("order_start", sizeof(uint64_t) * (kOrderBuckets + 2)));
+        C = static_cast<OrderCells*>(ctx->buf("order_cells", sizeof(OrderCells)));
         place = static_cast<int2*>(ctx->buf("order_place", sizeof(int2) * size_t(nq)));
         order = static_cast<int*>(ctx->buf("order", sizeof(int) * size_t(nq)));
     } catch (const Error&) {
         (void)hipGetLastError();
         return QueryOrder{};
     }
-    auto* extent = reinterpret_cast<unsigned int*>(start + kOrderBuckets + 1);
     ProfileScope ps(ctx, "gwn_query_order");
-    fill_u32(ctx, start, 0, 2 * (kOrderBuckets + 2));
-    const int samples = int(std::min<int64_t>(nq / 64, kOrderSamples));
-    hipLaunchKernelGGL(order_sample_kernel, dim3(samples), dim3(64), 0, ctx->stream, q, nq, T->cell, extent);
+    const QueryOrder O{order, &C->extent, unsigned(65536.f * 2.f * std::cbrt(64.f / float(nq)) * float(kOrderSamples))};
+    hipLaunchKernelGGL(order_sample_kernel, dim3(kOrderSamples), dim3(kOrderThreads), 0, ctx->stream, q, nq, T->cell, C);
     check_launch();
-    const QueryOrder O{order, extent, unsigned(65536.f * 2.f * std::cbrt(64.f / float(nq)) * float(samples))};
-    const unsigned blocks = std::min(grid_for(nq, 256), 2048u);
-    hipLaunchKernelGGL(order_count_kernel, dim3(blocks), dim3(256), 0, ctx->stream, q, nq, T->cell, O, place,
-                       start);
+    const unsigned blocks = std::min(grid_for(nq, kOrderThreads), 1024u);
+    hipLaunchKernelGGL(order_count_kernel, dim3(blocks), dim3(kOrderThreads), 0, ctx->stream, q, nq, T->cell, O.limit, C,
+                       place);
     check_launch();
-    exclusive_scan_i64(ctx, reinterpret_cast<int64_t*>(start), kOrderBuckets);
-    hipLaunchKernelGGL(order_scatter_kernel, dim3(blocks), dim3(256), 0, ctx->stream, place, nq, O, start,
-                       order);
+    hipLaunchKernelGGL(order_start_kernel, dim3(kOrderBuckets / kStartTile), dim3(kStartThreads), 0, ctx->stream, O, C);
+    check_launch();
+    hipLaunchKernelGGL(order_scatter_kernel, dim3(blocks), dim3(kOrderThreads), 0, ctx->stream, place, nq, O, C, order);
     check_launch();
     return O;
 }
