@@ -1027,9 +1027,14 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
                 ++sp;
             }
         }
+        if (full && kahan) {  // every lane with a point opened it: no masks to go by
 #pragma unroll
-        for (int h = 0; h < H; ++h)
-            if (H == 1 || mask[h]) add(part[h], h, mask[h]);
+            for (int h = 0; h < H; ++h) kahan_add(sum[h], comp[h], part[h]);
+        } else {
+#pragma unroll
+            for (int h = 0; h < H; ++h)
+                if (H == 1 || mask[h]) add(part[h], h, mask[h]);
+        }
     }
 #pragma unroll
     for (int h = 0; h < H; ++h) {
