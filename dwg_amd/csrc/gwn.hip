@@ -1307,12 +1307,25 @@ __global__ __launch_bounds__(kWalkWaves * 64) void gwn_ordered_walk_kernel(TreeA
 // Which walk explicit queries take.  Alone (gwn_walk_kernel), 64 lanes a query
 // below kWalkFew, where the waves do not fill the chip (1,000 of 100k sources:
 // 17 µs, with 8 lanes 48, shared 1,190), else 8 (32,000: 57 and 75 against
-// 1,380 µs; 100,000 with gradient: 0.17 against 2.5 ms).  From kShareValue on
-// (kShareGrad with the gradient) 64 to a shared walk, in spatial order: the
-// node records are then read once for 64 queries, which for 1M queries on the
-// surface takes half the time, while unordered ones (2M: 12.8 ms shared, 3.3 ms
-// alone) are put in order first
-constexpr int64_t kWalkFew = 40000, kShareValue = 196608, kShareGrad = 786432;
+// 1,380 µs; 100,000 with gradient: 0.17 against 2.5 ms).  From share_from on 64 to
+// a shared walk, in spatial order: the node records are then read once for 64
+// queries, which for 1M queries on the surface takes half the time, while unordered
+// ones (2M: 12.8 ms shared, 3.3 ms alone) are put in order first.
+constexpr int64_t kWalkFew = 40000;
+
+// A launch of shared walks lasts as long as its longest, which grow with the
+// tree, and lone walks cost the same for each query: sharing pays from a number of
+// queries on that grows with the sources.  Of queries in order and unordered
+// ones, near a surface, alone and shared (µs): 3,000 sources 150,000 70, 76 and 77,
+// 97; 200,000 88, 99 and 75, 104.  400,000 sources 200,000 246, 363 and 352, 378;
+// 300,000 336, 482 and 359, 368.  With gradient 3,000 sources 200,000 101, 113 and
+// 115, 150; 300,000 144, 160 and 132, 165.  30,000 sources 300,000 251, 289 and 276,
+// 340; 500,000 395, 467 and 322, 400.  1M sources 500,000 700, 962 and 920, 975;
+// 800,000 1,089, 1,479 and 1,156, 1,238
+static int64_t share_from(const dwg_octree* T, bool grad) {
+    const double n = double(T->n_points);
+    return int64_t(grad ? 62000.0 * std::pow(n, 1.0 / 6.0) : 82000.0 * std::pow(n, 1.0 / 12.0));
+}
 
 // The order: a counting sort by the Morton code of a 64³ grid over the tree's
 // cube.  Queries that come in order already are left as they are, which a
@@ -1739,7 +1752,7 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
         T->payload_bf16 = want_bf16;
     }
     const bool near64 = (flags & DWG_SCREENED) && (flags & DWG_NEAR_FP64);
-    if (Q.q && !count && !near64 && Q.nq < kShareValue) {
+    if (Q.q && !count && !near64 && Q.nq < share_from(T, false)) {
         if (Q.nq == 0) return;
         ProfileScope ps(ctx, (flags & DWG_SCREENED) ? "gwn_tree_screened" : "gwn_tree_plain");
         launch_walk<false>(ctx, T, Q.q, Q.nq, sigma, flags, out, nullptr);
@@ -1771,7 +1784,7 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
     const char* name = count ? "gwn_tree_terms" : (!Q.grid ? (scr ? "gwn_tree_screened" : "gwn_tree_plain")
                                                            : (scr ? "gwn_tree_grid_screened" : "gwn_tree_grid_plain"));
     // explicit points are put in order first, a part of them at a time
-    const bool in_order = Q.q && Q.nq >= kShareValue;
+    const bool in_order = Q.q && Q.nq >= share_from(T, false);
     const int64_t part = in_order ? order_part(Q.nq) : Q.nq;
     for (int64_t first = 0; first < Q.nq; first += part) {
         QueryArgs Qs = Q;
@@ -1860,7 +1873,7 @@ void gwn_tree_grad(dwg_ctx* ctx, const dwg_octree* Tc, const float* q, int64_t n
         T->payload_bf16 = false;
     }
     if (nq == 0) return;
-    if (nq < kShareGrad) {
+    if (nq < share_from(T, true)) {
         ProfileScope ps(ctx, "gwn_tree_grad");
         launch_walk<true>(ctx, T, q, nq, sigma, flags, out_w, out_g);
         return;

@@ -133,6 +133,30 @@ def test_screened_tree_gradient_of_a_query_that_is_no_number(ctx, nq):
     assert torch.equal(w, w0) and torch.equal(g, g0)
 
 
+@pytest.mark.parametrize("n", [1, 60, 3000, 100_000])
+@pytest.mark.parametrize("grad", [False, True])
+def test_points_share_walks_by_the_size_of_the_tree(ctx, n, grad):
+    # the last number of points that walk alone and the first that share walks,
+    # in order and not: each the sums of few points, by a walk of 64 lanes
+    P, N = shapes.sphere(n, 7)
+    rng = np.random.default_rng(n)
+    tree = gpu.Octree(ctx, P.astype(np.float64), None, max_depth=10)
+    tree.update(N.astype(np.float32), np.full(n, 0.5 / n, np.float32))
+    first = int(62000 * n ** (1 / 6) if grad else 82000 * n ** (1 / 12))
+    Q = rng.uniform(-1.2, 1.2, (first + 1, 3)).astype(np.float32)
+    sub = rng.permutation(first - 1)[:2000]
+    few = tree.eval_grad(Q[sub], 2.3, sigma=SIGMA) if grad else (tree.eval(Q[sub], 2.3, sigma=SIGMA),)
+    for ordered in (False, True):
+        at = np.lexsort((Q * 20).astype(int).T) if ordered else np.arange(len(Q))
+        back = torch.from_numpy(np.argsort(at)[sub]).cuda()
+        for nq in (first - 1, first, first + 1):
+            q = torch.from_numpy(Q[at]).cuda()
+            keep = back < nq
+            got = tree.eval_grad(q[:nq], 2.3, sigma=SIGMA) if grad else (tree.eval(q[:nq], 2.3, sigma=SIGMA),)
+            for g, f, tol in zip(got, few, (1e-5, 1e-4)):  # the tree's bounds against FP64
+                assert (g[back[keep]] - f[keep]).abs().max() <= tol * f.abs().max()
+
+
 @pytest.mark.parametrize("res,h", [((8, 4, 8), 0.05), ((33, 29, 31), 0.08), ((51, 53, 55), 0.02), ((401, 399, 1), 0.003),
                                    ((190, 181, 183), 0.005), ((195, 191, 185), 0.005)])
 @pytest.mark.parametrize("screened,bf16,radii", [(True, False, False), (True, True, True), (False, False, False),
