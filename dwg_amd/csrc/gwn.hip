@@ -465,9 +465,9 @@ void gwn_direct(dwg_ctx* ctx, const float* pts, const float* nrm, const float* a
     if (nq == 0) return;
     float4* sa = static_cast<float4*>(ctx->buf("direct_sa", sizeof(float4) * (n + 1)));
     float4* sb = static_cast<float4*>(ctx->buf("direct_sb", sizeof(float4) * (n + 1)));
-    double* part = direct_splits(n, nq, out_g ? 4 : 1) > 1
-                       ? static_cast<double*>(ctx->buf("direct_part", sizeof(double) * kDirectPartials))
-                       : nullptr;
+    // (also where this call does not split: one of the same sources that does may be
+    // recorded into a graph next, and can allocate nothing)
+    double* part = static_cast<double*>(ctx->buf("direct_part", sizeof(double) * kDirectPartials));
     direct_sums(ctx, sa, sb, part, pts, nrm, area, radii, n, q, nq, sigma, flags, out_w, out_g, true);
 }
 
@@ -1465,13 +1465,23 @@ __global__ __launch_bounds__(kOrderThreads) void order_scatter_kernel(const int2
     }
 }
 
-// The queries of one launch that shares walks, and where there is no memory to
-// order them the caller's order
+// the queries of one launch that shares walks
 static int64_t order_part(int64_t nq) {
     const int64_t parts = (nq + kOrderMost - 1) / kOrderMost;
     return ((nq + parts - 1) / parts + 63) / 64 * 64;
 }
 
+// A call that is recorded into a graph takes its points as they come: the scratch
+// of an order could not be allocated, or given back by a later call while the graph
+// still used it
+static bool recording(const dwg_ctx* ctx) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
+// the caller's order where there is no memory for another
 static QueryOrder query_order(dwg_ctx* ctx, const dwg_octree* T, const float* q, int64_t nq) {
     OrderCells* C = nullptr;
     int2* place = nullptr;
@@ -1784,7 +1794,7 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
     const char* name = count ? "gwn_tree_terms" : (!Q.grid ? (scr ? "gwn_tree_screened" : "gwn_tree_plain")
                                                            : (scr ? "gwn_tree_grid_screened" : "gwn_tree_grid_plain"));
     // explicit points are put in order first, a part of them at a time
-    const bool in_order = Q.q && Q.nq >= share_from(T, false);
+    const bool in_order = Q.q && Q.nq >= share_from(T, false) && !recording(ctx);
     const int64_t part = in_order ? order_part(Q.nq) : Q.nq;
     for (int64_t first = 0; first < Q.nq; first += part) {
         QueryArgs Qs = Q;
@@ -1879,12 +1889,13 @@ void gwn_tree_grad(dwg_ctx* ctx, const dwg_octree* Tc, const float* q, int64_t n
         return;
     }
     TreeArgs A{T->info, T->kid, T->cm_r, reinterpret_cast<const float*>(T->payload), T->sa, T->sb};
-    const int64_t part = order_part(nq);
+    const bool in_order = !recording(ctx);
+    const int64_t part = in_order ? order_part(nq) : nq;
     for (int64_t first = 0; first < nq; first += part) {
         const int64_t n = std::min(part, nq - first);
         const float* qs = q + 3 * first;
         float *w = out_w + first, *g = out_g ? out_g + 3 * first : nullptr;
-        const QueryOrder order = query_order(ctx, T, qs, n);
+        const QueryOrder order = in_order ? query_order(ctx, T, qs, n) : QueryOrder{};
         dim3 grid(grid_for((n + 63) / 64, kTreeWaves)), block(kTreeThreads);
         ProfileScope ps(ctx, "gwn_tree_grad");
         if (flags & DWG_SCREENED)

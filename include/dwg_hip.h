@@ -150,7 +150,8 @@ int dwg_octree_set_point_areas(dwg_ctx* ctx, dwg_octree* tree, const float* d_nr
  * TurboLibiGWN.cu:912-922; plain: TurboLibiGWNLaunch :900-910).  Many points are
  * brought into spatial order first where they are not in one (these and the
  * gradient's), with 12 B of context scratch a point, 204 MB at most; where that
- * cannot be allocated they are taken as they come. */
+ * cannot be allocated, and in a call recorded into a graph, they are taken as they
+ * come. */
 int dwg_gwn_tree(dwg_ctx* ctx, const dwg_octree* tree, const float* d_q, int64_t nq, float beta,
                  float sigma, uint32_t flags, float* d_out);
 /* Value and gradient ∇_q w of the Barnes-Hut sums at nq query points (new;

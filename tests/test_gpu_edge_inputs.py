@@ -315,3 +315,56 @@ def test_scratch_of_many_queries_is_bounded():
     assert torch.equal(out[-200_000:], want)
     del tree
     c.close()
+
+
+@pytest.mark.parametrize("kind,nq", [("tree", 200_000), ("tree_grad", 786_500), ("direct", 1000)])
+def test_sums_recorded_into_a_graph(kind, nq):
+    # a recorded call takes no scratch that it has to allocate, and none that a
+    # later call may give back: replayed after other work it gives the eager sums
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        c = gpu.Context(0)
+        P, N = shapes.sphere(3000, 4)
+        A = np.full(len(P), 1e-3, np.float32)
+        P, N, A = (torch.from_numpy(a.astype(np.float32)).cuda() for a in (P, N, A))
+        tree = gpu.Octree(c, P.cpu().numpy().astype(np.float64), None, max_depth=8)
+        tree.update(N, A)
+        Q = torch.rand((nq, 3), device="cuda") * 2 - 1
+        more = torch.rand((4 * nq + 300_000, 3), device="cuda") * 2 - 1
+        w, g = torch.empty(nq, device="cuda"), torch.empty((nq, 3), device="cuda")
+        p = [ctypes.c_void_p(t.data_ptr()) for t in (P, N, A, Q, w, g)]
+
+        def call(q, n, ow, og):
+            if kind == "tree":
+                rc = c.L.dwg_gwn_tree(c.h, tree.h, q, n, 2.3, SIGMA, 1, ow)
+            elif kind == "tree_grad":
+                rc = c.L.dwg_gwn_tree_grad(c.h, tree.h, q, n, 2.3, SIGMA, 1, ow, og)
+            else:
+                rc = c.L.dwg_gwn_direct(c.h, p[0], p[1], p[2], None, len(P), q, n, SIGMA, 1, ow, og)
+            c.check(rc)
+
+        def eager(q):
+            ow, og = torch.empty(len(q), device="cuda"), torch.empty((len(q), 3), device="cuda")
+            call(*(ctypes.c_void_p(t.data_ptr()) for t in (q,)), len(q),
+                 *(ctypes.c_void_p(t.data_ptr()) for t in (ow, og)))
+            return ow, og
+
+        # the far radii of these flags, and the packed sources' buffers
+        eager(more[:100] if kind != "direct" else more)
+        s.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            call(p[3], nq, p[4], p[5])
+        for i in range(3):
+            Q.copy_(torch.rand((nq, 3), device="cuda") * 2 - 1)
+            eager(more[: (i + 1) * len(more) // 3])  # scratch grows
+            w.fill_(-1)
+            graph.replay()
+            s.synchronize()
+            ow, og = eager(Q)
+            assert torch.equal(w, ow)
+            if kind != "tree":
+                assert torch.equal(g, og)
+        s.synchronize()
+        del tree
+        c.close()
