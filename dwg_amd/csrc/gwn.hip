@@ -81,15 +81,13 @@ __device__ __forceinline__ float add_rounded(float part, float x, float inv) {
     return part + t;
 }
 
-// max(r², s²), and s² where r² is no number (an s² never is): written as the
-// instruction, as the compiler would first quiet a possible signalling NaN of s².
-// UNIFORM: s² is the same in every lane and in a scalar register
-template <bool UNIFORM>
+// max(r², s²), and s² where r² is no number (an s² never is): the median with ∞,
+// which is the least of the numbers among three.  (Of a constant ∞ the compiler makes
+// a maximum, and one more instruction that quiets a signalling NaN of s².)
 __device__ __forceinline__ float screened_r2(float r2, float s2) {
-    float m;
-    if constexpr (UNIFORM) asm("v_max_f32 %0, %1, %2" : "=v"(m) : "s"(s2), "v"(r2));
-    else asm("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(s2), "v"(r2));
-    return m;
+    float inf;
+    asm("v_mov_b32 %0, 0x7f800000" : "=v"(inf));
+    return __builtin_amdgcn_fmed3f(r2, s2, inf);
 }
 
 // The direct sums' point term as such factors, a = (p, ·), b = (A·n/4π, s²);
@@ -104,7 +102,7 @@ __device__ __forceinline__ float gwn_term_split(float qx, float qy, float qz, co
     const float r2 = dist2(dx, dy, dz);
     bool ok;
     if constexpr (!SCREENED) return tree_term_split<false>(dx, dy, dz, r2, 0.f, b, sigma, sigma_l2e, inv, ok);
-    const float x = tree_term_split<true>(dx, dy, dz, screened_r2<true>(r2, b.w), 0.f, b, sigma, sigma_l2e, inv, ok);
+    const float x = tree_term_split<true>(dx, dy, dz, screened_r2(r2, b.w), 0.f, b, sigma, sigma_l2e, inv, ok);
     return r2 > 1e-20f ? x : 0.f;
 }
 
@@ -141,8 +139,8 @@ __device__ __forceinline__ bool near_field(float r2, float s) { return r2 < s * 
 // round twice at the sum's size (half of 2,000 queries next to one of 20,000
 // sources: RMS error of ∇w 11 % and maximum 37 % more).
 // A screened term at the guard, or whose distance is no number, has only zeros
-// (d may still be no number).  UNIFORM as in screened_r2.
-template <bool SCREENED, bool UNIFORM>
+// (d may still be no number).
+template <bool SCREENED>
 __device__ __forceinline__ void gwn_term_grad(float dx, float dy, float dz, float s2, const float4 b, float sigma,
                                               float sigma_l2e, float& dot, float& g, float& c) {
     const float r2 = dist2(dx, dy, dz);
@@ -154,7 +152,7 @@ __device__ __forceinline__ void gwn_term_grad(float dx, float dy, float dz, floa
     } else {
         const bool ok = r2 > 1e-20f;
         dot = ok ? dot : 0.0f;
-        const float rho2 = screened_r2<UNIFORM>(r2, s2);
+        const float rho2 = screened_r2(r2, s2);
         const float rho = fast_sqrt(rho2), irho = fast_rsq(rho2);
         const float er2 = fast_exp2(sigma_l2e * rho) * rho2;
         const float eps = kEpsScreened * kInv4Pi;
@@ -251,7 +249,7 @@ __device__ __forceinline__ void direct_grad(const float4* __restrict__ sa, const
     auto term = [&](const float4 a, const float4 b) {
         const float dx = a.x - qx, dy = a.y - qy, dz = a.z - qz;
         float dot, g, c;
-        gwn_term_grad<SCREENED, true>(dx, dy, dz, b.w, b, sigma, sl2e, dot, g, c);
+        gwn_term_grad<SCREENED>(dx, dy, dz, b.w, b, sigma, sl2e, dot, g, c);
         p[0] = __builtin_fmaf(g, dot, p[0]);
         p[1] += grad_component(c, dx, g, b.x);
         p[2] += grad_component(c, dy, g, b.y);
@@ -1088,7 +1086,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void gwn_walk_kernel(TreeArgs T, c
     auto add = [&](float dx, float dy, float dz, float s2, const float4 b) {
         if constexpr (GRAD) {
             float dot, g, c;
-            gwn_term_grad<SCREENED, false>(dx, dy, dz, s2, b, sigma, sl2e, dot, g, c);
+            gwn_term_grad<SCREENED>(dx, dy, dz, s2, b, sigma, sl2e, dot, g, c);
             sum[0] += double(g * dot);
             sum[1] += double(grad_component(c, dx, g, b.x));
             sum[2] += double(grad_component(c, dy, g, b.y));
@@ -1569,7 +1567,7 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_grad_kernel(TreeArgs T,
     float acc[4] = {0.f, 0.f, 0.f, 0.f}, comp[4] = {0.f, 0.f, 0.f, 0.f}, part[4] = {0.f, 0.f, 0.f, 0.f};
     auto add = [&](float dx, float dy, float dz, float s2, const float4 b, bool on) {
         float dot, g, c;
-        gwn_term_grad<SCREENED, false>(dx, dy, dz, s2, b, sigma, sl2e, dot, g, c);
+        gwn_term_grad<SCREENED>(dx, dy, dz, s2, b, sigma, sl2e, dot, g, c);
         g = on ? g : 0.f;
         c = on ? c : 0.f;
         part[0] = __builtin_fmaf(g, dot, part[0]);
