@@ -237,8 +237,12 @@ __device__ __forceinline__ void direct_value(const float4* __restrict__ sa, cons
     if (KAHAN) kahan_add(sum, comp, part); else sum += part;
 }
 
-// the sources [j0, j1) summed at q, value and gradient: s − c for each
-template <bool SCREENED, bool KAHAN>
+// the sources [j0, j1) summed at q, value and gradient: s − c for each.  UNROLL
+// terms of a tile at a time: 2, and 1 for plain sums that are not split (857 sources at
+// 1M queries, plain: 474 µs by 1, 512 by 2, 525 by 4; 3,000 at 300,000 664, 667 and
+// 639, screened 1,072, 1,029 and 1,105; 200,000 at 2,000, split, 352, 317 and 332,
+// screened 499, 489 and 519)
+template <bool SCREENED, bool KAHAN, int UNROLL>
 __device__ __forceinline__ void direct_grad(const float4* __restrict__ sa, const float4* __restrict__ sb, int64_t j0,
                                             int64_t j1, float qx, float qy, float qz, float sigma, float (&s)[4],
                                             float (&c)[4]) {
@@ -265,9 +269,7 @@ __device__ __forceinline__ void direct_grad(const float4* __restrict__ sa, const
 #pragma unroll
     for (int k = 0; k < 4; ++k) p[k] = 0.f;
     for (; j0 + kDirectTile <= j1; j0 += kDirectTile) {
-        // (857 sources at 1M queries, plain: 0.56 ms unrolled by 4, 0.53 by 2; 3,000
-        // at 300,000: 0.64 and 0.66; 200,000 at 2,000, screened: 0.52 and 0.51)
-#pragma unroll 2
+#pragma unroll UNROLL
         for (int j = 0; j < kDirectTile; ++j) term(sa[j0 + j], sb[j0 + j]);
         fold();
     }
@@ -298,7 +300,7 @@ __global__ __launch_bounds__(kDirectThreads) void gwn_direct_grad_kernel(
     const bool valid = i < nq;
     const float qx = valid ? q[3 * i] : 0.f, qy = valid ? q[3 * i + 1] : 0.f, qz = valid ? q[3 * i + 2] : 0.f;
     float s[4], c[4];
-    direct_grad<SCREENED, KAHAN>(sa, sb, 0, n, qx, qy, qz, sigma, s, c);
+    direct_grad<SCREENED, KAHAN, SCREENED ? 2 : 1>(sa, sb, 0, n, qx, qy, qz, sigma, s, c);
     if (valid) {
         out_w[i] = s[0] - c[0];
         out_g[3 * i] = s[1] - c[1];
@@ -340,7 +342,7 @@ __global__ __launch_bounds__(64) void gwn_direct_grad_split_kernel(const float4*
     const float qx = valid ? q[3 * i] : 0.f, qy = valid ? q[3 * i + 1] : 0.f, qz = valid ? q[3 * i + 2] : 0.f;
     const int64_t j0 = int64_t(blockIdx.y) * run, j1 = j0 + run < n ? j0 + run : n;
     float s[4], c[4];
-    direct_grad<SCREENED, KAHAN>(sa, sb, j0, j1, qx, qy, qz, sigma, s, c);
+    direct_grad<SCREENED, KAHAN, 2>(sa, sb, j0, j1, qx, qy, qz, sigma, s, c);
     if (valid) {
         double* o = part + int64_t(blockIdx.y) * 4 * nq;
 #pragma unroll
