@@ -533,7 +533,6 @@ dwg_octree::~dwg_octree() {
 
 namespace dwg {
 
-// EC/4π per node (FP64 prefix-sum difference, one rounding), into ec and
 // A leaf with one point is walked like a far dipole: its traversal record
 // holds the point (x, y, z), its payload the point's (A·n/4π, s²) and a zero
 // residual, so the walk reads the same words for both and evaluates the
@@ -550,8 +549,9 @@ __device__ __forceinline__ void write_point_leaf(int64_t i, const float4 a, cons
     cm_r[i].z = a.z;
 }
 
-// the node payload: words 0-3 of an internal node (EC/4π, s²); a leaf with
-// one point carries that point's term instead (write_point_leaf)
+// EC/4π per node (FP64 prefix-sum difference, one rounding), into ec and the node
+// payload: words 0-3 of an internal node (EC/4π, s²); a leaf with one point carries
+// that point's term instead (write_point_leaf)
 __global__ void node_ec_kernel(const int4* __restrict__ info, const Double3* __restrict__ scan, int64_t m,
                                const float4* __restrict__ sa, const float4* __restrict__ sb,
                                float4* __restrict__ ec, float4* __restrict__ payload, float4* __restrict__ cm_r) {

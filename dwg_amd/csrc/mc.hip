@@ -32,7 +32,6 @@ constexpr int kMcThreads = 256;
 struct McArgs {
     const float* f;
     int rx, ry, rz;
-    int64_t ncubes;
     float ox, oy, oz, h, iso;
 };
 
@@ -430,8 +429,7 @@ __global__ __launch_bounds__(kRunWaves * 64) void mc_fused_kernel(McArgs A, McBr
 
 static McArgs mc_args(const float* field, const dwg_grid* g, float iso, McBricks& B, int64_t& tiles) {
     DWG_REQUIRE(g && g->res[0] >= 2 && g->res[1] >= 2 && g->res[2] >= 2, "grid needs at least 2 samples per axis");
-    McArgs A{field, g->res[0], g->res[1], g->res[2], 0, g->origin[0], g->origin[1], g->origin[2], g->h, iso};
-    A.ncubes = int64_t(A.rx - 1) * (A.ry - 1) * (A.rz - 1);
+    const McArgs A{field, g->res[0], g->res[1], g->res[2], g->origin[0], g->origin[1], g->origin[2], g->h, iso};
     B = McBricks{(A.rx - 1 + kBx - 1) / kBx, (A.ry - 1 + kBy - 1) / kBy, (A.rz - 1 + kBz - 1) / kBz};
     tiles = int64_t(B.nbx) * B.nby * B.nbz;
     DWG_REQUIRE(tiles < (int64_t(1) << 31), "grid too large for the marching-cubes launch");

@@ -145,7 +145,6 @@ struct GemmArgs {
     float* C;
     int64_t sCi, sCj;
     int64_t M, N, K;
-    int accumulate;
 };
 
 // Lane layout of v_mfma_f32_32x32x16_bf16 (one wave, 32×32 += 32×16 · 16×32):
@@ -178,10 +177,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g, int64_t tile
     for (int r = 0; r < 16; ++r) {
         const int64_t i = ti * 32 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4);
         const int64_t j = tj * 32 + (lane & 31);
-        if (i < g.M && j < g.N) {
-            float* c = g.C + i * g.sCi + j * g.sCj;
-            *c = g.accumulate ? *c + acc[r] : acc[r];
-        }
+        if (i < g.M && j < g.N) g.C[i * g.sCi + j * g.sCj] = acc[r];
     }
 }
 
@@ -838,7 +834,7 @@ void mlp_init(dwg_ctx* ctx, const dwg_mlp* m, const float* p, int64_t n, const f
 
 void gemm_bf16_test(dwg_ctx* ctx, const uint16_t* A, int64_t sAi, int64_t sAk, const uint16_t* B, int64_t sBk,
                     int64_t sBj, float* C, int64_t M, int64_t N, int64_t K) {
-    gemm(ctx, {A, sAi, sAk, B, sBk, sBj, C, N, 1, M, N, K, 0});
+    gemm(ctx, {A, sAi, sAk, B, sBk, sBj, C, N, 1, M, N, K});
 }
 
 }  // namespace dwg

@@ -249,7 +249,7 @@ void radix_sort_pairs(dwg_ctx* ctx, const uint64_t* kin, const int* vin, uint64_
 }
 
 // Up to this many tiles (8M numbers) a block adds up the tiles before its own
-// itself, 64 kB at most and from L2: one launch of three, 4.5 µs back to back,
+// itself, 32 kB at most and from L2: one launch of three, 4.5 µs back to back,
 // is gone.  Beyond, these reads would grow with the square of the tiles.
 // Sums of FP64 keep the scan of the tiles, whose order of adding stays.
 constexpr int64_t kScanSums = 4096;

@@ -162,8 +162,8 @@ int dwg_gwn_tree(dwg_ctx* ctx, const dwg_octree* tree, const float* d_q, int64_t
  * d_out_grad (nq×3) may be NULL. */
 int dwg_gwn_tree_grad(dwg_ctx* ctx, const dwg_octree* tree, const float* d_q, int64_t nq, float beta,
                       float sigma, uint32_t flags, float* d_out_w, float* d_out_grad);
-/* The same sums at the octree's own points, evaluated in tree order (one
- * wave per 64 consecutive tree slots) and written in the caller's point order
+/* The same sums at the octree's own points, evaluated in tree order and
+ * written in the caller's point order
  * (the source self-evaluation of TurboScreenedDWGLaunch, TurboDWG.cu:536). */
 int dwg_gwn_tree_self(dwg_ctx* ctx, const dwg_octree* tree, float beta, float sigma, uint32_t flags,
                       float* d_out);

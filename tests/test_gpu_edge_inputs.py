@@ -368,3 +368,25 @@ def test_sums_recorded_into_a_graph(kind, nq):
         s.synchronize()
         del tree
         c.close()
+
+
+# 4096 tiles of 2048 numbers, of which every block adds up those before its own,
+# and one more, with a scan of their sums; tiles that are whole and not
+@pytest.mark.parametrize("n", [4096 * 2048 - 3, 4096 * 2048, 4096 * 2048 + 1])
+def test_learned_start_of_a_large_cloud(ctx, n):
+    """The subsample that a large cloud's patches are taken from (flags, scan,
+    gather) against the same from numpy."""
+    rng = np.random.default_rng(n)
+    P = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+    stride = np.uint32(-(-n // 50_000))
+    h = np.arange(n, dtype=np.uint32) * np.uint32(0x9E3779B1)
+    h ^= h >> np.uint32(16)
+    h *= np.uint32(0x85EBCA6B)
+    h ^= h >> np.uint32(13)
+    sub = torch.from_numpy(P[h % stride == 0]).cuda()
+    net = gpu.Mlp(ctx, 0)
+    q = torch.from_numpy(P).cuda()
+    got = net.init_normals(q, np.zeros(3))
+    sel = torch.from_numpy(rng.integers(0, n, 20_000)).cuda()
+    want = net.forward(net.patches_from(gpu.KnnIndex(ctx, sub, 17), q[sel]))
+    assert torch.equal(got[sel].abs(), want.abs())  # (turned away from the centre)
