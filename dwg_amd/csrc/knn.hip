@@ -1303,9 +1303,8 @@ __global__ __launch_bounds__(kDescWaves * 64) void knn_descent_kernel(
         const float qx = q[3 * i], qy = q[3 * i + 1], qz = q[3 * i + 2];
         const float cap = init_kth ? init_kth[t] : INFINITY;
         uint64_t list = kNoKey, kth = kNoKey;
-        float bound = cap;
-        // (a query that is no number walks nowhere)
-        int sp = uniform(qx == qx && qy == qy && qz == qz ? 1 : 0), steps = 0;
+        float bound = qx == qx && qy == qy && qz == qz ? cap : -1.f;  // below every distance for no number
+        int sp = 1, steps = 0;
         ent[0] = root;
         ed2[0] = 0.f;
         __builtin_amdgcn_wave_barrier();
@@ -1394,7 +1393,7 @@ __global__ __launch_bounds__(kDescWaves * 64) void knn_descent_kernel(
                     }
                     __builtin_amdgcn_wave_barrier();
                 }
-                if (kth != kNoKey) bound = fminf(cap, __uint_as_float(uint32_t(kth >> 32)));
+                bound = fminf(cap, __uint_as_float(uint32_t(kth >> 32)));  // (∞ while there are fewer)
             }
             __builtin_amdgcn_wave_barrier();
         }
