@@ -197,12 +197,12 @@ __device__ __forceinline__ int run_head(uint64_t starts, int lane) {
 // a run of lanes with one bucket takes its places with one atomic add.  The
 // second pass then needs no atomics (3M triangle centroids: count and scatter
 // 248 → 140 µs).
-template <class C>
-__device__ __forceinline__ int take_place(int bucket, C* __restrict__ counts) {
+__device__ __forceinline__ int take_place(int bucket, unsigned long long* __restrict__ counts) {
     const int lane = threadIdx.x & 63;
     const uint64_t starts = run_starts(bucket);
     int base = 0;
-    if (bucket >= 0 && ((starts >> lane) & 1ull)) base = int(atomicAdd(&counts[bucket], C(run_length(starts, lane))));
+    if (bucket >= 0 && ((starts >> lane) & 1ull))
+        base = int(atomicAdd(&counts[bucket], (unsigned long long)run_length(starts, lane)));
     const int head = run_head(starts, lane);
     return __shfl(base, head, 64) + (lane - head);
 }

@@ -1342,6 +1342,11 @@ constexpr int kOrderSamples = 256;  // runs, one a block of the first launch
 constexpr int kOrderThreads = 256;
 static_assert(kOrderSamples == kOrderThreads, "a block adds up the samples, one a thread");
 
+// Sources below which a walk is too short to put queries in order for: 300,000 and
+// 1M unordered ones as they come 45 and 101 µs over 100 sources, 73 and 168 over 200,
+// 111 and 260 over 400; in order 66 and 132, 72 and 142, 78 and 154
+constexpr int64_t kOrderSources = 200;
+
 // 12 B of scratch a query, and up to so many queries at a time: more are taken in
 // equal parts, so that the scratch a context keeps for this stays below 204 MB
 // and a query's number in 32 bits
@@ -1350,7 +1355,7 @@ constexpr int64_t kOrderMost = int64_t(1) << 24;
 struct OrderCells {
     uint32_t count[kOrderBuckets];  // queries of a bucket
     uint32_t start[kOrderBuckets];  // queries before a bucket
-    uint32_t sample[kOrderSamples]; // extent of a run relative to the cube, in 2^-16
+    uint32_t sample[kOrderSamples]; // extent of a run relative to the cube, times its part near it, in 2^-16
     uint32_t extent;                // their sum
 };
 constexpr int kOrderZero = kOrderBuckets / kOrderSamples;  // counts that a block of the first launch clears
@@ -1367,14 +1372,19 @@ __global__ __launch_bounds__(kOrderThreads) void order_sample_kernel(const float
     for (int k = threadIdx.x; k < kOrderZero; k += kOrderThreads) C->count[blockIdx.x * kOrderZero + k] = 0;
     if (threadIdx.x >= 64) return;
     const int64_t i = int64_t(blockIdx.x) * (nq / 64) / kOrderSamples * 64 + threadIdx.x;  // nq ≥ 64
+    const double4 c = cell[0];
+    const float w = float(c.w), x[3] = {q[3 * i], q[3 * i + 1], q[3 * i + 2]};
+    // (half the cube's width off it a point's walk is short in any company: such points
+    // have no extent, and a run counts by its other points)
+    const bool near = fmaxf(fmaxf(fabsf(x[0] - float(c.x)), fabsf(x[1] - float(c.y))), fabsf(x[2] - float(c.z))) <= w;
+    const float part = float(__builtin_popcountll(__builtin_amdgcn_ballot_w64(near))) * (1.f / 64.f);
     float e = 0.f;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        const float v = q[3 * i + d];
+        const float v = near ? x[d] : NAN;  // left out of the least
         e = fmaxf(e, -wave_min(-v) - wave_min(v));
     }
-    const float w = float(cell[0].w);
-    if (threadIdx.x == 0) C->sample[blockIdx.x] = uint32_t(65536.f * fminf(fmaxf(e / w, 0.f), 1.f));
+    if (threadIdx.x == 0) C->sample[blockIdx.x] = uint32_t(65536.f * fminf(fmaxf(e / w * part, 0.f), 1.f));
 }
 
 __device__ __forceinline__ int order_bucket(const float* __restrict__ q, int64_t i, const double4 c) {
@@ -1405,7 +1415,21 @@ __device__ __forceinline__ uint32_t block_sum(uint32_t v) {
     return v;
 }
 
-// (bucket, place in it) of every query: the scatter then needs no atomics
+// the lanes whose bucket is this lane's (−1: none)
+__device__ __forceinline__ uint64_t same_bucket(int b) {
+    uint64_t m = __builtin_amdgcn_ballot_w64(b >= 0);
+#pragma unroll
+    for (int k = 0; k < 3 * kOrderBits; ++k) {
+        const uint64_t ones = __builtin_amdgcn_ballot_w64((b >> k) & 1);
+        m &= (b >> k) & 1 ? ones : ~ones;
+    }
+    return m;
+}
+
+// (bucket, place in it) of every query: the scatter then needs no atomics.  The
+// lanes of a wave in one bucket take their places with one atomic add, as many
+// queries may lie in one (equal ones, or all beyond one corner of the cube: 300,000
+// took 0.78 ms one by one)
 __global__ __launch_bounds__(kOrderThreads) void order_count_kernel(const float* __restrict__ q, int64_t nq,
                                                                     const double4* __restrict__ cell, unsigned limit,
                                                                     OrderCells* __restrict__ C,
@@ -1414,11 +1438,16 @@ __global__ __launch_bounds__(kOrderThreads) void order_count_kernel(const float*
     if (blockIdx.x == 0 && threadIdx.x == 0) C->extent = extent;
     if (extent <= limit) return;
     const double4 root = cell[0];
+    const int lane = threadIdx.x & 63;
     for (int64_t i0 = int64_t(blockIdx.x) * kOrderThreads; i0 < nq; i0 += int64_t(gridDim.x) * kOrderThreads) {
         const int64_t i = i0 + threadIdx.x;
         const int b = i < nq ? order_bucket(q, i, root) : -1;
-        const int at = take_place(b, C->count);
-        if (i < nq) place[i] = make_int2(b, at);
+        const uint64_t same = same_bucket(b);
+        const int first = b >= 0 ? __builtin_ctzll(same) : lane;
+        uint32_t at = 0;
+        if (b >= 0 && lane == first) at = atomicAdd(&C->count[b], uint32_t(__builtin_popcountll(same)));
+        at = uint32_t(__shfl(int(at), first, 64)) + uint32_t(__builtin_popcountll(same & ((1ull << lane) - 1ull)));
+        if (i < nq) place[i] = make_int2(b, int(at));
     }
 }
 
@@ -1471,14 +1500,15 @@ static int64_t order_part(int64_t nq) {
     return ((nq + parts - 1) / parts + 63) / 64 * 64;
 }
 
-// A call that is recorded into a graph takes its points as they come: the scratch
-// of an order could not be allocated, or given back by a later call while the graph
-// still used it
-static bool recording(const dwg_ctx* ctx) {
+// Whether queries that share walks are looked at for an order.  A call that is
+// recorded into a graph takes them as they come: the scratch of an order could not
+// be allocated, or given back by a later call while the graph still used it
+static bool may_order(const dwg_ctx* ctx, const dwg_octree* T) {
+    if (T->n_points < kOrderSources) return false;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
     (void)hipGetLastError();
-    return true;
+    return false;
 }
 
 // the caller's order where there is no memory for another
@@ -1794,7 +1824,7 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
     const char* name = count ? "gwn_tree_terms" : (!Q.grid ? (scr ? "gwn_tree_screened" : "gwn_tree_plain")
                                                            : (scr ? "gwn_tree_grid_screened" : "gwn_tree_grid_plain"));
     // explicit points are put in order first, a part of them at a time
-    const bool in_order = Q.q && Q.nq >= share_from(T, false) && !recording(ctx);
+    const bool in_order = Q.q && Q.nq >= share_from(T, false) && may_order(ctx, T);
     const int64_t part = in_order ? order_part(Q.nq) : Q.nq;
     for (int64_t first = 0; first < Q.nq; first += part) {
         QueryArgs Qs = Q;
@@ -1889,7 +1919,7 @@ void gwn_tree_grad(dwg_ctx* ctx, const dwg_octree* Tc, const float* q, int64_t n
         return;
     }
     TreeArgs A{T->info, T->kid, T->cm_r, reinterpret_cast<const float*>(T->payload), T->sa, T->sb};
-    const bool in_order = !recording(ctx);
+    const bool in_order = may_order(ctx, T);
     const int64_t part = in_order ? order_part(nq) : nq;
     for (int64_t first = 0; first < nq; first += part) {
         const int64_t n = std::min(part, nq - first);

@@ -157,6 +157,28 @@ def test_points_share_walks_by_the_size_of_the_tree(ctx, n, grad):
                 assert (g[back[keep]] - f[keep]).abs().max() <= tol * f.abs().max()
 
 
+@pytest.mark.parametrize("n", [199, 200, 3000])
+@pytest.mark.parametrize("kind", ["equal", "far", "mixed"])
+def test_points_in_few_places_share_walks(ctx, n, kind):
+    # many points in one bucket of the order, or beyond the cube, among others
+    P, N = shapes.sphere(n, 7)
+    rng = np.random.default_rng(n)
+    tree = gpu.Octree(ctx, P.astype(np.float64), None, max_depth=10)
+    tree.update(N.astype(np.float32), np.full(n, 0.5 / n, np.float32))
+    nq = 200_001
+    Q = rng.uniform(-1.2, 1.2, (nq, 3)).astype(np.float32)
+    at = rng.uniform(size=nq)
+    if kind != "far":
+        Q[at < 0.4] = 0.3, -0.2, 1.01
+    if kind != "equal":
+        Q[at > 0.7] *= 40
+        Q[at > 0.98, rng.integers(0, 3)] = np.inf
+    sub = rng.permutation(nq)[:3000]
+    few, got = tree.eval(Q[sub], 2.3, sigma=SIGMA), tree.eval(Q, 2.3, sigma=SIGMA)[torch.from_numpy(sub).cuda()]
+    ok = torch.from_numpy(np.isfinite(Q[sub]).all(1)).cuda()
+    assert (got[ok] - few[ok]).abs().max() <= 1e-5 * few[ok].abs().max()  # the tree's bound against FP64
+
+
 @pytest.mark.parametrize("res,h", [((8, 4, 8), 0.05), ((33, 29, 31), 0.08), ((51, 53, 55), 0.02), ((401, 399, 1), 0.003),
                                    ((190, 181, 183), 0.005), ((195, 191, 185), 0.005)])
 @pytest.mark.parametrize("screened,bf16,radii", [(True, False, False), (True, True, True), (False, False, False),
