@@ -641,6 +641,10 @@ constexpr int kStack = tree_stack_entries(kMaxTreeLevel);  // the shared gradien
 // share a child's x and y products)
 constexpr int kPartsX = 2, kPartsY = 1, kPartsZ = 2;
 constexpr int kGridParts = kPartsX * kPartsY * kPartsZ;
+// the kernels' GRID of bricks of 2 × 2 × 1 parts, for grids of at most 4 points
+// along z, which would leave half of the others empty (over 3,000 sources 500×500×1
+// 94 → 69 µs, 2,000×2,000×1 1,033 → 559)
+constexpr int kFlatParts = kGridParts + 1;
 constexpr int kPointPts = 1;  // explicit queries per lane
 
 struct TreeArgs {
@@ -702,6 +706,7 @@ struct QueryArgs {
     float ox, oy, oz, h;
     int rx, ry, rz;
     int parts;       // 4×4×4 parts of a brick (grid walks): kGridParts or 1
+    bool flat;       // the kGridParts parts are kFlatParts' (grid walks)
     int bx, by, bz;  // bricks per axis
     int64_t n_bricks;
     int stack;  // walk stack entries (tree_stack_entries of the tree's depth)
@@ -714,8 +719,9 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
                                                                  int64_t* __restrict__ terms_out) {
     // grid walks: each lane evaluates kGridParts points (one per 4×4×4 part
     // of the brick), so that a pop, its loads and its pushes serve them all
-    constexpr int H = GRID ? GRID : kPointPts;
-    constexpr int PX = GRID == kGridParts ? kPartsX : 1, PY = GRID == kGridParts ? kPartsY : 1,
+    constexpr int H = GRID == kFlatParts ? kGridParts : GRID ? GRID : kPointPts;
+    constexpr int PX = GRID >= kGridParts ? kPartsX : 1,
+                  PY = GRID == kFlatParts ? kPartsZ : GRID == kGridParts ? kPartsY : 1,
                   PZ = GRID == kGridParts ? kPartsZ : 1;
     static_assert(kTreeWaves == 1, "one wave per block: the stack lives in the block's dynamic LDS");
     // the stack: Q.stack entries of (record, H lane masks), in dynamic LDS
@@ -770,11 +776,12 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
         }
     }
     uint64_t all[H];
-    bool any = false;
+    bool any = false, every = true;  // every: each part has points
 #pragma unroll
     for (int h = 0; h < H; ++h) {
         all[h] = __builtin_amdgcn_ballot_w64(valid[h]);
         any = any || all[h] != 0;
+        every = every && all[h] != 0;
     }
     if (!any) return;
     const float sl2e = sigma * kLog2e;
@@ -851,15 +858,16 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_kernel(TreeArgs T, Quer
     // the stack holds (traversal record of a node to open, lanes that open
     // it, per part): an internal node's first child, or a leaf's
     // (−count, begin).  In a grid walk the record's top bit says that every
-    // lane opens the node: its masks are then neither written nor read back
+    // lane opens the node: its masks are then neither written nor read back (not
+    // where a part lies beyond the grid, whose terms would be computed for nobody)
     constexpr int kAllLanes = BOX ? int(0x80000000u) : 0;
     int sp = 0;
     const int4 root = scalar_load(T.info, 0);
     if (root.x < 0) {
         leaf_sum(root.y, root.z, all);
     } else {
-        s_node_w[0] = make_int2(root.x, kAllLanes);
-        if (!BOX) {
+        s_node_w[0] = make_int2(root.x, every ? kAllLanes : 0);
+        if (!BOX || !every) {
 #pragma unroll
             for (int h = 0; h < H; ++h) s_mask_w[h] = all[h];
         }
@@ -1729,8 +1737,16 @@ static QueryArgs make_grid(const dwg_octree* T, const dwg_grid* g, bool whole_br
         Q.bz = (Q.rz + 4 * pz - 1) / (4 * pz);
         Q.n_bricks = int64_t(Q.bx) * Q.by * Q.bz;
     };
-    bricks(kGridParts, kPartsX, kPartsY, kPartsZ);
-    if (!whole_bricks && double(Q.n_bricks) < kWholeBricks * std::cbrt(double(T->n_points))) bricks(1, 1, 1, 1);
+    Q.flat = Q.rz <= 4;
+    if (Q.flat) bricks(kGridParts, kPartsX, kPartsZ, kPartsY);
+    else bricks(kGridParts, kPartsX, kPartsY, kPartsZ);
+    // (also at most 4 points along x, of which whole bricks leave half empty: 4×700×700
+    // over 3,000 sources 143 µs whole, 117 in parts, 3×1,500×1,500 over 100,000 BF16
+    // 453 and 417)
+    auto in_parts = [&]() {
+        return (Q.rx <= 4 && T->n_nodes > 1) || double(Q.n_bricks) < kWholeBricks * std::cbrt(double(T->n_points));
+    };
+    if (!whole_bricks && in_parts()) bricks(1, 1, 1, 1);
     Q.nq = int64_t(Q.rx) * Q.ry * Q.rz;
     return Q;
 }
@@ -1798,8 +1814,10 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
         launch_walk<false>(ctx, T, Q.q, Q.nq, sigma, flags, out, nullptr);
         return;
     }
-    const bool alone = Q.grid ? Q.nq < kGridAlone || (Q.nq < kGridAloneDense && 3 * T->n_points >= Q.nq)
-                              : Q.self_perm && Q.nq < kSelfAlone;
+    // (a tree that is one leaf has no walk to be alone on)
+    const bool alone = T->n_nodes > 1 &&
+                       (Q.grid ? Q.nq < kGridAlone || (Q.nq < kGridAloneDense && 3 * T->n_points >= Q.nq)
+                               : Q.self_perm && Q.nq < kSelfAlone);
     if (alone && !count && !near64) {
         const bool scr = flags & DWG_SCREENED, bf = flags & DWG_FAR_BF16;
         const TreeArgs A{T->info, T->kid, T->cm_r, reinterpret_cast<const float*>(T->payload), T->sa, T->sb};
@@ -1847,6 +1865,8 @@ static void launch_tree(dwg_ctx* ctx, const dwg_octree* Tc, const QueryArgs& Q, 
     do {                                             \
         if (!Q.grid)                                 \
             DWG_TREE_LAUNCH(S, C, B, 0, N);          \
+        else if (Q.flat)                             \
+            DWG_TREE_LAUNCH(S, C, B, kFlatParts, N); \
         else                                         \
             DWG_TREE_LAUNCH(S, C, B, kGridParts, N); \
     } while (0)

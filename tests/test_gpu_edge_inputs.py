@@ -180,7 +180,8 @@ def test_points_in_few_places_share_walks(ctx, n, kind):
 
 
 @pytest.mark.parametrize("res,h", [((8, 4, 8), 0.05), ((33, 29, 31), 0.08), ((51, 53, 55), 0.02), ((401, 399, 1), 0.003),
-                                   ((190, 181, 183), 0.005), ((195, 191, 185), 0.005)])
+                                   ((190, 181, 183), 0.005), ((195, 191, 185), 0.005), ((801, 803, 3), 0.003),
+                                   ((3, 500, 600), 0.004)])
 @pytest.mark.parametrize("screened,bf16,radii", [(True, False, False), (True, True, True), (False, False, False),
                                                  (False, True, False)])
 def test_compensated_grid_walk_equals_the_point_walk(ctx, res, h, screened, bf16, radii):
@@ -203,6 +204,7 @@ def test_compensated_grid_walk_equals_the_point_walk(ctx, res, h, screened, bf16
     many = Q if len(Q) > 200_000 else Q.repeat(200_000 // len(Q) + 1, 1)
     want = tree.eval(many, 2.3, **kw).cpu().numpy()[:len(Q)]
     np.testing.assert_array_equal(got, want)
+    assert tree.grid_terms(grid) == int(tree.terms(Q).sum())
 
 
 @pytest.mark.parametrize("leaf_size", [1, 8])
