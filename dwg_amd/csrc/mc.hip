@@ -184,25 +184,34 @@ static_assert(kRunX % kBx == 0 && kFacesZ <= 32 && kBy % kRunWaves == 0, "bits o
 // against 40.
 constexpr int kRowsAll = kBy, kRowsFew = kBy / kRunWaves;
 constexpr int64_t kRunFew = 8192;
+// The any-order pass writes a wave's triangles too, and of a field that crosses its
+// level in most cubes these are all the work: grids of fewer runs than these give a
+// wave 8 or 4 cubes along z instead of 16, reading the faces between two waves
+// twice.  A sphere and a noise field in µs by 16, 8 and 4: 64³ (32 runs) 44, 38, 34
+// and 180, 106, 72; 97³ (144) 49, 41, 44 and 201, 152, 128; 128³ (256) 47, 46, 56 and
+// 229, 182, 170; 192³ (864) 74, 69, 87 and 465, 429, 429; 256³ (2048) 82, 94, 138 and
+// 927, 906, 898
+constexpr int64_t kRunTiny = 256, kRunSmall = 2048;
 
-// the run of a wave, its rows, and the bits of the cubes that exist in a
-// lane's columns (0 past the grid along x)
+// a wave's part of a run, NZ cubes along z of ROWS rows, and the bits of the cubes
+// that exist in a lane's columns (0 past the grid along x)
 struct Run {
     int x0, y0, z0, ny;
     uint32_t cubes;
 };
 
-template <int ROWS>
+template <int ROWS, int NZ>
 __device__ __forceinline__ bool run_of_wave(const McArgs& A, const McBricks& B, Run& R) {
-    constexpr int W = kBy / ROWS;  // waves of a run
-    const int wave = threadIdx.x >> 6, nrx = (B.nbx * kBx + kRunX - 1) / kRunX;
-    const int64_t id = brick_of_block() * (kRunWaves / W) + wave / W;
+    constexpr int W = kBy / ROWS * (kBz / NZ);  // waves of a run
+    const int nrx = (B.nbx * kBx + kRunX - 1) / kRunX;
+    const int64_t wave = brick_of_block() * kRunWaves + (threadIdx.x >> 6), id = wave / W;
     if (id >= int64_t(nrx) * B.nby * B.nbz) return false;
+    const int w = int(wave % W);
     R.x0 = int(id % nrx) * kRunX;
-    R.y0 = int(id / nrx % B.nby) * kBy + (wave % W) * ROWS;
-    R.z0 = int(id / (int64_t(nrx) * B.nby)) * kBz;
-    R.ny = min(ROWS, A.ry - 1 - R.y0);  // none or less: a wave past the grid
-    R.cubes = R.x0 + int(threadIdx.x & 63) < A.rx - 1 ? (1u << min(kBz, A.rz - 1 - R.z0)) - 1u : 0u;
+    R.y0 = int(id / nrx % B.nby) * kBy + w % (kBy / ROWS) * ROWS;
+    R.z0 = int(id / (int64_t(nrx) * B.nby)) * kBz + w / (kBy / ROWS) * NZ;
+    R.ny = R.z0 < A.rz - 1 ? min(ROWS, A.ry - 1 - R.y0) : 0;  // none or less: a wave past the grid
+    R.cubes = R.x0 + int(threadIdx.x & 63) < A.rx - 1 ? (1u << min(NZ, max(A.rz - 1 - R.z0, 0))) - 1u : 0u;
     return true;
 }
 
@@ -210,7 +219,7 @@ __device__ __forceinline__ bool run_of_wave(const McArgs& A, const McBricks& B, 
 template <int ROWS>
 using RunBits = uint32_t[ROWS + 1][kRunX + 1];
 
-template <int ROWS>
+template <int ROWS, int NZ>
 __device__ __forceinline__ void run_bits(const McArgs& A, const Run& R, RunBits<ROWS>& bits) {
     const int lane = threadIdx.x & 63;
     // samples past the grid repeat its last one (no cube uses them)
@@ -221,7 +230,7 @@ __device__ __forceinline__ void run_bits(const McArgs& A, const Run& R, RunBits<
     for (int r = 0; r <= ROWS; ++r) col[r] = A.f + x + int64_t(A.rx) * min(R.y0 + r, A.ry - 1);
     uint32_t w[ROWS + 1] = {}, we = 0;
 #pragma unroll 4
-    for (int s = 0; s < kFacesZ; ++s) {
+    for (int s = 0; s <= NZ; ++s) {
         const int64_t z = plane * min(R.z0 + s, A.rz - 1);
         float v[ROWS + 1];
 #pragma unroll
@@ -271,10 +280,10 @@ __global__ __launch_bounds__(kRunWaves * 64) void mc_count_kernel(McArgs A, McBr
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     Run R;
-    const bool have = run_of_wave<ROWS>(A, B, R);
+    const bool have = run_of_wave<ROWS, kBz>(A, B, R);
     int cnt = 0;
     if (have && R.ny > 0) {
-        run_bits<ROWS>(A, R, s_bits[wave]);
+        run_bits<ROWS, kBz>(A, R, s_bits[wave]);
 #pragma unroll 1
         for (int r = 0; r < R.ny; ++r) {
             const RunColumn C = run_column<ROWS>(s_bits[wave], r, R.cubes);
@@ -358,7 +367,7 @@ __global__ __launch_bounds__(kMcThreads) void mc_emit_kernel(McArgs A, McBricks 
 // thread a column of 4 cubes, writing that column's triangles).
 constexpr int kFusedList = 256;  // cubes listed before their triangles are written
 
-template <int ROWS>
+template <int ROWS, int NZ>
 __global__ __launch_bounds__(kRunWaves * 64) void mc_fused_kernel(McArgs A, McBricks B,
                                                                    unsigned long long* __restrict__ ntri,
                                                                    int64_t capacity, float* __restrict__ cent,
@@ -372,9 +381,9 @@ __global__ __launch_bounds__(kRunWaves * 64) void mc_fused_kernel(McArgs A, McBr
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     Run R;
-    if (!run_of_wave<ROWS>(A, B, R) || R.ny <= 0) return;
+    if (!run_of_wave<ROWS, NZ>(A, B, R) || R.ny <= 0) return;
     uint32_t *cubes = s_cube[wave], *tri = s_tri[wave];
-    run_bits<ROWS>(A, R, s_bits[wave]);
+    run_bits<ROWS, NZ>(A, R, s_bits[wave]);
     int listed = 0, r = 0;
     RunColumn C = run_column<ROWS>(s_bits[wave], 0, R.cubes);
     uint32_t m = C.crossed;
@@ -452,12 +461,15 @@ int64_t marching_cubes_any_order(dwg_ctx* ctx, const float* field, const dwg_gri
     {
         ProfileScope ps(ctx, "mc_fused");
         const int64_t runs = mc_runs(B);
-        if (runs < kRunFew)
-            hipLaunchKernelGGL(mc_fused_kernel<kRowsFew>, dim3(unsigned(runs)), dim3(kRunWaves * 64), 0, ctx->stream,
-                               A, B, n, capacity, cent, nrm);
-        else
-            hipLaunchKernelGGL(mc_fused_kernel<kRowsAll>, dim3(grid_for(runs, kRunWaves)), dim3(kRunWaves * 64), 0,
-                               ctx->stream, A, B, n, capacity, cent, nrm);
+        // LAUNCH(rows, cubes along z) of a wave
+#define DWG_MC_FUSED(R, Z)                                                                                          \
+    hipLaunchKernelGGL((mc_fused_kernel<R, Z>), dim3(grid_for(runs * (kBy / (R)) * (kBz / (Z)), kRunWaves)),        \
+                       dim3(kRunWaves * 64), 0, ctx->stream, A, B, n, capacity, cent, nrm)
+        if (runs < kRunTiny) DWG_MC_FUSED(kRowsFew, kBz / 4);
+        else if (runs < kRunSmall) DWG_MC_FUSED(kRowsFew, kBz / 2);
+        else if (runs < kRunFew) DWG_MC_FUSED(kRowsFew, kBz);
+        else DWG_MC_FUSED(kRowsAll, kBz);
+#undef DWG_MC_FUSED
         check_launch();
     }
     const int64_t total = int64_t(read_scalar<unsigned long long>(ctx, n));

@@ -394,6 +394,19 @@ def test_sums_recorded_into_a_graph(kind, nq):
         c.close()
 
 
+# 240 runs of 64 cubes, 256, 2032 and 2048: by 4, 8 and 16 cubes along z a wave
+@pytest.mark.parametrize("res", [(65, 121, 257), (65, 129, 250), (65, 1017, 243), (65, 1025, 257)])
+def test_any_order_marching_cubes_by_runs(ctx, res):
+    # the rows of the ordered pass, bit for bit
+    x, y, z = (torch.arange(r, device="cuda", dtype=torch.float32) for r in res)
+    f = (torch.sin(0.3 * x)[None, None] + torch.sin(0.2 * y)[None, :, None] + torch.sin(0.25 * z)[:, None, None]).ravel()
+    grid = gpu.make_grid([-1.1, -0.9, -1.0], 0.05, res)
+    _, cent, nrm = gpu.marching_cubes(ctx, f, grid, 0.5)
+    c1, n1 = gpu.marching_cubes_any_order(ctx, f, grid, 0.5, capacity=len(cent))
+    rows = [torch.cat([c, m], 1).cpu().numpy().view(np.uint32) for c, m in ((cent, nrm), (c1, n1))]
+    assert len(rows[0]) > 100_000 and np.array_equal(*(r[np.lexsort(r.T[::-1])] for r in rows))
+
+
 # 4096 tiles of 2048 numbers, of which every block adds up those before its own,
 # and one more, with a scan of their sums; tiles that are whole and not
 @pytest.mark.parametrize("n", [4096 * 2048 - 3, 4096 * 2048, 4096 * 2048 + 1])
