@@ -166,10 +166,13 @@ __device__ __forceinline__ void gwn_term_grad(float dx, float dy, float dz, floa
 }
 
 // a component c·d − g·b of the gradient: 0 · d is 0 by this multiplication, also
-// for a d that is no number
+// for a d that is no number (plain terms have no zeros to keep, and the compiler
+// unrolls a loop with the instruction written out less)
+template <bool SCREENED>
 __device__ __forceinline__ float grad_component(float c, float d, float g, float b) {
     float cd;
-    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(cd) : "v"(c), "v"(d));
+    if constexpr (SCREENED) asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(cd) : "v"(c), "v"(d));
+    else cd = c * d;
     return __builtin_fmaf(-g, b, cd);
 }
 
@@ -239,9 +242,9 @@ __device__ __forceinline__ void direct_value(const float4* __restrict__ sa, cons
 
 // the sources [j0, j1) summed at q, value and gradient: s − c for each.  UNROLL
 // terms of a tile at a time: 2, and 1 for plain sums that are not split (857 sources at
-// 1M queries, plain: 474 µs by 1, 512 by 2, 525 by 4; 3,000 at 300,000 664, 667 and
-// 639, screened 1,072, 1,029 and 1,105; 200,000 at 2,000, split, 352, 317 and 332,
-// screened 499, 489 and 519)
+// 1M queries, plain: 489 µs by 1, 518 by 2, 528 by 4; 3,000 at 300,000 671, 667 and
+// 641, screened 1,073, 1,030 and 1,111; 200,000 at 2,000, split, 342, 318 and 333,
+// screened 499, 490 and 520)
 template <bool SCREENED, bool KAHAN, int UNROLL>
 __device__ __forceinline__ void direct_grad(const float4* __restrict__ sa, const float4* __restrict__ sb, int64_t j0,
                                             int64_t j1, float qx, float qy, float qz, float sigma, float (&s)[4],
@@ -255,9 +258,9 @@ __device__ __forceinline__ void direct_grad(const float4* __restrict__ sa, const
         float dot, g, c;
         gwn_term_grad<SCREENED>(dx, dy, dz, b.w, b, sigma, sl2e, dot, g, c);
         p[0] = __builtin_fmaf(g, dot, p[0]);
-        p[1] += grad_component(c, dx, g, b.x);
-        p[2] += grad_component(c, dy, g, b.y);
-        p[3] += grad_component(c, dz, g, b.z);
+        p[1] += grad_component<SCREENED>(c, dx, g, b.x);
+        p[2] += grad_component<SCREENED>(c, dy, g, b.y);
+        p[3] += grad_component<SCREENED>(c, dz, g, b.z);
     };
     auto fold = [&]() {
 #pragma unroll
@@ -1101,9 +1104,9 @@ __global__ __launch_bounds__(kWalkWaves * 64) void gwn_walk_kernel(TreeArgs T, c
             float dot, g, c;
             gwn_term_grad<SCREENED>(dx, dy, dz, s2, b, sigma, sl2e, dot, g, c);
             sum[0] += double(g * dot);
-            sum[1] += double(grad_component(c, dx, g, b.x));
-            sum[2] += double(grad_component(c, dy, g, b.y));
-            sum[3] += double(grad_component(c, dz, g, b.z));
+            sum[1] += double(grad_component<SCREENED>(c, dx, g, b.x));
+            sum[2] += double(grad_component<SCREENED>(c, dy, g, b.y));
+            sum[3] += double(grad_component<SCREENED>(c, dz, g, b.z));
         } else {
             float inv;
             bool ok;
@@ -1334,6 +1337,7 @@ constexpr int64_t kWalkFew = 40000;
 // 340; 500,000 395, 467 and 322, 400.  1M sources 500,000 700, 962 and 920, 975;
 // 800,000 1,089, 1,479 and 1,156, 1,238
 static int64_t share_from(const dwg_octree* T, bool grad) {
+    if (T->n_nodes == 1) return 0;  // a leaf has no walk to be alone on
     const double n = double(T->n_points);
     return int64_t(grad ? 62000.0 * std::pow(n, 1.0 / 6.0) : 82000.0 * std::pow(n, 1.0 / 12.0));
 }
@@ -1341,7 +1345,8 @@ static int64_t share_from(const dwg_octree* T, bool grad) {
 // The order: a counting sort by the Morton code of a 64³ grid over the tree's
 // cube.  Queries that come in order already are left as they are, which a
 // sample of runs of 64 decides: they come unsorted when such runs extend, on
-// average, over twice the side that 64 of nq uniform points fill.  (32³ and 128³
+// average, over four times the side that 64 of nq uniform points fill (in Morton
+// order they extend over 1.9 to 2.4 times, the rows of a grid 14 times).  (32³ and 128³
 // cells: 300,000 points over 400,000 sources 417 and 427 µs against 394 with 64³,
 // 1M points 690 and 611 against 602.)  Queries in order pay for the launches that
 // find it out, which are four for that reason: 8 to 10 µs (200,000 over 3,000 sources 66
@@ -1515,7 +1520,7 @@ static int64_t order_part(int64_t nq) {
 // recorded into a graph takes them as they come: the scratch of an order could not
 // be allocated, or given back by a later call while the graph still used it
 static bool may_order(const dwg_ctx* ctx, const dwg_octree* T) {
-    if (T->n_points < kOrderSources) return false;
+    if (T->n_points < kOrderSources || T->n_nodes == 1) return false;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
     (void)hipGetLastError();
@@ -1536,7 +1541,7 @@ static QueryOrder query_order(dwg_ctx* ctx, const dwg_octree* T, const float* q,
         return QueryOrder{};
     }
     ProfileScope ps(ctx, "gwn_query_order");
-    const QueryOrder O{order, &C->extent, unsigned(65536.f * 2.f * std::cbrt(64.f / float(nq)) * float(kOrderSamples))};
+    const QueryOrder O{order, &C->extent, unsigned(65536.f * 4.f * std::cbrt(64.f / float(nq)) * float(kOrderSamples))};
     hipLaunchKernelGGL(order_sample_kernel, dim3(kOrderSamples), dim3(kOrderThreads), 0, ctx->stream, q, nq, T->cell, C);
     check_launch();
     const unsigned blocks = std::min(grid_for(nq, kOrderThreads), 1024u);
@@ -1614,9 +1619,9 @@ __global__ __launch_bounds__(kTreeThreads) void gwn_tree_grad_kernel(TreeArgs T,
         g = on ? g : 0.f;
         c = on ? c : 0.f;
         part[0] = __builtin_fmaf(g, dot, part[0]);
-        part[1] += grad_component(c, dx, g, b.x);
-        part[2] += grad_component(c, dy, g, b.y);
-        part[3] += grad_component(c, dz, g, b.z);
+        part[1] += grad_component<SCREENED>(c, dx, g, b.x);
+        part[2] += grad_component<SCREENED>(c, dy, g, b.y);
+        part[3] += grad_component<SCREENED>(c, dz, g, b.z);
     };
     // (for the lanes that took part: adding a zero would move bits between the
     // sum and its compensation)
