@@ -165,14 +165,16 @@ __device__ __forceinline__ void gwn_term_grad(float dx, float dy, float dz, floa
     }
 }
 
-// a component c·d − g·b of the gradient: 0 · d is 0 by this multiplication, also
-// for a d that is no number (plain terms have no zeros to keep, and the compiler
-// unrolls a loop with the instruction written out less)
+// a component c·d − g·b of the gradient, of whose products one is rounded before
+// they meet.  Plain: the smaller, g·b (c·d next to a source is up to three times
+// as large).  Screened: c·d, as 0 · d is 0 by this multiplication, also for a d
+// that is no number (plain terms have no zeros to keep, and the compiler unrolls
+// a loop with the instruction written out less)
 template <bool SCREENED>
 __device__ __forceinline__ float grad_component(float c, float d, float g, float b) {
+    if constexpr (!SCREENED) return __builtin_fmaf(c, d, -(g * b));
     float cd;
-    if constexpr (SCREENED) asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(cd) : "v"(c), "v"(d));
-    else cd = c * d;
+    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(cd) : "v"(c), "v"(d));
     return __builtin_fmaf(-g, b, cd);
 }
 

@@ -88,6 +88,38 @@ def test_gradient_component_is_rounded_at_its_own_size(ctx, where, n, nq, screen
     assert np.abs(got - want).max() <= tiles * (16 * 1.25 + 63 * 0.5 + 1) * 2.0 ** -23
 
 
+def test_plain_gradient_rounds_the_smaller_product(ctx):
+    # Of a component c·d − g·b the product g·b is rounded before they meet.  The
+    # factors are read from the results: with a moment along x and x and z offsets
+    # that are powers of two, w is g and the z component c, each times a power; the
+    # moments (1, b, −b·dy/dz) leave d·b, and so both, as they are.
+    rng = np.random.default_rng(11)
+    f = np.float32
+    A, inv4pi = f(4 * np.pi), f(1 / (4 * np.pi))
+    moment = lambda v: f(f(A * v) * inv4pi)  # as the sources are packed
+    assert moment(f(1)) == 1
+    dx = f(2.0) ** np.arange(-2, 2, dtype=f)
+    checked = 0
+    for _ in range(2000):
+        dy, by = f(rng.integers(257, 1024) / 1024), f(rng.integers(257, 1024) / 1024)
+        bz = -dy * by
+        if moment(by) != by or moment(bz) != bz:
+            continue
+        q = np.stack([-dx, np.full(4, -dy), np.full(4, f(-1))], 1)
+        run = lambda n: [x.cpu().numpy() for x in ctx.gwn_direct(np.zeros((1, 3), f), np.array([n], f), np.array([A]),
+                                                                 q, screened=False, kahan=False, grad=True)]
+        w, grad = run((1, 0, 0))
+        g, c = w / dx, grad[:, 2]
+        w2, got = run((1, by, bz))
+        np.testing.assert_array_equal(w2, w)
+        want = c.astype(np.float64) * np.float64(dy) - (g * by).astype(np.float64)
+        np.testing.assert_array_equal(got[:, 1], want.astype(f))
+        checked += 4
+        if checked >= 400:
+            break
+    assert checked >= 200
+
+
 # one chain and split over the sources
 @pytest.mark.parametrize("n,nq", [(100, 7), (700, 300)])
 @pytest.mark.parametrize("kahan,near64", [(False, False), (True, False), (True, True)])
