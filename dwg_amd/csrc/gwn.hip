@@ -37,9 +37,9 @@ __device__ __forceinline__ float max_nonneg(float a, float b) {
 }
 
 // The tree walk's point and dipole terms in two factors, t = x · inv, from
-// d, r² = |d|² and s²: ρ² = max(r², s²), ρ = √ρ², ρ³ = ρ²·ρ; the screened
-// guard r > 1e-10 as r² > 1e-20
-template <bool SCREENED>
+// d, r² = |d|² and s²: ρ² = max(r², s²), ρ = √ρ², ρ³ = ρ²·ρ (ROOT:
+// ρ·ρ·ρ); the screened guard r > 1e-10 as r² > 1e-20
+template <bool SCREENED, bool ROOT = false>
 __device__ __forceinline__ float tree_term_split(float dx, float dy, float dz, float r2, float s2, const float4 b,
                                                  float sigma, float sigma_l2e, float& inv, bool& ok) {
     const float dot = __builtin_fmaf(dz, b.z, __builtin_fmaf(dy, b.y, dx * b.x));
@@ -51,7 +51,8 @@ __device__ __forceinline__ float tree_term_split(float dx, float dy, float dz, f
     } else {
         const float rho2 = max_nonneg(r2, s2);
         const float rho = fast_sqrt(rho2);
-        inv = fast_rcp(__builtin_fmaf(fast_exp2(sigma_l2e * rho), rho2 * rho, kEpsScreened * kInv4Pi));
+        const float rho3 = (ROOT ? rho * rho : rho2) * rho;
+        inv = fast_rcp(__builtin_fmaf(fast_exp2(sigma_l2e * rho), rho3, kEpsScreened * kInv4Pi));
         ok = r2 > 1e-20f;
         return __builtin_fmaf(sigma, rho, 1.0f) * dot;
     }
@@ -95,14 +96,18 @@ __device__ __forceinline__ float screened_r2(float r2, float s2) {
 // the other is always one.  With the product left to the sum's multiply-add it
 // takes 21 instructions screened (24 with ρ = max(r, s), ρ·ρ·ρ and a selected sum:
 // 10,000 sources at 2M queries 13.6 → 11.9 ms, the chip's whole issue rate).
-template <bool SCREENED>
+// ROOT: ρ³ as ρ·ρ·ρ, one more, for compensated sums, whose error is the factors':
+// the root's bias, which ρ²·ρ has once and e^{σρ}, 1 + σρ and ρ·ρ·ρ together, in
+// part cancels the reciprocal's (RMS error of 200,000 sources 6.5e-8 → 5.5e-8,
+// 292 → 322 µs at 2,000 queries; 10,000 at 2M 11.55 → 12.15 ms).
+template <bool SCREENED, bool ROOT>
 __device__ __forceinline__ float gwn_term_split(float qx, float qy, float qz, const float4 a, const float4 b,
                                                 float sigma, float sigma_l2e, float& inv) {
     const float dx = a.x - qx, dy = a.y - qy, dz = a.z - qz;
     const float r2 = dist2(dx, dy, dz);
     bool ok;
     if constexpr (!SCREENED) return tree_term_split<false>(dx, dy, dz, r2, 0.f, b, sigma, sigma_l2e, inv, ok);
-    const float x = tree_term_split<true>(dx, dy, dz, screened_r2(r2, b.w), 0.f, b, sigma, sigma_l2e, inv, ok);
+    const float x = tree_term_split<true, ROOT>(dx, dy, dz, screened_r2(r2, b.w), 0.f, b, sigma, sigma_l2e, inv, ok);
     return r2 > 1e-20f ? x : 0.f;
 }
 
@@ -132,12 +137,13 @@ __device__ __forceinline__ bool near_field(float r2, float s) { return r2 < s * 
 //             (∂ρ/∂q = −d/r), −g b for r < s;
 //             g' = (σε' − e^{σρ}ρ²(σ²ρ² + 3σρ + 3)) / D²  (no cancellation)
 // as the factors dot = d·b, g and c of w = g·dot, ∇w = c·d − g·b, with s2 the
-// squared screening radius (200,000 sources at 2,000 queries 540 → 487 µs with
-// selects on two factors instead of four results.  ρ = ρ²·ρ^-1 would save another
-// 5 %, for an error of w 8 to 13 % above the root's).  A component c·d − g·b is
-// formed before it joins its sum: its two products joined one by one, 460 µs,
-// round twice at the sum's size (half of 2,000 queries next to one of 20,000
-// sources: RMS error of ∇w 11 % and maximum 37 % more).
+// squared screening radius (200,000 sources at 2,000 queries 540 → 501 µs with
+// selects on two factors instead of four results.  Of that ρ·ρ takes 8, as ρ² in its
+// place adds 8 % to the RMS error of ∇w, and ρ^-1 as the root's reciprocal 5 %;
+// ρ = ρ²·ρ^-1 would save 5 % of the time for an error of w 8 to 13 % above the
+// root's).  A component c·d − g·b is formed before it joins its sum: its two products
+// joined one by one, 6 % faster, round twice at the sum's size (half of 2,000
+// queries next to one of 20,000 sources: RMS error of ∇w 11 % and maximum 37 % more).
 // A screened term at the guard, or whose distance is no number, has only zeros
 // (d may still be no number).
 template <bool SCREENED>
@@ -154,7 +160,7 @@ __device__ __forceinline__ void gwn_term_grad(float dx, float dy, float dz, floa
         dot = ok ? dot : 0.0f;
         const float rho2 = screened_r2(r2, s2);
         const float rho = fast_sqrt(rho2), irho = fast_rsq(rho2);
-        const float er2 = fast_exp2(sigma_l2e * rho) * rho2;
+        const float er2 = fast_exp2(sigma_l2e * rho) * (rho * rho);
         const float eps = kEpsScreened * kInv4Pi;
         const float inv = fast_rcp(__builtin_fmaf(er2, rho, eps));
         const float sr = sigma * rho;
@@ -220,7 +226,7 @@ __device__ __forceinline__ void direct_value(const float4* __restrict__ sa, cons
     near = 0.0;
     auto add = [&](float& part, const float4 a, const float4 b) {
         float inv;
-        float x = gwn_term_split<SCREENED>(qx, qy, qz, a, b, sigma, sl2e, inv);
+        float x = gwn_term_split<SCREENED, KAHAN>(qx, qy, qz, a, b, sigma, sl2e, inv);
         if constexpr (NEAR64) {
             const float dx = a.x - qx, dy = a.y - qy, dz = a.z - qz;
             const bool nr = near_field(dist2(dx, dy, dz), a.w);
@@ -246,7 +252,7 @@ __device__ __forceinline__ void direct_value(const float4* __restrict__ sa, cons
 // terms of a tile at a time: 2, and 1 for plain sums that are not split (857 sources at
 // 1M queries, plain: 489 µs by 1, 518 by 2, 528 by 4; 3,000 at 300,000 671, 667 and
 // 641, screened 1,073, 1,030 and 1,111; 200,000 at 2,000, split, 342, 318 and 333,
-// screened 499, 490 and 520)
+// screened, with a multiplication less, 499, 490 and 520)
 template <bool SCREENED, bool KAHAN, int UNROLL>
 __device__ __forceinline__ void direct_grad(const float4* __restrict__ sa, const float4* __restrict__ sb, int64_t j0,
                                             int64_t j1, float qx, float qy, float qz, float sigma, float (&s)[4],
@@ -471,7 +477,7 @@ void gwn_direct(dwg_ctx* ctx, const float* pts, const float* nrm, const float* a
     // one array: the partial sums (also where this call does not split: one of the
     // same sources that does may be recorded into a graph next, and can allocate
     // nothing), then the packed sources, each from a line of its own on (the scalar
-    // loads' lines: 200,000 sources at 2,000 queries 489 µs, 527 where they straddle)
+    // loads' lines: 200,000 sources at 2,000 queries 8 % slower where they straddle)
     const size_t parts = sizeof(double) * kDirectPartials, packed = (sizeof(float4) * size_t(n + 1) + 255) & ~size_t(255);
     char* mem = static_cast<char*>(ctx->buf("direct", parts + 2 * packed));
     double* part = reinterpret_cast<double*>(mem);

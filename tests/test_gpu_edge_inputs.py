@@ -121,6 +121,27 @@ def test_plain_gradient_rounds_the_smaller_product(ctx):
 
 
 # one chain and split over the sources
+@pytest.mark.parametrize("n", [1, 300])
+@pytest.mark.parametrize("grad,kahan", [(False, True), (True, True), (True, False)])
+def test_screened_factors_take_the_distance_by_its_root(ctx, n, grad, kahan):
+    # d·b = 1 at distances whose squares are the 4,096 numbers above 1: their roots
+    # are half as many numbers (the root's error of a unit adds one at either end),
+    # and so are the factors g = w
+    f = np.float32
+    m = 4096
+    dy = np.sqrt(np.arange(1, m + 1) * 2.0 ** -23).astype(f)
+    r2 = (1.0 + dy.astype(np.float64) ** 2).astype(f)
+    assert len(np.unique(r2)) == m and r2[-1] - 1 == f(m * 2.0 ** -23)
+    P, N, A = np.zeros((n, 3), f), np.zeros((n, 3), f), np.full(n, f(4 * np.pi))
+    P[:, 0] = N[0, 0] = 1
+    Q = np.zeros((m, 3), f)
+    Q[:, 1] = -dy
+    w = ctx.gwn_direct(P, N, A, Q, sigma=SIGMA, screened=True, kahan=kahan, grad=grad)
+    w = (w[0] if grad else w).cpu().numpy()
+    assert len(np.unique(w)) <= m // 2 + 3
+
+
+# one chain and split over the sources
 @pytest.mark.parametrize("n,nq", [(100, 7), (700, 300)])
 @pytest.mark.parametrize("kahan,near64", [(False, False), (True, False), (True, True)])
 def test_screened_direct_sums_leave_out_what_is_no_number(ctx, n, nq, kahan, near64):
